@@ -51,6 +51,28 @@ __global__ void set_counters_kernel(int32_t *pos, int32_t *step, int32_t p, int3
     *step = s;
   }
 }
+// the state yscv_hip_decoder_reset sets, carried to the device as kernel arguments: no copy, no wait
+struct ResetState {
+  int32_t tokens[16];
+  int32_t batch, pos;
+};
+__global__ void reset_state_kernel(int32_t *tokens, int32_t *pos, int32_t *step, ResetState r) {
+  const int i = threadIdx.x;
+  if (i < r.batch) tokens[i] = r.tokens[i];
+  if (i == 0) {
+    *pos = r.pos;
+    *step = 0;
+  }
+}
+// a piece of a prompt, likewise
+constexpr int kPromptPiece = 896;
+struct PromptPiece {
+  int32_t tokens[kPromptPiece];
+};
+__global__ void __launch_bounds__(kPromptPiece) store_prompt_kernel(int32_t *dst, int n, PromptPiece p) {
+  const int i = threadIdx.x;
+  if (i < n) dst[i] = p.tokens[i];
+}
 __global__ void fill_i32_kernel(int32_t *p, size_t n, int32_t v) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
 }
@@ -128,6 +150,14 @@ struct yscv_hip_decoder {
   size_t ws_bytes = 0;
   int32_t *tokens = nullptr, *history = nullptr, *pos = nullptr, *step = nullptr;
   int batch = 0;
+  // what *pos and *step hold once everything enqueued so far has run: every call knows how far it moves them, so the
+  // bounds checks of a run need no read-back
+  int32_t pos_host = 0, step_host = 0;
+  hipStream_t last_stream = nullptr;  // stream of the last call that enqueued work on the decoder's state
+  void *pf_buf = nullptr;             // activations and partial sums of the prompt pass, kept between prompts
+  size_t pf_bytes = 0;
+  int32_t *prompt = nullptr;          // device copy of the prompt being processed
+  int32_t prompt_cap = 0;
   int kv_dtype = YSCV_HIP_KV_F16;
   bool finalized = false;
   hipGraph_t graph = nullptr;
@@ -196,6 +226,8 @@ static void decoder_free(yscv_hip_decoder *d) {
   (void)hipFree(d->ao);
   (void)hipFree(d->act);
   (void)hipFree(d->ws);
+  (void)hipFree(d->pf_buf);
+  (void)hipFree(d->prompt);
   (void)hipFree(d->tokens);
   (void)hipFree(d->history);
   (void)hipFree(d->pos);
@@ -210,6 +242,13 @@ static void decoder_free(yscv_hip_decoder *d) {
   (void)hipFree(d->p_abort);
   (void)hipFree(d->p_trace);
   delete d;
+}
+
+// The decoder's state is used in the order of the calls: a call on another stream than the one before waits for it.
+static hipError_t enter_stream(yscv_hip_decoder *d, hipStream_t s) {
+  if (s == d->last_stream) return hipSuccess;
+  d->last_stream = s;
+  return hipDeviceSynchronize();
 }
 
 #define DEC_HIP(expr)                                                                                \
@@ -884,10 +923,15 @@ int32_t yscv_hip_decoder_reset(yscv_hip_decoder *d, int32_t batch, int32_t start
   YSCV_REQUIRE(batch >= 1 && batch <= c.max_batch, "batch %d out of range 1..%d", batch, c.max_batch);
   YSCV_REQUIRE(start_pos >= 0 && start_pos < c.max_ctx, "start position %d out of range", start_pos);
   d->batch = batch;
-  DEC_HIP(hipMemcpy(d->tokens, tokens_host, (size_t)batch * 4, hipMemcpyHostToDevice));
-  DEC_HIP(hipMemcpy(d->pos, &start_pos, 4, hipMemcpyHostToDevice));
-  const int32_t zero = 0;
-  DEC_HIP(hipMemcpy(d->step, &zero, 4, hipMemcpyHostToDevice));
+  DEC_HIP(enter_stream(d, nullptr));
+  ResetState r{};
+  memcpy(r.tokens, tokens_host, (size_t)batch * 4);
+  r.batch = batch;
+  r.pos = start_pos;
+  hipLaunchKernelGGL(reset_state_kernel, dim3(1), dim3(64), 0, nullptr, d->tokens, d->pos, d->step, r);
+  DEC_HIP(hipGetLastError());
+  d->pos_host = start_pos;
+  d->step_host = 0;
   return YSCV_HIP_OK;
 }
 
@@ -898,10 +942,7 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
   YSCV_REQUIRE(n_steps >= 0, "negative step count");
   hipStream_t s = as_stream(stream);
   // host-side bound check: the cache must hold every position this run appends
-  int32_t pos = 0, step = 0;
-  DEC_HIP(hipStreamSynchronize(s));
-  DEC_HIP(hipMemcpy(&pos, d->pos, 4, hipMemcpyDeviceToHost));
-  DEC_HIP(hipMemcpy(&step, d->step, 4, hipMemcpyDeviceToHost));
+  const int32_t pos = d->pos_host, step = d->step_host;
   YSCV_REQUIRE(pos + n_steps <= d->cfg.max_ctx, "KV cache overflow: position %d + %d steps > max_ctx %d", pos, n_steps,
                d->cfg.max_ctx);
   YSCV_REQUIRE(step + n_steps <= d->cfg.max_steps, "token history overflow: %d + %d > max_steps %d", step, n_steps,
@@ -917,6 +958,7 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
     if (d->has_bias) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "the single-launch decode path has no q / k / v bias");
     if (d->batch != 1) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "the single-launch decode path runs batch 1 only");
     if (n_steps == 0) return YSCV_HIP_OK;
+    DEC_HIP(enter_stream(d, s));
     // A tag is ((epoch + step) * (layers + 2) + 1 + layer) modulo 2^24.  Before the tag space wraps, the exchange
     // buffers are cleared and the epoch starts again, so an entry left from half a million steps ago can never be taken
     // for a fresh one.
@@ -930,13 +972,20 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
     }
     YSCV_TRY(launch_persist_decode(d->pm, n_steps, pos, step, d->cfg.max_steps, d->epoch, s));
     d->epoch += (uint32_t)n_steps;
+    d->pos_host += n_steps;
+    d->step_host += n_steps;
     // position and step counters live on the device for the multi-kernel path: keep them in step
     hipLaunchKernelGGL(set_counters_kernel, dim3(1), dim3(64), 0, s, d->pos, d->step, pos + n_steps, step + n_steps);
     DEC_HIP(hipGetLastError());
     return YSCV_HIP_OK;
   }
+  DEC_HIP(enter_stream(d, s));
   if (!use_graph) {
-    for (int i = 0; i < n_steps; i++) YSCV_TRY(enqueue_step(d, d->batch, s));
+    for (int i = 0; i < n_steps; i++) {
+      YSCV_TRY(enqueue_step(d, d->batch, s));
+      d->pos_host++;
+      d->step_host++;
+    }
     return YSCV_HIP_OK;
   }
   if (!d->graph_exec || d->graph_batch != d->batch) {
@@ -956,7 +1005,11 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
     if (e != hipSuccess) return set_error(YSCV_HIP_ERR_DEVICE, "graph capture failed: %s", hipGetErrorString(e));
     d->graph_batch = d->batch;
   }
-  for (int i = 0; i < n_steps; i++) DEC_HIP(hipGraphLaunch(d->graph_exec, s));
+  for (int i = 0; i < n_steps; i++) {
+    DEC_HIP(hipGraphLaunch(d->graph_exec, s));
+    d->pos_host++;
+    d->step_host++;
+  }
   return YSCV_HIP_OK;
 }
 
@@ -1142,25 +1195,25 @@ int32_t yscv_hip_decoder_set_qkv_bias(yscv_hip_decoder *d, int32_t layer, const 
   return YSCV_HIP_OK;
 }
 
+static int32_t keep_prefill_buffer(yscv_hip_decoder *d, size_t bytes) {
+  if (bytes <= d->pf_bytes) return YSCV_HIP_OK;
+  (void)hipFree(d->pf_buf);  // waits for the passes that use it
+  d->pf_buf = nullptr;
+  d->pf_bytes = 0;
+  DEC_HIP(hipMalloc(&d->pf_buf, bytes));
+  d->pf_bytes = bytes;
+  return YSCV_HIP_OK;
+}
+
 // The prompt pass: every projection sees all rows at once (the MFMA GEMM above 16 rows), attention is causal over the
 // cache, and only the last row goes through the final norm and the LM head.
 static int32_t prefill_chunk(yscv_hip_decoder *d, const int32_t *tokens_dev, int rows, int start_pos, bool last, hipStream_t s) {
   const auto &c = d->cfg;
   const size_t R = (size_t)rows, D = c.d_model, hq = (size_t)c.n_heads * c.head_dim;
   const size_t qkv_n = (size_t)(c.n_heads + 2 * c.n_kv_heads) * c.head_dim, ff = c.d_ff;
-  StreamBuf h, xn, qkv, ao, act;
-  YSCV_TRY(h.alloc(R * D * 4, s));
-  YSCV_TRY(xn.alloc(R * D * 2, s));
-  YSCV_TRY(qkv.alloc(R * qkv_n * 2, s));
-  YSCV_TRY(ao.alloc(R * hq * 2, s));
-  YSCV_TRY(act.alloc(R * ff * 2, s));
   const bool i8 = d->kv_dtype == YSCV_HIP_KV_I8;
   const int t_ctx = (start_pos + rows + 31) / 32 * 32;
-  StreamBuf tk, tv;
-  if (i8) {
-    YSCV_TRY(tk.alloc((size_t)c.n_kv_heads * t_ctx * c.head_dim * 2, s));
-    YSCV_TRY(tv.alloc((size_t)c.n_kv_heads * t_ctx * c.head_dim * 2, s));
-  }
+  const size_t t_bytes = i8 ? (size_t)c.n_kv_heads * t_ctx * c.head_dim * 2 : 0;
   // one scratch for all projections of the pass (prepared activations are not needed: the rows are fp16 already; what
   // remains are the K-split partial sums of the short-prompt shapes)
   size_t ws_bytes = 0;
@@ -1169,34 +1222,48 @@ static int32_t prefill_chunk(yscv_hip_decoder *d, const int32_t *tokens_dev, int
     YSCV_TRY(int4_workspace_bytes(w, R, YSCV_HIP_F16, 0, &b));
     ws_bytes = b > ws_bytes ? b : ws_bytes;
   }
-  StreamBuf pws;
-  if (ws_bytes > 0) YSCV_TRY(pws.alloc(ws_bytes, s));
-  YSCV_TRY(launch_embed(tokens_dev, d->emb, rows, (int)D, c.vocab, h.as<float>(), s));
+  // the pass's buffers, one behind the other in the block the decoder keeps
+  size_t need = 0;
+  auto place = [&need](size_t bytes) {
+    const size_t at = need;
+    need += round_up(bytes, 256);
+    return at;
+  };
+  const size_t at_h = place(R * D * 4), at_xn = place(R * D * 2), at_qkv = place(R * qkv_n * 2), at_ao = place(R * hq * 2),
+               at_act = place(R * ff * 2), at_tk = place(t_bytes), at_tv = place(t_bytes), at_ws = place(ws_bytes);
+  YSCV_TRY(keep_prefill_buffer(d, need));
+  char *base = static_cast<char *>(d->pf_buf);
+  float *h = reinterpret_cast<float *>(base + at_h);
+  _Float16 *xn = reinterpret_cast<_Float16 *>(base + at_xn), *qkv = reinterpret_cast<_Float16 *>(base + at_qkv),
+           *ao = reinterpret_cast<_Float16 *>(base + at_ao), *act = reinterpret_cast<_Float16 *>(base + at_act),
+           *tk = reinterpret_cast<_Float16 *>(base + at_tk), *tv = reinterpret_cast<_Float16 *>(base + at_tv);
+  void *pws = base + at_ws;
+  YSCV_TRY(launch_embed(tokens_dev, d->emb, rows, (int)D, c.vocab, h, s));
   for (auto &L : d->layers) {
-    YSCV_TRY(launch_rmsnorm(h.as<float>(), L.attn_norm, rows, (int)D, c.rms_eps, xn.as<_Float16>(), s));
-    YSCV_TRY(int4_run_ws(L.wqkv, xn.p, YSCV_HIP_F16, qkv.p, YSCV_HIP_F16, R, 0, EPI_STORE, pws.p, ws_bytes, s));
-    if (L.qkv_bias) YSCV_TRY(launch_bias_add_f16(qkv.as<_Float16>(), L.qkv_bias, R, qkv_n, s));
+    YSCV_TRY(launch_rmsnorm(h, L.attn_norm, rows, (int)D, c.rms_eps, xn, s));
+    YSCV_TRY(int4_run_ws(L.wqkv, xn, YSCV_HIP_F16, qkv, YSCV_HIP_F16, R, 0, EPI_STORE, pws, ws_bytes, s));
+    if (L.qkv_bias) YSCV_TRY(launch_bias_add_f16(qkv, L.qkv_bias, R, qkv_n, s));
     if (i8) {
       // the quantised append, and attention over what the int8 cache returns for every position so far (fp16 scratch)
-      YSCV_TRY(launch_prefill_rope_append_i8(qkv.as<_Float16>(), rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta,
-                                             c.max_ctx, L.kc8, L.ks, L.vc8, L.vs, t_ctx, tk.as<_Float16>(), tv.as<_Float16>(), s));
-      YSCV_TRY(launch_gqa_cache(qkv.as<_Float16>(), tk.as<_Float16>(), tv.as<_Float16>(), nullptr, rows, start_pos, c.n_heads,
-                                c.n_kv_heads, c.head_dim, t_ctx, ao.as<_Float16>(), s));
+      YSCV_TRY(launch_prefill_rope_append_i8(qkv, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta,
+                                             c.max_ctx, L.kc8, L.ks, L.vc8, L.vs, t_ctx, tk, tv, s));
+      YSCV_TRY(launch_gqa_cache(qkv, tk, tv, nullptr, rows, start_pos, c.n_heads,
+                                c.n_kv_heads, c.head_dim, t_ctx, ao, s));
     } else {
-      YSCV_TRY(launch_prefill_rope_append(qkv.as<_Float16>(), rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta,
+      YSCV_TRY(launch_prefill_rope_append(qkv, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta,
                                           c.max_ctx, L.kc, L.vc, s));
-      YSCV_TRY(launch_gqa_cache(qkv.as<_Float16>(), L.kc, L.vc, nullptr, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim,
-                                c.max_ctx, ao.as<_Float16>(), s));
+      YSCV_TRY(launch_gqa_cache(qkv, L.kc, L.vc, nullptr, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim,
+                                c.max_ctx, ao, s));
     }
     // the residual update and SwiGLU ride on the projections' epilogues (both kernels have them: the skinny kernel up to
     // 16 rows, the LDS-ring GEMM above)
-    YSCV_TRY(int4_run_ws(L.wo, ao.p, YSCV_HIP_F16, h.p, YSCV_HIP_F32, R, 0, EPI_ADD_F32, pws.p, ws_bytes, s));
-    YSCV_TRY(launch_rmsnorm(h.as<float>(), L.ffn_norm, rows, (int)D, c.rms_eps, xn.as<_Float16>(), s));
-    YSCV_TRY(int4_run_ws(L.wgu, xn.p, YSCV_HIP_F16, act.p, YSCV_HIP_F16, R, 0, EPI_SWIGLU, pws.p, ws_bytes, s));
-    YSCV_TRY(int4_run_ws(L.wdown, act.p, YSCV_HIP_F16, h.p, YSCV_HIP_F32, R, 0, EPI_ADD_F32, pws.p, ws_bytes, s));
+    YSCV_TRY(int4_run_ws(L.wo, ao, YSCV_HIP_F16, h, YSCV_HIP_F32, R, 0, EPI_ADD_F32, pws, ws_bytes, s));
+    YSCV_TRY(launch_rmsnorm(h, L.ffn_norm, rows, (int)D, c.rms_eps, xn, s));
+    YSCV_TRY(int4_run_ws(L.wgu, xn, YSCV_HIP_F16, act, YSCV_HIP_F16, R, 0, EPI_SWIGLU, pws, ws_bytes, s));
+    YSCV_TRY(int4_run_ws(L.wdown, act, YSCV_HIP_F16, h, YSCV_HIP_F32, R, 0, EPI_ADD_F32, pws, ws_bytes, s));
   }
   if (last) {
-    YSCV_TRY(launch_rmsnorm(h.as<float>() + (R - 1) * D, d->final_norm, 1, (int)D, c.rms_eps, d->xn, s));
+    YSCV_TRY(launch_rmsnorm(h + (R - 1) * D, d->final_norm, 1, (int)D, c.rms_eps, d->xn, s));
     YSCV_TRY(int4_run_ws(d->lm_head, d->xn, YSCV_HIP_F16, d->logits, YSCV_HIP_F32, 1, 1, EPI_STORE, d->ws, d->ws_bytes, s));
   }
   return YSCV_HIP_OK;
@@ -1214,20 +1281,33 @@ int32_t yscv_hip_decoder_prefill(yscv_hip_decoder *d, const int32_t *tokens_host
     YSCV_REQUIRE(tokens_host[i] >= 0 && tokens_host[i] < c.vocab, "token %d outside the vocabulary (%d)", tokens_host[i], c.vocab);
   hipStream_t s = as_stream(stream);
   d->batch = 1;
-  StreamBuf toks;
-  YSCV_TRY(toks.alloc((size_t)n_tokens * 4, s));
-  DEC_HIP(hipMemcpyAsync(toks.p, tokens_host, (size_t)n_tokens * 4, hipMemcpyHostToDevice, s));
-  DEC_HIP(hipStreamSynchronize(s));  // tokens_host is the caller's again
+  DEC_HIP(enter_stream(d, s));
+  if (n_tokens > d->prompt_cap) {
+    (void)hipFree(d->prompt);
+    d->prompt = nullptr;
+    d->prompt_cap = 0;
+    DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->prompt), (size_t)n_tokens * 4));
+    d->prompt_cap = n_tokens;
+  }
+  for (int32_t t0 = 0; t0 < n_tokens; t0 += kPromptPiece) {
+    PromptPiece piece;
+    const int n = n_tokens - t0 < kPromptPiece ? n_tokens - t0 : kPromptPiece;
+    memcpy(piece.tokens, tokens_host + t0, (size_t)n * 4);
+    hipLaunchKernelGGL(store_prompt_kernel, dim3(1), dim3(kPromptPiece), 0, s, d->prompt + t0, n, piece);
+    DEC_HIP(hipGetLastError());
+  }
   const int chunk = d->prefill_rows;  // rows per pass: bounds the activation buffers
   for (int32_t r0 = 0; r0 < n_tokens; r0 += chunk) {
     const int rows = n_tokens - r0 < chunk ? n_tokens - r0 : chunk;
-    YSCV_TRY(prefill_chunk(d, toks.as<int32_t>() + r0, rows, start_pos + r0, r0 + rows == n_tokens, s));
+    YSCV_TRY(prefill_chunk(d, d->prompt + r0, rows, start_pos + r0, r0 + rows == n_tokens, s));
   }
   // as after reset(last token, start_pos + n - 1) + one decode step: the pick is the next input, position and step advance
   hipLaunchKernelGGL(set_counters_kernel, dim3(1), dim3(64), 0, s, d->pos, d->step, start_pos + n_tokens - 1, 0);
   DEC_HIP(hipGetLastError());
   YSCV_TRY(launch_argmax(d->logits, 1, c.vocab, d->tokens, d->history, d->step, c.max_steps, s));
   YSCV_TRY(launch_advance(d->pos, d->step, s));
+  d->pos_host = start_pos + n_tokens;
+  d->step_host = 1;
   d->last_path = 1;
   return YSCV_HIP_OK;
 }

@@ -133,6 +133,7 @@ class Decoder:
         ids = np.ascontiguousarray(input_ids, dtype=np.uint32)
         cfg = capi.GenerateConfig(max_tokens, temperature, top_k, top_p, 0 if eos_token_id is None else 1,
                                   0 if eos_token_id is None else int(eos_token_id), repetition_penalty)
+        self.batch = 1  # as after reset(): logits() and tokens() return one row
         out = np.zeros(max(max_tokens, 1), np.uint32)
         n = C.c_size_t(0)
         lib().decoder_generate(self._h, _p(ids), C.c_size_t(ids.size), C.byref(cfg), _p(out), C.byref(n))
