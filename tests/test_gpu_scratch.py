@@ -1,0 +1,88 @@
+"""Scratch blocks the library keeps per stream: calls of growing and shrinking size on more streams than there are
+blocks, from several threads on one stream, and inside a captured graph give what they give one at a time."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _weight(K, rng, n, k, g=64):
+    return K.PackedInt4Weight(rng.integers(0, 256, n * k // 2, dtype=np.uint8), rng.uniform(0.005, 0.02, n * (k // g)).astype(np.float16),
+                              g, n, k, nibble_format=K.NIBBLE_UNSIGNED)
+
+
+def test_more_streams_than_blocks_and_growing_requests():
+    import torch
+
+    from yscv_amd import kernels as K
+
+    rng = np.random.default_rng(1)
+    w = _weight(K, rng, 208, 960)  # 960 is no multiple of 512: prepared activations in the scratch
+    xs = [torch.from_numpy(rng.standard_normal((m, 960)).astype(np.float32)).half().cuda() for m in (3, 700, 40, 5000, 77, 1, 300, 20, 64, 9, 2500, 130)]
+    want = [w.matmul(x, out_dtype=torch.float32).clone() for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(11)]
+    got = []
+    for rnd in range(3):
+        for i, x in enumerate(xs):
+            with torch.cuda.stream(streams[(i * 5 + rnd) % len(streams)]):
+                got.append((i, w.matmul(x, out_dtype=torch.float32)))
+    torch.cuda.synchronize()
+    for i, y in got:
+        assert torch.equal(y, want[i]), i
+
+
+def test_threads_on_one_stream():
+    import torch
+
+    from yscv_amd import kernels as K
+
+    rng = np.random.default_rng(2)
+    w = _weight(K, rng, 272, 1344)
+    xs = [torch.from_numpy(rng.standard_normal((50 + 30 * t, 1344)).astype(np.float32)).half().cuda() for t in range(4)]
+    want = [w.matmul(x, out_dtype=torch.float32).clone() for x in xs]
+    torch.cuda.synchronize()
+    got = [[] for _ in xs]
+
+    def worker(t):
+        for _ in range(50):
+            got[t].append(w.matmul(xs[t], out_dtype=torch.float32))
+
+    threads = [threading.Thread(target=worker, args=(t,)) for t in range(len(xs))]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join(timeout=60)
+    assert not any(th.is_alive() for th in threads)
+    torch.cuda.synchronize()
+    for t, ys in enumerate(got):
+        assert len(ys) == 50 and all(torch.equal(y, want[t]) for y in ys), t
+
+
+def test_captured_call_keeps_its_own_memory():
+    import torch
+
+    from yscv_amd import kernels as K
+
+    rng = np.random.default_rng(3)
+    w = _weight(K, rng, 208, 960)
+    x = torch.from_numpy(rng.standard_normal((90, 960)).astype(np.float32)).half().cuda()
+    other = torch.from_numpy(rng.standard_normal((4000, 960)).astype(np.float32)).half().cuda()
+    want = w.matmul(x, out_dtype=torch.float32).clone()
+    out = torch.empty_like(want)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        w.matmul(x, out=out)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            w.matmul(x, out=out)
+    for _ in range(4):
+        out.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        w.matmul(other)  # another call's scratch between the replays
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)

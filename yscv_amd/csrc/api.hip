@@ -53,8 +53,8 @@ int32_t init_context(int device) {
     YSCV_HIP_TRY(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
     g_scratch_ptr[device] = p;
   }
-  // Calls without a caller-provided workspace take their scratch from the stream-ordered allocator; keeping freed
-  // blocks in its pool makes that a sub-microsecond operation instead of a trip to the driver per call.
+  // Scratch beyond what scratch.hip keeps comes from the stream-ordered allocator; keeping freed blocks in its pool
+  // saves the trip to the driver per call.
   hipMemPool_t pool = nullptr;
   if (hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess && pool != nullptr) {
     uint64_t keep = UINT64_MAX;
@@ -133,7 +133,7 @@ static Int4Scratch int4_scratch_layout(const yscv_hip_int4_weight *w, const void
   return L;
 }
 
-int32_t int4_workspace_bytes(const yscv_hip_int4_weight *w, size_t m, int x_dtype, int force, size_t *bytes) {
+int32_t int4_workspace_bytes(const yscv_hip_int4_weight *w, size_t m, int x_dtype, int force, size_t *bytes, const void *x) {
   const Context *ctx = nullptr;
   YSCV_TRY(ensure_context(&ctx));
   YSCV_REQUIRE(w != nullptr && bytes != nullptr, "null argument");
@@ -142,14 +142,15 @@ int32_t int4_workspace_bytes(const yscv_hip_int4_weight *w, size_t m, int x_dtyp
     return YSCV_HIP_OK;
   }
   // a 16-byte aligned pointer stands in for the activation: alignment is checked again at run time
-  Int4Scratch L = int4_scratch_layout(w, reinterpret_cast<const void *>(uintptr_t(256)), x_dtype, m, force, ctx->num_cus);
+  if (!x) x = reinterpret_cast<const void *>(uintptr_t(256));
+  Int4Scratch L = int4_scratch_layout(w, x, x_dtype, m, force, ctx->num_cus);
   *bytes = L.total + L.opt_bytes;
   return YSCV_HIP_OK;
 }
 
 // Runs the int4 path: activation preparation if needed, then the skinny or the GEMM kernel.
-// `ws` may be null: scratch then comes from the stream-ordered allocator, so concurrent callers
-// on different streams never share it.
+// `ws` may be null: scratch then comes from the blocks the library keeps per stream (scratch.hip), so concurrent
+// callers on different streams never share it.
 int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y, int y_dtype, size_t m,
                     int force /*0 auto, 1 skinny, 2 gemm*/, int epi, void *ws, size_t ws_bytes, hipStream_t s,
                     const NormFold *nf) {
@@ -190,7 +191,7 @@ int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, v
     }
   }
   char *scratch = static_cast<char *>(ws);
-  bool own = false;
+  Scratch own;
   size_t have = ws_bytes;
   if (L.total + L.opt_bytes > 0) {
     if (scratch) {
@@ -198,8 +199,8 @@ int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, v
       YSCV_REQUIRE((reinterpret_cast<uintptr_t>(scratch) & 255) == 0, "workspace must be 256-byte aligned");
     } else {
       have = L.total + L.opt_bytes;
-      YSCV_HIP_TRY(hipMallocAsync(reinterpret_cast<void **>(&scratch), have, s));
-      own = true;
+      YSCV_TRY(own.take(have, s));
+      scratch = own.as<char>();
     }
   }
   // the GEMM's K-split partials sit behind everything else
@@ -222,21 +223,10 @@ int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, v
     run_split = 1;
     xl = nullptr;
   }
-  int32_t st = YSCV_HIP_OK;
   if (!L.direct)
-    st = launch_x_prep(x, x_dtype, m, w->k, L.k_pad, run_split, const_cast<_Float16 *>(xh), xl, row_scale, s);
-  if (st == YSCV_HIP_OK) {
-    if (L.skinny)
-      st = launch_int4_skinny(w, L.plan, xh, xl, xraw, row_scale, L.k_pad, L.split, y, y_dtype, m, partial, epi, s, nf);
-    else
-      st = launch_int4_gemm(w, xh, xl, row_scale, L.k_pad, run_split, y, y_dtype, m, s, epi, gemm_partial, L.opt_bytes);
-  }
-  if (own) {
-    hipError_t fe = hipFreeAsync(scratch, s);
-    YSCV_TRY(st);
-    YSCV_HIP_TRY(fe);
-  }
-  return st;
+    YSCV_TRY(launch_x_prep(x, x_dtype, m, w->k, L.k_pad, run_split, const_cast<_Float16 *>(xh), xl, row_scale, s));
+  if (L.skinny) return launch_int4_skinny(w, L.plan, xh, xl, xraw, row_scale, L.k_pad, L.split, y, y_dtype, m, partial, epi, s, nf);
+  return launch_int4_gemm(w, xh, xl, row_scale, L.k_pad, run_split, y, y_dtype, m, s, epi, gemm_partial, L.opt_bytes);
 }
 
 static int32_t int4_run(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y, int y_dtype,
@@ -422,6 +412,7 @@ extern "C" {
 int32_t yscv_hip_init(int32_t device_index) { return init_context(device_index); }
 
 int32_t yscv_hip_shutdown(void) {
+  release_scratch();
   drop_context();
   return YSCV_HIP_OK;
 }
@@ -769,7 +760,7 @@ int32_t yscv_hip_dynamic_quantize_linear(const float *x_dev, size_t len, uint8_t
   YSCV_TRY(ensure_context(nullptr));
   YSCV_REQUIRE(scale_zp_dev != nullptr, "null scale/zero-point pointer");
   YSCV_REQUIRE(len == 0 || (x_dev && y_dev), "null pointer");
-  return launch_dynamic_quantize_linear(x_dev, len, y_dev, scale_zp_dev, as_stream(stream));
+  return launch_dynamic_quantize_linear(x_dev, len, y_dev, false, scale_zp_dev, scale_zp_dev + 1, nullptr, as_stream(stream));
 }
 
 int32_t yscv_hip_quantize_linear_f32_to_i8_dispatch(const float *data, size_t len, float scale, float zero_point,
@@ -831,7 +822,7 @@ int32_t yscv_hip_dynamic_quantize_linear_host(const float *x, size_t len, uint8_
   YSCV_TRY(dy.alloc(len));
   YSCV_TRY(dsz.alloc(2 * sizeof(float)));
   if (len) YSCV_HIP_TRY(hipMemcpy(dx.p, x, len * sizeof(float), hipMemcpyHostToDevice));
-  YSCV_TRY(launch_dynamic_quantize_linear(dx.as<float>(), len, dy.as<uint8_t>(), dsz.as<float>(), nullptr));
+  YSCV_TRY(launch_dynamic_quantize_linear(dx.as<float>(), len, dy.p, false, dsz.as<float>(), dsz.as<float>() + 1, nullptr, nullptr));
   float sz[2];
   YSCV_HIP_TRY(hipMemcpy(sz, dsz.p, sizeof(sz), hipMemcpyDeviceToHost));
   if (len) YSCV_HIP_TRY(hipMemcpy(y, dy.p, len, hipMemcpyDeviceToHost));

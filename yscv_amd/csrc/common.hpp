@@ -77,30 +77,25 @@ struct DevBuf {
   }
 };
 
-// Scratch from the stream-ordered allocator: allocation and release are queued on the stream like the kernels that
-// use the memory, so the call that owns the buffer can return without waiting for the device.
-struct StreamBuf {
+// Scratch of one call on one stream, usable by everything the call enqueues until the object goes out of scope; the
+// call can return without waiting for the device (scratch.hip).  One per call: a second one on the same stream inside
+// its lifetime would wait for itself.
+struct ScratchSlot;
+struct Scratch {
   void *p = nullptr;
   hipStream_t s = nullptr;
-  ~StreamBuf() {
-    if (p) (void)hipFreeAsync(p, s);
-  }
-  int32_t alloc(size_t bytes, hipStream_t stream) {
-    if (bytes == 0) bytes = 4;
-    s = stream;
-    hipError_t e = hipMallocAsync(&p, bytes, s);
-    if (e != hipSuccess) {
-      p = nullptr;
-      return set_error(e == hipErrorOutOfMemory ? YSCV_HIP_ERR_OOM : YSCV_HIP_ERR_DEVICE,
-                       "hipMallocAsync(%zu) failed: %s", bytes, hipGetErrorString(e));
-    }
-    return YSCV_HIP_OK;
-  }
+  ScratchSlot *slot = nullptr;
+  Scratch() = default;
+  Scratch(const Scratch &) = delete;
+  Scratch &operator=(const Scratch &) = delete;
+  ~Scratch();
+  int32_t take(size_t bytes, hipStream_t stream);
   template <typename T>
-  T *as() const {
-    return static_cast<T *>(p);
+  T *as(size_t byte_offset = 0) const {
+    return reinterpret_cast<T *>(static_cast<char *>(p) + byte_offset);
   }
 };
+void release_scratch();
 
 inline size_t ceil_div(size_t a, size_t b) { return (a + b - 1) / b; }
 inline size_t round_up(size_t a, size_t b) { return ceil_div(a, b) * b; }

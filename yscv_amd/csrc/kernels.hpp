@@ -127,7 +127,8 @@ int32_t launch_int4_mid(const yscv_hip_int4_weight *w, const _Float16 *xh, const
                         int y_dtype, size_t m, hipStream_t s, int epi, float *partial, size_t partial_bytes);
 
 // Whole int4 call (activation preparation + kernel) with caller-provided scratch; ws may be null.
-int32_t int4_workspace_bytes(const yscv_hip_int4_weight *w, size_t m, int x_dtype, int force, size_t *bytes);
+// (x: the activations, whose alignment decides whether they are used in place; null = 16-byte aligned ones)
+int32_t int4_workspace_bytes(const yscv_hip_int4_weight *w, size_t m, int x_dtype, int force, size_t *bytes, const void *x = nullptr);
 int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y, int y_dtype, size_t m,
                     int force, int epi, void *ws, size_t ws_bytes, hipStream_t s, const NormFold *nf = nullptr);
 
@@ -168,8 +169,11 @@ int32_t launch_quantize_f32_to_int4(const float *x, size_t len, float scale, int
 int32_t launch_requant(const int32_t *acc, size_t len, size_t c, const int32_t *corr,
                        const float *composite_v, float composite, float y_zp, int round_mode,
                        int lo, int hi, int relu, void *out, hipStream_t s);
-int32_t launch_dynamic_quantize_linear(const float *x, size_t len, uint8_t *y, float *scale_zp,
-                                       hipStream_t s);
+// y: uint8 values, or the same values as f32 when y_f32.  partial: dql_partial_bytes() of scratch for the block ranges, or
+// null (taken from the scratch blocks then)
+size_t dql_partial_bytes(size_t len);
+int32_t launch_dynamic_quantize_linear(const float *x, size_t len, void *y, bool y_f32, float *scale_out, float *zp_out,
+                                       float *partial, hipStream_t s);
 
 int32_t launch_kv_i8_quantize_rows(const float *src, size_t rows, size_t kv_dim, int8_t *data, float *scales, hipStream_t s);
 int32_t launch_kv_i8_dequantize_rows(const int8_t *data, const float *scales, size_t rows, size_t kv_dim, float *out,

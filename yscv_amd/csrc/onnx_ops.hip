@@ -172,15 +172,6 @@ __global__ void dequantize_linear_f32_kernel(const float *__restrict__ q, size_t
   }
 }
 
-__global__ void u8_to_f32_kernel(const uint8_t *__restrict__ q, size_t len, const float *__restrict__ scale_zp,
-                                 float *__restrict__ y, float *__restrict__ scale_out, float *__restrict__ zp_out) {
-  GRID_STRIDE(i, len) y[i] = (float)q[i];
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *scale_out = scale_zp[0];
-    *zp_out = scale_zp[1];
-  }
-}
-
 // [d0][d1] -> [d1][d0]
 __global__ void transpose_f32_kernel(const float *__restrict__ in, size_t d0, size_t d1, float *__restrict__ out) {
   __shared__ float tile[32][33];
@@ -281,9 +272,9 @@ struct MatmulArgs {
 int32_t run_fast(const MatmulArgs &g) {
   if (g.b_packed) {
     // the usual case, a weight packed at load time: cast kernel + GEMM whose epilogue writes the f32 carriers, the
-    // int8 copy of A in stream-ordered scratch -- nothing here waits for the device
-    StreamBuf a8;
-    YSCV_TRY(a8.alloc(g.m * g.k, g.s));
+    // int8 copy of A in scratch -- nothing here waits for the device
+    Scratch a8;
+    YSCV_TRY(a8.take(g.m * g.k, g.s));
     hipLaunchKernelGGL(cast_as_i8_kernel, dim3(grid_for(g.m * g.k)), dim3(256), 0, g.s, g.a, g.m * g.k, 0, a8.as<int8_t>());
     YSCV_HIP_TRY(hipGetLastError());
     I8Epilogue ep{};
@@ -559,23 +550,18 @@ int32_t yscv_hip_exec_qdq_matmul(const float *x_dev, size_t m, float a_scale, co
   hipStream_t s = as_stream(stream);
   // QuantizeLinear (zero point 0) into a scratch int8 matrix, then the GEMM whose epilogue requantises with the
   // QLinearMatMul fast-path expression and dequantises again
-  int8_t *a8 = nullptr;
-  YSCV_HIP_TRY(hipMallocAsync(reinterpret_cast<void **>(&a8), m * b->k, s));
-  int32_t st = launch_quantize_linear_i8(x_dev, m * b->k, a_scale, 0.0f, a8, s);
-  if (st == YSCV_HIP_OK) {
-    I8Epilogue ep{};
-    ep.mode = 2;
-    ep.composite = (a_scale * b_scale) / y_scale;
-    ep.y_zp = y_zp;
-    ep.round_mode = YSCV_HIP_ROUND_HALF_AWAY;
-    ep.lo = -128;
-    ep.hi = 127;
-    ep.dq_scale = y_scale;
-    st = launch_i8_gemm(a8, 0, 0, b, m, out_dev, ep, s);
-  }
-  const hipError_t fe = hipFreeAsync(a8, s);
-  YSCV_TRY(st);
-  YSCV_HIP_TRY(fe);
+  Scratch a8;
+  YSCV_TRY(a8.take(m * b->k, s));
+  YSCV_TRY(launch_quantize_linear_i8(x_dev, m * b->k, a_scale, 0.0f, a8.as<int8_t>(), s));
+  I8Epilogue ep{};
+  ep.mode = 2;
+  ep.composite = (a_scale * b_scale) / y_scale;
+  ep.y_zp = y_zp;
+  ep.round_mode = YSCV_HIP_ROUND_HALF_AWAY;
+  ep.lo = -128;
+  ep.hi = 127;
+  ep.dq_scale = y_scale;
+  YSCV_TRY(launch_i8_gemm(a8.p, 0, 0, b, m, out_dev, ep, s));
   g_qlinear_fast.fetch_add(1, std::memory_order_relaxed);
   return YSCV_HIP_OK;
 }
@@ -589,28 +575,15 @@ int32_t yscv_hip_exec_dql_matmul_integer(const float *x_dev, size_t m, const ysc
   YSCV_REQUIRE(x_dev && out_dev, "null x / out pointer");
   hipStream_t s = as_stream(stream);
   const size_t len = m * b->k;
-  // uint8 A and {scale, zero point} in one stream-ordered scratch block; nothing returns to the host
-  uint8_t *scratch = nullptr;
+  // uint8 A and the block ranges of the quantiser in one scratch block; nothing returns to the host
   const size_t a_bytes = round_up(len, 256);
-  YSCV_HIP_TRY(hipMallocAsync(reinterpret_cast<void **>(&scratch), a_bytes + 256, s));
-  float *scale_zp = reinterpret_cast<float *>(scratch + a_bytes);
-  int32_t st = launch_dynamic_quantize_linear(x_dev, len, scratch, scale_zp, s);
-  if (st == YSCV_HIP_OK) {
-    I8Epilogue ep{};
-    ep.mode = 3;                   // f32(acc): MatMulInteger's output carrier (linear.rs:693-697)
-    ep.a_zp_dev = scale_zp + 1;    // the zero point stays on the device: the GEMM folds (128 - zp) * colsum(b) itself
-    st = launch_i8_gemm(scratch, 1, 0, b, m, out_dev, ep, s);
-  }
-  hipError_t e1 = hipSuccess, e2 = hipSuccess;
-  if (st == YSCV_HIP_OK) {
-    e1 = hipMemcpyAsync(y_scale_dev, scale_zp, sizeof(float), hipMemcpyDeviceToDevice, s);
-    e2 = hipMemcpyAsync(y_zp_dev, scale_zp + 1, sizeof(float), hipMemcpyDeviceToDevice, s);
-  }
-  const hipError_t fe = hipFreeAsync(scratch, s);
-  YSCV_TRY(st);
-  YSCV_HIP_TRY(e1);
-  YSCV_HIP_TRY(e2);
-  YSCV_HIP_TRY(fe);
+  Scratch scratch;
+  YSCV_TRY(scratch.take(a_bytes + dql_partial_bytes(len), s));
+  YSCV_TRY(launch_dynamic_quantize_linear(x_dev, len, scratch.p, false, y_scale_dev, y_zp_dev, scratch.as<float>(a_bytes), s));
+  I8Epilogue ep{};
+  ep.mode = 3;               // f32(acc): MatMulInteger's output carrier (linear.rs:693-697)
+  ep.a_zp_dev = y_zp_dev;    // the zero point stays on the device: the GEMM folds (128 - zp) * colsum(b) itself
+  YSCV_TRY(launch_i8_gemm(scratch.p, 1, 0, b, m, out_dev, ep, s));
   g_mmi_fallback.fetch_add(1, std::memory_order_relaxed);
   return YSCV_HIP_OK;
 }
@@ -633,21 +606,18 @@ int32_t yscv_hip_exec_matmul_nbits(const void *a_dev, int32_t a_dtype, size_t m,
   hipStream_t s = as_stream(stream);
   if (bias_dev == nullptr) return yscv_hip_int4_matmul(b, a_dev, a_dtype, y_dev, y_dtype, m, stream);
   // with a bias the product is kept in f32 until the bias is added, then rounded once to the output type
-  float *acc = nullptr;
+  // (one scratch block for that product and whatever the matmul itself needs)
   const bool in_place = y_dtype == YSCV_HIP_F32;
-  if (in_place) acc = static_cast<float *>(y_dev);
-  else YSCV_HIP_TRY(hipMallocAsync(reinterpret_cast<void **>(&acc), m * n * sizeof(float), s));
-  int32_t st = yscv_hip_int4_matmul(b, a_dev, a_dtype, acc, YSCV_HIP_F32, m, stream);
-  if (st == YSCV_HIP_OK) {
-    hipLaunchKernelGGL(bias_cast_kernel, dim3(grid_for(m * n)), dim3(256), 0, s, acc, m, n, bias_dev, y_dev, y_dtype);
-    if (hipGetLastError() != hipSuccess) st = set_error(YSCV_HIP_ERR_DEVICE, "MatMulNBits: bias kernel launch failed");
-  }
-  if (!in_place) {
-    const hipError_t fe = hipFreeAsync(acc, s);
-    YSCV_TRY(st);
-    YSCV_HIP_TRY(fe);
-  }
-  return st;
+  const size_t acc_bytes = in_place ? 0 : round_up(m * n * sizeof(float), 256);
+  size_t ws_bytes = 0;
+  YSCV_TRY(int4_workspace_bytes(b, m, a_dtype, 0, &ws_bytes, a_dev));
+  Scratch scratch;
+  YSCV_TRY(scratch.take(acc_bytes + ws_bytes, s));
+  float *acc = in_place ? static_cast<float *>(y_dev) : scratch.as<float>();
+  YSCV_TRY(int4_run_ws(b, a_dev, a_dtype, acc, YSCV_HIP_F32, m, 0, EPI_STORE, ws_bytes ? scratch.as<char>(acc_bytes) : nullptr, ws_bytes, s));
+  hipLaunchKernelGGL(bias_cast_kernel, dim3(grid_for(m * n)), dim3(256), 0, s, acc, m, n, bias_dev, y_dev, y_dtype);
+  if (hipGetLastError() != hipSuccess) return set_error(YSCV_HIP_ERR_DEVICE, "MatMulNBits: bias kernel launch failed");
+  return YSCV_HIP_OK;
 }
 
 int32_t yscv_hip_exec_gemm_int4(const float *a_dev, size_t m, const yscv_hip_int4_weight *b, const float *c_dev,
@@ -701,15 +671,7 @@ int32_t yscv_hip_exec_dynamic_quantize_linear(const float *x_dev, size_t len, fl
   YSCV_TRY(ensure_context(nullptr));
   YSCV_REQUIRE(y_scale_dev && y_zp_dev, "null scale / zero-point pointer");
   YSCV_REQUIRE(len == 0 || (x_dev && y_dev), "null pointer");
-  hipStream_t s = as_stream(stream);
-  StreamBuf q, sz;  // released in stream order: the call does not wait for the device
-  YSCV_TRY(q.alloc(len, s));
-  YSCV_TRY(sz.alloc(2 * sizeof(float), s));
-  YSCV_TRY(launch_dynamic_quantize_linear(x_dev, len, q.as<uint8_t>(), sz.as<float>(), s));
-  hipLaunchKernelGGL(u8_to_f32_kernel, dim3(grid_for(len)), dim3(256), 0, s, q.as<uint8_t>(), len, sz.as<float>(),
-                     y_dev, y_scale_dev, y_zp_dev);
-  YSCV_HIP_TRY(hipGetLastError());
-  return YSCV_HIP_OK;
+  return launch_dynamic_quantize_linear(x_dev, len, y_dev, true, y_scale_dev, y_zp_dev, nullptr, as_stream(stream));
 }
 
 }  // extern "C"

@@ -142,10 +142,11 @@ __global__ void __launch_bounds__(256) dql_minmax_kernel(const float *__restrict
   }
 }
 
+template <typename T>
 __global__ void __launch_bounds__(256) dql_quantize_kernel(const float *__restrict__ x, size_t len,
                                                            const float *__restrict__ minmax, int nparts,
-                                                           uint8_t *__restrict__ y,
-                                                           float *__restrict__ scale_zp) {
+                                                           T *__restrict__ y, float *__restrict__ scale_out,
+                                                           float *__restrict__ zp_out) {
   __shared__ float smin[4], smax[4];
   float mn = 3.40282347e+38f, mx = -3.40282347e+38f;
   for (int i = threadIdx.x; i < nparts; i += blockDim.x) {
@@ -176,32 +177,39 @@ __global__ void __launch_bounds__(256) dql_quantize_kernel(const float *__restri
   float zp = round_half_away_f(__fsub_rn(0.0f, __fdiv_rn(mn, scale)));
   if (zp == zp) zp = fminf(fmaxf(zp, 0.0f), 255.0f);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    scale_zp[0] = scale;
-    scale_zp[1] = zp;
+    *scale_out = scale;
+    *zp_out = zp;
   }
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < len;
        i += (size_t)gridDim.x * blockDim.x) {
     float v = __fadd_rn(__fdiv_rn(x[i], scale), zp);
-    y[i] = (uint8_t)clamp_cast(round_half_away_f(v), 0.0f, 255.0f);
+    y[i] = (T)(uint8_t)clamp_cast(round_half_away_f(v), 0.0f, 255.0f);
   }
 }
 
-int32_t launch_dynamic_quantize_linear(const float *x, size_t len, uint8_t *y, float *scale_zp,
-                                       hipStream_t s) {
-  int blocks = (int)ceil_div(len, (size_t)1024);
-  if (blocks > DQL_BLOCKS) blocks = DQL_BLOCKS;
-  if (blocks < 1) blocks = 1;
-  float *minmax = nullptr;
-  YSCV_HIP_TRY(hipMallocAsync(reinterpret_cast<void **>(&minmax), sizeof(float) * 2 * blocks, s));
-  hipLaunchKernelGGL(dql_minmax_kernel, dim3(blocks), dim3(256), 0, s, x, len, minmax);
-  hipError_t e1 = hipGetLastError();
-  hipLaunchKernelGGL(dql_quantize_kernel, dim3(blocks), dim3(256), 0, s, x, len, minmax, blocks, y,
-                     scale_zp);
-  hipError_t e2 = hipGetLastError();
-  hipError_t e3 = hipFreeAsync(minmax, s);
-  YSCV_HIP_TRY(e1);
-  YSCV_HIP_TRY(e2);
-  YSCV_HIP_TRY(e3);
+static int dql_blocks(size_t len) {
+  const size_t blocks = ceil_div(len, (size_t)1024);
+  return blocks > DQL_BLOCKS ? DQL_BLOCKS : (blocks < 1 ? 1 : (int)blocks);
+}
+size_t dql_partial_bytes(size_t len) { return sizeof(float) * 2 * dql_blocks(len); }
+
+int32_t launch_dynamic_quantize_linear(const float *x, size_t len, void *y, bool y_f32, float *scale_out, float *zp_out,
+                                       float *partial, hipStream_t s) {
+  const int blocks = dql_blocks(len);
+  Scratch own;
+  if (!partial) {
+    YSCV_TRY(own.take(dql_partial_bytes(len), s));
+    partial = own.as<float>();
+  }
+  hipLaunchKernelGGL(dql_minmax_kernel, dim3(blocks), dim3(256), 0, s, x, len, partial);
+  YSCV_HIP_TRY(hipGetLastError());
+  if (y_f32)
+    hipLaunchKernelGGL(dql_quantize_kernel<float>, dim3(blocks), dim3(256), 0, s, x, len, partial, blocks, static_cast<float *>(y),
+                       scale_out, zp_out);
+  else
+    hipLaunchKernelGGL(dql_quantize_kernel<uint8_t>, dim3(blocks), dim3(256), 0, s, x, len, partial, blocks,
+                       static_cast<uint8_t *>(y), scale_out, zp_out);
+  YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
 
