@@ -173,6 +173,17 @@ EXPORTED_SYMBOLS = sorted(list(_SIGNATURES) + list(_SPECIAL))
 _lib = None
 
 
+def stream_ptr() -> int:
+    """hipStream_t of torch's current stream.  torch.cuda.current_stream() builds a Stream object (3 us a call, as much as
+    a kernel launch); the raw accessor returns the handle itself."""
+    import torch
+
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch._C._cuda_getDevice())
+
+
 class _Checked:
     """Wraps the CDLL so that every status-returning call raises YscvHipError on failure."""
 

@@ -10,10 +10,11 @@ from __future__ import annotations
 import ctypes as C
 
 import numpy as np
+import torch
 
 from . import capi
 from .capi import (BF16, EPILOGUE_ADD_F32, EPILOGUE_STORE, EPILOGUE_SWIGLU, F16, F32, NIBBLE_SIGNED, NIBBLE_UNSIGNED,
-                   ROUND_HALF_AWAY, ROUND_TIES_EVEN, lib)
+                   ROUND_HALF_AWAY, ROUND_TIES_EVEN, lib, stream_ptr)
 
 _sz = C.c_size_t
 
@@ -26,16 +27,11 @@ def _ptr(a: np.ndarray):
     return a.ctypes.data_as(C.c_void_p)
 
 
+_DTYPE_CODE = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
+
+
 def _torch_dtype_code(t) -> int:
-    import torch
-
-    return {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}[t.dtype]
-
-
-def _stream_ptr():
-    import torch
-
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return _DTYPE_CODE[t.dtype]
 
 
 # ---- host-slice entry points (exact Rust argument lists) ---------------------------------
@@ -126,27 +122,23 @@ def dynamic_quantize_linear(x):
 
 def kv_i8_quantize_rows(src):
     """KvCache int8 append (runner/kv_cache.rs:45-61): src CUDA f32 [rows][kv_dim] -> (int8 [rows][kv_dim], f32 [rows])."""
-    import torch
-
     assert src.is_cuda and src.dtype == torch.float32 and src.dim() == 2
     src = src.contiguous()
     rows, kv_dim = int(src.shape[0]), int(src.shape[1])
     data = torch.empty(rows, kv_dim, device=src.device, dtype=torch.int8)
     scales = torch.empty(rows, device=src.device, dtype=torch.float32)
     lib().kv_i8_quantize_rows(C.c_void_p(src.data_ptr()), _sz(rows), _sz(kv_dim), C.c_void_p(data.data_ptr()),
-                              C.c_void_p(scales.data_ptr()), _stream_ptr())
+                              C.c_void_p(scales.data_ptr()), stream_ptr())
     return data, scales
 
 
 def kv_i8_dequantize_rows(data, scales):
     """KvCache int8 read (runner/kv_cache.rs:64-79)."""
-    import torch
-
     assert data.is_cuda and data.dtype == torch.int8 and data.dim() == 2 and scales.dtype == torch.float32
     rows, kv_dim = int(data.shape[0]), int(data.shape[1])
     out = torch.empty(rows, kv_dim, device=data.device, dtype=torch.float32)
     lib().kv_i8_dequantize_rows(C.c_void_p(data.contiguous().data_ptr()), C.c_void_p(scales.contiguous().data_ptr()), _sz(rows),
-                                _sz(kv_dim), C.c_void_p(out.data_ptr()), _stream_ptr())
+                                _sz(kv_dim), C.c_void_p(out.data_ptr()), stream_ptr())
     return out
 
 
@@ -212,14 +204,12 @@ class PackedInt4Weight:
         """quantize_matmul_weights_int4_packed (quantize/packed_int4.rs:50-128) for one initialiser: weight is a CUDA
         f32 tensor of shape [K, N] (MatMul, Gemm transB=0) or, with transposed_nk, [N, K] (Gemm transB=1).
         Returns None for a weight the reference skips (K % group_size != 0 or K * N < 32)."""
-        import torch
-
         assert weight.is_cuda and weight.dtype == torch.float32 and weight.dim() == 2
         weight = weight.contiguous()
         d0, d1 = int(weight.shape[0]), int(weight.shape[1])
         h = C.c_void_p()
         lib().int4_weight_from_f32(C.c_void_p(weight.data_ptr()), _sz(d0), _sz(d1), 1 if transposed_nk else 0,
-                                   _sz(group_size), _stream_ptr(), C.byref(h))
+                                   _sz(group_size), stream_ptr(), C.byref(h))
         if not h:
             return None
         self = cls.__new__(cls)
@@ -250,9 +240,7 @@ class PackedInt4Weight:
 
     def workspace_bytes(self, m: int, x_dtype) -> int:
         """Scratch yscv_hip_int4_matmul_ws needs for m rows of activations of torch dtype x_dtype (0 = none)."""
-        import torch
-
-        code = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}[x_dtype]
+        code = _DTYPE_CODE[x_dtype]
         b = _sz()
         lib().int4_workspace_bytes(self._h, _sz(m), code, C.byref(b))
         return b.value
@@ -262,23 +250,21 @@ class PackedInt4Weight:
         x.shape[:-1] + [m_w], like exec_matmul's int4 branch (runner/linear.rs:269-270).  With `workspace` (a CUDA
         uint8 tensor of at least workspace_bytes(m, x.dtype), 256-byte aligned) the call allocates nothing
         (yscv_hip_int4_matmul_ws, mode auto only)."""
-        import torch
-
-        assert x.is_cuda and x.shape[-1] == self.k
+        # (pointers and sizes go to ctypes as plain integers: at decode sizes the call is as long as its host side)
+        shape = x.shape
+        assert x.is_cuda and shape[-1] == self.k
         x = x.contiguous()
         m = x.numel() // self.k
-        odt = out_dtype or x.dtype
         if out is None:
-            out = torch.empty(*x.shape[:-1], self.m_w, device=x.device, dtype=odt)
+            out = x.new_empty((*shape[:-1], self.m_w), dtype=out_dtype or x.dtype)
+        args = (self._h, x.data_ptr(), _DTYPE_CODE[x.dtype], out.data_ptr(), _DTYPE_CODE[out.dtype], m)
         if workspace is not None:
             assert mode == "auto" and workspace.is_cuda and workspace.dtype == torch.uint8
-            lib().int4_matmul_ws(self._h, C.c_void_p(x.data_ptr()), _torch_dtype_code(x), C.c_void_p(out.data_ptr()),
-                                 _torch_dtype_code(out), _sz(m), C.c_void_p(workspace.data_ptr()),
-                                 _sz(workspace.numel()), _stream_ptr())
-            return out
-        fn = {"auto": lib().int4_matmul, "gemv": lib().int4_gemv, "gemm": lib().int4_gemm}[mode]
-        fn(self._h, C.c_void_p(x.data_ptr()), _torch_dtype_code(x), C.c_void_p(out.data_ptr()),
-           _torch_dtype_code(out), _sz(m), _stream_ptr())
+            lib().int4_matmul_ws(*args, workspace.data_ptr(), workspace.numel(), stream_ptr())
+        elif mode == "auto":
+            lib().int4_matmul(*args, stream_ptr())
+        else:
+            {"gemv": lib().int4_gemv, "gemm": lib().int4_gemm}[mode](*args, stream_ptr())
         return out
 
     def matmul_static(self, x, out):
@@ -288,7 +274,7 @@ class PackedInt4Weight:
         m = x.numel() // self.k
         assert out.numel() == m * self.m_w
         lib().int4_matmul_static(self._h, C.c_void_p(x.data_ptr()), _torch_dtype_code(x), C.c_void_p(out.data_ptr()),
-                                 _torch_dtype_code(out), _sz(m), _stream_ptr())
+                                 _torch_dtype_code(out), _sz(m), stream_ptr())
         return out
 
     def matmul_fused(self, x, out, epilogue: int):
@@ -300,7 +286,7 @@ class PackedInt4Weight:
         m = x.numel() // self.k
         assert out.is_contiguous() and out.numel() == m * (self.m_w // 2 if epilogue == 2 else self.m_w)
         lib().int4_matmul_fused(self._h, C.c_void_p(x.data_ptr()), _torch_dtype_code(x), C.c_void_p(out.data_ptr()),
-                                _torch_dtype_code(out), _sz(m), int(epilogue), _stream_ptr())
+                                _torch_dtype_code(out), _sz(m), int(epilogue), stream_ptr())
         return out
 
     def close(self):
@@ -345,32 +331,26 @@ class PackedI8B:
 
     def matmul(self, a, a_zp: int = 0, out=None):
         """a: CUDA tensor [m][k] int8 or uint8 -> int32 [m][n] (exact)."""
-        import torch
-
         assert a.is_cuda and a.dim() == 2 and a.shape[1] == self._k and a.dtype in (torch.int8, torch.uint8)
         a = a.contiguous()
         m = a.shape[0]
         if out is None:
-            out = torch.empty(m, self._n, device=a.device, dtype=torch.int32)
-        lib().int8_matmul(C.c_void_p(a.data_ptr()), int(a.dtype == torch.uint8), int(a_zp), self._h, _sz(m),
-                          C.c_void_p(out.data_ptr()), _stream_ptr())
+            out = a.new_empty((m, self._n), dtype=torch.int32)
+        lib().int8_matmul(a.data_ptr(), a.dtype == torch.uint8, int(a_zp), self._h, m, out.data_ptr(), stream_ptr())
         return out
 
     def matmul_requant(self, a, a_zp, composite, y_zp, round_mode, clamp_lo, clamp_hi, corr=None, out=None):
         """Fused GEMM + requantize.  composite: float or CUDA f32 tensor [n]; corr: CUDA i32 [n] or None."""
-        import torch
-
         assert a.is_cuda and a.dim() == 2 and a.shape[1] == self._k and a.dtype in (torch.int8, torch.uint8)
         a = a.contiguous()
         m = a.shape[0]
         if out is None:
-            out = torch.empty(m, self._n, device=a.device, dtype=torch.int8 if clamp_lo < 0 else torch.uint8)
-        comp_v, comp_s = (None, float(composite)) if not hasattr(composite, "data_ptr") else (composite, 0.0)
-        lib().int8_matmul_requant(C.c_void_p(a.data_ptr()), int(a.dtype == torch.uint8), int(a_zp), self._h, _sz(m),
-                                  C.c_void_p(corr.data_ptr()) if corr is not None else None,
-                                  C.c_void_p(comp_v.data_ptr()) if comp_v is not None else None,
-                                  C.c_float(comp_s), C.c_float(y_zp), int(round_mode), int(clamp_lo), int(clamp_hi),
-                                  C.c_void_p(out.data_ptr()), _stream_ptr())
+            out = a.new_empty((m, self._n), dtype=torch.int8 if clamp_lo < 0 else torch.uint8)
+        per_column = hasattr(composite, "data_ptr")
+        lib().int8_matmul_requant(a.data_ptr(), a.dtype == torch.uint8, int(a_zp), self._h, m,
+                                  corr.data_ptr() if corr is not None else None,
+                                  composite.data_ptr() if per_column else None, 0.0 if per_column else float(composite),
+                                  float(y_zp), int(round_mode), int(clamp_lo), int(clamp_hi), out.data_ptr(), stream_ptr())
         return out
 
     def close(self):
