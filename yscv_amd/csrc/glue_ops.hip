@@ -9,10 +9,10 @@
 // query positions per call with a causal limit (prompt ingestion), K / V either as the operator's tensors or as the
 // decoder's fp16 cache.
 //
-// Three forms of the attention kernel share the arithmetic below: gqa_generic_kernel (a workgroup owns 16 queries of
-// one head, the key blocks are split over its waves: decode and short query counts), gqa_rows_kernel (a wave owns 32
-// queries and walks every key block: the operator from 64 queries on) and gqa_shared_kv_kernel (the prompt pass over
-// the decoder's cache: the waves of a workgroup share each stage of K / V through LDS).
+// Three forms of the attention kernel share the arithmetic below: gqa_generic_kernel (the decoder's cache, decode and
+// short query counts: a workgroup owns 16 queries of one head, the key blocks are split over its waves),
+// gqa_shared_kv_kernel (the prompt pass over the cache: the waves of a workgroup share each stage of K / V through LDS)
+// and gqa_flat_kernel (the operator on f32 tensors).
 // gqa_generic_kernel: a workgroup of four waves owns 16 query positions of one head.  Wave w walks the key blocks
 // w, w + 4, ... of 16 positions each:
 //   S^T = K Q^T   rows = positions, columns = queries: hd / 32 x v_mfma_f32_16x16x32_f16, A = 16 cache rows as they lie
@@ -26,7 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
-#include <type_traits>
+#include <mutex>
 
 #include "int4_common.hpp"
 #include "decoder.hpp"
@@ -78,11 +78,12 @@ __device__ __forceinline__ void store4<float>(float *p, float a, float b, float 
 
 constexpr int GQA_WAVES = 4;
 
-template <int HD, typename TQ, typename TKV, typename TO, bool V_SLAB, bool FUSE = false>
+template <int HD, bool FUSE = false>
 __global__ void __launch_bounds__(64 * GQA_WAVES) gqa_generic_kernel(GqaArgs p) {
   static_assert(HD % 32 == 0 && HD >= 32 && HD <= 128, "head width (the merge buffer must fit the static LDS limit)");
-  static_assert(!FUSE || (V_SLAB && std::is_same<TQ, _Float16>::value && std::is_same<TKV, _Float16>::value),
-                "the fused form works on the decoder's fp16 buffers");
+  using TQ = _Float16;
+  using TKV = _Float16;
+  using TO = _Float16;
   constexpr int KK = HD / 32, DT = HD / 16;
   __shared__ float m_s[GQA_WAVES][16], l_s[GQA_WAVES][16];
   __shared__ float o_s[GQA_WAVES][16][HD + 4];
@@ -169,16 +170,8 @@ __global__ void __launch_bounds__(64 * GQA_WAVES) gqa_generic_kernel(GqaArgs p) 
     for (int kk = 0; kk < KK; kk++) kf[kk] = load8<TKV>(krow + 32 * kk + 8 * c);
 #pragma unroll
     for (int t = 0; t < DT; t++) {
-      if constexpr (V_SLAB) {
-        const _Float16 *vp = reinterpret_cast<const _Float16 *>(vbase) + ((size_t)((p0 + 4 * c) >> 3) * HD + 16 * t + r) * 8 + ((4 * c) & 7);
-        vf[t] = *reinterpret_cast<const half4_t *>(vp);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int pos = min(p0 + 4 * c + e, Sk - 1);
-          vf[t][e] = (_Float16)vbase[(size_t)pos * p.v_s + 16 * t + r];
-        }
-      }
+      const _Float16 *vp = vbase + ((size_t)((p0 + 4 * c) >> 3) * HD + 16 * t + r) * 8 + ((4 * c) & 7);
+      vf[t] = *reinterpret_cast<const half4_t *>(vp);
     }
   };
   half8_t kf[KK], kn[KK];
@@ -279,134 +272,12 @@ __global__ void __launch_bounds__(64 * GQA_WAVES) gqa_generic_kernel(GqaArgs p) 
   }
 }
 
-// Many query positions (prompt pass, or the operator with a long seq_q): a wave owns 32 consecutive queries of one
-// head and walks every key block itself -- each K / V load then feeds two query tiles, and nothing is merged at the
-// end.  A workgroup's four waves take neighbouring query ranges of the same head, so their K / V requests meet in
-// the CU's cache.  Same arithmetic per (query, position) as gqa_generic_kernel.
-template <int HD, typename TQ, typename TKV, typename TO, bool V_SLAB>
-__global__ void __launch_bounds__(64 * GQA_WAVES) gqa_rows_kernel(GqaArgs p) {
-  static_assert(HD % 32 == 0 && HD >= 32 && HD <= 128, "head width");
-  constexpr int KK = HD / 32, DT = HD / 16, QT = 2;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r = lane & 15, c = lane >> 4;
-  // late query ranges see the most keys: they are dispatched first, so that the grid does not end on its longest workgroups
-  const int q0 = (((int)gridDim.x - 1 - (int)blockIdx.x) * GQA_WAVES + wave) * 16 * QT, h = blockIdx.y, b = blockIdx.z;
-  if (q0 >= p.Sq) return;  // no barrier in this kernel
-  const int kvh = h / (p.Hq / p.Hkv);
-  const int Sk = p.Sk;
-  int qi[QT], lim_q[QT];
-  half8_t qf[QT][KK];
-#pragma unroll
-  for (int u = 0; u < QT; u++) {
-    qi[u] = min(q0 + 16 * u + r, p.Sq - 1);
-    lim_q[u] = p.causal_base < 0 ? Sk - 1 : min(Sk - 1, p.causal_base + qi[u]);
-    const TQ *qrow = static_cast<const TQ *>(p.q) + (size_t)b * p.q_b + (size_t)qi[u] * p.q_s + (size_t)h * HD;
-#pragma unroll
-    for (int kk = 0; kk < KK; kk++) qf[u][kk] = load8<TQ>(qrow + 32 * kk + 8 * c);
-  }
-  const int lim_wave = p.causal_base < 0 ? Sk - 1 : min(Sk - 1, p.causal_base + min(q0 + 16 * QT - 1, p.Sq - 1));
-  const int nblocks = lim_wave / 16 + 1;
-  const TKV *kbase = static_cast<const TKV *>(p.k) + (size_t)b * p.k_b + (size_t)kvh * p.k_h;
-  const TKV *vbase = static_cast<const TKV *>(p.v) + (size_t)b * p.v_b + (size_t)kvh * p.v_h;
-  float m_run[QT], l_run[QT];
-  float4_t o_acc[QT][DT];
-#pragma unroll
-  for (int u = 0; u < QT; u++) {
-    m_run[u] = -INFINITY;
-    l_run[u] = 0.0f;
-#pragma unroll
-    for (int t = 0; t < DT; t++) o_acc[u][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  }
-  auto load_block = [&](int blk, half8_t (&kf)[KK], half4_t (&vf)[DT]) {
-    const int p0 = blk * 16;
-    const TKV *krow = kbase + (size_t)min(p0 + r, Sk - 1) * p.k_s;
-#pragma unroll
-    for (int kk = 0; kk < KK; kk++) kf[kk] = load8<TKV>(krow + 32 * kk + 8 * c);
-#pragma unroll
-    for (int t = 0; t < DT; t++) {
-      if constexpr (V_SLAB) {
-        const _Float16 *vp = reinterpret_cast<const _Float16 *>(vbase) + ((size_t)((p0 + 4 * c) >> 3) * HD + 16 * t + r) * 8 + ((4 * c) & 7);
-        vf[t] = *reinterpret_cast<const half4_t *>(vp);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int pos = min(p0 + 4 * c + e, Sk - 1);
-          vf[t][e] = (_Float16)vbase[(size_t)pos * p.v_s + 16 * t + r];
-        }
-      }
-    }
-  };
-  half8_t kf[KK], kn[KK];
-  half4_t vf[DT], vn[DT];
-  load_block(0, kf, vf);
-  for (int blk = 0; blk < nblocks; blk++) {
-    const int p0 = blk * 16;
-    const bool more = blk + 1 < nblocks;
-    if (more) load_block(blk + 1, kn, vn);
-    half4_t vv[DT];
-#pragma unroll
-    for (int t = 0; t < DT; t++) {
-      vv[t] = vf[t];
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-        if (p0 + 4 * c + e >= Sk) vv[t][e] = (_Float16)0.0f;  // 0 * NaN would poison the sum
-    }
-#pragma unroll
-    for (int u = 0; u < QT; u++) {
-      float4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int kk = 0; kk < KK; kk++) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[kk], qf[u][kk], s, 0, 0, 0);
-      float sv[4], mx = -INFINITY;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        sv[e] = (p0 + 4 * c + e <= lim_q[u]) ? s[e] * p.scale : -INFINITY;
-        mx = fmaxf(mx, sv[e]);
-      }
-      mx = max_xor16_xor32(mx);
-      const float m_new = fmaxf(m_run[u], mx);
-      float pe[4], sum = 0.0f;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        pe[e] = (sv[e] == -INFINITY) ? 0.0f : __expf(sv[e] - m_new);
-        sum += pe[e];
-      }
-      sum = sum_xor16_xor32(sum);
-      const float alpha = (m_run[u] == -INFINITY) ? 0.0f : __expf(m_run[u] - m_new);
-      l_run[u] = l_run[u] * alpha + sum;
-      m_run[u] = m_new;
-      const half4_t pf = {(_Float16)pe[0], (_Float16)pe[1], (_Float16)pe[2], (_Float16)pe[3]};
-#pragma unroll
-      for (int t = 0; t < DT; t++) {
-        o_acc[u][t] = o_acc[u][t] * alpha;
-        o_acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(vv[t], pf, o_acc[u][t], 0, 0, 0);
-      }
-    }
-    if (more) {
-#pragma unroll
-      for (int kk = 0; kk < KK; kk++) kf[kk] = kn[kk];
-#pragma unroll
-      for (int t = 0; t < DT; t++) vf[t] = vn[t];
-    }
-  }
-  // lane (r, c) holds O^T[16 t + 4c + e][query r] of each query tile: four consecutive channels per store
-  TO *obase = static_cast<TO *>(p.out) + (size_t)b * p.o_b + (size_t)h * HD;
-#pragma unroll
-  for (int u = 0; u < QT; u++) {
-    if (q0 + 16 * u + r >= p.Sq) continue;
-    const float inv = l_run[u] > 0.0f ? 1.0f / l_run[u] : 0.0f;
-    TO *orow = obase + (size_t)(q0 + 16 * u + r) * p.o_s;
-#pragma unroll
-    for (int t = 0; t < DT; t++)
-      store4<TO>(orow + 16 * t + 4 * c, o_acc[u][t][0] * inv, o_acc[u][t][1] * inv, o_acc[u][t][2] * inv, o_acc[u][t][3] * inv);
-  }
-}
-
 // Prompt pass over the decoder's fp16 cache: the four waves of a workgroup take the same key range -- query heads
 // that share a kv head (as many of them as divide four), else neighbouring 32-query ranges of one head -- so a
 // stage of 32 cache positions is fetched once per workgroup into LDS (K rows with their 16-byte pieces XOR-swizzled
 // so that the 16 rows a fragment read touches fall into 16 different bank groups; V as its slabs lie in memory) and
-// read from there by all four: a quarter of the L2 traffic of gqa_rows_kernel, which is what bounds that kernel at
-// prompt lengths in the thousands.  Two stage buffers: the next stage's pieces are requested into registers before
+// read from there by all four: a quarter of the L2 traffic of waves that fetch for themselves, which bounds such a
+// kernel at prompt lengths in the thousands.  Two stage buffers: the next stage's pieces are requested into registers before
 // this stage's arithmetic and written to the other buffer behind it, one barrier per stage.  Arithmetic per
 // (query, position) as in gqa_generic_kernel; the running output is rescaled only where some query's maximum moved
 // (a factor of exactly one otherwise).
@@ -614,27 +485,14 @@ int32_t gqa_launch_shared_kv(const GqaArgs &a, int hd, hipStream_t s) {
   return YSCV_HIP_OK;
 }
 
-template <typename TQ, typename TKV, typename TO, bool V_SLAB>
-int32_t gqa_launch(const GqaArgs &a, int hd, hipStream_t s) {
-  // many queries and a host-known context: one wave per 32 queries, no split over the keys
-  if (a.Sq >= 64 && a.sk_minus_1 == nullptr) {
-    const dim3 grid((unsigned)((a.Sq + 32 * GQA_WAVES - 1) / (32 * GQA_WAVES)), (unsigned)a.Hq, (unsigned)a.B), block(64 * GQA_WAVES);
-    switch (hd) {
-      case 32: hipLaunchKernelGGL((gqa_rows_kernel<32, TQ, TKV, TO, V_SLAB>), grid, block, 0, s, a); break;
-      case 64: hipLaunchKernelGGL((gqa_rows_kernel<64, TQ, TKV, TO, V_SLAB>), grid, block, 0, s, a); break;
-      case 96: hipLaunchKernelGGL((gqa_rows_kernel<96, TQ, TKV, TO, V_SLAB>), grid, block, 0, s, a); break;
-      case 128: hipLaunchKernelGGL((gqa_rows_kernel<128, TQ, TKV, TO, V_SLAB>), grid, block, 0, s, a); break;
-      default: return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention: head width %d (supported: 32, 64, 96, 128)", hd);
-    }
-    YSCV_HIP_TRY(hipGetLastError());
-    return YSCV_HIP_OK;
-  }
+// few query rows against the decoder's cache
+int32_t gqa_launch_cache(const GqaArgs &a, int hd, hipStream_t s) {
   const dim3 grid((unsigned)((a.Sq + 15) / 16), (unsigned)a.Hq, (unsigned)a.B), block(64 * GQA_WAVES);
   switch (hd) {
-    case 32: hipLaunchKernelGGL((gqa_generic_kernel<32, TQ, TKV, TO, V_SLAB>), grid, block, 0, s, a); break;
-    case 64: hipLaunchKernelGGL((gqa_generic_kernel<64, TQ, TKV, TO, V_SLAB>), grid, block, 0, s, a); break;
-    case 96: hipLaunchKernelGGL((gqa_generic_kernel<96, TQ, TKV, TO, V_SLAB>), grid, block, 0, s, a); break;
-    case 128: hipLaunchKernelGGL((gqa_generic_kernel<128, TQ, TKV, TO, V_SLAB>), grid, block, 0, s, a); break;
+    case 32: hipLaunchKernelGGL((gqa_generic_kernel<32>), grid, block, 0, s, a); break;
+    case 64: hipLaunchKernelGGL((gqa_generic_kernel<64>), grid, block, 0, s, a); break;
+    case 96: hipLaunchKernelGGL((gqa_generic_kernel<96>), grid, block, 0, s, a); break;
+    case 128: hipLaunchKernelGGL((gqa_generic_kernel<128>), grid, block, 0, s, a); break;
     default: return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention: head width %d (supported: 32, 64, 96, 128)", hd);
   }
   YSCV_HIP_TRY(hipGetLastError());
@@ -645,13 +503,420 @@ int32_t gqa_launch(const GqaArgs &a, int hd, hipStream_t s) {
 int32_t gqa_launch_fused_decode(const GqaArgs &a, int hd, hipStream_t s) {
   const dim3 grid(1, (unsigned)a.Hq, (unsigned)a.B), block(64 * GQA_WAVES);
   switch (hd) {
-    case 32: hipLaunchKernelGGL((gqa_generic_kernel<32, _Float16, _Float16, _Float16, true, true>), grid, block, 0, s, a); break;
-    case 64: hipLaunchKernelGGL((gqa_generic_kernel<64, _Float16, _Float16, _Float16, true, true>), grid, block, 0, s, a); break;
-    case 96: hipLaunchKernelGGL((gqa_generic_kernel<96, _Float16, _Float16, _Float16, true, true>), grid, block, 0, s, a); break;
-    case 128: hipLaunchKernelGGL((gqa_generic_kernel<128, _Float16, _Float16, _Float16, true, true>), grid, block, 0, s, a); break;
+    case 32: hipLaunchKernelGGL((gqa_generic_kernel<32, true>), grid, block, 0, s, a); break;
+    case 64: hipLaunchKernelGGL((gqa_generic_kernel<64, true>), grid, block, 0, s, a); break;
+    case 96: hipLaunchKernelGGL((gqa_generic_kernel<96, true>), grid, block, 0, s, a); break;
+    case 128: hipLaunchKernelGGL((gqa_generic_kernel<128, true>), grid, block, 0, s, a); break;
     default: return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention: head width %d (supported: 32, 64, 96, 128)", hd);
   }
   YSCV_HIP_TRY(hipGetLastError());
+  return YSCV_HIP_OK;
+}
+
+// ---- the GroupQueryAttention operator --------------------------------------------------------------------------------
+// The GroupQueryAttention operator on f32 tensors (no mask).  The `group` query heads of a kv head and the query
+// positions together are the rows of one problem per (sequence, kv head): R = group * Sq rows against Sk keys, so a
+// single decode position of four heads fills one row tile instead of four.  A workgroup of eight waves is RW row waves
+// (16 QT rows each) times KS = 8 / RW key groups; a key group streams its stages of KB keys through LDS, converted to
+// fp16 on the way in and V transposed into slabs of eight positions per channel, where all its row waves read them.
+// What bounds it is the f32 K / V every workgroup has to take in (512 KB for 512 keys of 128 channels, 115 GB/s per CU
+// from L2), so a workgroup gets as many rows as still leave one workgroup per CU, the waves left over split the keys
+// and are merged through LDS, and where even that leaves CUs idle (decode: 8 workgroups) the keys are split over the
+// grid too, with the partial results merged by a second kernel.  512 queries x 512 keys, 32 heads over 8 of 128: 21 us,
+// against 88 for the kernel before (one wave per 32 rows of one head, V gathered by single values); one query x 2048
+// keys: 9.5 + 5.7 us against 70.  Of the 21 us, 5 pass before the first stage is in LDS, 12 are four rounds of stages
+// (2 048 cycles each for the f32 K / V alone at 64 bytes per cycle and CU), 3 the merge and the stores.
+// QT: row tiles per wave; RW 1 is the form for few rows (wave-private stages: no barrier in the loop).
+template <int HD, int RW, int QT>
+struct FlatCfg {
+  static constexpr int KS = 8 / RW, T = 64 * RW;        // key groups, threads of one
+  static constexpr int KB = RW <= 2 ? 32 : 16 * RW;     // keys per stage: the same registers per thread whatever RW
+  static constexpr int NBUF = RW == 1 ? 1 : 2;
+  static constexpr int PITCH = HD > 64 ? 16 : (HD > 32 ? 8 : 4);  // K row pitch in 16-byte pieces
+  static constexpr int K_BYTES = KB * PITCH * 16, V_BYTES = (KB / 8) * HD * 16, ST_BYTES = K_BYTES + V_BYTES;
+  static constexpr int ROWS = RW * 16 * QT;
+  static constexpr int OP = HD + 4;                      // floats per row of the merge buffer
+  static constexpr int MERGE_BYTES = KS > 1 ? KS * ROWS * (OP + 2) * 4 : 0;
+  static constexpr int LDS = KS * NBUF * ST_BYTES > MERGE_BYTES ? KS * NBUF * ST_BYTES : MERGE_BYTES;
+};
+
+struct FlatArgs {
+  const float *q, *k, *v;
+  float *out, *part;       // part: [b * Hkv][gs][R][HD + 2] when gs > 1 (un-normalised output, maximum, sum)
+  int Sq, Sk, Hq, Hkv, group, R, gs;
+  int v16;                 // v is 16-byte aligned
+  uint32_t magic;          // ceil(2^32 / group): row / group = the high half of row * magic (0: divide)
+  float scale;             // log2(e) / sqrt(head width)
+};
+
+template <int HD, int RW, int QT>
+__global__ void __launch_bounds__(512) gqa_flat_kernel(FlatArgs p) {
+  using C = FlatCfg<HD, RW, QT>;
+  constexpr int KK = HD / 32, DT = HD / 16, KB = C::KB, PITCH = C::PITCH, RPW = 16 / PITCH, CPR = HD / 8, T = C::T, KS = C::KS;
+  constexpr int K_PIECES = KB * CPR, V_UNITS = (KB / 8) * (HD / 4);  // V unit: eight positions x four channels
+  constexpr int K_LD = (K_PIECES + T - 1) / T, V_LD = (V_UNITS + T - 1) / T;
+  extern __shared__ __attribute__((aligned(16))) uint8_t flat_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, c = lane >> 4;
+  const int kg = wave / RW, rw = wave % RW, gt = tid - kg * T;  // key group, row wave, thread of the group
+  // kv heads are the fast grid dimension: with eight of them the workgroups of one share an XCD, and its L2 holds one head
+  const int nb = blockIdx.x, b = nb / p.Hkv, kvh = nb % p.Hkv, gs = blockIdx.z;
+  const int row0 = (int)blockIdx.y * C::ROWS + rw * 16 * QT;
+  uint8_t *lds = flat_lds + kg * C::NBUF * C::ST_BYTES;
+  const size_t q_s = (size_t)p.Hq * HD, kv_s = (size_t)p.Hkv * HD;
+  const float *kbase = p.k + (size_t)b * p.Sk * kv_s + (size_t)kvh * HD;
+  const float *vbase = p.v + (size_t)b * p.Sk * kv_s + (size_t)kvh * HD;
+  const int stages = (p.Sk + KB - 1) / KB, st_lo = (int)((long long)stages * gs / p.gs), st_hi = (int)((long long)stages * (gs + 1) / p.gs);
+  const int iters = (st_hi - st_lo + KS - 1) / KS;
+
+  // where row `row` of this problem starts in q and out
+  auto row_offset = [&](int row) {
+    const int qpos = p.magic ? (int)__umulhi((uint32_t)row, p.magic) : row / p.group;
+    return ((size_t)b * p.Sq + qpos) * q_s + (size_t)(kvh * p.group + row - qpos * p.group) * HD;
+  };
+  float4_t kr[K_LD][2], vr[V_LD][8];
+  // A stage's base is wave-uniform and a lane's byte offsets inside a whole stage are the same for every stage: 32 bits
+  // each, worked out once.  In the last stage rows past the end repeat the last key (their positions are masked).
+  const uint32_t ks = (uint32_t)kv_s * 4u;  // bytes from one key to the next
+  uint32_t koff[K_LD], voff[V_LD];
+#pragma unroll
+  for (int j = 0; j < K_LD; j++) koff[j] = (uint32_t)(gt + T * j) / CPR * ks + (uint32_t)(gt + T * j) % CPR * 32u;
+#pragma unroll
+  for (int j = 0; j < V_LD; j++) voff[j] = (uint32_t)(gt + T * j) / (HD / 4) * 8u * ks + (uint32_t)(gt + T * j) % (HD / 4) * 16u;
+  auto fetch = [&](int st) {
+    const char *kst = reinterpret_cast<const char *>(kbase) + (size_t)st * KB * ks, *vst = reinterpret_cast<const char *>(vbase) + (size_t)st * KB * ks;
+    if (p.v16 && (st + 1) * KB <= p.Sk) {  // uniform
+      // (opaque to the optimiser, or it hoists base + offset out of the loop as 64-bit addresses per lane and load)
+#pragma unroll
+      for (int j = 0; j < K_LD; j++) asm volatile("" : "+v"(koff[j]));
+#pragma unroll
+      for (int j = 0; j < V_LD; j++) asm volatile("" : "+v"(voff[j]));
+#pragma unroll
+      for (int j = 0; j < K_LD; j++) {
+        if (K_PIECES % T == 0 || gt + T * j < K_PIECES) {
+          kr[j][0] = *reinterpret_cast<const float4_t *>(kst + koff[j]);
+          kr[j][1] = *reinterpret_cast<const float4_t *>(kst + 16 + koff[j]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < V_LD; j++) {
+        if (V_UNITS % T == 0 || gt + T * j < V_UNITS) {
+#pragma unroll
+          for (int e = 0; e < 8; e++) vr[j][e] = *reinterpret_cast<const float4_t *>(vst + e * ks + voff[j]);
+        }
+      }
+      return;
+    }
+    const uint32_t last = (uint32_t)min(KB, p.Sk - st * KB) - 1u;
+#pragma unroll
+    for (int j = 0; j < K_LD; j++) {
+      const uint32_t idx = (uint32_t)(gt + T * j);
+      if (K_PIECES % T == 0 || idx < (uint32_t)K_PIECES) {
+        const char *src = kst + (min(idx / CPR, last) * ks + idx % CPR * 32u);
+        kr[j][0] = *reinterpret_cast<const float4_t *>(src);
+        kr[j][1] = *reinterpret_cast<const float4_t *>(src + 16);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < V_LD; j++) {
+      const uint32_t idx = (uint32_t)(gt + T * j);
+      if (V_UNITS % T == 0 || idx < (uint32_t)V_UNITS) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const float *src = reinterpret_cast<const float *>(vst + (min(idx / (HD / 4) * 8 + e, last) * ks + idx % (HD / 4) * 16u));
+#pragma unroll
+          for (int u = 0; u < 4; u++) vr[j][e][u] = src[u];
+        }
+      }
+    }
+  };
+  auto stash = [&](int buf, int st) {
+    uint8_t *base = lds + buf * C::ST_BYTES;
+    const int left = p.Sk - st * KB;  // keys of the stage that exist; the V of the others is 0 (0 * inf would not be)
+#pragma unroll
+    for (int j = 0; j < K_LD; j++) {
+      const int idx = gt + T * j;
+      if (K_PIECES % T == 0 || idx < K_PIECES) {
+        const int row = idx / CPR, piece = idx % CPR;
+        half8_t h;
+#pragma unroll
+        for (int e = 0; e < 8; e++) h[e] = (_Float16)kr[j][e >> 2][e & 3];
+        *reinterpret_cast<half8_t *>(base + (row * PITCH + (piece ^ ((((row >> 3) & 3) * 4 + (row & 3)) / RPW))) * 16) = h;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < V_LD; j++) {
+      const int idx = gt + T * j;
+      if (V_UNITS % T == 0 || idx < V_UNITS) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          half8_t h;
+#pragma unroll
+          for (int e = 0; e < 8; e++) h[e] = (_Float16)vr[j][e][u];
+          if (left < KB) {  // uniform
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+              if (idx / (HD / 4) * 8 + e >= left) h[e] = (_Float16)0.0f;
+          }
+          *reinterpret_cast<half8_t *>(base + C::K_BYTES + (idx * 4 + u) * 16) = h;
+        }
+      }
+    }
+  };
+
+  int st = st_lo + kg;
+  const bool any = st < st_hi;
+  if (any) fetch(st);
+
+  half8_t qf[QT][KK];
+#pragma unroll
+  for (int u = 0; u < QT; u++) {
+    const int row = min(row0 + 16 * u + r, p.R - 1);  // rows past the end repeat the last one and are not stored
+    const float *qrow = p.q + row_offset(row);
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) qf[u][kk] = load8<float>(qrow + 32 * kk + 8 * c);
+  }
+  float m_run[QT], l_run[QT];
+  float4_t o_acc[QT][DT];
+#pragma unroll
+  for (int u = 0; u < QT; u++) {
+    m_run[u] = -INFINITY;
+    l_run[u] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < DT; t++) o_acc[u][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  const bool active = row0 < p.R;  // uniform in the wave
+
+  // 32 keys of a stage; layout and arithmetic as in gqa_shared_kv_kernel.  The scores of all row tiles come first and V
+  // is read behind them: K and V fragments together would not fit beside the next stage's loads in flight.
+  auto compute32 = [&](const uint8_t *base, int sub, int p0) {
+    half8_t pf[QT];
+    {
+      half8_t kf[2][KK];
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const int row = 8 * (r >> 2) + 4 * j + (r & 3);
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++)
+          kf[j][kk] = *reinterpret_cast<const half8_t *>(base + ((sub * 32 + row) * PITCH + ((4 * kk + c) ^ (r / RPW))) * 16);
+      }
+      const bool tail = p0 + 32 > p.Sk;  // uniform
+#pragma unroll
+      for (int u = 0; u < QT; u++) {
+        float4_t s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++) {
+          s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[0][kk], qf[u][kk], s0, 0, 0, 0);
+          s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[1][kk], qf[u][kk], s1, 0, 0, 0);
+        }
+        // softmax in powers of two: the scale (log2(e) in it) and the maximum go into one fma per score
+        float sv[8], mx = -INFINITY, pe[8], sum = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) sv[e] = e < 4 ? s0[e & 3] : s1[e & 3];
+        if (tail) {
+#pragma unroll
+          for (int e = 0; e < 8; e++)
+            if (p0 + 8 * c + e >= p.Sk) sv[e] = -INFINITY;  // (an existing key's scores repeated)
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) mx = fmaxf(mx, sv[e]);
+        const float m_new = fmaxf(m_run[u], max_xor16_xor32(mx) * p.scale);
+        const float m_sub = m_new == -INFINITY ? 0.0f : m_new;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          pe[e] = __builtin_amdgcn_exp2f(fmaf(sv[e], p.scale, -m_sub));
+          sum += pe[e];
+        }
+        sum = sum_xor16_xor32(sum);
+        const float alpha = __builtin_amdgcn_exp2f(m_run[u] - m_sub);
+        l_run[u] = l_run[u] * alpha + sum;
+        m_run[u] = m_new;
+        pf[u] = half8_t{(_Float16)pe[0], (_Float16)pe[1], (_Float16)pe[2], (_Float16)pe[3],
+                        (_Float16)pe[4], (_Float16)pe[5], (_Float16)pe[6], (_Float16)pe[7]};
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+          for (int t = 0; t < DT; t++) o_acc[u][t] = o_acc[u][t] * alpha;
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    half8_t vv[DT];
+#pragma unroll
+    for (int t = 0; t < DT; t++) vv[t] = *reinterpret_cast<const half8_t *>(base + C::K_BYTES + ((sub * 4 + c) * HD + 16 * t + r) * 16);
+#pragma unroll
+    for (int u = 0; u < QT; u++)
+#pragma unroll
+      for (int t = 0; t < DT; t++) o_acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[t], pf[u], o_acc[u][t], 0, 0, 0);
+  };
+  auto compute = [&](int stage_index, int buf) {
+    if (!active) return;
+#pragma unroll 1
+    for (int sub = 0; sub < KB / 32; sub++) {
+      const int p0 = stage_index * KB + sub * 32;
+      if (p0 < p.Sk) compute32(lds + buf * C::ST_BYTES, sub, p0);
+    }
+  };
+
+  if constexpr (RW == 1) {
+    // the wave's own stages: LDS serves a wave's accesses in order, only the compiler must keep that order
+    for (; st < st_hi; st += KS) {
+      stash(0, st);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (st + KS < st_hi) fetch(st + KS);
+      compute(st, 0);
+      asm volatile("" ::: "memory");
+    }
+  } else {
+    if (any) stash(0, st);
+    __syncthreads();
+    for (int it = 0; it < iters; it++, st += KS) {  // uniform in the workgroup
+      const bool more = st + KS < st_hi;
+      if (more) fetch(st + KS);
+      if (st < st_hi) compute(st, it & 1);
+      if (more) stash((it + 1) & 1, st + KS);
+      __syncthreads();
+    }
+  }
+
+  // lane (r, c) holds O^T[16 t + 4c + e][row r]
+  const size_t part_row0 = ((size_t)nb * p.gs + gs) * p.R;
+  if constexpr (KS == 1) {
+#pragma unroll
+    for (int u = 0; u < QT; u++) {
+      const int row = row0 + 16 * u + r;
+      if (row >= p.R) continue;
+      float *dst;
+      float f = 1.0f;
+      if (p.gs > 1) {
+        dst = p.part + (part_row0 + row) * (HD + 2);
+        if (c == 0) {
+          dst[HD] = m_run[u];
+          dst[HD + 1] = l_run[u];
+        }
+#pragma unroll
+        for (int t = 0; t < DT; t++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) dst[16 * t + 4 * c + e] = o_acc[u][t][e];
+        continue;
+      }
+      dst = p.out + row_offset(row);
+      f = l_run[u] > 0.0f ? 1.0f / l_run[u] : 0.0f;
+#pragma unroll
+      for (int t = 0; t < DT; t++) store4<float>(dst + 16 * t + 4 * c, o_acc[u][t][0] * f, o_acc[u][t][1] * f, o_acc[u][t][2] * f, o_acc[u][t][3] * f);
+    }
+  } else {
+    // merge the key groups through LDS (the stages are done with it)
+    __syncthreads();
+    float *o_s = reinterpret_cast<float *>(flat_lds);                       // [KS][ROWS][OP]
+    float *ml = o_s + KS * C::ROWS * C::OP;                                 // [KS][ROWS][2]
+#pragma unroll
+    for (int u = 0; u < QT; u++) {
+      const int lr = rw * 16 * QT + 16 * u + r;
+      float *dst = o_s + (kg * C::ROWS + lr) * C::OP;
+#pragma unroll
+      for (int t = 0; t < DT; t++) *reinterpret_cast<float4_t *>(dst + 16 * t + 4 * c) = o_acc[u][t];
+      if (c == 0) {
+        ml[(kg * C::ROWS + lr) * 2] = m_run[u];
+        ml[(kg * C::ROWS + lr) * 2 + 1] = l_run[u];
+      }
+    }
+    __syncthreads();
+    for (int idx = tid; idx < C::ROWS * (HD / 4); idx += 512) {
+      const int lr = idx / (HD / 4), d4 = idx % (HD / 4) * 4, row = (int)blockIdx.y * C::ROWS + lr;
+      if (row >= p.R) continue;
+      float M = -INFINITY, L = 0.0f;
+#pragma unroll
+      for (int g = 0; g < KS; g++) M = fmaxf(M, ml[(g * C::ROWS + lr) * 2]);
+      float4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int g = 0; g < KS; g++) {
+        const float mg = ml[(g * C::ROWS + lr) * 2];
+        const float f = mg == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mg - M);
+        L += ml[(g * C::ROWS + lr) * 2 + 1] * f;
+        o += *reinterpret_cast<const float4_t *>(o_s + (g * C::ROWS + lr) * C::OP + d4) * f;
+      }
+      if (p.gs > 1) {
+        float *dst = p.part + (part_row0 + row) * (HD + 2);
+        if (d4 == 0) {
+          dst[HD] = M;
+          dst[HD + 1] = L;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) dst[d4 + e] = o[e];
+        continue;
+      }
+      const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+      store4<float>(p.out + row_offset(row) + d4, o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv);
+    }
+  }
+}
+
+// merges the grid's key splits: one thread per (row, channel)
+__global__ void __launch_bounds__(256) gqa_flat_merge_kernel(FlatArgs p, int hd, int total_rows) {
+  const int idx = (int)(blockIdx.x * 256 + threadIdx.x), grow = idx / hd, ch = idx % hd;
+  if (grow >= total_rows) return;
+  const int nb = grow / p.R, row = grow % p.R;
+  const size_t step = (size_t)p.R * (hd + 2);
+  const float *src = p.part + ((size_t)nb * p.gs * p.R + row) * (hd + 2);
+  float M = -INFINITY, L = 0.0f, o = 0.0f;
+  for (int g = 0; g < p.gs; g++) M = fmaxf(M, src[g * step + hd]);
+  for (int g = 0; g < p.gs; g++) {
+    const float mg = src[g * step + hd];
+    const float f = mg == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mg - M);
+    L += src[g * step + hd + 1] * f;
+    o += src[g * step + ch] * f;
+  }
+  p.out[((size_t)(nb / p.Hkv) * p.Sq + row / p.group) * p.Hq * hd + (size_t)(nb % p.Hkv * p.group + row % p.group) * hd + ch] =
+      L > 0.0f ? o / L : 0.0f;
+}
+
+template <int HD, int RW, int QT>
+int32_t gqa_flat_go(const FlatArgs &p, int nbs, hipStream_t s) {
+  using C = FlatCfg<HD, RW, QT>;
+  static std::once_flag once;
+  static hipError_t attr_err = hipSuccess;
+  std::call_once(once, [] {
+    attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(gqa_flat_kernel<HD, RW, QT>), hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+  });
+  YSCV_HIP_TRY(attr_err);
+  hipLaunchKernelGGL((gqa_flat_kernel<HD, RW, QT>), dim3((unsigned)nbs, (unsigned)((p.R + C::ROWS - 1) / C::ROWS), (unsigned)p.gs), dim3(512),
+                     C::LDS, s, p);
+  YSCV_HIP_TRY(hipGetLastError());
+  return YSCV_HIP_OK;
+}
+
+template <int HD>
+int32_t gqa_flat_launch(FlatArgs p, int B, int num_cus, hipStream_t s) {
+  const int nbs = B * p.Hkv;
+  // Rows per workgroup: the most that still give every CU a workgroup (K / V are taken in once per workgroup); 16 rows
+  // and a split of the keys over the grid where no choice does.
+  auto wgs = [&](int rows) { return nbs * ((p.R + rows - 1) / rows); };
+  const int rw = wgs(256) >= num_cus ? 8 : (wgs(128) >= num_cus ? 4 : (wgs(64) >= num_cus ? 2 : 1));
+  p.gs = 1;
+  Scratch part;
+  if (rw == 1) {
+    // a split pays where it takes whole rounds of stages off the longest workgroup (a stage: about 1 us; the second
+    // kernel about 4): at least two rounds of the eight key groups each
+    const int rounds = (p.Sk + 32 * 8 - 1) / (32 * 8), room = num_cus / wgs(16);
+    int gs = rounds < room ? rounds : room;
+    if (gs >= 2 && rounds >= 2) {
+      if (gs > 64) gs = 64;
+      p.gs = gs;
+      YSCV_TRY(part.take((size_t)nbs * gs * p.R * (HD + 2) * sizeof(float), s));
+      p.part = part.as<float>();
+    }
+  }
+  switch (rw) {
+    case 8: YSCV_TRY((gqa_flat_go<HD, 8, 2>(p, nbs, s))); break;
+    case 4: YSCV_TRY((gqa_flat_go<HD, 4, 2>(p, nbs, s))); break;
+    case 2: YSCV_TRY((gqa_flat_go<HD, 2, 2>(p, nbs, s))); break;
+    default: YSCV_TRY((gqa_flat_go<HD, 1, 1>(p, nbs, s))); break;
+  }
+  if (p.gs > 1) {
+    const size_t total = (size_t)nbs * p.R * HD;
+    hipLaunchKernelGGL(gqa_flat_merge_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p, HD, nbs * p.R);
+    YSCV_HIP_TRY(hipGetLastError());
+  }
   return YSCV_HIP_OK;
 }
 
@@ -661,15 +926,39 @@ __global__ void __launch_bounds__(256) rms_norm_f32_kernel(const float *__restri
   __shared__ float red[4];
   const float *row = x + (size_t)blockIdx.x * d;
   float *out = y + (size_t)blockIdx.x * d;
+  // HBM-bound: the row stays in registers between its two uses (up to KEEP x 1024 values, sixteen bytes per lane and
+  // load); longer, odd or unaligned rows are read twice
+  constexpr int KEEP = 8;
+  const bool vec = (d & 3) == 0 && d <= KEEP * 1024 &&
+                   ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(gamma)) & 15) == 0;
+  float4_t v[KEEP];
   float ss = 0.0f;
-  for (int i = threadIdx.x; i < d; i += 256) ss += row[i] * row[i];
+  if (vec) {
+#pragma unroll
+    for (int j = 0; j < KEEP; j++) {
+      const int i = (j * 256 + (int)threadIdx.x) * 4;
+      v[j] = i < d ? *reinterpret_cast<const float4_t *>(row + i) : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int j = 0; j < KEEP; j++) ss += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
+  } else {
+    for (int i = threadIdx.x; i < d; i += 256) ss += row[i] * row[i];
+  }
   ss = wave_sum(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
   ss = red[0] + red[1] + red[2] + red[3];
   // rms = sqrt(sum / n + eps); inv_rms = 1 / rms; y = x * inv_rms * gamma (ops/norm.rs:1507-1516, in that order)
   const float inv_rms = 1.0f / sqrtf(ss / (float)d + eps);
-  for (int i = threadIdx.x; i < d; i += 256) out[i] = row[i] * inv_rms * gamma[i];
+  if (vec) {
+#pragma unroll
+    for (int j = 0; j < KEEP; j++) {
+      const int i = (j * 256 + (int)threadIdx.x) * 4;
+      if (i < d) *reinterpret_cast<float4_t *>(out + i) = v[j] * inv_rms * *reinterpret_cast<const float4_t *>(gamma + i);
+    }
+  } else {
+    for (int i = threadIdx.x; i < d; i += 256) out[i] = row[i] * inv_rms * gamma[i];
+  }
 }
 
 // ---- rotate-half RoPE in place on [seq][heads][d] f32 ------------------------------------------------------------
@@ -833,7 +1122,7 @@ int32_t launch_gqa_cache(const _Float16 *qkv, const _Float16 *kc, const _Float16
   // prompt mode with enough rows: the kernel that stages K / V in LDS for four waves (its K rows must be contiguous
   // 16-byte pieces, which the cache's are)
   if (!pos_ptr && rows >= 64 && (max_ctx & 7) == 0) return gqa_launch_shared_kv(a, hd, s);
-  return gqa_launch<_Float16, _Float16, _Float16, true>(a, hd, s);
+  return gqa_launch_cache(a, hd, s);
 }
 
 extern "C" {
@@ -883,30 +1172,33 @@ int32_t yscv_hip_gqa_attention_dev(const float *q, const float *k, const float *
                "GroupQueryAttention: tensors must be 16-byte aligned");
   if (batch == 0 || seq_q == 0) return YSCV_HIP_OK;
   YSCV_REQUIRE(seq_k > 0, "GroupQueryAttention: no key positions");
-  GqaArgs a{};
-  a.q = q;
-  a.k = k;
-  a.v = v;
-  a.out = out;
-  a.q_s = (long long)(num_q_heads * d_head);
-  a.q_b = (long long)seq_q * a.q_s;
-  a.k_s = (long long)(num_kv_heads * d_head);
-  a.k_b = (long long)seq_k * a.k_s;
-  a.k_h = (long long)d_head;
-  a.v_s = a.k_s;
-  a.v_b = a.k_b;
-  a.v_h = a.k_h;
-  a.o_s = a.q_s;
-  a.o_b = a.q_b;
-  a.B = (int)batch;
-  a.Sq = (int)seq_q;
-  a.Sk = (int)seq_k;
-  a.Hq = (int)num_q_heads;
-  a.Hkv = (int)num_kv_heads;
-  a.causal_base = -1;
-  a.sk_minus_1 = nullptr;
-  a.scale = 1.0f / sqrtf((float)d_head);
-  return gqa_launch<float, float, float, false>(a, (int)d_head, as_stream(stream));
+  const Context *ctx = nullptr;
+  YSCV_TRY(ensure_context(&ctx));
+  FlatArgs p{};
+  p.q = q;
+  p.k = k;
+  p.v = v;
+  p.out = out;
+  p.Sq = (int)seq_q;
+  p.Sk = (int)seq_k;
+  p.Hq = (int)num_q_heads;
+  p.Hkv = (int)num_kv_heads;
+  p.group = (int)(num_q_heads / num_kv_heads);
+  p.v16 = (reinterpret_cast<uintptr_t>(v) & 15) == 0;
+  p.scale = 1.44269504f / sqrtf((float)d_head);
+  // exact while row * group < 2^32
+  p.magic = p.group > 1 && p.group <= 256 ? (uint32_t)((((uint64_t)1 << 32) + p.group - 1) / p.group) : 0;
+  const uint64_t rows = (uint64_t)p.group * seq_q;
+  YSCV_REQUIRE(rows <= (uint64_t)65535 * 256 && batch * num_kv_heads < ((uint64_t)1 << 31) && batch * num_q_heads * seq_q * d_head < ((uint64_t)1 << 38),
+               "GroupQueryAttention: shape too large");
+  p.R = (int)rows;
+  switch (d_head) {
+    case 32: return gqa_flat_launch<32>(p, (int)batch, ctx->num_cus, as_stream(stream));
+    case 64: return gqa_flat_launch<64>(p, (int)batch, ctx->num_cus, as_stream(stream));
+    case 96: return gqa_flat_launch<96>(p, (int)batch, ctx->num_cus, as_stream(stream));
+    case 128: return gqa_flat_launch<128>(p, (int)batch, ctx->num_cus, as_stream(stream));
+    default: return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention: head width %zu (supported: 32, 64, 96, 128)", d_head);
+  }
 }
 
 }  // extern "C"
