@@ -1,4 +1,5 @@
 // C ABI of the yscv_hip library (declarations and contracts: include/yscv_hip.h).
+#include <algorithm>
 #include <vector>
 
 #include "int4_common.hpp"
@@ -86,48 +87,63 @@ static bool valid_act_dtype(int d) { return d == YSCV_HIP_F32 || d == YSCV_HIP_F
 static size_t dtype_size(int d) { return d == YSCV_HIP_F32 ? 4 : 2; }
 
 // Scratch layout of one int4 call: [xh][xl][row_scale][partial], each part rounded to 256 B.
-// A fp16 activation whose row stride already equals the padded K needs no preparation at all, and neither does an
-// f32 or bf16 one on its way to the skinny kernel, which normalises (and for f32 splits) it on the fly.
+// Activations on 16-byte alignment need no preparation on their way to the skinny kernel (which normalises f32 and bf16,
+// and splits f32, on the fly), nor as fp16 to the GEMMs with fp16-prepared activations, which end their k loop with the
+// data.  The exact-scale GEMM takes rows padded to whole 512-k slices.
 struct Int4Scratch {
   bool direct;       // x is used in place as the fp16 `hi` operand
   bool skinny;
+  bool fast16;       // above 16 rows: one fp16 operand (int4_ksplit.hip / int4_gemm_ring.hip), else the exact-scale GEMM
   int split;
-  size_t k_pad;
+  size_t ldx;        // row stride of the activations the kernel reads
   SkinnyPlan plan;
   size_t xh_bytes, rs_bytes, part_bytes, total;
-  size_t opt_bytes;  // behind `total`: the K-split partials of the LDS-ring GEMM (0 when that launch is not split)
+  size_t opt_bytes;  // behind `total`: partial sums of a K split above 16 rows (0 when that launch is not split)
 };
 
 // f32 activations on the exact-scale route with 16 < m <= this many rows run as 16-row skinny calls
 constexpr size_t kChunkedSkinnyMaxRows = 128;
 
-static Int4Scratch int4_scratch_layout(const yscv_hip_int4_weight *w, const void *x, int x_dtype, size_t m,
-                                       int force, int num_cus) {
+// y == null asks for the size of a workspace: activations of a K that is no multiple of 512 may then come on any alignment
+static Int4Scratch int4_scratch_layout(const yscv_hip_int4_weight *w, const void *x, int x_dtype, const void *y, int y_dtype,
+                                       size_t m, int force, int num_cus) {
   Int4Scratch L{};
   L.skinny = force == 1 || (force == 0 && m <= 16);
-  L.k_pad = w->ktp * 128;
-  L.direct = (x_dtype == YSCV_HIP_F16 || L.skinny) && L.k_pad == w->k &&
-             (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-  L.split = x_dtype == YSCV_HIP_F32 ? 2 : 1;
+  const size_t k_pad = w->ktp * 128;
+  const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (y != nullptr || k_pad == w->k);
+  // f32 activations with more than 16 rows against a weight whose scales are stored as fp16 (the MatMulNBits form) go
+  // as ONE fp16 operand: those kernels fold the group scale into fp16 weights (2^-11 relative per weight), which a lo
+  // half of the activations could not refine, and are 3.5x (prefill shapes) to 14x (few rows, wide N) faster than the
+  // exact-scale kernel.  Weights with f32 scales -- what packed_int4_gemm_dispatch hands over -- keep the exact-scale
+  // kernel with hi + lo activations: the reference's own test holds that entry point to 1e-3 absolute
+  // (int4_matmul.rs:816-855).
+  L.fast16 = !L.skinny && m > 16 && (x_dtype != YSCV_HIP_F32 || w->scale_dtype == YSCV_HIP_F16) && y != nullptr &&
+             int4_gemm_ring_eligible(w, reinterpret_cast<const _Float16 *>(uintptr_t(256)), y, y_dtype, 1, m, round_up(w->k, 64));
+  L.split = x_dtype == YSCV_HIP_F32 && !L.fast16 ? 2 : 1;
+  if (L.skinny || L.fast16) {
+    const bool any_k = L.skinny || w->k % 64 == 0 || int4_ksplit_takes(w, m, num_cus);  // (the LDS-ring GEMM's stages are 64 k)
+    // (the skinny kernel's form for more than four f32 rows reads its 512-k slices whole)
+    L.direct = aligned && any_k && (x_dtype == YSCV_HIP_F16 || (L.skinny && (x_dtype == YSCV_HIP_BF16 || m <= 4 || k_pad == w->k)));
+    L.ldx = L.direct ? w->k : (L.fast16 ? round_up(w->k, 64) : k_pad);
+  } else {
+    L.direct = aligned && x_dtype == YSCV_HIP_F16 && k_pad == w->k;
+    L.ldx = k_pad;
+  }
   if (L.skinny) L.plan = plan_int4_skinny(w, m, L.split, num_cus);
-  L.xh_bytes = L.direct ? 0 : round_up(m * L.k_pad * sizeof(_Float16), 256);
+  L.xh_bytes = L.direct ? 0 : round_up(m * L.ldx * sizeof(_Float16), 256);
   L.rs_bytes = L.direct ? 0 : round_up(m * sizeof(float), 256);
   L.part_bytes = L.skinny ? round_up(L.plan.partial_bytes, 256) : 0;
   L.total = L.xh_bytes * L.split + L.rs_bytes + L.part_bytes;
-  // partial sums of whichever kernel takes the rows above 16: the register-resident one up to 32 rows where its
-  // parts fit the cap, else the LDS-ring GEMM's K split
-  if (L.skinny) {
-    L.opt_bytes = 0;
-  } else if (m <= 32 && int4_mid_partial_bytes(w, m) <= kMidPartialCap) {
-    const size_t ring = int4_gemm_ring_partial_bytes(w, m, num_cus);  // the ring takes over if the mid kernel cannot (alignment)
-    const size_t mid = int4_mid_partial_bytes(w, m);
-    L.opt_bytes = round_up(mid > ring ? mid : ring, 256);
-  } else {
-    L.opt_bytes = round_up(int4_gemm_ring_partial_bytes(w, m, num_cus), 256);
+  if (!L.skinny) {
+    // whichever kernel takes the rows above 16; the LDS-ring GEMM takes over where the other one cannot
+    size_t opt = int4_gemm_ring_partial_bytes(w, m, num_cus);
+    if (int4_ksplit_takes(w, m, num_cus)) opt = std::max(opt, int4_ksplit_partial_bytes(w, m, num_cus));
+    else if (m <= 32 && int4_mid_partial_bytes(w, m) <= kKsplitPartialCap) opt = std::max(opt, int4_mid_partial_bytes(w, m));
+    L.opt_bytes = round_up(opt, 256);
   }
   if (!L.skinny && force == 0 && x_dtype == YSCV_HIP_F32 && m <= kChunkedSkinnyMaxRows) {
     // this call may run as 16-row skinny calls (see int4_run_ws): the scratch must cover one of those too
-    const Int4Scratch c = int4_scratch_layout(w, x, x_dtype, 16, 1, num_cus);
+    const Int4Scratch c = int4_scratch_layout(w, x, x_dtype, y, y_dtype, 16, 1, num_cus);
     if (c.total > L.total) L.total = c.total;
   }
   return L;
@@ -143,7 +159,7 @@ int32_t int4_workspace_bytes(const yscv_hip_int4_weight *w, size_t m, int x_dtyp
   }
   // a 16-byte aligned pointer stands in for the activation: alignment is checked again at run time
   if (!x) x = reinterpret_cast<const void *>(uintptr_t(256));
-  Int4Scratch L = int4_scratch_layout(w, x, x_dtype, m, force, ctx->num_cus);
+  Int4Scratch L = int4_scratch_layout(w, x, x_dtype, nullptr, YSCV_HIP_F32, m, force, ctx->num_cus);
   *bytes = L.total + L.opt_bytes;
   return YSCV_HIP_OK;
 }
@@ -169,7 +185,7 @@ int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, v
     return launch_int4_generic(w, x, x_dtype, y, y_dtype, m, s);
   }
   note_int4_fast();
-  Int4Scratch L = int4_scratch_layout(w, x, x_dtype, m, force, ctx->num_cus);
+  Int4Scratch L = int4_scratch_layout(w, x, x_dtype, y, y_dtype, m, force, ctx->num_cus);
   // above 16 rows the LDS-ring GEMM (16-bit activations) has the add and SwiGLU epilogues; the exact-scale kernel has none
   if (!L.skinny && epi != EPI_STORE && !(x_dtype != YSCV_HIP_F32 && nf == nullptr))
     return set_error(YSCV_HIP_ERR_UNSUPPORTED, "fused epilogues above 16 rows need 16-bit activations");
@@ -178,9 +194,7 @@ int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, v
   // 5-10 x faster than the exact-scale GEMM kernel there: that one keeps a 64 x 256 tile per workgroup and cannot fill
   // the GPU with so few rows (m = 64 against 14336 x 4096: 432 us; four skinny passes: about 60 us).
   if (!L.skinny && force == 0 && x_dtype == YSCV_HIP_F32 && m <= kChunkedSkinnyMaxRows) {
-    const bool ring_ok = w->scale_dtype == YSCV_HIP_F16 &&
-                         int4_gemm_ring_eligible(w, reinterpret_cast<const _Float16 *>(uintptr_t(256)), y, y_dtype, 1, m, L.k_pad);
-    if (!ring_ok) {
+    if (!L.fast16) {
       const size_t ysz = dtype_size(y_dtype);
       for (size_t r0 = 0; r0 < m; r0 += 16) {
         const size_t rows = m - r0 < 16 ? m - r0 : 16;
@@ -211,22 +225,10 @@ int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, v
   _Float16 *xl = (!L.direct && L.split == 2) ? reinterpret_cast<_Float16 *>(scratch + L.xh_bytes) : nullptr;
   float *row_scale = L.direct ? nullptr : reinterpret_cast<float *>(scratch + L.xh_bytes * L.split);
   float *partial = L.part_bytes ? reinterpret_cast<float *>(scratch + L.xh_bytes * L.split + L.rs_bytes) : nullptr;
-  // f32 activations with more than 16 rows against a weight whose scales are stored as fp16 (the MatMulNBits form) go
-  // to the LDS-ring GEMM as ONE fp16 operand: that kernel folds the group scale into fp16 weights (2^-11 relative per
-  // weight), which a lo half of the activations could not refine, and it is 3.5x (prefill shapes) to 14x (few rows,
-  // wide N) faster than the exact-scale kernel.  Weights with f32 scales -- what packed_int4_gemm_dispatch hands
-  // over -- keep the exact-scale kernel with hi + lo activations: the reference's own test holds that entry point
-  // to 1e-3 absolute (int4_matmul.rs:816-855).  The scratch keeps the size of the two-operand form.
-  int run_split = L.split;
-  if (!L.skinny && x_dtype == YSCV_HIP_F32 && m > 16 && w->scale_dtype == YSCV_HIP_F16 &&
-      int4_gemm_ring_eligible(w, xh, y, y_dtype, 1, m, L.k_pad)) {
-    run_split = 1;
-    xl = nullptr;
-  }
   if (!L.direct)
-    YSCV_TRY(launch_x_prep(x, x_dtype, m, w->k, L.k_pad, run_split, const_cast<_Float16 *>(xh), xl, row_scale, s));
-  if (L.skinny) return launch_int4_skinny(w, L.plan, xh, xl, xraw, row_scale, L.k_pad, L.split, y, y_dtype, m, partial, epi, s, nf);
-  return launch_int4_gemm(w, xh, xl, row_scale, L.k_pad, run_split, y, y_dtype, m, s, epi, gemm_partial, L.opt_bytes);
+    YSCV_TRY(launch_x_prep(x, x_dtype, m, w->k, L.ldx, L.split, const_cast<_Float16 *>(xh), xl, row_scale, s));
+  if (L.skinny) return launch_int4_skinny(w, L.plan, xh, xl, xraw, row_scale, L.ldx, L.split, y, y_dtype, m, partial, epi, s, nf);
+  return launch_int4_gemm(w, xh, xl, row_scale, L.ldx, L.split, y, y_dtype, m, s, epi, gemm_partial, L.opt_bytes);
 }
 
 static int32_t int4_run(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y, int y_dtype,
@@ -514,7 +516,7 @@ int32_t yscv_hip_int4_matmul_static(const yscv_hip_int4_weight *w, const void *x
   void *ws = ctx->device < kMaxDevices ? g_scratch_ptr[ctx->device] : nullptr;
   if (ws == nullptr) return set_error(YSCV_HIP_ERR_DEVICE, "the static scratch of device %d was never resolved", ctx->device);
   if (w->tiled) {
-    const Int4Scratch L = int4_scratch_layout(w, x_dev, x_dtype, m, 0, ctx->num_cus);
+    const Int4Scratch L = int4_scratch_layout(w, x_dev, x_dtype, y_dev, y_dtype, m, 0, ctx->num_cus);
     if (L.total + L.opt_bytes > (size_t)YSCV_HIP_STATIC_SCRATCH_BYTES)
       return set_error(YSCV_HIP_ERR_INVALID_ARG,
                        "this call needs %zu bytes of scratch, the static scratch holds %zu: use yscv_hip_int4_matmul_ws",

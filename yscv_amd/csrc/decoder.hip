@@ -475,7 +475,7 @@ static int32_t finish_setup(yscv_hip_decoder *d) {
       for (auto *w : {L.wqkv, L.wgu}) ok = ok && consumes(w);
     ok = ok && consumes(d->lm_head);
     for (auto &L : d->layers) ok = ok && L.wo->tiled && L.wdown->tiled;
-    // every projection takes its fp16 activations as they are (no padded copy with a row scale of its own)
+    // models with a width that is no multiple of 512 keep the separate norms: their parity bar was set with those rounding points
     auto direct = [](const yscv_hip_int4_weight *w) { return w->ktp * 128 == w->k; };
     for (auto &L : d->layers)
       for (auto *w : {L.wqkv, L.wo, L.wgu, L.wdown}) ok = ok && direct(w);

@@ -254,10 +254,14 @@ int32_t launch_int4_gemm(const yscv_hip_int4_weight *w, const _Float16 *xh, cons
                          const float *row_scale, size_t k_pad, int split, void *y, int y_dtype, size_t m,
                          hipStream_t s, int epi, float *partial, size_t partial_bytes) {
   if (!w->tiled) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "int4 GEMM kernel needs the tiled layout");
-  // 16-bit activations: the LDS-ring kernel from the first row count the skinny kernel does not take (rows are
-  // padded to its 128-row tile; with few rows the weights are still streamed exactly once)
-  // 17 .. 32 rows: the register-resident kernel of int4_mid.hip where its partial sums (if any) have their scratch
-  if (m > 16 && m <= 32 && int4_mid_eligible(w, xh, y, y_dtype, split, m, k_pad, kMidPartialCap)) {
+  // one fp16 operand: the K-split kernel while its tiles fit the CUs at once, the LDS-ring kernel above
+  const Context *ctx = nullptr;
+  YSCV_TRY(ensure_context(&ctx));
+  if (m > 16 && int4_ksplit_takes(w, m, ctx->num_cus) && int4_gemm_ring_eligible(w, xh, y, y_dtype, split, m, round_up(k_pad, 64)))
+    return launch_int4_ksplit(w, xh, row_scale, k_pad, y, y_dtype, m, s, epi, partial, partial_bytes);
+  // 17 .. 32 rows of a wider weight: the register-resident kernel where its partial sums (if any) have their scratch
+  // (LM head of 128 256 rows: 79 us against 85)
+  if (m > 16 && m <= 32 && int4_mid_eligible(w, xh, y, y_dtype, split, m, kKsplitPartialCap)) {
     const size_t need = int4_mid_partial_bytes(w, m);
     if (need == 0 || (partial != nullptr && partial_bytes >= need))
       return launch_int4_mid(w, xh, row_scale, k_pad, y, y_dtype, m, s, epi, partial, partial_bytes);

@@ -46,7 +46,8 @@ struct RingArgs {
   int col0, ldy;   // first column of this launch (a multiple of the tile width); row stride of y
   int nt, kt, ktp;
   int chunks, chunk_div;
-  int k_pad;
+  int ldx;         // row stride of xh
+  int stages;      // 64-k stages that hold data; the rows of xh reach to the end of the last one
   int y_dtype;
   int epi;         // EPI_STORE, EPI_ADD_F32 (y f32, y += product) or EPI_SWIGLU (y [m][n / 2] = silu(gate) * up, columns 2i / 2i+1)
   // K split (shapes with fewer tiles than CUs): the workgroups of split j multiply 128-k tiles j * kt_per .. and
@@ -227,7 +228,8 @@ __global__ void __launch_bounds__(256 + 64 * NP) int4_gemm_ring_kernel(RingArgs 
   const int m0 = tm * BM, n0 = p.col0 + tn * BN;
   const int kt_lo = ksplit * p.kt_per;
   const int kt_n = min(p.kt - kt_lo, p.kt_per);
-  const int nstages = kt_n * (4 / KS), st_base = kt_lo * (4 / KS);  // this workgroup's stages are st_base + 0 .. nstages - 1
+  const int st_base = kt_lo * (4 / KS);
+  const int nstages = min(kt_n * (4 / KS), p.stages - st_base);  // this workgroup's stages are st_base + 0 .. nstages - 1
 
   float4_t acc[MT][NT];  // MMA waves only; the producers never touch it
   const int wm = (wave >> 1) & 1, wn = wave & 1;
@@ -256,7 +258,7 @@ __global__ void __launch_bounds__(256 + 64 * NP) int4_gemm_ring_kernel(RingArgs 
       const int h = q & 1, row8 = lane >> 3;
       const int chunk = (lane & 7) ^ (4 * h + (row8 >> 1));
       const int row = min(m0 + (q >> 1) * 16 + 8 * h + row8, p.m - 1);
-      aoff[j] = (uint32_t)(((size_t)row * p.k_pad + chunk * 8) * sizeof(_Float16));
+      aoff[j] = (uint32_t)(((size_t)row * p.ldx + chunk * 8) * sizeof(_Float16));
     }
     const uint32_t woff = lane * 16, soff = r * SC::SC_BYTES, zoff = r * SC::ZP_BYTES;
     const uint8_t *wbase[WT], *sbase[WT], *zbase[WT];
@@ -565,12 +567,7 @@ int32_t ring_launch_one(const RingArgs &a, hipStream_t s) {
   const unsigned grid = (unsigned)((super_blocks * splits + 7) / 8) * 8 * 32;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(256 + 64 * NP), LDS, s, a, tiles_m, tiles_n, sbm_log2);
   YSCV_HIP_TRY(hipGetLastError());
-  if (a.partial) {
-    const size_t work = (size_t)a.m * ((a.n + 3) / 4);
-    const unsigned fb = (unsigned)std::min<size_t>((work + 255) / 256, 4096);
-    hipLaunchKernelGGL(ring_finalize_kernel, dim3(fb), dim3(256), 0, s, a.partial, (int)splits, a.m, a.n, a.y, a.y_dtype, a.epi, a.ldy);
-    YSCV_HIP_TRY(hipGetLastError());
-  }
+  if (a.partial) return launch_int4_partial_sum(a.partial, (int)splits, a.m, a.n, a.y, a.y_dtype, a.epi, s);
   return YSCV_HIP_OK;
 }
 
@@ -585,10 +582,19 @@ int32_t ring_launch_gm(const RingArgs &a, int gm, bool sf16, hipStream_t s) {
 
 }  // namespace
 
+int32_t launch_int4_partial_sum(const float *partial, int splits, int m, int n, void *y, int y_dtype, int epi, hipStream_t s) {
+  const size_t work = (size_t)m * ((n + 3) / 4);
+  const unsigned fb = (unsigned)std::min<size_t>((work + 255) / 256, 4096);
+  hipLaunchKernelGGL(ring_finalize_kernel, dim3(fb), dim3(256), 0, s, partial, splits, m, n, y, y_dtype, epi, n);
+  YSCV_HIP_TRY(hipGetLastError());
+  return YSCV_HIP_OK;
+}
+
 bool int4_gemm_ring_eligible(const yscv_hip_int4_weight *w, const _Float16 *xh, const void *y, int y_dtype, int split, size_t m,
                              size_t k_pad) {
   if (!w->tiled || split != 1) return false;
   if ((reinterpret_cast<uintptr_t>(xh) & 15) != 0) return false;
+  if (k_pad < round_up(w->k, 64)) return false;  // a stage is 64 k
   if (m * k_pad * sizeof(_Float16) >= ((size_t)1 << 32)) return false;  // per-lane offsets are 32 bits wide
   const size_t align = y_dtype == YSCV_HIP_F32 ? 16 : 8;
   return (reinterpret_cast<uintptr_t>(y) & (align - 1)) == 0;
@@ -729,7 +735,8 @@ int32_t launch_int4_gemm_ring(const yscv_hip_int4_weight *w, const _Float16 *xh,
   a.ktp = (int)w->ktp;
   a.chunks = (int)w->chunks;
   a.chunk_div = w->gm == GM128 ? (int)(w->g / 128) : 1;
-  a.k_pad = (int)k_pad;
+  a.ldx = (int)k_pad;
+  a.stages = (int)ceil_div(w->k, (size_t)64);
   a.y_dtype = y_dtype;
   a.partial = nullptr;
   a.kt_per = (int)w->kt;

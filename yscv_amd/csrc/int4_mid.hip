@@ -11,7 +11,7 @@
 // GEMM folds it) and feeds it to RT MFMAs.  Nothing but the partial sums of the waves goes through LDS: RT x 1 KiB per
 // wave and block, two buffers, one LDS-only barrier per block; the waves' sums are added in a fixed order.
 // A workgroup covers 8 x TPWM x 128 = 4096 k; a longer K is cut into parts over blockIdx.y whose f32 products go to
-// partial[part][m][n] (the caller's workspace) and are added, epilogue included, by mid_finalize_kernel.
+// partial[part][m][n] (the caller's workspace) and are added, epilogue included, by the LDS-ring GEMM's second kernel.
 // (The same kernel with four row tiles and 256 k per wave, for 33 .. 64 rows, was slower than the LDS-ring GEMM with
 // its K split on the prompt-pass shapes -- 3.86 against 3.56 ms for 64 tokens -- and is not instantiated.)
 // The MFMA is issued with the weights as the A operand (D = W_frag x X_frag): a lane holds four consecutive columns
@@ -36,7 +36,7 @@ struct MidArgs {
   const float *row_scale;  // null: 1
   void *y;
   float *partial;  // [parts][m][n] when K is cut into parts, else null
-  int m, n, nt, ktp, chunks, chunk_div, k_pad, y_dtype, epi, ldy;
+  int m, n, nt, ktp, chunks, chunk_div, k, ldx, y_dtype, epi, ldy;
 };
 
 template <int GM, bool SF16>
@@ -111,12 +111,12 @@ __global__ void __launch_bounds__(512, 1) int4_mid_kernel(MidArgs a) {
     const int row = min(rt * 16 + r, a.m - 1);  // rows past m repeat the last one and are not stored
 #pragma unroll
     for (int j = 0; j < TPWM; j++) {
-      const bool live = t0 + j < a.ktp;
-      const _Float16 *src = a.xh + (size_t)row * a.k_pad + (size_t)tl[j] * 128 + c * 8;
+      const _Float16 *src = a.xh + (size_t)row * a.ldx + c * 8;
 #pragma unroll
       for (int ks = 0; ks < 4; ks++) {
-        half8_t v = *reinterpret_cast<const half8_t *>(src + ks * 32);
-        if (!live) v = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        const int kk = (t0 + j) * 128 + ks * 32;  // K is a multiple of 32: inside K or behind it, the same for every lane
+        half8_t v = *reinterpret_cast<const half8_t *>(src + min(kk, a.k - 32));
+        if (kk >= a.k) v = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
         xa[j][ks][rt] = v;
       }
     }
@@ -213,40 +213,6 @@ __global__ void __launch_bounds__(512, 1) int4_mid_kernel(MidArgs a) {
   }
 }
 
-// Adds the K parts in a fixed order and applies the epilogue: four columns per thread.
-__global__ void __launch_bounds__(256) mid_finalize_kernel(const float *__restrict__ partial, int parts, int m, int n, void *y,
-                                                           int y_dtype, int epi, int ldy) {
-  const int chunks = (n + 3) / 4;
-  const size_t total = (size_t)m * chunks;
-  for (size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x; idx < total; idx += (size_t)gridDim.x * blockDim.x) {
-    const int row = (int)(idx / chunks), col = (int)(idx % chunks) * 4;
-    const bool whole = col + 4 <= n && (n & 3) == 0;
-    float4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int j = 0; j < parts; j++) {
-      const float *src = partial + ((size_t)j * m + row) * n + col;
-      if (whole) {
-        v += *reinterpret_cast<const float4_t *>(src);
-      } else {
-        for (int e = 0; e < 4; e++)
-          if (col + e < n) v[e] += src[e];
-      }
-    }
-    const size_t o = (size_t)row * ldy + col;
-    if (epi == EPI_SWIGLU) {
-      const size_t oh = (size_t)row * (ldy >> 1) + (col >> 1);
-      store_out(y, oh, mid_silu(v[0]) * v[1], y_dtype);
-      if (col + 2 < n) store_out(y, oh + 1, mid_silu(v[2]) * v[3], y_dtype);
-    } else if (epi == EPI_ADD_F32) {
-      float *dst = reinterpret_cast<float *>(y) + o;
-      for (int e = 0; e < 4; e++)
-        if (col + e < n) dst[e] += v[e];
-    } else {
-      for (int e = 0; e < 4; e++)
-        if (col + e < n) store_out(y, o + e, v[e], y_dtype);
-    }
-  }
-}
-
 template <int RT, int TPWM, int GM, bool SF16, bool HAS_ZP, int P>
 int32_t mid_launch_one(const MidArgs &a, int parts, int cus, hipStream_t s) {
   constexpr int LDS = 2 * 8 * RT * 64 * 16;
@@ -262,12 +228,7 @@ int32_t mid_launch_one(const MidArgs &a, int parts, int cus, hipStream_t s) {
   nparts = nparts < 1 ? 1 : (nparts > a.nt ? a.nt : nparts);
   hipLaunchKernelGGL(kern, dim3((unsigned)nparts, (unsigned)parts), dim3(512), LDS, s, a);
   YSCV_HIP_TRY(hipGetLastError());
-  if (a.partial != nullptr) {
-    const size_t work = (size_t)a.m * ((a.n + 3) / 4);
-    const unsigned fb = (unsigned)std::min<size_t>((work + 255) / 256, 4096);
-    hipLaunchKernelGGL(mid_finalize_kernel, dim3(fb), dim3(256), 0, s, a.partial, parts, a.m, a.n, a.y, a.y_dtype, a.epi, a.ldy);
-    YSCV_HIP_TRY(hipGetLastError());
-  }
+  if (a.partial != nullptr) return launch_int4_partial_sum(a.partial, parts, a.m, a.n, a.y, a.y_dtype, a.epi, s);
   return YSCV_HIP_OK;
 }
 
@@ -299,15 +260,15 @@ size_t int4_mid_partial_bytes(const yscv_hip_int4_weight *w, size_t m) {
 // 17 .. 32 rows of fp16-prepared activations against a tiled weight.  A workgroup covers 4096 k; a longer K needs the
 // partial-sum scratch: the kernel is taken where that scratch stays within `max_partial_bytes`.
 bool int4_mid_eligible(const yscv_hip_int4_weight *w, const _Float16 *xh, const void *y, int y_dtype, int split, size_t m,
-                       size_t k_pad, size_t max_partial_bytes) {
+                       size_t max_partial_bytes) {
   if (!w->tiled || split != 1 || m <= 16 || m > 32) return false;
-  if ((reinterpret_cast<uintptr_t>(xh) & 15) != 0 || (k_pad & 7) != 0) return false;
+  if ((reinterpret_cast<uintptr_t>(xh) & 15) != 0) return false;
   const size_t align = y_dtype == YSCV_HIP_F32 ? 16 : 8;
   if ((reinterpret_cast<uintptr_t>(y) & (align - 1)) != 0) return false;
   return int4_mid_partial_bytes(w, m) <= max_partial_bytes;
 }
 
-int32_t launch_int4_mid(const yscv_hip_int4_weight *w, const _Float16 *xh, const float *row_scale, size_t k_pad, void *y,
+int32_t launch_int4_mid(const yscv_hip_int4_weight *w, const _Float16 *xh, const float *row_scale, size_t ldx, void *y,
                         int y_dtype, size_t m, hipStream_t s, int epi, float *partial, size_t partial_bytes) {
   if (epi == EPI_ADD_F32 && y_dtype != YSCV_HIP_F32) return set_error(YSCV_HIP_ERR_INVALID_ARG, "the add epilogue updates an f32 tensor");
   if (epi == EPI_SWIGLU && (w->n & 1)) return set_error(YSCV_HIP_ERR_INVALID_ARG, "SwiGLU epilogue needs an even row count");
@@ -332,7 +293,8 @@ int32_t launch_int4_mid(const yscv_hip_int4_weight *w, const _Float16 *xh, const
   a.ktp = (int)w->ktp;
   a.chunks = (int)w->chunks;
   a.chunk_div = w->gm == GM128 ? (int)(w->g / 128) : 1;
-  a.k_pad = (int)k_pad;
+  a.k = (int)w->k;
+  a.ldx = (int)ldx;
   a.y_dtype = y_dtype;
   a.epi = epi;
   a.ldy = (int)w->n;

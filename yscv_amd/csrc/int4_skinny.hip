@@ -49,8 +49,8 @@ struct SkinnyArgs {
   const uint8_t *tzps;  // null: zero point 8 everywhere
   const _Float16 *xh;
   const _Float16 *xl;
-  const float *xf;     // raw f32 activations (row stride k_pad) for the kernels that split them themselves, else null
-  const uint16_t *xb;  // raw bf16 activations (row stride k_pad), else null
+  const float *xf;     // raw f32 activations for the kernels that split them themselves, else null
+  const uint16_t *xb;  // raw bf16 activations, else null
   const float *row_scale;
   void *y;
   float *partial;  // [ksg][m][n] when ksg > 1
@@ -58,7 +58,7 @@ struct SkinnyArgs {
   int nt, ktp;     // tile counts; ktp = 128-k tiles per 16-row block as stored (multiple of TPW)
   int chunks;      // scale chunks per 16-row block
   int chunk_div;   // GM128: tiles per scale chunk (group_size / 128)
-  int k_pad;       // row stride of xh / xl, = ktp * 128
+  int k, ldx;      // K (a multiple of 32) and the row stride of the activations; the weights hold zeros behind K
   int y_dtype;
   int ksg;
   int epi;         // EPI_STORE / EPI_ADD_F32 / EPI_SWIGLU
@@ -234,6 +234,12 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
   // ---- activations -> registers, in A-operand order ------------------------------------------
   // MFMA row `r` carries batch row m when r == 4*(m / NI) + (m % NI): the useful results then sit
   // in the first NI of the four accumulator registers of each lane.
+  // K is a multiple of 32, so a 32-k block lies inside K or behind it, the same for every lane: blocks behind it read the
+  // last one and are zeroed.  Only the wave that holds the end of such a K looks (a branch of its own around all its loads:
+  // in the other waves sixteen loads share one address and differ in constant offsets).
+  const bool whole = (t0 + TPW) * 128 <= a.k;  // uniform in the wave
+  auto block_k = [&](int t, int j) { return min((t0 + t) * 128 + j * 32, a.k - 32); };
+  auto block_in = [&](int t, int j) { return (t0 + t) * 128 + j * 32 < a.k; };
   half8_t xa[TPW][4][SPLIT];
   float slice_scale = 1.0f;  // RAWX: what this wave's products of the row it loads must be multiplied by
   {
@@ -246,12 +252,25 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
       // bf16 activations straight from the caller: the wave scales its own 512-k slice of every row by a power of
       // two (abs-max to [2^14, 2^15)), which makes every bf16 value an exact fp16 one (8 significant bits; only
       // values below 2^-29 of the slice maximum are lost); the power of two is undone on the wave's partial sums.
-      const uint16_t *src = a.xb + (size_t)(valid ? mrow : 0) * a.k_pad + (size_t)t0 * 128 + c * 8;
+      const uint16_t *src = a.xb + (size_t)(valid ? mrow : 0) * a.ldx + c * 8;
       uint4_t raw[TPW][4];
+      if (whole) {
+        src += (size_t)t0 * 128;
 #pragma unroll
-      for (int t = 0; t < TPW; t++)
+        for (int t = 0; t < TPW; t++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) raw[t][j] = *reinterpret_cast<const uint4_t *>(src + t * 128 + j * 32);
+          for (int j = 0; j < 4; j++) raw[t][j] = *reinterpret_cast<const uint4_t *>(src + t * 128 + j * 32);
+      } else {
+#pragma unroll
+        for (int t = 0; t < TPW; t++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) raw[t][j] = *reinterpret_cast<const uint4_t *>(src + block_k(t, j));
+#pragma unroll
+        for (int t = 0; t < TPW; t++)
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            if (!block_in(t, j)) raw[t][j] = uint4_t{0, 0, 0, 0};
+      }
       uint32_t amax_bits = 0;  // |bf16| orders like its bit pattern
 #pragma unroll
       for (int t = 0; t < TPW; t++)
@@ -298,10 +317,15 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
       // partial sums.  Lanes without a row read row 0 and discard it (unconditional loads: one round trip for all).
       const int srow = lane >> 4, q = lane & 15;
       const bool svalid = wave_active && srow < a.m;
-      const float *src = a.xf + (size_t)(svalid ? srow : 0) * a.k_pad + (size_t)t0 * 128 + q * 32;
+      const bool k_in = t0 * 128 + q * 32 < a.k;
+      const float *src = a.xf + (size_t)(svalid ? srow : 0) * a.ldx + (k_in ? t0 * 128 + q * 32 : 0);
       float4_t raw[8];
 #pragma unroll
       for (int e = 0; e < 8; e++) raw[e] = *reinterpret_cast<const float4_t *>(src + 4 * e);
+      if (!k_in) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) raw[e] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      }
       float amax = 0.0f;
 #pragma unroll
       for (int e = 0; e < 8; e++)
@@ -352,7 +376,8 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
       // hi + lo; the power of two is undone on the wave's partial sums before they meet the other slices.
       // Idle lanes read row 0 and discard it: every load is unconditional, so all of them are in flight together
       // instead of one round trip per guarded load.
-      const float *src = a.xf + (size_t)(valid ? mrow : 0) * a.k_pad + (size_t)t0 * 128 + c * 8;
+      // (K a multiple of 512: the launcher checks)
+      const float *src = a.xf + (size_t)(valid ? mrow : 0) * a.ldx + (size_t)t0 * 128 + c * 8;
       float amax = 0.0f;
 #pragma unroll
       for (int t = 0; t < TPW; t++)
@@ -397,20 +422,43 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
         }
       }
     } else {
-      const size_t row_off = (size_t)(valid ? mrow : 0) * a.k_pad;
+      const size_t row_off = (size_t)(valid ? mrow : 0) * a.ldx + c * 8;
       const half8_t hz = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (whole) {
+#pragma unroll
+        for (int t = 0; t < TPW; t++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const size_t off = row_off + (size_t)(t0 + t) * 128 + j * 32;
+            xa[t][j][0] = *reinterpret_cast<const half8_t *>(a.xh + off);
+            if constexpr (SPLIT == 2) xa[t][j][1] = *reinterpret_cast<const half8_t *>(a.xl + off);
+          }
+      } else {
+#pragma unroll
+        for (int t = 0; t < TPW; t++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const size_t off = row_off + block_k(t, j);
+            xa[t][j][0] = *reinterpret_cast<const half8_t *>(a.xh + off);
+            if constexpr (SPLIT == 2) xa[t][j][1] = *reinterpret_cast<const half8_t *>(a.xl + off);
+          }
+#pragma unroll
+        for (int t = 0; t < TPW; t++)
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            if (!block_in(t, j)) {
+              xa[t][j][0] = hz;
+              if constexpr (SPLIT == 2) xa[t][j][1] = hz;
+            }
+      }
 #pragma unroll
       for (int t = 0; t < TPW; t++) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-          const size_t off = row_off + (size_t)(t0 + t) * 128 + j * 32 + c * 8;
-          half8_t h = *reinterpret_cast<const half8_t *>(a.xh + off);
-          if (!valid) h = hz;
-          if constexpr (OFFSET) h = h * pre;  // slots that meet 1024 + 16 q carry x / 16 (a power of two)
-          xa[t][j][0] = h;
+          if (!valid) xa[t][j][0] = hz;
+          if constexpr (OFFSET) xa[t][j][0] = xa[t][j][0] * pre;  // slots that meet 1024 + 16 q carry x / 16 (a power of two)
           if constexpr (SPLIT == 2) {
-            half8_t l = *reinterpret_cast<const half8_t *>(a.xl + off);
-            xa[t][j][1] = valid ? l : hz;
+            if (!valid) xa[t][j][1] = hz;
           }
         }
       }
@@ -896,13 +944,13 @@ static int32_t launch_gm(const SkinnyArgs &a, const SkinnyPlan &plan, int gm, bo
 }
 
 int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan, const _Float16 *xh,
-                           const _Float16 *xl, const void *xraw, const float *row_scale, size_t k_pad, int split,
+                           const _Float16 *xl, const void *xraw, const float *row_scale, size_t ldx, int split,
                            void *y, int y_dtype, size_t m, float *partial, int epi, hipStream_t s, const NormFold *nf) {
   if (!w->tiled) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "skinny int4 kernel needs the tiled layout");
   if (m == 0 || m > 16) return set_error(YSCV_HIP_ERR_INVALID_ARG, "skinny int4 kernel handles 1 <= m <= 16, got %zu", m);
   if (plan.ksg > 1 && !partial) return set_error(YSCV_HIP_ERR_INVALID_ARG, "k-split needs a partial buffer");
-  if (k_pad != w->ktp * 128)
-    return set_error(YSCV_HIP_ERR_INVALID_ARG, "activation row stride %zu != padded K %zu", k_pad, w->ktp * 128);
+  if (ldx < w->k || w->k % 32 != 0 || (split == 2 && xraw && m > 4 && w->k % 512 != 0))
+    return set_error(YSCV_HIP_ERR_INVALID_ARG, "activation row stride %zu for K %zu", ldx, w->k);
   SkinnyArgs a;
   a.tiles = w->tiles;
   a.tscales = w->tscales;
@@ -920,7 +968,8 @@ int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan
   a.ktp = (int)w->ktp;
   a.chunks = (int)w->chunks;
   a.chunk_div = w->gm == GM128 ? (int)(w->g / 128) : 1;
-  a.k_pad = (int)k_pad;
+  a.k = (int)w->k;
+  a.ldx = (int)ldx;
   a.y_dtype = y_dtype;
   a.ksg = plan.ksg;
   a.epi = epi;

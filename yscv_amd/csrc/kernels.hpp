@@ -91,10 +91,10 @@ struct SkinnyPlan {
   size_t partial_bytes;
 };
 SkinnyPlan plan_int4_skinny(const yscv_hip_int4_weight *w, size_t m, int split, int num_cus);
-// xraw != null: raw activations with row stride k_pad, f32 when split == 2 and bf16 when split == 1; the kernel
-// normalises (and for f32 splits) them itself and xh, xl, row_scale are not used
+// ldx: row stride of the activations, at least k.  xraw != null: raw activations, f32 when split == 2 and bf16 when
+// split == 1; the kernel normalises (and for f32 splits) them itself and xh, xl, row_scale are not used
 int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan, const _Float16 *xh,
-                           const _Float16 *xl, const void *xraw, const float *row_scale, size_t k_pad, int split,
+                           const _Float16 *xl, const void *xraw, const float *row_scale, size_t ldx, int split,
                            void *y, int y_dtype, size_t m, float *partial, int epi, hipStream_t s,
                            const NormFold *nf = nullptr);
 int32_t launch_int4_generic(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y,
@@ -116,15 +116,24 @@ int32_t launch_int4_gemm_ring(const yscv_hip_int4_weight *w, const _Float16 *xh,
                               size_t partial_bytes = 0);
 size_t int4_gemm_ring_partial_bytes(const yscv_hip_int4_weight *w, size_t m, int num_cus);
 
-// 17 .. 32 rows (int4_mid.hip): K split over the waves with all rows' activations in registers, the weights streamed
-// once.  With K > 4096 K is also cut into parts over workgroups whose f32 partial sums need
-// int4_mid_partial_bytes() of scratch; the kernel is used where that stays within kMidPartialCap.
-constexpr size_t kMidPartialCap = (size_t)16 << 20;
+// A few dozen to a few hundred rows of fp16-prepared activations (int4_ksplit.hip): taken while its tiles fit the CUs at once.
+// A launch that is also split over K needs int4_ksplit_partial_bytes() of scratch (at most kKsplitPartialCap; without it the
+// launch runs unsplit).
+constexpr size_t kKsplitPartialCap = (size_t)16 << 20;
+bool int4_ksplit_takes(const yscv_hip_int4_weight *w, size_t m, int num_cus);
+size_t int4_ksplit_partial_bytes(const yscv_hip_int4_weight *w, size_t m, int num_cus);
+int32_t launch_int4_ksplit(const yscv_hip_int4_weight *w, const _Float16 *xh, const float *row_scale, size_t ldx, void *y, int y_dtype,
+                           size_t m, hipStream_t s, int epi, float *partial, size_t partial_bytes);
+// 17 .. 32 rows against a weight with more column blocks than that kernel takes at once (int4_mid.hip): K split over the
+// waves with all rows' activations in registers, the weights streamed once.  With K > 4096 K is also cut into parts over
+// workgroups whose f32 partial sums need int4_mid_partial_bytes() of scratch (at most kKsplitPartialCap).
 size_t int4_mid_partial_bytes(const yscv_hip_int4_weight *w, size_t m);
 bool int4_mid_eligible(const yscv_hip_int4_weight *w, const _Float16 *xh, const void *y, int y_dtype, int split, size_t m,
-                       size_t k_pad, size_t max_partial_bytes);
-int32_t launch_int4_mid(const yscv_hip_int4_weight *w, const _Float16 *xh, const float *row_scale, size_t k_pad, void *y,
+                       size_t max_partial_bytes);
+int32_t launch_int4_mid(const yscv_hip_int4_weight *w, const _Float16 *xh, const float *row_scale, size_t ldx, void *y,
                         int y_dtype, size_t m, hipStream_t s, int epi, float *partial, size_t partial_bytes);
+// y = epilogue(sum over the splits of partial[split][m][n]), fixed order (y rows of n, or n / 2 for SwiGLU)
+int32_t launch_int4_partial_sum(const float *partial, int splits, int m, int n, void *y, int y_dtype, int epi, hipStream_t s);
 
 // Whole int4 call (activation preparation + kernel) with caller-provided scratch; ws may be null.
 // (x: the activations, whose alignment decides whether they are used in place; null = 16-byte aligned ones)
