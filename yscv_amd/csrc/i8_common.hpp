@@ -1,0 +1,67 @@
+// Shared by the int8 GEMM kernels (i8_gemm.hip, i8_ksplit.hip): arguments and the per-element epilogue arithmetic.
+#pragma once
+
+#include "int4_common.hpp"
+#include "kernels.hpp"
+
+namespace yscv {
+
+// ---- rounding helpers (bit-exact with the reference's two rules) -----------------------
+// f32::round: half away from zero.  v - trunc(v) is exact, so the comparison is too.
+__device__ __forceinline__ float round_half_away(float v) {
+  float t = truncf(v);
+  float d = fabsf(__fsub_rn(v, t));
+  return (d >= 0.5f) ? __fadd_rn(t, copysignf(1.0f, v)) : t;
+}
+
+__device__ __forceinline__ int requant_one(int32_t acc, int32_t corr, float comp, float y_zp, int round_mode,
+                                           float lo, float hi) {
+  int32_t a = (int32_t)((uint32_t)acc + (uint32_t)corr);         // wrapping_add
+  float v = __fadd_rn(__fmul_rn((float)a, comp), y_zp);          // two roundings, never an FMA
+  float r = round_mode == YSCV_HIP_ROUND_HALF_AWAY ? round_half_away(v) : rintf(v);
+  if (r != r) return 0;                                          // clamp keeps NaN, `as i8` -> 0
+  r = fminf(fmaxf(r, lo), hi);
+  return (int)r;
+}
+
+// requantise, then DequantizeLinear of the quantised value: (q - y_zp) * dq_scale (crates/yscv-onnx/src/runner/misc.rs:124-128)
+__device__ __forceinline__ int32_t requant_dequant_bits(int32_t acc, int32_t corr, float comp, float y_zp, int round_mode,
+                                                        float lo, float hi, float dq_scale) {
+  const int q = requant_one(acc, corr, comp, y_zp, round_mode, lo, hi);
+  return __float_as_int(__fmul_rn(__fsub_rn((float)q, y_zp), dq_scale));
+}
+
+// requantise and keep the value as an f32 carrier, the form exec_qlinear_matmul returns (crates/yscv-onnx/src/runner/
+// linear.rs:481-485): clamp keeps a NaN
+__device__ __forceinline__ int32_t requant_f32_bits(int32_t acc, int32_t corr, float comp, float y_zp, int round_mode,
+                                                    float lo, float hi) {
+  int32_t a = (int32_t)((uint32_t)acc + (uint32_t)corr);
+  float v = __fadd_rn(__fmul_rn((float)a, comp), y_zp);
+  float r = round_mode == YSCV_HIP_ROUND_HALF_AWAY ? round_half_away(v) : rintf(v);
+  if (r == r) r = fminf(fmaxf(r, lo), hi);
+  return __float_as_int(r);
+}
+
+struct I8Args {
+  const uint8_t *a;   // [m][k]
+  const int8_t *frag; // packed B
+  const int32_t *col_sum;
+  void *out;
+  const int32_t *corr;
+  const float *composite_v;
+  float composite, y_zp, dq_scale;
+  int round_mode, lo, hi, mode;  // as I8Epilogue::mode
+  int m, n, k;
+  int lda;          // row stride of a in bytes (k, or kp for a padded copy)
+  int ksteps;       // kp / 64
+  int a_xor;        // 0x80808080 for uint8 activations, 0 for int8
+  int zp_mul;       // multiplies col_sum in the epilogue
+  const float *a_zp_dev;  // null, or the uint8 zero point of A as an f32 in device memory (then zp_mul = 128 - that)
+};
+
+// Shapes whose tiles leave the ring kernel's grid short of the CUs (i8_ksplit.hip): 16-byte aligned a with an lda that is a
+// multiple of 64, m * lda below 2 GiB.
+bool i8_ksplit_takes(size_t m, size_t n, size_t ksteps, int num_cus);
+int32_t launch_i8_ksplit(const I8Args &p, int num_cus, hipStream_t s);
+
+}  // namespace yscv

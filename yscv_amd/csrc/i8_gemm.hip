@@ -19,8 +19,7 @@
 #include <mutex>
 #include <utility>
 
-#include "int4_common.hpp"
-#include "kernels.hpp"
+#include "i8_common.hpp"
 
 namespace yscv {
 
@@ -69,58 +68,6 @@ int32_t launch_i8_pack_b(const int8_t *b_kn, size_t k, size_t n, size_t kp, size
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
-
-// ---- rounding helpers (bit-exact with the reference's two rules) -----------------------
-// f32::round: half away from zero.  v - trunc(v) is exact, so the comparison is too.
-__device__ __forceinline__ float round_half_away(float v) {
-  float t = truncf(v);
-  float d = fabsf(__fsub_rn(v, t));
-  return (d >= 0.5f) ? __fadd_rn(t, copysignf(1.0f, v)) : t;
-}
-
-__device__ __forceinline__ int requant_one(int32_t acc, int32_t corr, float comp, float y_zp, int round_mode,
-                                           float lo, float hi) {
-  int32_t a = (int32_t)((uint32_t)acc + (uint32_t)corr);         // wrapping_add
-  float v = __fadd_rn(__fmul_rn((float)a, comp), y_zp);          // two roundings, never an FMA
-  float r = round_mode == YSCV_HIP_ROUND_HALF_AWAY ? round_half_away(v) : rintf(v);
-  if (r != r) return 0;                                          // clamp keeps NaN, `as i8` -> 0
-  r = fminf(fmaxf(r, lo), hi);
-  return (int)r;
-}
-
-// requantise, then DequantizeLinear of the quantised value: (q - y_zp) * dq_scale (crates/yscv-onnx/src/runner/misc.rs:124-128)
-__device__ __forceinline__ int32_t requant_dequant_bits(int32_t acc, int32_t corr, float comp, float y_zp, int round_mode,
-                                                        float lo, float hi, float dq_scale) {
-  const int q = requant_one(acc, corr, comp, y_zp, round_mode, lo, hi);
-  return __float_as_int(__fmul_rn(__fsub_rn((float)q, y_zp), dq_scale));
-}
-
-// requantise and keep the value as an f32 carrier, the form exec_qlinear_matmul returns (crates/yscv-onnx/src/runner/
-// linear.rs:481-485): clamp keeps a NaN
-__device__ __forceinline__ int32_t requant_f32_bits(int32_t acc, int32_t corr, float comp, float y_zp, int round_mode,
-                                                    float lo, float hi) {
-  int32_t a = (int32_t)((uint32_t)acc + (uint32_t)corr);
-  float v = __fadd_rn(__fmul_rn((float)a, comp), y_zp);
-  float r = round_mode == YSCV_HIP_ROUND_HALF_AWAY ? round_half_away(v) : rintf(v);
-  if (r == r) r = fminf(fmaxf(r, lo), hi);
-  return __float_as_int(r);
-}
-
-struct I8Args {
-  const uint8_t *a;   // [m][k]
-  const int8_t *frag; // packed B
-  const int32_t *col_sum;
-  void *out;
-  const int32_t *corr;
-  const float *composite_v;
-  float composite, y_zp, dq_scale;
-  int round_mode, lo, hi, mode;  // as I8Epilogue::mode
-  int m, n, k;
-  int ksteps;       // kp / 64
-  int a_xor;        // 0x80808080 for uint8 activations, 0 for int8
-  int zp_mul;       // multiplies col_sum in the epilogue
-  const float *a_zp_dev;  // null, or the uint8 zero point of A as an f32 in device memory (then zp_mul = 128 - that)
-};
 
 template <bool VEC>
 __global__ void __launch_bounds__(I8_THREADS) i8_gemm_kernel(I8Args p) {
@@ -384,10 +331,10 @@ __global__ void __launch_bounds__(I8R_THREADS) i8_gemm_ring_kernel(I8Args p, int
           const int h = q & 1, row8 = lane >> 3;
           const int chunk = (lane & 7) ^ (4 * h + (row8 >> 1));
           const int row = min(m0 + (q / KS) * 16 + 8 * h + row8, p.m - 1);
-          src[j] = p.a + (size_t)row * p.k + chunk * 16;
+          src[j] = p.a + (size_t)row * p.lda + chunk * 16;
         } else {
           const int row = min(m0 + (q / KS) * 16 + r, p.m - 1);
-          src[j] = p.a + (size_t)row * p.k + c * 16;
+          src[j] = p.a + (size_t)row * p.lda + c * 16;
         }
       } else {
         const int gnt = min(n0 / 16 + (q - 2 * MT * KS) / KS, nt_total - 1);
@@ -594,8 +541,36 @@ int32_t launch_ring(const I8Args &p, size_t m, size_t n, hipStream_t s) {
   return YSCV_HIP_OK;
 }
 
+// rows of k bytes on any alignment -> rows of kp bytes (a multiple of 64), zeros behind k
+__global__ void __launch_bounds__(256) i8_pad_rows_kernel(const uint8_t *__restrict__ a, size_t m, int k, int kp, uint8_t *__restrict__ out) {
+  const int chunks = kp / 16;
+  const size_t total = m * chunks;
+  for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
+    const size_t row = i / (unsigned)chunks;
+    const int k0 = (int)(i % (unsigned)chunks) * 16;
+    const uint8_t *src = a + row * k + k0;
+    uint4_t v = {0, 0, 0, 0};
+    if (k0 + 16 <= k) {
+      __builtin_memcpy(&v, src, 16);  // one load; any alignment
+    } else {
+      for (int e = 0; k0 + e < k; e++) v[e >> 2] |= (uint32_t)src[e] << (8 * (e & 3));
+    }
+    reinterpret_cast<uint4_t *>(out)[i] = v;
+  }
+}
+
+// 32-bit offsets reach every row of A and the result takes 16-byte stores; anything else goes to i8_gemm_kernel
+static bool i8_fast_rows(size_t m, size_t kp, const void *out) {
+  return m * kp < ((size_t)1 << 31) && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+}
+
+size_t i8_gemm_pad_bytes(const yscv_hip_i8_weight *b, size_t m, const void *a, const void *out) {
+  if (!i8_fast_rows(m, b->kp, out) || (b->k == b->kp && (reinterpret_cast<uintptr_t>(a) & 15) == 0)) return 0;
+  return m * b->kp;
+}
+
 int32_t launch_i8_gemm(const void *a, int a_is_u8, int a_zp, const yscv_hip_i8_weight *b, size_t m,
-                       void *out, const I8Epilogue &ep, hipStream_t s) {
+                       void *out, const I8Epilogue &ep, hipStream_t s, void *pad) {
   I8Args p;
   p.a = static_cast<const uint8_t *>(a);
   p.frag = b->frag;
@@ -617,14 +592,28 @@ int32_t launch_i8_gemm(const void *a, int a_is_u8, int a_zp, const yscv_hip_i8_w
   p.a_xor = a_is_u8 ? (int)0x80808080u : 0;
   p.zp_mul = a_is_u8 ? (128 - a_zp) : -a_zp;
   p.a_zp_dev = ep.a_zp_dev;
-  const bool aligned = (reinterpret_cast<uintptr_t>(a) & 15) == 0;
-  const bool out_ok = (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-  if (b->k % 64 == 0 && aligned && out_ok && m * b->k < ((size_t)1 << 31)) {
-    // 128 x 128 tiles halve the LDS fill per MFMA; 64 x 128 tiles are for shapes that would not fill the CUs otherwise
+  p.lda = (int)b->k;
+  if (i8_fast_rows(m, b->kp, out)) {
+    Scratch own;
+    if (const size_t pad_bytes = i8_gemm_pad_bytes(b, m, a, out)) {
+      // K = 3001, 512 rows x 4096: a copy in kp-byte rows and the kernels below; the general kernel fetches such rows byte by byte
+      if (pad == nullptr) {
+        YSCV_TRY(own.take(pad_bytes, s));
+        pad = own.p;
+      }
+      const size_t blocks = ceil_div(pad_bytes / 16, (size_t)256);
+      hipLaunchKernelGGL(i8_pad_rows_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, p.a, m, p.k, (int)b->kp,
+                         static_cast<uint8_t *>(pad));
+      YSCV_HIP_TRY(hipGetLastError());
+      p.a = static_cast<const uint8_t *>(pad);
+      p.lda = (int)b->kp;
+    }
     const Context *ctx = nullptr;
     YSCV_TRY(ensure_context(&ctx));
+    if (i8_ksplit_takes(m, b->n, (size_t)p.ksteps, ctx->num_cus)) return launch_i8_ksplit(p, ctx->num_cus, s);
+    // 128 x 128 tiles halve the LDS fill per MFMA; 64 x 128 tiles are for shapes that would not fill the CUs otherwise
     const size_t big_tiles = ceil_div(m, (size_t)128) * ceil_div(b->n, (size_t)128);
-    const bool wide_a = b->k % 128 == 0;  // k-steps come in pairs: A is fetched as whole 128-byte lines
+    const bool wide_a = b->kp % 128 == 0;  // k-steps come in pairs: A is fetched as whole 128-byte lines
     if (big_tiles >= (size_t)ctx->num_cus)
       return wide_a ? launch_ring<4, 4, 2, 4, true>(p, m, b->n, s) : launch_ring<4, 4, 2, 4, false>(p, m, b->n, s);
     return wide_a ? launch_ring<2, 4, 4, 3, true>(p, m, b->n, s) : launch_ring<2, 4, 4, 3, false>(p, m, b->n, s);

@@ -169,7 +169,10 @@ struct I8Epilogue {
   const float *a_zp_dev = nullptr;  // uint8 A only: its zero point as an f32 in device memory, used instead of a_zp
 };
 int32_t launch_i8_gemm(const void *a, int a_is_u8, int a_zp, const yscv_hip_i8_weight *b, size_t m,
-                       void *out, const I8Epilogue &ep, hipStream_t s);
+                       void *out, const I8Epilogue &ep, hipStream_t s, void *pad = nullptr);
+// What launch_i8_gemm needs at `pad` (16-byte aligned) to copy rows of a K that is no multiple of 64, or A off 16-byte
+// alignment: 0 for others.  With a null pad it takes a scratch block itself, so a caller that holds one must pass its own.
+size_t i8_gemm_pad_bytes(const yscv_hip_i8_weight *b, size_t m, const void *a, const void *out);
 
 // ---- elementwise ---------------------------------------------------------------------
 int32_t launch_quantize_linear_i8(const float *x, size_t len, float scale, float zp, int8_t *out,

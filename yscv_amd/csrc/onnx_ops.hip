@@ -274,7 +274,8 @@ int32_t run_fast(const MatmulArgs &g) {
     // the usual case, a weight packed at load time: cast kernel + GEMM whose epilogue writes the f32 carriers, the
     // int8 copy of A in scratch -- nothing here waits for the device
     Scratch a8;
-    YSCV_TRY(a8.take(g.m * g.k, g.s));
+    const size_t a8_bytes = round_up(g.m * g.k, 256);
+    YSCV_TRY(a8.take(a8_bytes + i8_gemm_pad_bytes(g.b_packed, g.m, nullptr, g.out), g.s));
     hipLaunchKernelGGL(cast_as_i8_kernel, dim3(grid_for(g.m * g.k)), dim3(256), 0, g.s, g.a, g.m * g.k, 0, a8.as<int8_t>());
     YSCV_HIP_TRY(hipGetLastError());
     I8Epilogue ep{};
@@ -288,7 +289,7 @@ int32_t run_fast(const MatmulArgs &g) {
     } else {
       ep.mode = 3;
     }
-    return launch_i8_gemm(a8.p, 0, 0, g.b_packed, g.m, g.out, ep, g.s);
+    return launch_i8_gemm(a8.p, 0, 0, g.b_packed, g.m, g.out, ep, g.s, a8.as<char>(a8_bytes));
   }
   DevBuf a8, b8, acc;
   YSCV_TRY(a8.alloc(g.m * g.k));
@@ -551,7 +552,8 @@ int32_t yscv_hip_exec_qdq_matmul(const float *x_dev, size_t m, float a_scale, co
   // QuantizeLinear (zero point 0) into a scratch int8 matrix, then the GEMM whose epilogue requantises with the
   // QLinearMatMul fast-path expression and dequantises again
   Scratch a8;
-  YSCV_TRY(a8.take(m * b->k, s));
+  const size_t a8_bytes = round_up(m * b->k, 256);
+  YSCV_TRY(a8.take(a8_bytes + i8_gemm_pad_bytes(b, m, nullptr, out_dev), s));
   YSCV_TRY(launch_quantize_linear_i8(x_dev, m * b->k, a_scale, 0.0f, a8.as<int8_t>(), s));
   I8Epilogue ep{};
   ep.mode = 2;
@@ -561,7 +563,7 @@ int32_t yscv_hip_exec_qdq_matmul(const float *x_dev, size_t m, float a_scale, co
   ep.lo = -128;
   ep.hi = 127;
   ep.dq_scale = y_scale;
-  YSCV_TRY(launch_i8_gemm(a8.p, 0, 0, b, m, out_dev, ep, s));
+  YSCV_TRY(launch_i8_gemm(a8.p, 0, 0, b, m, out_dev, ep, s, a8.as<char>(a8_bytes)));
   g_qlinear_fast.fetch_add(1, std::memory_order_relaxed);
   return YSCV_HIP_OK;
 }
@@ -578,12 +580,13 @@ int32_t yscv_hip_exec_dql_matmul_integer(const float *x_dev, size_t m, const ysc
   // uint8 A and the block ranges of the quantiser in one scratch block; nothing returns to the host
   const size_t a_bytes = round_up(len, 256);
   Scratch scratch;
-  YSCV_TRY(scratch.take(a_bytes + dql_partial_bytes(len), s));
+  const size_t pad_at = a_bytes + round_up(dql_partial_bytes(len), 256);
+  YSCV_TRY(scratch.take(pad_at + i8_gemm_pad_bytes(b, m, nullptr, out_dev), s));
   YSCV_TRY(launch_dynamic_quantize_linear(x_dev, len, scratch.p, false, y_scale_dev, y_zp_dev, scratch.as<float>(a_bytes), s));
   I8Epilogue ep{};
   ep.mode = 3;               // f32(acc): MatMulInteger's output carrier (linear.rs:693-697)
   ep.a_zp_dev = y_zp_dev;    // the zero point stays on the device: the GEMM folds (128 - zp) * colsum(b) itself
-  YSCV_TRY(launch_i8_gemm(scratch.p, 1, 0, b, m, out_dev, ep, s));
+  YSCV_TRY(launch_i8_gemm(scratch.p, 1, 0, b, m, out_dev, ep, s, scratch.as<char>(pad_at)));
   g_mmi_fallback.fetch_add(1, std::memory_order_relaxed);
   return YSCV_HIP_OK;
 }
