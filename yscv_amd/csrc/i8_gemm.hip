@@ -213,8 +213,6 @@ __global__ void __launch_bounds__(I8_THREADS) i8_gemm_kernel(I8Args p) {
 // processing of the loads.  The MFMA is issued with the operands swapped, D = Bfrag x Afrag, which yields the
 // transposed tile: a lane holds four consecutive columns of one row of C.  The finished tile goes through LDS so
 // that all eight waves store whole rows of it (512 contiguous bytes of int32, 128 of requantised bytes).
-// Workgroups are numbered so that the ones sharing an XCD (id mod 8) cover a contiguous range of n-tiles over
-// all m-tiles: an XCD's L2 holds its slice of B once.
 typedef __attribute__((address_space(3))) void lds_void;
 #define I8_AS1(ptr) ((const void __attribute__((address_space(1))) *)(ptr))
 constexpr int I8R_THREADS = 512;
@@ -260,7 +258,7 @@ __device__ __forceinline__ void i8_frags_wait(I8Frags<MT, NT> &f) {
 // (i & 7) ^ g of row i / 8 with g = 4 h + (i / 8) / 2 (h = which eight rows of the 16-row group), so that the sixteen
 // lanes which later read one k-chunk of sixteen rows in one ds_read_b128 pass hit sixteen different 16-byte slots.
 template <int MT, int NT, int KS, int S, bool WIDE_A>
-__global__ void __launch_bounds__(I8R_THREADS) i8_gemm_ring_kernel(I8Args p, int tiles_m, int tiles_n, int sbm_log2) {
+__global__ void __launch_bounds__(I8R_THREADS) i8_gemm_ring_kernel(I8Args p, int tiles_m, int tiles_n) {
   constexpr int BM = 32 * MT, BN = 32 * NT;
   constexpr int A_BYTES = 2 * MT * KS * 1024, STAGE = 2 * (MT + NT) * KS * 1024;
   constexpr int PER_WAVE = (MT + NT) * KS / 2;  // 1 KiB chunks a producer wave fetches per stage
@@ -278,15 +276,13 @@ __global__ void __launch_bounds__(I8R_THREADS) i8_gemm_ring_kernel(I8Args p, int
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, c = lane >> 4;
 
-  // XCD-aware tile numbering: the grid of tiles is cut into super-blocks of 32 tiles, 2^sbm_log2 (at most 8) along
-  // m; workgroup ids that share an XCD (id mod 8) walk through one super-block at a time, so the 32 workgroups an
-  // XCD runs together share row panels of A and column panels of B in its L2.
-  const int sbm = 1 << sbm_log2, sbn = 32 >> sbm_log2;
-  const int sb_m = (tiles_m + sbm - 1) >> sbm_log2;
-  const int j_in_xcd = (int)(blockIdx.x >> 3);
-  const int sb = (j_in_xcd >> 5) * 8 + (int)(blockIdx.x & 7);
-  const int tm = (sb % sb_m) * sbm + (j_in_xcd & (sbm - 1)), tn = (sb / sb_m) * sbn + ((j_in_xcd & 31) >> sbm_log2);
-  if (tm >= tiles_m || tn >= tiles_n) return;
+  // XCD-aware tile numbering: tiles are numbered down bands of eight row tiles, column by column; an XCD (workgroup ids equal
+  // modulo 8) takes an eighth of them in a row: the neighbours that it runs together share row panels of A and column panels
+  // of B in its L2, and no XCD has more than its share.
+  const int tiles = tiles_m * tiles_n, share = (tiles + 7) >> 3, t = (int)(blockIdx.x & 7) * share + (int)(blockIdx.x >> 3);
+  if (t >= tiles) return;
+  const int band = t / (8 * tiles_n), in_band = t - band * 8 * tiles_n, band_rows = min(8, tiles_m - 8 * band);
+  const int tn = in_band / band_rows, tm = 8 * band + in_band % band_rows;
   const int m0 = tm * BM, n0 = tn * BN;
   const int nt_total = (p.n + 15) / 16;
   const int nstages = (p.ksteps + KS - 1) / KS;
@@ -531,12 +527,8 @@ int32_t launch_ring(const I8Args &p, size_t m, size_t n, hipStream_t s) {
   if (attr_err != hipSuccess)
     return set_error(YSCV_HIP_ERR_DEVICE, "cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(attr_err));
   const int tiles_m = (int)ceil_div(m, (size_t)(32 * MT)), tiles_n = (int)ceil_div(n, (size_t)(32 * NT));
-  int sbm_log2 = 3;
-  while (sbm_log2 > 0 && (1 << sbm_log2) > tiles_m) sbm_log2--;
-  const int sbm = 1 << sbm_log2, sbn = 32 >> sbm_log2;
-  const int super_blocks = ((tiles_m + sbm - 1) / sbm) * ((tiles_n + sbn - 1) / sbn);
-  const unsigned grid = (unsigned)((super_blocks + 7) / 8) * 8 * 32;
-  hipLaunchKernelGGL((i8_gemm_ring_kernel<MT, NT, KS, S, WIDE_A>), dim3(grid), dim3(I8R_THREADS), LDS, s, p, tiles_m, tiles_n, sbm_log2);
+  const unsigned grid = (unsigned)((tiles_m * tiles_n + 7) / 8 * 8);
+  hipLaunchKernelGGL((i8_gemm_ring_kernel<MT, NT, KS, S, WIDE_A>), dim3(grid), dim3(I8R_THREADS), LDS, s, p, tiles_m, tiles_n);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }

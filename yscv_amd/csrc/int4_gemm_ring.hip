@@ -191,7 +191,7 @@ __device__ __forceinline__ void g4_wait_vm_n() {
 }
 
 template <int MT, int NT, int KS, int SA, int NP, int GM, bool SF16>
-__global__ void __launch_bounds__(256 + 64 * NP) int4_gemm_ring_kernel(RingArgs p, int tiles_m, int tiles_n, int sbm_log2) {
+__global__ void __launch_bounds__(256 + 64 * NP) int4_gemm_ring_kernel(RingArgs p, int tiles_m, int tiles_n) {
   constexpr int THREADS = 256 + 64 * NP;
   constexpr int BM = 32 * MT, BN = 32 * NT;
   constexpr int A_BYTES = 2 * MT * KS * 1024, B_BYTES = 2 * NT * KS * 1024;  // one stage of each operand
@@ -212,19 +212,16 @@ __global__ void __launch_bounds__(256 + 64 * NP) int4_gemm_ring_kernel(RingArgs 
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, c = lane >> 4;
 
-  // XCD-aware tile numbering: the grid of tiles is cut into super-blocks of 32 tiles, 2^sbm_log2 (at most 8) along
-  // m; workgroup ids that share an XCD (id mod 8) walk through one super-block at a time, so the 32 workgroups an
-  // XCD runs together share row panels of A and column panels of B in its L2.
-  // With a K split the (super-block, split) pairs are numbered the same way: the splits of one super-block land on
-  // different XCDs (a shape with a single super-block would otherwise keep all its workgroups on one).
-  const int sbm = 1 << sbm_log2, sbn = 32 >> sbm_log2;
-  const int sb_m = (tiles_m + sbm - 1) >> sbm_log2;
-  const int sb_count = sb_m * ((tiles_n + sbn - 1) / sbn);
-  const int j_in_xcd = (int)(blockIdx.x >> 3);
-  const int pair = (j_in_xcd >> 5) * 8 + (int)(blockIdx.x & 7);
-  const int sb = pair % sb_count, ksplit = pair / sb_count;
-  const int tm = (sb % sb_m) * sbm + (j_in_xcd & (sbm - 1)), tn = (sb / sb_m) * sbn + ((j_in_xcd & 31) >> sbm_log2);
-  if (tm >= tiles_m || tn >= tiles_n || ksplit >= p.splits) return;
+  // XCD-aware tile numbering: tiles are numbered down bands of eight row tiles, column by column, the parts of a K split one
+  // behind the other; an XCD (workgroup ids equal modulo 8) takes an eighth of them in a row: the neighbours that it runs
+  // together share row panels of A and column panels of B in its L2, and no XCD has more than its share.
+  const int tiles = tiles_m * tiles_n, all = tiles * p.splits, share = (all + 7) >> 3;
+  int t = (int)(blockIdx.x & 7) * share + (int)(blockIdx.x >> 3);
+  if (t >= all) return;
+  const int ksplit = t / tiles;
+  t -= ksplit * tiles;
+  const int band = t / (8 * tiles_n), in_band = t - band * 8 * tiles_n, band_rows = min(8, tiles_m - 8 * band);
+  const int tn = in_band / band_rows, tm = 8 * band + in_band % band_rows;
   const int m0 = tm * BM, n0 = p.col0 + tn * BN;
   const int kt_lo = ksplit * p.kt_per;
   const int kt_n = min(p.kt - kt_lo, p.kt_per);
@@ -559,13 +556,9 @@ int32_t ring_launch_one(const RingArgs &a, hipStream_t s) {
   if (attr_err != hipSuccess)
     return set_error(YSCV_HIP_ERR_DEVICE, "cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(attr_err));
   const int tiles_m = (int)ceil_div((size_t)a.m, (size_t)(32 * MT)), tiles_n = (int)ceil_div((size_t)(a.n - a.col0), (size_t)(32 * NT));
-  int sbm_log2 = 3;
-  while (sbm_log2 > 0 && (1 << sbm_log2) > tiles_m) sbm_log2--;
-  const int sbm = 1 << sbm_log2, sbn = 32 >> sbm_log2;
-  const int super_blocks = ((tiles_m + sbm - 1) / sbm) * ((tiles_n + sbn - 1) / sbn);
   const unsigned splits = (unsigned)a.splits;
-  const unsigned grid = (unsigned)((super_blocks * splits + 7) / 8) * 8 * 32;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256 + 64 * NP), LDS, s, a, tiles_m, tiles_n, sbm_log2);
+  const unsigned grid = ((unsigned)(tiles_m * tiles_n) * splits + 7) / 8 * 8;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256 + 64 * NP), LDS, s, a, tiles_m, tiles_n);
   YSCV_HIP_TRY(hipGetLastError());
   if (a.partial) return launch_int4_partial_sum(a.partial, (int)splits, a.m, a.n, a.y, a.y_dtype, a.epi, s);
   return YSCV_HIP_OK;
@@ -679,23 +672,16 @@ RingPlan ring_plan(size_t m, size_t n, size_t kt, size_t cus) {
   // K split: a shape whose tiles cover at most half the CUs is cut along k, each part with at least four 128-k tiles
   // (eight stages), as long as the f32 partial sums stay within 16 MB and, together with a prepared fp16 copy of the
   // activations, within 31 MB (they travel in the caller's workspace; yscv_hip_int4_matmul_static has 32 MB for
-  // both).  The workgroups of one
-  // (super-block, split) pair share an XCD, eight pairs run side by side: the number of splits is the one with the
-  // shortest estimated time, rounds of eight pairs x (a part's k-tiles at 0.9 us each + 5 us to start and end a
-  // workgroup), + 5 us for the kernel that adds the parts.
+  // both).  The number of splits is the one with the shortest estimated time, rounds over the CUs x (a part's k-tiles at
+  // 0.9 us each + 5 us to start and end a workgroup), + 5 us for the kernel that adds the parts.
   if (tiles * 2 <= cus && kt >= 8) {
-    const size_t bm = pl.one == 3 ? 32 : (pl.one == 4 ? 64 : (pl.one == 2 ? 256 : 128)), bn = pl.one == 1 ? 256 : 128;
-    const size_t tiles_m = ceil_div(m, bm), tiles_n = ceil_div(n, bn);
-    size_t sbm = 8;
-    while (sbm > 1 && sbm > tiles_m) sbm >>= 1;
-    const size_t sb = ceil_div(tiles_m, sbm) * ceil_div(tiles_n, 32 / sbm);
-    size_t best_ks = 1, best_t = ceil_div(sb, (size_t)8) * (kt * 18 + 100);  // units of 0.05 us
+    size_t best_ks = 1, best_t = kt * 18 + 100;  // units of 0.05 us
     const size_t x_bytes = m * kt * 128 * sizeof(_Float16);
     const size_t room = x_bytes >= ((size_t)31 << 20) ? 0 : ((size_t)31 << 20) - x_bytes;
     const size_t cap = room < ((size_t)16 << 20) ? room : ((size_t)16 << 20);
     for (size_t ks = 2; ks <= 16 && ks <= kt / 4; ks++) {
       if (ks * m * n * sizeof(float) > cap) break;
-      const size_t t = ceil_div(sb * ks, (size_t)8) * (ceil_div(kt, ks) * 18 + 100) + 100;
+      const size_t t = ceil_div(tiles * ks, cus) * (ceil_div(kt, ks) * 18 + 100) + 100;
       if (t < best_t) {
         best_t = t;
         best_ks = ks;
