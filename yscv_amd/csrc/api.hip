@@ -104,11 +104,23 @@ struct Int4Scratch {
 // f32 activations on the exact-scale route with 16 < m <= this many rows run as 16-row skinny calls
 constexpr size_t kChunkedSkinnyMaxRows = 128;
 
+static Int4Scratch int4_scratch_layout(const yscv_hip_int4_weight *w, const void *x, int x_dtype, const void *y, int y_dtype, size_t m,
+                                       int force, int num_cus);
+// Rows of one launch of that route: all of them, or the most groups of 16 whose scratch stays within that of one group or
+// 16 MB (the static-scratch entry point has 32 MB)
+static size_t int4_chunked_rows(const yscv_hip_int4_weight *w, const void *x, int x_dtype, const void *y, int y_dtype, size_t m,
+                                int num_cus, size_t room = (size_t)16 << 20) {
+  size_t rows = round_up(m, 16);
+  room = std::max(room, int4_scratch_layout(w, x, x_dtype, y, y_dtype, 16, 3, num_cus).total);
+  while (rows > 16 && int4_scratch_layout(w, x, x_dtype, y, y_dtype, rows, 3, num_cus).total > room) rows -= 16;
+  return rows;
+}
+
 // y == null asks for the size of a workspace: activations of a K that is no multiple of 512 may then come on any alignment
 static Int4Scratch int4_scratch_layout(const yscv_hip_int4_weight *w, const void *x, int x_dtype, const void *y, int y_dtype,
                                        size_t m, int force, int num_cus) {
   Int4Scratch L{};
-  L.skinny = force == 1 || (force == 0 && m <= 16);
+  L.skinny = force == 1 || force == 3 || (force == 0 && m <= 16);
   const size_t k_pad = w->ktp * 128;
   const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (y != nullptr || k_pad == w->k);
   // f32 activations with more than 16 rows against a weight whose scales are stored as fp16 (the MatMulNBits form) go
@@ -142,9 +154,8 @@ static Int4Scratch int4_scratch_layout(const yscv_hip_int4_weight *w, const void
     L.opt_bytes = round_up(opt, 256);
   }
   if (!L.skinny && force == 0 && x_dtype == YSCV_HIP_F32 && m <= kChunkedSkinnyMaxRows) {
-    // this call may run as 16-row skinny calls (see int4_run_ws): the scratch must cover one of those too
-    const Int4Scratch c = int4_scratch_layout(w, x, x_dtype, y, y_dtype, 16, 1, num_cus);
-    if (c.total > L.total) L.total = c.total;
+    // this call may run on the skinny kernel (see int4_run_ws): the scratch must cover a launch of that too
+    L.total = std::max(L.total, int4_scratch_layout(w, x, x_dtype, y, y_dtype, int4_chunked_rows(w, x, x_dtype, y, y_dtype, m, num_cus), 3, num_cus).total);
   }
   return L;
 }
@@ -168,7 +179,7 @@ int32_t int4_workspace_bytes(const yscv_hip_int4_weight *w, size_t m, int x_dtyp
 // `ws` may be null: scratch then comes from the blocks the library keeps per stream (scratch.hip), so concurrent
 // callers on different streams never share it.
 int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y, int y_dtype, size_t m,
-                    int force /*0 auto, 1 skinny, 2 gemm*/, int epi, void *ws, size_t ws_bytes, hipStream_t s,
+                    int force /*0 auto, 1 skinny, 2 gemm, 3 skinny in groups of 16 rows (f32)*/, int epi, void *ws, size_t ws_bytes, hipStream_t s,
                     const NormFold *nf) {
   const Context *ctx = nullptr;
   YSCV_TRY(ensure_context(&ctx));
@@ -190,16 +201,20 @@ int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, v
   if (!L.skinny && epi != EPI_STORE && !(x_dtype != YSCV_HIP_F32 && nf == nullptr))
     return set_error(YSCV_HIP_ERR_UNSUPPORTED, "fused epilogues above 16 rows need 16-bit activations");
   // f32 activations that stay on the exact-scale route (f32 scales, or an output the ring GEMM cannot take): up to
-  // 128 rows go through the skinny kernel 16 rows at a time.  Each pass streams the weights again, which is still
-  // 5-10 x faster than the exact-scale GEMM kernel there: that one keeps a 64 x 256 tile per workgroup and cannot fill
-  // the GPU with so few rows (m = 64 against 14336 x 4096: 432 us; four skinny passes: about 60 us).
+  // 128 rows go through the skinny kernel in groups of 16 rows, side by side in one launch.  Each group streams the weights
+  // again, which is still 5-10 x faster than the exact-scale GEMM kernel there: that one keeps a 64 x 256 tile per workgroup
+  // and cannot fill the GPU with so few rows (m = 64 against 14336 x 4096: 432 us; four skinny passes: about 60 us).
+  // One launch instead of one per group (us, m x n x k): 81 x 358 x 5056 155 -> 19.5, 100 x 1000 x 1024 44 -> 10, 24 x 60000 x
+  // 1024 52 -> 36, 128 x 14336 x 4096 138 -> 111: a launch and the ramp per group, and most CUs idle where N is small.
   if (!L.skinny && force == 0 && x_dtype == YSCV_HIP_F32 && m <= kChunkedSkinnyMaxRows) {
     if (!L.fast16) {
       const size_t ysz = dtype_size(y_dtype);
-      for (size_t r0 = 0; r0 < m; r0 += 16) {
-        const size_t rows = m - r0 < 16 ? m - r0 : 16;
+      const size_t step = ws ? int4_chunked_rows(w, x, x_dtype, y, y_dtype, m, ctx->num_cus, std::min(ws_bytes, (size_t)16 << 20))
+                             : int4_chunked_rows(w, x, x_dtype, y, y_dtype, m, ctx->num_cus);
+      for (size_t r0 = 0; r0 < m; r0 += step) {
+        const size_t rows = std::min(m - r0, step);
         YSCV_TRY(int4_run_ws(w, static_cast<const char *>(x) + r0 * w->k * sizeof(float), x_dtype,
-                             static_cast<char *>(y) + r0 * w->n * ysz, y_dtype, rows, 1, epi, ws, ws_bytes, s));
+                             static_cast<char *>(y) + r0 * w->n * ysz, y_dtype, rows, rows > 16 ? 3 : 1, epi, ws, ws_bytes, s));
       }
       return YSCV_HIP_OK;
     }

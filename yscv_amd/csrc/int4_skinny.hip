@@ -145,6 +145,18 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
   nc.init();
 
   // ---- per-wave stream pointers (advance by one grid stride of 16-row blocks per iteration) ----
+  // more than 16 rows (f32 only): blockIdx.z takes sixteen of them
+  const int m_all = a.m;
+  if constexpr (SPLIT == 2 && NI == 4) {
+    const int r0 = (int)blockIdx.z * 16;
+    a.m = min(16, a.m - r0);
+    if (a.xf) a.xf += (size_t)r0 * a.ldx;
+    a.xh += (size_t)r0 * a.ldx;
+    a.xl += (size_t)r0 * a.ldx;
+    if (a.row_scale) a.row_scale += r0;
+    if (a.partial) a.partial += (size_t)r0 * a.n;
+    a.y = static_cast<char *>(a.y) + (size_t)r0 * a.n * (a.y_dtype == YSCV_HIP_F32 ? 4 : 2);
+  }
   const int stride = gridDim.x;
   const size_t w_step = (size_t)stride * a.ktp * kTileBytes;
   const size_t s_step = (size_t)stride * a.chunks * 16 * SC_BYTES;
@@ -640,7 +652,7 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
       const int mrow = c * NI + i;
       const bool live = mrow < a.m && col < a.n;
       if (a.ksg > 1) {
-        if (live) a.partial[((size_t)blockIdx.y * a.m + mrow) * a.n + col] = v;
+        if (live) a.partial[((size_t)blockIdx.y * m_all + mrow) * a.n + col] = v;
       } else {
         float rsv = rs[0];
 #pragma unroll
@@ -870,6 +882,12 @@ SkinnyPlan plan_int4_skinny(const yscv_hip_int4_weight *w, size_t m, int split, 
   return p;
 }
 
+// groups of 16 rows: the f32 form takes several side by side
+template <int SPLIT, int NI>
+static unsigned skinny_groups(const SkinnyArgs &a) {
+  return SPLIT == 2 && NI == 4 ? (unsigned)((a.m + 15) / 16) : 1u;
+}
+
 template <int SPLIT, int NI, int GM, bool SF16, bool HAS_ZP, int P>
 static int32_t launch_p(const SkinnyArgs &a, const SkinnyPlan &plan, hipStream_t s) {
   constexpr int UB = skinny_ub(NI, P);
@@ -887,20 +905,20 @@ static int32_t launch_p(const SkinnyArgs &a, const SkinnyPlan &plan, hipStream_t
         if (attr_err != hipSuccess)
           return set_error(YSCV_HIP_ERR_DEVICE, "cannot reserve LDS for the activation staging: %s", hipGetErrorString(attr_err));
       }
-      hipLaunchKernelGGL((int4_skinny_kernel<SPLIT, NI, GM, SF16, HAS_ZP, P, 1>), dim3(plan.grid_x, plan.ksg),
+      hipLaunchKernelGGL((int4_skinny_kernel<SPLIT, NI, GM, SF16, HAS_ZP, P, 1>), dim3(plan.grid_x, plan.ksg, skinny_groups<SPLIT, NI>(a)),
                          dim3(plan.waves * 64), lds + stage, s, a);
       YSCV_HIP_TRY(hipGetLastError());
       return YSCV_HIP_OK;
     }
   } else {
     if (a.xb != nullptr) {
-      hipLaunchKernelGGL((int4_skinny_kernel<SPLIT, NI, GM, SF16, HAS_ZP, P, 2>), dim3(plan.grid_x, plan.ksg),
+      hipLaunchKernelGGL((int4_skinny_kernel<SPLIT, NI, GM, SF16, HAS_ZP, P, 2>), dim3(plan.grid_x, plan.ksg, skinny_groups<SPLIT, NI>(a)),
                          dim3(plan.waves * 64), lds, s, a);
       YSCV_HIP_TRY(hipGetLastError());
       return YSCV_HIP_OK;
     }
   }
-  hipLaunchKernelGGL((int4_skinny_kernel<SPLIT, NI, GM, SF16, HAS_ZP, P, 0>), dim3(plan.grid_x, plan.ksg),
+  hipLaunchKernelGGL((int4_skinny_kernel<SPLIT, NI, GM, SF16, HAS_ZP, P, 0>), dim3(plan.grid_x, plan.ksg, skinny_groups<SPLIT, NI>(a)),
                      dim3(plan.waves * 64), lds, s, a);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
@@ -947,7 +965,8 @@ int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan
                            const _Float16 *xl, const void *xraw, const float *row_scale, size_t ldx, int split,
                            void *y, int y_dtype, size_t m, float *partial, int epi, hipStream_t s, const NormFold *nf) {
   if (!w->tiled) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "skinny int4 kernel needs the tiled layout");
-  if (m == 0 || m > 16) return set_error(YSCV_HIP_ERR_INVALID_ARG, "skinny int4 kernel handles 1 <= m <= 16, got %zu", m);
+  if (m == 0 || (m > 16 && (split != 2 || epi != EPI_STORE || nf)))
+    return set_error(YSCV_HIP_ERR_INVALID_ARG, "skinny int4 kernel handles 1 <= m <= 16, got %zu", m);
   if (plan.ksg > 1 && !partial) return set_error(YSCV_HIP_ERR_INVALID_ARG, "k-split needs a partial buffer");
   if (ldx < w->k || w->k % 32 != 0 || (split == 2 && xraw && m > 4 && w->k % 512 != 0))
     return set_error(YSCV_HIP_ERR_INVALID_ARG, "activation row stride %zu for K %zu", ldx, w->k);
