@@ -53,6 +53,21 @@ __global__ void __launch_bounds__(64 * WAVES) i8_ksplit_kernel(I8Args p, int til
   const int pairs = (p.ksteps + 1) >> 1;
   const int q_lo = pairs * wave / WAVES, q_hi = pairs * (wave + 1) / WAVES;
 
+  // The per-column terms of the epilogue: a thread stores the same four columns of every row it stores, so they are requested
+  // once and ahead of the loop (197 x 3072 x 768 requantised: 8.3 us with these loads behind it, 7.0 with them here).
+  constexpr int CPR = 4 * NT;  // pieces of four columns in a row of the tile
+  static_assert(64 * WAVES % CPR == 0, "a thread keeps its columns from row to row");
+  const int col = nb0 * 16 + tid % CPR * 4;
+  int32_t zc[4], corr[4];
+  float comp[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int cc = min(col + e, p.n - 1);
+    zc[e] = p.col_sum[cc];
+    corr[e] = p.corr ? p.corr[cc] : 0;
+    comp[e] = p.composite_v ? p.composite_v[cc] : p.composite;
+  }
+
   int4_t acc[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; i++)
@@ -139,7 +154,7 @@ __global__ void __launch_bounds__(64 * WAVES) i8_ksplit_kernel(I8Args p, int til
   }
 
   // ---- the waves' tiles meet in LDS and leave as whole rows ------------------------------------------------------------
-  constexpr int RS = iks_row_ints(NT), ROWS = 16 * MT, CPR = 4 * NT;
+  constexpr int RS = iks_row_ints(NT), ROWS = 16 * MT;
   __syncthreads();  // every wave has read its last slot
   int32_t *red = reinterpret_cast<int32_t *>(iks_ring);
 #pragma unroll
@@ -151,21 +166,14 @@ __global__ void __launch_bounds__(64 * WAVES) i8_ksplit_kernel(I8Args p, int til
   const int zp_mul = p.a_zp_dev ? 128 - (int)p.a_zp_dev[0] : p.zp_mul;
   const bool vec = (p.n & 3) == 0;
   for (int u = tid; u < ROWS * CPR; u += 64 * WAVES) {
-    const int lrow = u / CPR, row = m0 + lrow, col = nb0 * 16 + u % CPR * 4;
+    const int lrow = u / CPR, row = m0 + lrow;
     if (row >= p.m || col >= p.n) continue;
-    const int32_t *src = red + lrow * RS + u % CPR * 4;
+    const int32_t *src = red + lrow * RS + tid % CPR * 4;
     int4_t v = *reinterpret_cast<const int4_t *>(src);
 #pragma unroll
     for (int w = 1; w < WAVES; w++) v += *reinterpret_cast<const int4_t *>(src + w * ROWS * RS);
-    int32_t corr[4];
-    float comp[4];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int cc = min(col + e, p.n - 1);
-      v[e] = (int32_t)((uint32_t)v[e] + (uint32_t)zp_mul * (uint32_t)p.col_sum[cc]);
-      corr[e] = p.corr ? p.corr[cc] : 0;
-      comp[e] = p.composite_v ? p.composite_v[cc] : p.composite;
-    }
+    for (int e = 0; e < 4; e++) v[e] = (int32_t)((uint32_t)v[e] + (uint32_t)zp_mul * (uint32_t)zc[e]);
     const size_t o = (size_t)row * p.n + col;
     if (p.mode == 1) {
       uint32_t packed = 0;
