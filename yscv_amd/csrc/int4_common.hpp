@@ -101,14 +101,16 @@ struct NibbleConsts {
   }
 };
 
-// raw fp16 forms of the 8 weights of one word: {1024+q0, 1024+q1, 1024+16 q2, 1024+16 q3, ...}
-__device__ __forceinline__ half8_t extract8(uint32_t s, const NibbleConsts &nc) {
+// raw fp16 forms of the 8 weights of one word: {1024+q0, 1024+q1, 64+q2, 64+q3, ...} (magic_hi: 0x54005400, in a register
+// like the others).  In [64, 128) the last bit of an fp16 is 1/16, so 0x5400 | (q << 4) is 64 + q: the activations meet
+// both forms as they are.
+__device__ __forceinline__ half8_t extract8(uint32_t s, const NibbleConsts &nc, uint32_t magic_hi) {
   U32H2 r0, r1, r2, r3;
   const uint32_t s2 = s >> 8;
   r0.u = (s & nc.lo) | nc.magic;
-  r1.u = (s & nc.hi) | nc.magic;
+  r1.u = (s & nc.hi) | magic_hi;
   r2.u = (s2 & nc.lo) | nc.magic;
-  r3.u = (s2 & nc.hi) | nc.magic;
+  r3.u = (s2 & nc.hi) | magic_hi;
   half8_t out;
   out[0] = r0.h[0];
   out[1] = r0.h[1];

@@ -15,16 +15,17 @@
 //     already in MFMA A-operand order: the inner loop reads neither LDS nor L2 for them;
 //   * v_mfma_f32_16x16x32_f16 does the dot products (A = up to 16 activation rows, B = 16 weight
 //     rows), one MFMA per 32-k block = one quantisation group when group_size is 32;
-//   * nibbles become fp16 with one v_and_or_b32 per pair: 0x6400 | q = 1024 + q and
-//     0x6400 | (q << 4) = 1024 + 16 q.  For symmetric weights (zero point 8) and fp16/bf16
-//     activations the offsets are not subtracted per weight: the activation slots that meet the
-//     16 q form are pre-divided by 16, and the offset term sum_k x_k * (1024 + 8 or 1024 + 128)
+//   * nibbles become fp16 with one v_and_or_b32 per pair.  For symmetric weights (zero point 8)
+//     and fp16/bf16 activations that is all: 0x6400 | q = 1024 + q, 0x5400 | (q << 4) = 64 + q, and
+//     the offsets are not subtracted per weight.  The offset term sum_k x_k * (1024 + 8 or 64 + 8)
 //     -- which does not depend on the weight row -- is computed once per kernel by the same MFMA
-//     against a constant operand.  With m <= 4 it is subtracted from each group's result; with
+//     against a constant operand.  The activations stay as they are, whatever their magnitude: the
+//     one form 0x6400 | (q << 4) = 1024 + 16 q for the high nibbles would want x / 16 against it, and
+//     an fp16 x below 2^-10 loses bits there (2e-2 of a row of standard deviation 1e-5).  With m <= 4 it is subtracted from each group's result; with
 //     m > 4 (four useful accumulators per lane) the products -offset[row][block] * scale[n][block]
 //     of a whole 16-row block are added by four v_mfma_f32_16x16x4_f32 at the end of the block.
-//     With explicit zero points or f32 activations the offsets are subtracted exactly in fp16
-//     before the MFMA;
+//     With explicit zero points or f32 activations both nibbles take 0x6400 and the offsets are
+//     subtracted exactly in fp16 before the MFMA;
 //   * group scales are applied in fp32 to the MFMA result (acc += scale * D);
 //   * K is split across the wavefronts of a workgroup (each wave owns 512 k of the activations);
 //     the per-wave partial sums meet in LDS behind an LDS-only barrier, once per four 16-row blocks
@@ -143,6 +144,8 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
   const int t0 = (wave_active ? slice : 0) * TPW;  // first 128-k tile of the slice
   NibbleConsts nc;
   nc.init();
+  uint32_t magic_hi = 0x54005400u;
+  if constexpr (OFFSET) asm volatile("" : "+v"(magic_hi));  // as NibbleConsts
 
   // ---- per-wave stream pointers (advance by one grid stride of 16-row blocks per iteration) ----
   // more than 16 rows (f32 only): blockIdx.z takes sixteen of them
@@ -258,8 +261,6 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
     const int i = r & 3;
     const int mrow = (r >> 2) * NI + i;
     const bool valid = wave_active && (i < NI) && (mrow < a.m);
-    const half8_t pre = {(_Float16)1.0f, (_Float16)1.0f, (_Float16)0.0625f, (_Float16)0.0625f,
-                         (_Float16)1.0f, (_Float16)1.0f, (_Float16)0.0625f, (_Float16)0.0625f};
     if constexpr (XM == 2) {
       // bf16 activations straight from the caller: the wave scales its own 512-k slice of every row by a power of
       // two (abs-max to [2^14, 2^15)), which makes every bf16 value an exact fp16 one (8 significant bits; only
@@ -317,7 +318,6 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
             h[2 * e + 1] = (_Float16)(__uint_as_float(wd & 0xFFFF0000u) * up);
           }
           if (!valid) h = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-          if constexpr (OFFSET) h = h * pre;
           xa[t][j][0] = h;
         }
       }
@@ -468,7 +468,6 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           if (!valid) xa[t][j][0] = hz;
-          if constexpr (OFFSET) xa[t][j][0] = xa[t][j][0] * pre;  // slots that meet 1024 + 16 q carry x / 16 (a power of two)
           if constexpr (SPLIT == 2) {
             if (!valid) xa[t][j][1] = hz;
           }
@@ -503,15 +502,15 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
 #pragma unroll
   for (int i = 0; i < NI; i++)
     acc_scale[i] = RAWX ? __shfl(slice_scale, (XM == 1 && NI == 1) ? 16 * c : 4 * c + i, 64) : 1.0f;
-  // offset term of every 32-k block: sum_k x'_k * (1024 + 8 | 1024 + 128), same register layout as D
+  // offset term of every 32-k block: sum_k x_k * (1024 + 8 | 64 + 8), same register layout as D
   float corr1[OFFSET1 ? TPW : 1][4];
   // OFFSETC: minus the offset term of MFMA row r and 32-k block (t, j = c), i.e. in the A-operand layout of
   // v_mfma_f32_16x16x4_f32: at the end of a 16-row block, four of those MFMAs (one per tile, B = the scale that
   // applies to weight row r in 32-k block c) add sum_blocks -offset * scale to all four accumulators at once.
   float ncorr_a[OFFSETC ? TPW : 1];
   if constexpr (OFFSET) {
-    const half8_t bc = {(_Float16)1032.0f, (_Float16)1032.0f, (_Float16)1152.0f, (_Float16)1152.0f,
-                        (_Float16)1032.0f, (_Float16)1032.0f, (_Float16)1152.0f, (_Float16)1152.0f};
+    const half8_t bc = {(_Float16)1032.0f, (_Float16)1032.0f, (_Float16)72.0f, (_Float16)72.0f,
+                        (_Float16)1032.0f, (_Float16)1032.0f, (_Float16)72.0f, (_Float16)72.0f};
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
       float sel = 0.0f;
@@ -548,7 +547,7 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
         for (int j = 0; j < 4; j++) {
           half8_t b;
           if constexpr (OFFSET) {
-            b = extract8(tr.w[t][j], nc);
+            b = extract8(tr.w[t][j], nc, magic_hi);
           } else {
             half2_t c1 = {(_Float16)(-1032.0f), (_Float16)(-1032.0f)};
             half2_t c2 = {(_Float16)(-72.0f), (_Float16)(-72.0f)};
@@ -577,7 +576,7 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
         const bool group_end = GM == GM32 || (GM == GM64 && (j & 1)) || (GM == GM128 && j == 3);
         half8_t b;
         if constexpr (OFFSET) {
-          b = extract8(tr.w[t][j], nc);
+          b = extract8(tr.w[t][j], nc, magic_hi);
           if constexpr (OFFSET1) csum = group_start ? corr1[t][j] : csum + corr1[t][j];
         } else {
           half2_t c1 = {(_Float16)(-1032.0f), (_Float16)(-1032.0f)};
