@@ -12,8 +12,11 @@ from isa_lint import copies_of_inflight_registers, scratch_bytes_per_kernel
 CSRC = os.path.join(os.path.dirname(__file__), "..", "yscv_amd", "csrc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Xclang", "-target-feature",
          "-Xclang", "-packed-fp32-ops", "-S", "--cuda-device-only"]
-# the sources with asm loads whose wait is a separate statement, and their extra flags in the Makefile
-SOURCES = {"int4_gemm_ring.hip": [], "decode_persistent.hip": [], "i8_gemm.hip": ["-ffp-contract=off"]}
+# the sources with asm loads or hand-counted waits, and their extra flags in the Makefile
+SOURCES = {"int4_gemm_ring.hip": [], "decode_persistent.hip": [], "i8_gemm.hip": ["-ffp-contract=off"], "int4_gemm_wide.hip": [],
+           "int4_ksplit.hip": [], "i8_ksplit.hip": ["-ffp-contract=off"], "glue_ops.hip": []}
+# kernels whose pipeline counts on every value staying in registers
+PIPELINED = ("gemm_ring_kernel", "gemm_wide_kernel", "int4_ksplit_kernel", "i8_ksplit_kernel", "gqa_flat_kernel")
 
 
 def test_checker_sees_a_copy_between_load_and_wait():
@@ -41,21 +44,25 @@ def test_no_register_of_a_load_in_flight_is_moved(tmp_path):
         assert proc.returncode == 0, proc.stdout[-2000:]
         return name, out.read_text()
 
-    with ThreadPoolExecutor(max_workers=3) as pool:
+    with ThreadPoolExecutor(max_workers=4) as pool:
         results = list(pool.map(compile_one, SOURCES.items()))
-    report = []
+    report, seen = [], set()
     for name, text in results:
         hits = copies_of_inflight_registers(text)
         if hits:
             report.append(f"{name}: {len(hits)} moves of registers whose load is in flight, first {hits[0]}")
-        # The LDS-ring GEMMs count their loads in flight with literal wait counts and name the registers of pending
-        # loads in asm statements: an instantiation that spills (a tile whose accumulators, fragments and epilogue terms
-        # exceed the 256 registers two waves per SIMD leave each) gets scratch traffic on the same counter and spill
-        # code the pipeline was not written for.  Every instantiation in the library must fit its registers.
-        for kern, scratch in scratch_bytes_per_kernel(text).items():
-            if ("gemm_ring_kernel" in kern) and scratch != 0:
+        # These kernels count their loads in flight with literal wait counts, name the registers of pending loads in asm
+        # statements or hold the next stage's loads in registers over the current one: an instantiation that spills (a
+        # tile whose accumulators, fragments and epilogue terms exceed the 256 registers two waves per SIMD leave each)
+        # gets scratch traffic on the same counter and spill code the pipeline was not written for.  Every instantiation
+        # in the library must fit its registers.
+        kernels = scratch_bytes_per_kernel(text)
+        seen.update(p for p in PIPELINED if any(p in kern for kern in kernels))
+        for kern, scratch in kernels.items():
+            if any(p in kern for p in PIPELINED) and scratch != 0:
                 report.append(f"{name}: {kern} uses {scratch} bytes of scratch per lane (register spills in a pipelined kernel)")
     assert not report, "\n".join(report)
+    assert seen == set(PIPELINED)  # a renamed kernel would otherwise drop out unnoticed
 
 
 def test_scratch_parser():
