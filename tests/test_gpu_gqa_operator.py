@@ -49,6 +49,25 @@ def test_operator_against_float32(B, Sq, Sk, hq, hkv, d):
     assert torch.equal(got, ops.exec_grouped_query_attention(q, k, v, hq, hkv))
 
 
+@pytest.mark.parametrize("B,Sq,hq,hkv", [
+    (1, (1 << 24) - 1, 2, 1),   # more rows per kv head than one launch takes: the second one starts inside the sequence
+    (65535, 1, 130, 130),       # more (sequence, kv head) problems than one launch takes
+])
+def test_more_rows_or_problems_than_one_launch_takes(B, Sq, hq, hkv):
+    import torch
+
+    from yscv_amd import onnx_ops as ops
+
+    q = torch.randn(B, Sq, hq * 32, device="cuda")
+    k = torch.randn(B, 1, hkv * 32, device="cuda")
+    # one key: the result is its value (rounded to fp16) over the softmax sum, one weight: 2^(s - round(s)) in f32, where
+    # |s| is below 16 (32 channels ~N(0, 1), scaled), so 1 up to 16 * 2^-24, and one more rounding
+    v = torch.randn(B, 1, hkv * 32, device="cuda").half().float()
+    got = ops.exec_grouped_query_attention(q, k, v, hq, hkv)
+    want = v.view(B, 1, hkv, 1, 32).expand(B, 1, hkv, hq // hkv, 32).reshape(B, 1, hq * 32)
+    assert bool(((got - want).abs() <= 17 * 2.0**-24 * want.abs()).all())
+
+
 def test_values_on_four_byte_alignment():
     import torch
 

@@ -543,7 +543,7 @@ struct FlatCfg {
 struct FlatArgs {
   const float *q, *k, *v;
   float *out, *part;       // part: [b * Hkv][gs][R][HD + 2] when gs > 1 (un-normalised output, maximum, sum)
-  int Sq, Sk, Hq, Hkv, group, R, gs;
+  int Sq, Sk, Hq, Hkv, group, R, gs;  // Sq: query positions from one sequence to the next; R: rows of this launch
   int v16;                 // v is 16-byte aligned
   uint32_t magic;          // ceil(2^32 / group): row / group = the high half of row * magic (0: divide)
   float scale;             // log2(e) / sqrt(head width)
@@ -1180,10 +1180,6 @@ int32_t yscv_hip_gqa_attention_dev(const float *q, const float *k, const float *
   const Context *ctx = nullptr;
   YSCV_TRY(ensure_context(&ctx));
   FlatArgs p{};
-  p.q = q;
-  p.k = k;
-  p.v = v;
-  p.out = out;
   p.Sq = (int)seq_q;
   p.Sk = (int)seq_k;
   p.Hq = (int)num_q_heads;
@@ -1193,17 +1189,28 @@ int32_t yscv_hip_gqa_attention_dev(const float *q, const float *k, const float *
   p.scale = 1.44269504f / sqrtf((float)d_head);
   // exact while row * group < 2^32
   p.magic = p.group > 1 && p.group <= 256 ? (uint32_t)((((uint64_t)1 << 32) + p.group - 1) / p.group) : 0;
-  const uint64_t rows = (uint64_t)p.group * seq_q;
-  YSCV_REQUIRE(rows <= (uint64_t)65535 * 256 && batch * num_kv_heads < ((uint64_t)1 << 31) && batch * num_q_heads * seq_q * d_head < ((uint64_t)1 << 38),
-               "GroupQueryAttention: shape too large");
-  p.R = (int)rows;
-  switch (d_head) {
-    case 32: return gqa_flat_launch<32>(p, (int)batch, ctx->num_cus, as_stream(stream));
-    case 64: return gqa_flat_launch<64>(p, (int)batch, ctx->num_cus, as_stream(stream));
-    case 96: return gqa_flat_launch<96>(p, (int)batch, ctx->num_cus, as_stream(stream));
-    case 128: return gqa_flat_launch<128>(p, (int)batch, ctx->num_cus, as_stream(stream));
-    default: return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention: head width %zu (supported: 32, 64, 96, 128)", d_head);
+  // What one launch takes: 2^22 problems (2^32 threads along x) and 65535 workgroups of 256 rows along y.  Sequences and
+  // query positions beyond that go in further launches.
+  const size_t b_step = std::max<size_t>(1, ((size_t)1 << 22) / num_kv_heads), q_step = (size_t)65535 * 256 / p.group;
+  for (size_t b0 = 0; b0 < batch; b0 += b_step) {
+    for (size_t q0 = 0; q0 < seq_q; q0 += q_step) {
+      const int bs = (int)std::min(b_step, batch - b0);
+      p.R = p.group * (int)std::min(q_step, seq_q - q0);
+      const size_t q_at = (b0 * seq_q + q0) * num_q_heads * d_head, kv_at = b0 * seq_k * num_kv_heads * d_head;
+      p.q = q + q_at;
+      p.out = out + q_at;
+      p.k = k + kv_at;
+      p.v = v + kv_at;
+      switch (d_head) {
+        case 32: YSCV_TRY(gqa_flat_launch<32>(p, bs, ctx->num_cus, as_stream(stream))); break;
+        case 64: YSCV_TRY(gqa_flat_launch<64>(p, bs, ctx->num_cus, as_stream(stream))); break;
+        case 96: YSCV_TRY(gqa_flat_launch<96>(p, bs, ctx->num_cus, as_stream(stream))); break;
+        case 128: YSCV_TRY(gqa_flat_launch<128>(p, bs, ctx->num_cus, as_stream(stream))); break;
+        default: return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention: head width %zu (supported: 32, 64, 96, 128)", d_head);
+      }
+    }
   }
+  return YSCV_HIP_OK;
 }
 
 }  // extern "C"
