@@ -85,3 +85,51 @@ def test_f32_operators_with_copied_rows(m, k, n):
     assert float(scale) == float(s2) and float(zp) == float(z2)
     want = (q.cpu().numpy().astype(np.float64).reshape(m, k) - float(zp)) @ b.astype(np.float64)
     assert np.array_equal(got.cpu().numpy().reshape(m, n), want.astype(np.float32))
+
+
+def test_a_long_matrix_is_copied_in_bounded_pieces():
+    """800 MB of rows with a K that is no multiple of 64: the copy stays within the 64 MB block that is kept."""
+    import torch
+
+    from yscv_amd import kernels as K
+
+    rng = np.random.default_rng(3)
+    m, k, n = 200_003, 4001, 48
+    b = rng.integers(-127, 128, (k, n), dtype=np.int8)
+    w = K.pack_i8_b_for_matmul(b, k, n)
+    a = torch.randint(0, 256, (m, k), device="cuda", dtype=torch.uint8)
+    out = torch.empty(m, n, device="cuda", dtype=torch.int32)
+    free = torch.cuda.mem_get_info()[0]
+    w.matmul(a, a_zp=7, out=out)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= 160 << 20  # the block and what the allocator rounds up to
+    step = (64 << 20) // 4032 // 16 * 16
+    rows = [0, m - 1] + [r for at in range(step, m, step) for r in (at - 1, at)]
+    want = _exact(a[rows].cpu().numpy(), b, 7)
+    assert np.array_equal(out[rows].cpu().numpy(), want.astype(np.int32))
+
+
+@pytest.mark.parametrize("m,k,n", [(40, 77, 130), (300, 1001, 520)])
+def test_capture_of_rows_that_would_be_copied(m, k, n):
+    """A graph needs no memory for them: the kernel that reads any row runs there, with the same bytes as a result."""
+    import torch
+
+    from yscv_amd import kernels as K
+
+    rng = np.random.default_rng(m)
+    a, b = _inputs(torch, rng, m, k, n, False)
+    w = K.pack_i8_b_for_matmul(b, k, n)
+    at = torch.from_numpy(a).cuda()
+    out = torch.zeros(m, n, dtype=torch.int32, device="cuda")
+    w.matmul(at, a_zp=9, out=out)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        w.matmul(at, a_zp=9, out=out)
+    for turn in range(3):
+        new = torch.from_numpy(rng.integers(0, 256, (m, k), dtype=np.uint8))
+        at.copy_(new)
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), _exact(new.numpy(), b, 9).astype(np.int32)), turn

@@ -96,6 +96,7 @@ struct Scratch {
   }
 };
 void release_scratch();
+bool stream_capturing(hipStream_t s);  // s is being captured into a graph (the default stream never is)
 
 inline size_t ceil_div(size_t a, size_t b) { return (a + b - 1) / b; }
 inline size_t round_up(size_t a, size_t b) { return ceil_div(a, b) * b; }

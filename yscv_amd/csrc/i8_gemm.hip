@@ -556,9 +556,28 @@ static bool i8_fast_rows(size_t m, size_t kp, const void *out) {
   return m * kp < ((size_t)1 << 31) && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
 }
 
+// Rows of A that are copied at a time: the copy stays within 64 MB (a block of scratch.hip that is kept), whole 16-row
+// tiles so that every piece of the result starts on 16 bytes.
+static size_t i8_copy_rows(size_t m, size_t kp) {
+  const size_t rows = (((size_t)64 << 20) / kp) / 16 * 16;
+  return m < rows ? m : rows;
+}
+
 size_t i8_gemm_pad_bytes(const yscv_hip_i8_weight *b, size_t m, const void *a, const void *out) {
   if (!i8_fast_rows(m, b->kp, out) || (b->k == b->kp && (reinterpret_cast<uintptr_t>(a) & 15) == 0)) return 0;
-  return m * b->kp;
+  return i8_copy_rows(m, b->kp) * b->kp;
+}
+
+// the matrix kernels on rows of p.lda bytes, whole 64-byte steps on 16-byte alignment
+static int32_t i8_gemm_rows(const I8Args &p, const yscv_hip_i8_weight *b, int num_cus, hipStream_t s) {
+  const size_t m = (size_t)p.m;
+  if (i8_ksplit_takes(m, b->n, (size_t)p.ksteps, num_cus)) return launch_i8_ksplit(p, num_cus, s);
+  // 128 x 128 tiles halve the LDS fill per MFMA; 64 x 128 tiles are for shapes that would not fill the CUs otherwise
+  const size_t big_tiles = ceil_div(m, (size_t)128) * ceil_div(b->n, (size_t)128);
+  const bool wide_a = b->kp % 128 == 0;  // k-steps come in pairs: A is fetched as whole 128-byte lines
+  if (big_tiles >= (size_t)num_cus)
+    return wide_a ? launch_ring<4, 4, 2, 4, true>(p, m, b->n, s) : launch_ring<4, 4, 2, 4, false>(p, m, b->n, s);
+  return wide_a ? launch_ring<2, 4, 4, 3, true>(p, m, b->n, s) : launch_ring<2, 4, 4, 3, false>(p, m, b->n, s);
 }
 
 int32_t launch_i8_gemm(const void *a, int a_is_u8, int a_zp, const yscv_hip_i8_weight *b, size_t m,
@@ -585,31 +604,36 @@ int32_t launch_i8_gemm(const void *a, int a_is_u8, int a_zp, const yscv_hip_i8_w
   p.zp_mul = a_is_u8 ? (128 - a_zp) : -a_zp;
   p.a_zp_dev = ep.a_zp_dev;
   p.lda = (int)b->k;
-  if (i8_fast_rows(m, b->kp, out)) {
+  const Context *ctx = nullptr;
+  YSCV_TRY(ensure_context(&ctx));
+  const bool in_place = b->k == b->kp && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
+  if (in_place && i8_fast_rows(m, b->kp, out)) return i8_gemm_rows(p, b, ctx->num_cus, s);
+  if (const size_t pad_bytes = i8_gemm_pad_bytes(b, m, a, out)) {
+    // a copy in kp-byte rows and the kernels above: the general kernel fetches such rows byte by byte (whole op, that kernel
+    // -> this: 512 x 4096 x 3001 88 -> 20 us, 64 x 1003 x 1001 32 -> 8.7, 1500 x 3000 x 5000 254 -> 65).  That kernel needs
+    // no memory, so it runs where there is none for the copy and under capture, where the graph would keep it.
     Scratch own;
-    if (const size_t pad_bytes = i8_gemm_pad_bytes(b, m, a, out)) {
-      // a copy in kp-byte rows and the kernels below: the general kernel fetches such rows byte by byte (whole op, that kernel
-      // -> this: 512 x 4096 x 3001 88 -> 20 us, 64 x 1003 x 1001 32 -> 8.7, 1500 x 3000 x 5000 254 -> 65)
-      if (pad == nullptr) {
-        YSCV_TRY(own.take(pad_bytes, s));
-        pad = own.p;
-      }
-      const size_t blocks = ceil_div(pad_bytes / 16, (size_t)256);
-      hipLaunchKernelGGL(i8_pad_rows_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, p.a, m, p.k, (int)b->kp,
-                         static_cast<uint8_t *>(pad));
-      YSCV_HIP_TRY(hipGetLastError());
-      p.a = static_cast<const uint8_t *>(pad);
-      p.lda = (int)b->kp;
+    if (pad == nullptr && !stream_capturing(s)) {
+      if (own.take(pad_bytes, s) == YSCV_HIP_OK) pad = own.p;
+      else (void)hipGetLastError();
     }
-    const Context *ctx = nullptr;
-    YSCV_TRY(ensure_context(&ctx));
-    if (i8_ksplit_takes(m, b->n, (size_t)p.ksteps, ctx->num_cus)) return launch_i8_ksplit(p, ctx->num_cus, s);
-    // 128 x 128 tiles halve the LDS fill per MFMA; 64 x 128 tiles are for shapes that would not fill the CUs otherwise
-    const size_t big_tiles = ceil_div(m, (size_t)128) * ceil_div(b->n, (size_t)128);
-    const bool wide_a = b->kp % 128 == 0;  // k-steps come in pairs: A is fetched as whole 128-byte lines
-    if (big_tiles >= (size_t)ctx->num_cus)
-      return wide_a ? launch_ring<4, 4, 2, 4, true>(p, m, b->n, s) : launch_ring<4, 4, 2, 4, false>(p, m, b->n, s);
-    return wide_a ? launch_ring<2, 4, 4, 3, true>(p, m, b->n, s) : launch_ring<2, 4, 4, 3, false>(p, m, b->n, s);
+    if (pad != nullptr) {
+      const size_t step = i8_copy_rows(m, b->kp), out_row = b->n * (ep.mode == 1 ? 1 : 4);
+      I8Args piece = p;
+      piece.a = static_cast<const uint8_t *>(pad);
+      piece.lda = (int)b->kp;
+      for (size_t r0 = 0; r0 < m; r0 += step) {
+        const size_t rows = m - r0 < step ? m - r0 : step;
+        const size_t blocks = ceil_div(rows * b->kp / 16, (size_t)256);
+        hipLaunchKernelGGL(i8_pad_rows_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, p.a + r0 * b->k, rows,
+                           p.k, (int)b->kp, static_cast<uint8_t *>(pad));
+        YSCV_HIP_TRY(hipGetLastError());
+        piece.m = (int)rows;
+        piece.out = static_cast<char *>(out) + r0 * out_row;
+        YSCV_TRY(i8_gemm_rows(piece, b, ctx->num_cus, s));
+      }
+      return YSCV_HIP_OK;
+    }
   }
   dim3 grid((unsigned)ceil_div(b->n, (size_t)I8_BN), (unsigned)ceil_div(m, (size_t)I8_BM));
   const bool vec = (b->k % 16 == 0) && ((reinterpret_cast<uintptr_t>(a) & 15) == 0);

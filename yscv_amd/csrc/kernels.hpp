@@ -175,8 +175,9 @@ struct I8Epilogue {
 };
 int32_t launch_i8_gemm(const void *a, int a_is_u8, int a_zp, const yscv_hip_i8_weight *b, size_t m,
                        void *out, const I8Epilogue &ep, hipStream_t s, void *pad = nullptr);
-// What launch_i8_gemm needs at `pad` (16-byte aligned) to copy rows of a K that is no multiple of 64, or A off 16-byte
-// alignment: 0 for others.  With a null pad it takes a scratch block itself, so a caller that holds one must pass its own.
+// What launch_i8_gemm uses at `pad` (16-byte aligned) to copy rows of a K that is no multiple of 64, or A off 16-byte
+// alignment: at most 64 MB, 0 for others.  With a null pad it takes a scratch block itself, so a caller that holds one must
+// pass its own; where there is none (no memory, a stream under capture) it runs the kernel that needs none.
 size_t i8_gemm_pad_bytes(const yscv_hip_i8_weight *b, size_t m, const void *a, const void *out);
 
 // ---- elementwise ---------------------------------------------------------------------

@@ -59,15 +59,16 @@ static int32_t alloc_failed(hipError_t e, size_t bytes) {
                    bytes, hipGetErrorString(e));
 }
 
+bool stream_capturing(hipStream_t s) {
+  if (s == nullptr) return false;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
 int32_t Scratch::take(size_t bytes, hipStream_t stream) {
   s = stream;
   if (bytes == 0) bytes = 4;
-  bool keep = bytes <= kKeep;
-  if (keep && stream != nullptr) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    keep = hipStreamIsCapturing(stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
-  }
-  if (!keep) {
+  if (bytes > kKeep || stream_capturing(stream)) {
     const hipError_t e = hipMallocAsync(&p, bytes, stream);
     if (e != hipSuccess) {
       p = nullptr;
