@@ -535,7 +535,8 @@ int32_t yscv_hip_decoder_reset(yscv_hip_decoder *d, int32_t batch, int32_t start
  * (each path is within the float bar of the int4 kernels against the reference arithmetic) and a greedy pick can
  * differ where two logits are that close.  A caller that needs one arithmetic for every batch size names the path
  * instead of passing AUTO; yscv_hip_decoder_last_path tells which one a call took.  Fails if the KV cache or the
- * token history would overflow (KvCache::append returns an error in the same situation, kv_cache.rs:160-185). */
+ * token history would overflow (KvCache::append returns an error in the same situation, kv_cache.rs:160-185), and with
+ * YSCV_HIP_ERR_UNSUPPORTED on a stream that is being captured (use_graph 1 captures and replays its own step). */
 #define YSCV_HIP_DECODE_AUTO 3
 int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_graph, void *stream);
 /* The prompt phase of the decode loop (apps/llm-bench/src/main.rs:403-470 times it apart from the decode phase): feeds
@@ -547,7 +548,8 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
  * results agree with token-by-token feeding to the float bar of the int4 kernels (the GEMM folds the group scale into
  * fp16 weights where the decode kernel applies it in fp32).  With an int8 cache every row is quantised as the decode
  * step quantises it (scales over all kv heads of the position) and attention reads what the cache returns for each
- * position, q * scale of its row, earlier positions included.  tokens_host is read before the call returns. */
+ * position, q * scale of its row, earlier positions included.  tokens_host is read before the call returns.
+ * YSCV_HIP_ERR_UNSUPPORTED on a stream that is being captured. */
 int32_t yscv_hip_decoder_prefill(yscv_hip_decoder *d, const int32_t *tokens_host, int32_t n_tokens, int32_t start_pos,
                                  void *stream);
 /* Rows of the prompt that yscv_hip_decoder_prefill takes through the layers in one pass (default 4096).  A longer

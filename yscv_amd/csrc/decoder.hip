@@ -251,6 +251,13 @@ static hipError_t enter_stream(yscv_hip_decoder *d, hipStream_t s) {
   return hipDeviceSynchronize();
 }
 
+// The host keeps the position and the step the decoder is at and passes them, and a prompt's tokens, with the call: a graph
+// would replay the numbers of the call that was captured.
+static int32_t refuse_capture(hipStream_t s) {
+  if (!stream_capturing(s)) return YSCV_HIP_OK;
+  return set_error(YSCV_HIP_ERR_UNSUPPORTED, "decoder calls cannot be captured into a graph: position and tokens of a call are kept on the host");
+}
+
 #define DEC_HIP(expr)                                                                                \
   do {                                                                                               \
     hipError_t _e = (expr);                                                                          \
@@ -941,6 +948,7 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
   YSCV_REQUIRE(d->batch >= 1, "call yscv_hip_decoder_reset first");
   YSCV_REQUIRE(n_steps >= 0, "negative step count");
   hipStream_t s = as_stream(stream);
+  YSCV_TRY(refuse_capture(s));
   // host-side bound check: the cache must hold every position this run appends
   const int32_t pos = d->pos_host, step = d->step_host;
   YSCV_REQUIRE(pos + n_steps <= d->cfg.max_ctx, "KV cache overflow: position %d + %d steps > max_ctx %d", pos, n_steps,
@@ -1280,6 +1288,7 @@ int32_t yscv_hip_decoder_prefill(yscv_hip_decoder *d, const int32_t *tokens_host
   for (int32_t i = 0; i < n_tokens; i++)
     YSCV_REQUIRE(tokens_host[i] >= 0 && tokens_host[i] < c.vocab, "token %d outside the vocabulary (%d)", tokens_host[i], c.vocab);
   hipStream_t s = as_stream(stream);
+  YSCV_TRY(refuse_capture(s));
   d->batch = 1;
   DEC_HIP(enter_stream(d, s));
   if (n_tokens > d->prompt_cap) {
