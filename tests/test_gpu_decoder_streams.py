@@ -52,3 +52,62 @@ def test_a_captured_stream_is_refused_and_nothing_moves(mode):
         want.run(PCFG["max_steps"], **MODES[mode])
         dec.run(PCFG["max_steps"] - 2, **MODES[mode])
         assert np.array_equal(dec.tokens(0, PCFG["max_steps"]), want.tokens(0, PCFG["max_steps"]))
+
+
+def _hip():
+    """The runtime this process already has loaded."""
+    import ctypes as C
+
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip = C.CDLL(path)
+    hip.hipStreamCreateWithFlags.argtypes = [C.POINTER(C.c_void_p), C.c_uint]
+    hip.hipStreamDestroy.argtypes = [C.c_void_p]
+    return hip, C
+
+
+@pytest.mark.parametrize("mode", MODES)
+def test_calls_on_changing_streams_follow_each_other(mode):
+    """reset, run, run_projections and prefill on the default stream, on streams that do not wait for it, and on streams that
+    are destroyed right behind the call (their handles come back for the next ones), with no wait in between."""
+    import torch
+
+    dec = _decoder()
+    prompt = np.arange(60, dtype=np.int32) * 7 % PCFG["vocab"]
+    kw = MODES[mode]
+
+    def drive(streams):
+        dec.reset([9], 0)
+        for s in streams[:5]:
+            dec.run(3, stream=s(), **kw)
+        first = dec.tokens(0, 15).copy(), dec.logits().copy()
+        dec.prefill(prompt, stream=streams[5]())
+        dec.run(4, stream=streams[6](), **kw)
+        dec.reset([11], 64)
+        dec.run(6, stream=streams[7](), **kw)
+        last = dec.tokens(0, 6).copy(), dec.logits().copy()
+        dec.prefill(prompt, stream=streams[8]())
+        dec.run_projections(1, stream=streams[9]())  # leaves the cache and the tokens alone
+        dec.run(5, stream=streams[10](), **kw)
+        return first, last, (dec.tokens(0, 6).copy(), dec.logits().copy())
+
+    want = drive([lambda: None] * 11)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    hip, C = _hip()
+    alive = []
+
+    def fresh():  # the stream before this one is destroyed now, right behind the call that used it
+        while alive:
+            assert hip.hipStreamDestroy(alive.pop()) == 0
+        h = C.c_void_p()
+        assert hip.hipStreamCreateWithFlags(C.byref(h), 1) == 0  # hipStreamNonBlocking
+        alive.append(h)
+        return h.value
+
+    on_a, on_b, default = (lambda: a.cuda_stream), (lambda: b.cuda_stream), (lambda: None)
+    for streams in ([on_a, on_b, on_a, on_a, default, on_b, on_a, on_b, default, on_a, on_b], [fresh] * 11,
+                    [default, fresh, fresh, default, on_a, fresh, default, fresh, on_b, default, fresh]):
+        for (tok, log), (wtok, wlog) in zip(drive(streams), want):
+            assert np.array_equal(tok, wtok) and np.array_equal(log, wlog)
+    torch.cuda.synchronize()
+    while alive:
+        assert hip.hipStreamDestroy(alive.pop()) == 0
