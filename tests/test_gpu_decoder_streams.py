@@ -111,3 +111,57 @@ def test_calls_on_changing_streams_follow_each_other(mode):
     torch.cuda.synchronize()
     while alive:
         assert hip.hipStreamDestroy(alive.pop()) == 0
+
+
+def test_a_failed_call_leaves_the_state_as_it_was():
+    import torch
+
+    from yscv_amd.capi import YscvHipError
+
+    side = torch.cuda.Stream()
+    dec = _decoder()
+    dec.reset([9], 500)
+    dec.run(12, auto=True)
+    want = dec.tokens(0, 12).copy()
+    for kw in MODES.values():
+        dec.reset([9], 500)
+        dec.run(5, stream=side.cuda_stream, **kw)
+        for bad in (lambda: dec.run(8, stream=side.cuda_stream, **kw),           # past the end of the context
+                    lambda: dec.run(1000, **kw),
+                    lambda: dec.run(-1, **kw),
+                    lambda: dec.prefill([1, PCFG["vocab"]], stream=side.cuda_stream),  # no such token
+                    lambda: dec.prefill([1] * 20, start_pos=500),
+                    lambda: dec.reset([1], PCFG["max_ctx"]),
+                    lambda: dec.reset([1, 2, 3], 0)):
+            with pytest.raises(YscvHipError):
+                bad()
+        dec.batch = 1
+        dec.run(7, stream=side.cuda_stream, **kw)
+        if "persistent" in kw or "auto" in kw:
+            assert np.array_equal(dec.tokens(0, 12), want)
+        else:
+            assert dec.tokens(0, 12).shape == (12, 1)
+        with pytest.raises(YscvHipError):
+            dec.run(1, **kw)  # position 512 of 512
+
+
+@pytest.mark.parametrize("n", [895, 896, 897, 1793])
+def test_prompts_around_the_pieces_they_travel_in(n):
+    """A prompt goes to the device in pieces of 896 tokens and its buffers are kept: the logits of one pass against the same
+    tokens in two calls that share no piece boundary, with longer and shorter prompts in between."""
+    import torch
+
+    side = torch.cuda.Stream()
+    dec = _decoder(max_ctx=2048)
+    rng = np.random.default_rng(n)
+    prompt = rng.integers(0, PCFG["vocab"], n).astype(np.int32)
+    dec.prefill(prompt, stream=side.cuda_stream)
+    one, first = dec.logits().copy(), dec.tokens(0, 1).copy()
+    dec.prefill(rng.integers(0, PCFG["vocab"], 40).astype(np.int32))
+    dec.prefill(rng.integers(0, PCFG["vocab"], 2000).astype(np.int32))
+    dec.prefill(prompt[:500])
+    dec.prefill(prompt[500:], start_pos=500, stream=side.cuda_stream)
+    two = dec.logits().copy()
+    assert np.abs(one - two).max() < 1e-2 * np.abs(one).max()
+    dec.prefill(prompt)
+    assert np.array_equal(dec.logits(), one) and np.array_equal(dec.tokens(0, 1), first)
