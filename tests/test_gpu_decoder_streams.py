@@ -113,6 +113,21 @@ def test_calls_on_changing_streams_follow_each_other(mode):
         assert hip.hipStreamDestroy(alive.pop()) == 0
 
 
+def test_a_step_is_captured_again_behind_replays_under_way():
+    """Changing the batch drops the captured step; its replays run to their end first."""
+    import torch
+
+    a, b = _decoder(), _decoder()
+    side = torch.cuda.Stream()
+    for turn in range(4):
+        for tokens in ([9 + turn], [9 + turn, 40 + turn]):
+            a.reset(tokens, 0)
+            a.run(20, stream=side.cuda_stream)  # graph replays; the next turn's capture comes right behind them
+        b.reset([9 + turn, 40 + turn], 0)
+        b.run(20, use_graph=False)
+        assert np.array_equal(a.tokens(0, 20), b.tokens(0, 20)) and np.array_equal(a.logits(), b.logits())
+
+
 def test_a_failed_call_leaves_the_state_as_it_was():
     import torch
 

@@ -186,9 +186,13 @@ struct yscv_hip_decoder {
 };
 
 // A captured step holds the addresses of the weights and of the workspace as they were at capture time: whatever
-// frees or replaces one of them drops the graph, and the next graph run captures again.
+// frees or replaces one of them drops the graph, and the next graph run captures again.  Replays of it may still be under
+// way (no call waits for them): they are waited for first.
 static void drop_graph(yscv_hip_decoder *d) {
-  if (d->graph_exec) (void)hipGraphExecDestroy(d->graph_exec);
+  if (d->graph_exec) {
+    (void)hipDeviceSynchronize();
+    (void)hipGraphExecDestroy(d->graph_exec);
+  }
   if (d->graph) (void)hipGraphDestroy(d->graph);
   d->graph_exec = nullptr;
   d->graph = nullptr;
