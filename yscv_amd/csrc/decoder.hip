@@ -1363,6 +1363,8 @@ int32_t yscv_hip_decoder_prefill(yscv_hip_decoder *d, const int32_t *tokens_host
   // as after reset(last token, start_pos + n - 1) + one decode step: the pick is the next input, position and step advance
   hipLaunchKernelGGL(set_counters_kernel, dim3(1), dim3(64), 0, s, d->pos, d->step, start_pos + n_tokens - 1, 0);
   DEC_HIP(hipGetLastError());
+  d->pos_host = start_pos + n_tokens - 1;
+  d->step_host = 0;
   YSCV_TRY(launch_argmax(d->logits, 1, c.vocab, d->tokens, d->history, d->step, c.max_steps, s));
   YSCV_TRY(launch_advance(d->pos, d->step, s));
   d->pos_host = start_pos + n_tokens;
