@@ -28,3 +28,26 @@ def test_fp16_rows_of_any_magnitude(n, k, g, std):
         # x (1024 + q) are up to 160 times the group's product, over a few roundings: 160 * 2^-24 * 5.  Above, the
         # weights are rounded to fp16.
         assert rel < (5e-5 if m <= 16 else 6e-4), (m, rel)
+
+
+def test_single_launch_decoder_with_small_activations():
+    """The LM head of the single-launch decode path behind a norm whose gain leaves values of about 1e-5: against the
+    multi-kernel path with its norms as launches of their own, which rounds the same fp16 (the folded norm rounds a quarter
+    of it, whose last bit is four times as coarse).  That last bit is 2^-24: rounding is 2^-24 / sqrt(12) of 1e-5, 1.7e-3 of
+    the result, on each side, and the paths' other rounding points add about 1e-3."""
+    from test_gpu_decoder import PCFG
+    from yscv_amd import lib
+    from yscv_amd.decoder import Decoder
+
+    dec = Decoder(**PCFG)
+    dec.init_random(seed=3, nibbles=(1, 15))
+    dec.set_norm(0, "final", np.full(PCFG["d_model"], 1e-5, np.float32))
+    dec.finalize()
+    lib().decoder_debug_set_folded_norm(dec._h, 0)
+    logits = {}
+    for name, kw in {"graph": dict(use_graph=True), "single": dict(persistent=True)}.items():
+        dec.reset([9], 0)
+        dec.run(1, **kw)
+        logits[name] = dec.logits()[0].astype(np.float64)
+    rel = np.linalg.norm(logits["single"] - logits["graph"]) / np.linalg.norm(logits["graph"])
+    assert rel < 5e-3, rel

@@ -20,9 +20,10 @@
 // of the A operand carry 16 different k-blocks of the activation (row i = k-block i of the wave's
 // 512-k fragment), and the 16 columns of B carry 8 weight rows x 2 k-blocks, so each MFMA produces
 // the dot products of 8 rows over two k-blocks in rows {j, j+4, ...} of D; the lanes that hold a
-// useful element apply the group scale in fp32.  Weights stay exact integers (0x6400 | q = 1024 + q);
-// the offset term sum_k x_k * (1024 + 8) is computed once per fragment by the same MFMA against a
-// constant operand and subtracted per group.
+// useful element apply the group scale in fp32.  Weights stay exact integers (0x6400 | q = 1024 + q,
+// 0x5400 | (q << 4) = 64 + q for the high nibbles, so that x meets both as it is: see int4_skinny.hip);
+// the offset term sum_k x_k * (1024 + 8 or 64 + 8) is computed once per fragment by the same MFMA
+// against a constant operand and subtracted per group.
 //
 // Semantics of the glue (tolerance-checked against the numpy restatement, like the multi-kernel path):
 // RMSNorm crates/yscv-kernels/src/ops/norm.rs:1497-1518, RoPE ops/rope.rs:24-117, grouped-query
@@ -508,14 +509,14 @@ __device__ GEMV_INL GemvState gemv_stage(GemvArgs a, GemvState st) {
   // becomes one three-register v_and_or_b32 instead of two literal-operand instructions.  (An inline-asm
   // v_and_or_b32 is not an option: the hazard recognizer does not see it overwrite a register that a
   // matrix instruction is still writing.)
-  uint32_t magic = 0x64006400u, mask_lo = 0x000F000Fu, mask_hi = 0x00F000F0u;
-  asm volatile("" : "+v"(magic), "+v"(mask_lo), "+v"(mask_hi));
+  uint32_t magic = 0x64006400u, magic_hi = 0x54005400u, mask_lo = 0x000F000Fu, mask_hi = 0x00F000F0u;
+  asm volatile("" : "+v"(magic), "+v"(magic_hi), "+v"(mask_lo), "+v"(mask_hi));
   const uint32_t tag = a.tag;
   half8_t xa[MAXF];
   float4_t z[MAXF];
   float rstd = 1.0f;
-  const half8_t bc = {(_Float16)1032.0f, (_Float16)1032.0f, (_Float16)1152.0f, (_Float16)1152.0f,
-                      (_Float16)1032.0f, (_Float16)1032.0f, (_Float16)1152.0f, (_Float16)1152.0f};
+  const half8_t bc = {(_Float16)1032.0f, (_Float16)1032.0f, (_Float16)72.0f, (_Float16)72.0f,
+                      (_Float16)1032.0f, (_Float16)1032.0f, (_Float16)72.0f, (_Float16)72.0f};
   const bool normed = a.ss != nullptr;
   // ---- activation fragments (A operand: row i = k-block i of the fragment) ------------------------------
   // A `normed` vector holds fp16(h * gamma * 2^-e) with the exponent e of each 8-row block in the top byte
@@ -574,10 +575,6 @@ __device__ GEMV_INL GemvState gemv_stage(GemvArgs a, GemvState st) {
           u2.h = half2_t{(_Float16)((float)u2.h[0] * fac), (_Float16)((float)u2.h[1] * fac)};
           u3.h = half2_t{(_Float16)((float)u3.h[0] * fac), (_Float16)((float)u3.h[1] * fac)};
         }
-        // the slots that meet 1024 + 16 q carry x / 16 (exact: a power of two)
-        const half2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-        u1.h = u1.h * sixteenth;
-        u3.h = u3.h * sixteenth;
         xa[f] = half8_t{u0.h[0], u0.h[1], u1.h[0], u1.h[1], u2.h[0], u2.h[1], u3.h[0], u3.h[1]};
         const float4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
         z[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[f], bc, zero, 0, 0, 0);  // offset term of every k-block
@@ -628,9 +625,9 @@ __device__ GEMV_INL GemvState gemv_stage(GemvArgs a, GemvState st) {
       U32H2 q0, q1, q2, q3;
       const uint32_t s = w0[j], s2 = s >> 8;
       q0.u = (s & mask_lo) | magic;
-      q1.u = (s & mask_hi) | magic;
+      q1.u = (s & mask_hi) | magic_hi;
       q2.u = (s2 & mask_lo) | magic;
-      q3.u = (s2 & mask_hi) | magic;
+      q3.u = (s2 & mask_hi) | magic_hi;
       const half8_t b = {q0.h[0], q0.h[1], q1.h[0], q1.h[1], q2.h[0], q2.h[1], q3.h[0], q3.h[1]};
       const float4_t dd = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf, b, zero, 0, 0, 0);
       d0[j] = dd[j];
@@ -641,9 +638,9 @@ __device__ GEMV_INL GemvState gemv_stage(GemvArgs a, GemvState st) {
         U32H2 q0, q1, q2, q3;
         const uint32_t s = w1[j], s2 = s >> 8;
         q0.u = (s & mask_lo) | magic;
-        q1.u = (s & mask_hi) | magic;
+        q1.u = (s & mask_hi) | magic_hi;
         q2.u = (s2 & mask_lo) | magic;
-        q3.u = (s2 & mask_hi) | magic;
+        q3.u = (s2 & mask_hi) | magic_hi;
         const half8_t b = {q0.h[0], q0.h[1], q1.h[0], q1.h[1], q2.h[0], q2.h[1], q3.h[0], q3.h[1]};
         const float4_t dd = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf, b, zero, 0, 0, 0);
         d1[j] = dd[j];
