@@ -24,6 +24,7 @@
 #include <stdint.h>
 
 #include "../../include/yscv_hip.h"
+#include "kernels.hpp"
 
 namespace yscv {
 
@@ -167,6 +168,40 @@ __device__ __forceinline__ void store_out(void *y, size_t idx, float v, int dtyp
     reinterpret_cast<_Float16 *>(y)[idx] = (_Float16)v;
   } else {
     reinterpret_cast<uint16_t *>(y)[idx] = float_to_bf16_bits(v);
+  }
+}
+
+__device__ __forceinline__ float silu(float g) { return g / (1.0f + __expf(-g)); }
+
+// Columns col .. col + 3 of one row into y (rows of ldy columns, n of them in use) through the epilogue `epi`; col is a
+// multiple of 4, `whole` says that all four exist and lie on their vector's alignment.  Every element has one writer.
+__device__ __forceinline__ void store_cols4(void *y, int y_dtype, int epi, int ldy, int n, int row, int col, bool whole, float4_t v) {
+  const size_t o = (size_t)row * ldy + col;
+  if (epi == EPI_SWIGLU) {
+    // columns col .. col + 3 are gate, up, gate, up of two channels (n is even)
+    const size_t oh = (size_t)row * (ldy >> 1) + (col >> 1);
+    store_out(y, oh, silu(v[0]) * v[1], y_dtype);
+    if (col + 2 < n) store_out(y, oh + 1, silu(v[2]) * v[3], y_dtype);
+  } else if (epi == EPI_ADD_F32) {
+    float *dst = reinterpret_cast<float *>(y) + o;
+    if (whole) {
+      *reinterpret_cast<float4_t *>(dst) = *reinterpret_cast<const float4_t *>(dst) + v;
+    } else {
+      for (int e = 0; e < 4; e++)
+        if (col + e < n) dst[e] += v[e];
+    }
+  } else if (whole && y_dtype == YSCV_HIP_F32) {
+    *reinterpret_cast<float4_t *>(reinterpret_cast<float *>(y) + o) = v;
+  } else if (whole && y_dtype == YSCV_HIP_F16) {
+    *reinterpret_cast<half4_t *>(reinterpret_cast<_Float16 *>(y) + o) = half4_t{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+  } else if (whole) {
+    uint2 b;
+    b.x = (uint32_t)float_to_bf16_bits(v[0]) | ((uint32_t)float_to_bf16_bits(v[1]) << 16);
+    b.y = (uint32_t)float_to_bf16_bits(v[2]) | ((uint32_t)float_to_bf16_bits(v[3]) << 16);
+    *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(y) + o) = b;
+  } else {
+    for (int e = 0; e < 4; e++)
+      if (col + e < n) store_out(y, o + e, v[e], y_dtype);
   }
 }
 

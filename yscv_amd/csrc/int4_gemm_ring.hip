@@ -30,8 +30,6 @@ namespace yscv {
 namespace {
 
 __device__ const float kOne = 1.0f;  // stands in for an absent row-scale vector
-__device__ __forceinline__ float ring_silu(float g) { return g / (1.0f + __expf(-g)); }
-
 typedef __attribute__((address_space(3))) void lds_void;
 #define G4_AS1(ptr) ((const void __attribute__((address_space(1))) *)(ptr))
 
@@ -480,8 +478,8 @@ __global__ void __launch_bounds__(256 + 64 * NP) int4_gemm_ring_kernel(RingArgs 
       } else if (p.epi == EPI_SWIGLU) {
         // columns col .. col + 3 are gate, up, gate, up of two channels (n is even, col a multiple of 4)
         const size_t oh = (size_t)row * (p.ldy >> 1) + (col >> 1);
-        store_out(p.y, oh, ring_silu(v[0]) * v[1], p.y_dtype);
-        if (col + 2 < p.n) store_out(p.y, oh + 1, ring_silu(v[2]) * v[3], p.y_dtype);
+        store_out(p.y, oh, silu(v[0]) * v[1], p.y_dtype);
+        if (col + 2 < p.n) store_out(p.y, oh + 1, silu(v[2]) * v[3], p.y_dtype);
       } else if (p.epi == EPI_ADD_F32) {
         float *dst = reinterpret_cast<float *>(p.y) + o;  // every element has one writer in a launch
         if (vec) {
@@ -531,8 +529,8 @@ __global__ void __launch_bounds__(256) ring_finalize_kernel(const float *__restr
     const size_t o = (size_t)row * ldy + col;
     if (epi == EPI_SWIGLU) {
       const size_t oh = (size_t)row * (ldy >> 1) + (col >> 1);
-      store_out(y, oh, ring_silu(v[0]) * v[1], y_dtype);
-      if (col + 2 < n) store_out(y, oh + 1, ring_silu(v[2]) * v[3], y_dtype);
+      store_out(y, oh, silu(v[0]) * v[1], y_dtype);
+      if (col + 2 < n) store_out(y, oh + 1, silu(v[2]) * v[3], y_dtype);
     } else if (epi == EPI_ADD_F32) {
       float *dst = reinterpret_cast<float *>(y) + o;
       for (int e = 0; e < 4; e++)

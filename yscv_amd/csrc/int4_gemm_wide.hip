@@ -24,8 +24,6 @@ namespace yscv {
 
 namespace {
 
-__device__ __forceinline__ float wide_silu(float g) { return g / (1.0f + __expf(-g)); }
-
 constexpr int WG_MT = 8, WG_NT = 4, WG_WM = 2, WG_WN = 4;  // MFMA tiles of a wave, waves of a workgroup
 constexpr int WG_BM = 16 * WG_MT * WG_WM, WG_BN = 16 * WG_NT * WG_WN, WG_THREADS = 64 * WG_WM * WG_WN;
 constexpr int WG_XSLOT = WG_BM * 128, WG_XSLOTS = 3;  // activations of 64 k
@@ -63,35 +61,6 @@ template <int N>
 __device__ __forceinline__ void wide_barrier() {
   // this wave's loads of the stage have landed and its fragment reads of the last one have returned; then everyone's
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-__device__ __forceinline__ void wide_store(const WideArgs &p, int row, int col, bool whole, float4_t v) {
-  const size_t o = (size_t)row * p.ldy + col;
-  if (p.epi == EPI_SWIGLU) {
-    const size_t oh = (size_t)row * (p.ldy >> 1) + (col >> 1);
-    store_out(p.y, oh, wide_silu(v[0]) * v[1], p.y_dtype);
-    if (col + 2 < p.n) store_out(p.y, oh + 1, wide_silu(v[2]) * v[3], p.y_dtype);
-  } else if (p.epi == EPI_ADD_F32) {
-    float *dst = reinterpret_cast<float *>(p.y) + o;
-    if (whole) {
-      *reinterpret_cast<float4_t *>(dst) = *reinterpret_cast<const float4_t *>(dst) + v;
-    } else {
-      for (int e = 0; e < 4; e++)
-        if (col + e < p.n) dst[e] += v[e];
-    }
-  } else if (whole && p.y_dtype == YSCV_HIP_F32) {
-    *reinterpret_cast<float4_t *>(reinterpret_cast<float *>(p.y) + o) = v;
-  } else if (whole && p.y_dtype == YSCV_HIP_F16) {
-    *reinterpret_cast<half4_t *>(reinterpret_cast<_Float16 *>(p.y) + o) = half4_t{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-  } else if (whole) {
-    uint2 b;
-    b.x = (uint32_t)float_to_bf16_bits(v[0]) | ((uint32_t)float_to_bf16_bits(v[1]) << 16);
-    b.y = (uint32_t)float_to_bf16_bits(v[2]) | ((uint32_t)float_to_bf16_bits(v[3]) << 16);
-    *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.y) + o) = b;
-  } else {
-    for (int e = 0; e < 4; e++)
-      if (col + e < p.n) store_out(p.y, o + e, v[e], p.y_dtype);
-  }
 }
 
 template <int GM, bool SF16, bool HAS_ZP>
@@ -312,7 +281,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) int4_gemm_wide_kernel(WideArgs 
       if (row < p.m && col < p.n) {
         float4_t v = *reinterpret_cast<const float4_t *>(red + (4 * q + c) * WG_RS + 4 * r);
         if (p.row_scale) v = v * p.row_scale[row];
-        wide_store(p, row, col, vec, v);
+        store_cols4(p.y, p.y_dtype, p.epi, p.ldy, p.n, row, col, vec, v);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

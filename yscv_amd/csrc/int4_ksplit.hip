@@ -26,8 +26,6 @@ namespace yscv {
 
 namespace {
 
-__device__ __forceinline__ float ks_silu(float g) { return g / (1.0f + __expf(-g)); }
-
 struct KsArgs {
   const uint8_t *tiles;
   const void *tscales;
@@ -63,44 +61,18 @@ __device__ __forceinline__ uint32_t ks_load_zp(const uint8_t *p) {
   return *p;
 }
 
-// four consecutive columns of one row through the epilogue
+// four consecutive columns of one row: a partial sum, or the result through the epilogue
 __device__ __forceinline__ void ks_store(const KsArgs &p, int part, int row, int col, bool whole, float4_t v) {
-  if (p.partial) {
-    float *dst = p.partial + ((size_t)part * p.m + row) * p.n + col;
-    if (whole) {
-      *reinterpret_cast<float4_t *>(dst) = v;
-    } else {
-      for (int e = 0; e < 4; e++)
-        if (col + e < p.n) dst[e] = v[e];
-    }
+  if (!p.partial) {
+    store_cols4(p.y, p.y_dtype, p.epi, p.n, p.n, row, col, whole, v);
     return;
   }
-  const size_t o = (size_t)row * p.n + col;
-  if (p.epi == EPI_SWIGLU) {
-    // columns col .. col + 3 are gate, up, gate, up of two channels (n is even, col a multiple of 4)
-    const size_t oh = (size_t)row * (p.n >> 1) + (col >> 1);
-    store_out(p.y, oh, ks_silu(v[0]) * v[1], p.y_dtype);
-    if (col + 2 < p.n) store_out(p.y, oh + 1, ks_silu(v[2]) * v[3], p.y_dtype);
-  } else if (p.epi == EPI_ADD_F32) {
-    float *dst = reinterpret_cast<float *>(p.y) + o;
-    if (whole) {
-      *reinterpret_cast<float4_t *>(dst) = *reinterpret_cast<const float4_t *>(dst) + v;
-    } else {
-      for (int e = 0; e < 4; e++)
-        if (col + e < p.n) dst[e] += v[e];
-    }
-  } else if (whole && p.y_dtype == YSCV_HIP_F32) {
-    *reinterpret_cast<float4_t *>(reinterpret_cast<float *>(p.y) + o) = v;
-  } else if (whole && p.y_dtype == YSCV_HIP_F16) {
-    *reinterpret_cast<half4_t *>(reinterpret_cast<_Float16 *>(p.y) + o) = half4_t{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-  } else if (whole) {
-    uint2 b;
-    b.x = (uint32_t)float_to_bf16_bits(v[0]) | ((uint32_t)float_to_bf16_bits(v[1]) << 16);
-    b.y = (uint32_t)float_to_bf16_bits(v[2]) | ((uint32_t)float_to_bf16_bits(v[3]) << 16);
-    *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.y) + o) = b;
+  float *dst = p.partial + ((size_t)part * p.m + row) * p.n + col;
+  if (whole) {
+    *reinterpret_cast<float4_t *>(dst) = v;
   } else {
     for (int e = 0; e < 4; e++)
-      if (col + e < p.n) store_out(p.y, o + e, v[e], p.y_dtype);
+      if (col + e < p.n) dst[e] = v[e];
   }
 }
 

@@ -26,8 +26,6 @@ namespace yscv {
 
 namespace {
 
-__device__ __forceinline__ float mid_silu(float g) { return g / (1.0f + __expf(-g)); }
-
 struct MidArgs {
   const uint8_t *tiles;
   const void *tscales;
@@ -175,8 +173,8 @@ __global__ void __launch_bounds__(512, 1) int4_mid_kernel(MidArgs a) {
         } else if (a.epi == EPI_SWIGLU) {
           // columns col .. col + 3 are gate, up, gate, up of two channels (n is even, col a multiple of 4)
           const size_t oh = (size_t)out_row * (a.ldy >> 1) + (col >> 1);
-          store_out(a.y, oh, mid_silu(v[0]) * v[1], a.y_dtype);
-          if (col + 2 < a.n) store_out(a.y, oh + 1, mid_silu(v[2]) * v[3], a.y_dtype);
+          store_out(a.y, oh, silu(v[0]) * v[1], a.y_dtype);
+          if (col + 2 < a.n) store_out(a.y, oh + 1, silu(v[2]) * v[3], a.y_dtype);
         } else if (a.epi == EPI_ADD_F32) {
           float *dst = reinterpret_cast<float *>(a.y) + (size_t)out_row * a.ldy + col;
           if (whole) {

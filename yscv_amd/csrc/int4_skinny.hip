@@ -40,8 +40,6 @@
 
 namespace yscv {
 
-__device__ __forceinline__ float silu(float g) { return g / (1.0f + __expf(-g)); }
-
 constexpr int TPW = 4;  // 128-k tiles per wave: 512 k of activations live in 64 VGPRs (hi)
 
 struct SkinnyArgs {
