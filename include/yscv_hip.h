@@ -358,7 +358,7 @@ int32_t yscv_hip_exec_qdq_matmul(const float *x_dev, size_t m, float a_scale, co
 /* DynamicQuantizeLinear feeding MatMulInteger, the pair ONNX Runtime's dynamic quantisation emits (exec_dynamic_quantize_linear,
  * crates/yscv-onnx/src/runner/misc.rs:241-289, then exec_matmul_integer with a_zero_point = the y_zero_point just computed,
  * runner/linear.rs:648-737), as one call: x_dev [m][k] f32 is reduced to its range, quantised to uint8 once into
- * stream-ordered scratch, and multiplied against the prepacked int8 weight (b_zero_point 0); the zero point never leaves
+ * scratch kept per stream, and multiplied against the prepacked int8 weight (b_zero_point 0); the zero point never leaves
  * the device (the GEMM's epilogue reads it there and folds (128 - zp) * colsum(b)), the f32 carriers of the quantised
  * activations are never written, no range scan and no host synchronisation.  out_dev [m][n] = f32 of the exact integer sum
  * of (a_q - zp) * b; *y_scale_dev, *y_zp_dev as DynamicQuantizeLinear returns them.  Bit-identical to the two operators

@@ -13,8 +13,8 @@
 // 2 MT MFMAs and its decode never competes with them for issue slots.  The activation pieces of SA stages form a
 // ring (SA - 1 stages in flight hide the memory latency); decoded weights need two slots only because they are
 // written just before the stage is published, with one s_barrier per stage.
-// The scale is folded into the fp16 weight (relative rounding 2^-11 per weight, exact when the scales are stored
-// as fp16), so any group size costs the same; results stay inside the int4 tolerance (max-abs <= 1e-3 sqrt(K)
+// The scale is folded into the fp16 weight, fp16((q - zp) * s) with a relative rounding of 2^-11 per weight (the product of a
+// five-bit and an eleven-bit number has up to fifteen), so any group size costs the same; results stay inside the int4 tolerance (max-abs <= 1e-3 sqrt(K)
 // max|x|) by more than an order of magnitude.  f32 activations keep the exact-scale kernel of int4_gemm.hip.
 // The MFMA is issued with the operands swapped (D = Wfrag x Xfrag): a lane holds four consecutive columns of one
 // row of y; the finished tile goes through LDS so that whole rows are stored.
@@ -619,8 +619,8 @@ RingPlan ring_plan(size_t m, size_t n, size_t kt, size_t cus) {
     // weight feeds twice as many MFMAs).  A workgroup needs about 1.72 / 1.63 times as long for them as for a
     // 128 x 128 tile; they pay when the tiles come in rounds over the CUs and the larger ones need sufficiently fewer
     // rounds.  When the last round of the best shape would leave most CUs idle, the columns of its whole rounds go to
-    // one launch and the rest to a second one with the shape that suits the rest (config 3: three rounds of
-    // 256 x 128 tiles, then one round of 128 x 128 tiles, instead of three and a half rounds).
+    // one launch and the rest to a second one with the shape that suits the rest (2048 rows x 14336 columns in 256 x 128
+    // tiles: three rounds, then one round of 128 x 128 tiles, instead of three and a half).
     struct Shape {
       size_t bm, bn, cost;
       int code;
@@ -628,7 +628,8 @@ RingPlan ring_plan(size_t m, size_t n, size_t kt, size_t cus) {
     // cost: time of one tile in hundredths of a 128 x 128 tile's (measured on K 4096: 40 us; the 64-row tile 30 us).
     // The 64-row tile decodes every weight twice as often per MFMA; it pays where it fills CUs that the taller tiles
     // would leave idle (512 rows against N 4096: 256 tiles instead of 128).
-    // The 256 x 256 tile of int4_gemm_wide.hip takes 110 us where two rounds of 256 x 128 tiles take 138.
+    // The 256 x 256 tile of int4_gemm_wide.hip takes 110 us where two rounds of 256 x 128 tiles take 138 (weights without
+    // zero points; with them its gain depends on the clock, see its header).
     const Shape shapes[5] = {{128, 128, 100, 0}, {128, 256, 172, 1}, {256, 128, 163, 2}, {256, 256, 280, 5}, {64, 128, 75, 4}};
     auto allowed = [&](const Shape &sh) { return sh.code == 2 ? m > 128 : (sh.code == 5 ? m > 256 : true); };
     // best single shape for columns [c0, n): cost of its rounds over the CUs

@@ -11,8 +11,11 @@
 // the LDS-ring GEMM), weights and scales in two of 128 k.  One barrier per 64 k; half a k-step's MFMAs are issued behind it
 // and cover the first fragment reads of the next stage.
 // The group scale is folded into fp16 weights as in the LDS-ring GEMM, products are added in the same order: same results.
-// us of the whole op, weights from HBM, without -> with this kernel (m x n x k): 2048 x 8192 x 4096 146 -> 128, 2048 x 28672 x
-// 4096 469 -> 423, 2048 x 14336 x 4096 with zero points 256 -> 240, 700 x 24000 x 2048 131 -> 98, 1700 x 13000 x 3072 187 -> 152.
+// us of the whole op, planned without -> with this kernel (m x n x k, fp16 rows), in bursts of six calls 50 ms apart | replayed
+// for 1.5 s, the clock settled: 2048 x 8192 x 4096 137 -> 120 | 134 -> 114, 2048 x 14336 x 4096 248 -> 228 | 240 -> 210, 2048 x
+// 28672 x 4096 525 -> 472 | 456 -> 408, 700 x 24000 x 2048 95 -> 84 | 90 -> 79.  With zero points (two more instructions per
+// pair of weights, and the bf16 rows prepared first: 9 us of it) the decode takes back most of it: 2048 x 14336 x 4096 in
+// 128-groups 254 -> 266 | 242 -> 233: slower while the clock is still coming up behind an idle stretch, faster once it is there.
 // A stage takes 1.43 us (1.09 without the decode) where its MFMAs take 1.05 at the rate a registers-only loop reaches.
 #include <mutex>
 #include <type_traits>

@@ -12,10 +12,11 @@
 // barrier until the eight partial tiles are added (fixed order) and stored as whole rows.
 // (Fragments loaded straight into registers are sixteen rows x 64 bytes per load with neighbouring lanes in different
 // rows: 30 GB/s per CU, a quarter of what whole lines get; 64 rows x 4096 x 4096 took 12.3 us that way.)
-// Time of the whole op, LDS-ring kernel before -> this one, K 4096: 32 rows x 4096 13.8 -> 7.9 us, 64 x 4096 17.0 -> 9.1,
-// 128 x 4096 18.6 -> 11.4, 256 x 4096 22.1 -> 15.9, 64 x 14336 22.0 -> 17.1; K 1024: 128 x 1024 10.8 -> 4.7.
-// The group scale is folded into fp16 weights as in the LDS-ring GEMM (exact for scales stored as fp16, 2^-11 per weight
-// otherwise).  The MFMA is issued with the weights as the A operand: a lane holds four consecutive columns of a row.
+// us per call, nodes of one graph with a caller's workspace, the kernels before (LDS-ring; up to 32 rows int4_mid.hip) ->
+// this one, fp16 rows, 32-groups, K 4096: 32 rows x 4096 10.9 -> 6.5, 64 x 4096 15.7 -> 7.9, 128 x 4096 17.0 -> 9.9, 256 x
+// 4096 21.0 -> 15.1, 64 x 14336 21.1 -> 15.9; 128 x 1024 x 1024 9.8 -> 4.4.  (Called one by one, with the scratch the library
+// then took per call: 21.7 -> 6.9, 25 -> 8.3, 25 -> 10.2, 25.4 -> 15.1, 25.5 -> 16.2, 9.5 -> 4.5.)
+// The group scale is folded into fp16 weights as in the LDS-ring GEMM: fp16((q - zp) * s), rounded to 2^-11 per weight.  The MFMA is issued with the weights as the A operand: a lane holds four consecutive columns of a row.
 #include <mutex>
 #include <type_traits>
 
