@@ -19,8 +19,8 @@ def test_more_streams_than_blocks_and_growing_requests():
     from yscv_amd import kernels as K
 
     rng = np.random.default_rng(1)
-    w = _weight(K, rng, 208, 960)  # 960 is no multiple of 512: prepared activations in the scratch
-    xs = [torch.from_numpy(rng.standard_normal((m, 960)).astype(np.float32)).half().cuda() for m in (3, 700, 40, 5000, 77, 1, 300, 20, 64, 9, 2500, 130)]
+    w = _weight(K, rng, 208, 960)  # bf16 rows above 16 are prepared in the scratch, and K is cut into parts there
+    xs = [torch.from_numpy(rng.standard_normal((m, 960)).astype(np.float32)).bfloat16().cuda() for m in (3, 700, 40, 5000, 77, 1, 300, 20, 64, 9, 2500, 130)]
     want = [w.matmul(x, out_dtype=torch.float32).clone() for x in xs]
     torch.cuda.synchronize()
     streams = [torch.cuda.Stream() for _ in range(11)]
@@ -41,7 +41,7 @@ def test_threads_on_one_stream():
 
     rng = np.random.default_rng(2)
     w = _weight(K, rng, 272, 1344)
-    xs = [torch.from_numpy(rng.standard_normal((50 + 30 * t, 1344)).astype(np.float32)).half().cuda() for t in range(4)]
+    xs = [torch.from_numpy(rng.standard_normal((50 + 30 * t, 1344)).astype(np.float32)).bfloat16().cuda() for t in range(4)]
     want = [w.matmul(x, out_dtype=torch.float32).clone() for x in xs]
     torch.cuda.synchronize()
     got = [[] for _ in xs]
@@ -68,8 +68,8 @@ def test_captured_call_keeps_its_own_memory():
 
     rng = np.random.default_rng(3)
     w = _weight(K, rng, 208, 960)
-    x = torch.from_numpy(rng.standard_normal((90, 960)).astype(np.float32)).half().cuda()
-    other = torch.from_numpy(rng.standard_normal((4000, 960)).astype(np.float32)).half().cuda()
+    x = torch.from_numpy(rng.standard_normal((90, 960)).astype(np.float32)).bfloat16().cuda()
+    other = torch.from_numpy(rng.standard_normal((4000, 960)).astype(np.float32)).bfloat16().cuda()
     want = w.matmul(x, out_dtype=torch.float32).clone()
     out = torch.empty_like(want)
     side = torch.cuda.Stream()
