@@ -119,7 +119,7 @@ int32_t Scratch::take(size_t bytes, hipStream_t stream) {
 
 Scratch::~Scratch() {
   if (slot) {
-    if (slot->end) (void)hipEventRecord(slot->end, s);
+    if (slot->end && hipEventRecord(slot->end, s) != hipSuccess) (void)hipStreamSynchronize(s);
     slot->busy.unlock();
   } else if (p) {
     (void)hipFreeAsync(p, s);
