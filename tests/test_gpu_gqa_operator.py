@@ -93,3 +93,13 @@ def test_rms_norm_widths(rows, d):
     odd = torch.empty(rows * d + 1, device="cuda")
     odd[1:] = x.reshape(-1)
     assert float((ops.rms_norm(odd[1:].view(rows, d), gamma, 1e-5).double() - want).abs().max() / want.abs().max()) < 1e-6
+
+
+def test_rms_norm_of_more_rows_than_one_launch_takes():
+    import torch
+
+    from yscv_amd import onnx_ops as ops
+
+    x, gamma = torch.randn((1 << 24) + 5, 4, device="cuda"), torch.rand(4, device="cuda") + 0.5
+    want = x / torch.sqrt(x.square().mean(-1, keepdim=True) + 1e-5) * gamma
+    assert float((ops.rms_norm(x, gamma, 1e-5) - want).abs().max()) < 1e-5  # f32 against f32, |want| up to 3

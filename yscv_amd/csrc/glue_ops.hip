@@ -25,6 +25,7 @@
 // enter the MFMAs as fp16, like the decoder's own kernels (tolerance-checked against the f32 restatement).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -1137,9 +1138,12 @@ int32_t yscv_hip_rms_norm_dev(const float *x, const float *gamma, size_t rows, s
   YSCV_REQUIRE(x && gamma && y, "null argument");
   YSCV_REQUIRE(std::isfinite(eps) && eps > 0.0f, "rms_norm: epsilon must be finite and > 0");
   YSCV_REQUIRE(d > 0 && d < ((size_t)1 << 31) && rows < ((size_t)1 << 31), "rms_norm: bad shape %zu x %zu", rows, d);
-  if (rows == 0) return YSCV_HIP_OK;
-  hipLaunchKernelGGL(rms_norm_f32_kernel, dim3((unsigned)rows), dim3(256), 0, as_stream(stream), x, gamma, (int)d, eps, y);
-  YSCV_HIP_TRY(hipGetLastError());
+  const size_t step = (size_t)1 << 23;  // a grid holds less than 2^32 threads
+  for (size_t r0 = 0; r0 < rows; r0 += step) {
+    hipLaunchKernelGGL(rms_norm_f32_kernel, dim3((unsigned)std::min(step, rows - r0)), dim3(256), 0, as_stream(stream), x + r0 * d, gamma,
+                       (int)d, eps, y + r0 * d);
+    YSCV_HIP_TRY(hipGetLastError());
+  }
   return YSCV_HIP_OK;
 }
 
