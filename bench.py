@@ -425,12 +425,11 @@ def extra_kernels(torch, stream_ptr):
         fl = 2.0 * m * k * n
         sweep["m%d" % m] = {"us": round(t * 1e6, 1), "weight_GB/s": round(wbytes / t / 1e9, 0),
                             "frac_of_hbm_peak": round(wbytes / t / 1e9 / HBM_PEAK_GBS, 3),
-                            "TFLOP/s": round(fl / t / 1e12, 1), "frac_of_mfma_peak": round(fl / t / 1e12 / MFMA_BF16_PEAK, 4),
-                            "kernel": "int4_skinny_kernel" if m <= 16 else ("int4_mid_kernel" if m <= 32 else "int4_gemm_ring_kernel")}
+                            "TFLOP/s": round(fl / t / 1e12, 1), "frac_of_mfma_peak": round(fl / t / 1e12 / MFMA_BF16_PEAK, 4)}
     out["config5_lm_head_sweep_k4096_n128256"] = sweep
 
     # where the skinny kernel hands over to the MFMA GEMM: both kernels on either side of m = 16 (event-timed eager
-    # calls: the forced modes take their scratch from the stream-ordered allocator)
+    # calls: the forced modes take the library's own scratch)
     def teager(fn, reps=20):
         for _ in range(3):
             fn()
@@ -471,7 +470,7 @@ def bench_prefill(dec, torch, cfg, n_tokens, params):
     import numpy as np
 
     prompt = np.random.default_rng(11).integers(0, cfg["vocab"], n_tokens).astype(np.int32)
-    dec.prefill(prompt)  # warm-up: kernel images, the stream-ordered pool's first allocations
+    dec.prefill(prompt)  # warm-up: kernel images, the buffers the decoder keeps
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     reps = 3
@@ -482,7 +481,7 @@ def bench_prefill(dec, torch, cfg, n_tokens, params):
     fl = 2.0 * (params - cfg["vocab"] * cfg["d_model"]) * n_tokens  # the LM head sees the last row only
     return {"ms": round(t * 1e3, 2), "prompt_tok/s": round(n_tokens / t, 0), "TFLOP/s_projections": round(fl / t / 1e12, 1),
             "frac_of_mfma_peak": round(fl / t / 1e12 / MFMA_BF16_PEAK, 4),
-            "note": "host-timed whole call (token upload, per-call scratch from the stream-ordered pool, every launch), "
+            "note": "host-timed whole call (token upload, every launch; buffers kept from the first call), "
                     "one pass over all 32 layers; feeding the same prompt through the decode step takes n x ms_per_step"}
 
 
