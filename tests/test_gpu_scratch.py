@@ -86,3 +86,48 @@ def test_captured_call_keeps_its_own_memory():
         w.matmul(other)  # another call's scratch between the replays
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("where", ["used before", "new", "default", "growing"])
+def test_a_call_beside_a_capture_of_another_stream(where):
+    """Calls on one stream while another is captured (torch's default mode watches the whole process for calls that may not
+    happen meanwhile): they run, and the capture goes on."""
+    import ctypes as C
+
+    import torch
+
+    from yscv_amd import BF16, kernels as K, lib
+
+    rng = np.random.default_rng(4)
+    w = _weight(K, rng, 256, 512)
+    x = torch.from_numpy(rng.standard_normal((24, 512)).astype(np.float32)).bfloat16().cuda()
+    want = w.matmul(x)
+    got, z = torch.zeros_like(want), torch.zeros(4, device="cuda")
+    captured, other = torch.cuda.Stream(), torch.cuda.default_stream() if where == "default" else torch.cuda.Stream()
+    long_x = torch.from_numpy(rng.standard_normal((9000, 512)).astype(np.float32)).bfloat16().cuda()
+    long_want = w.matmul(long_x)
+    long_got = torch.zeros_like(long_want)
+
+    def call_long():
+        lib().int4_matmul(w._h, C.c_void_p(long_x.data_ptr()), BF16, C.c_void_p(long_got.data_ptr()), BF16, C.c_size_t(9000),
+                          C.c_void_p(other.cuda_stream))
+
+    def call():
+        lib().int4_matmul(w._h, C.c_void_p(x.data_ptr()), BF16, C.c_void_p(got.data_ptr()), BF16, C.c_size_t(24), C.c_void_p(other.cuda_stream))
+
+    if where != "new":
+        call()
+    torch.cuda.synchronize()
+    got.zero_()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=captured):
+        z += 1
+        for _ in range(3):
+            call()
+        if where == "growing":
+            call_long()  # more than the block holds
+    g.replay()
+    torch.cuda.synchronize()
+    assert where != "growing" or torch.equal(long_got, long_want)
+    assert z.tolist() == [1.0] * 4 and torch.equal(got, want)

@@ -3,7 +3,7 @@
 // A hipMallocAsync / hipFreeAsync pair costs 15 us of host time on this runtime, as much as the kernels of a small call
 // together (24 bf16 rows x 256 x 512: 26.5 us a call against 11.7 with the caller's own workspace), so blocks are kept.  On
 // the default stream a block costs nothing measurable (7.9 us a call, 8.2 with the caller's workspace), on another stream 4 us
-// (12.3): the capture query, the wait for the last use, the event behind this one.
+// (12.1): the capture query, the wait for the last use, the event behind this one.
 // There is one block for the default stream and eight for other streams (least recently used one first when
 // a ninth stream comes).  A block is used by one call at a time: its lock is held from the first launch that uses it to
 // the last, so two threads on one stream cannot interleave their launches, and the stream runs them in that order.
@@ -83,9 +83,9 @@ int32_t Scratch::take(size_t bytes, hipStream_t stream) {
   slot->busy.lock();
   int device = 0;
   hipError_t e = hipGetDevice(&device);
-  // (an event belongs to one device: another one's is drained on the host and dropped with the block)
-  if (e == hipSuccess && slot->end && slot->device == device && hipEventQuery(slot->end) != hipSuccess)
-    e = hipStreamWaitEvent(stream, slot->end, 0);
+  // (an event belongs to one device: another one's is drained on the host and dropped with the block.  The event is not
+  // asked whether it has passed: such a query ends the capture that another stream may be under.)
+  if (e == hipSuccess && slot->end && slot->device == device) e = hipStreamWaitEvent(stream, slot->end, 0);
   if (e == hipSuccess && slot->p && (slot->device != device || slot->cap < bytes)) {
     if (slot->device == device) {
       e = hipFreeAsync(slot->p, stream);  // behind the wait above, so behind its last use
