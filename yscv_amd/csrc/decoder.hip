@@ -7,6 +7,7 @@
 #include <cmath>
 #include <vector>
 
+#include "decode_layers.hpp"
 #include "decoder.hpp"
 #include "int4_common.hpp"
 #include "kernels.hpp"
@@ -183,19 +184,35 @@ struct yscv_hip_decoder {
   size_t p_exch_entries = 0;
   uint32_t epoch = 1;          // tag epoch of the next persistent step; tags are 24 bits wide: see yscv_hip_decoder_run
   unsigned long long *p_trace = nullptr;  // stage timestamps (builds with YSCV_PERSIST_TRACE only)
+  // small models at batch 1, YSCV_HIP_DECODE_AUTO: all layers of a step in one launch (decode_layers.hip), a graph of its own
+  bool layers_ok = false;      // the shape is supported, the buffers exist and the weights are laid out as it reads them
+  LayersModel lm{};
+  LayersLayer *l_table = nullptr;
+  unsigned long long *l_exch = nullptr;
+  size_t l_exch_entries = 0;
+  uint32_t *l_count = nullptr;
+  uint32_t l_steps = 0;        // what *l_count holds once everything enqueued so far has run
+  uint32_t *l_give_up = nullptr;  // pinned host memory
+  int l_last_pos = -1;         // position of the last step when it was one of these: its activations are in the exchange buffer
+  hipGraph_t l_graph = nullptr;
+  hipGraphExec_t l_graph_exec = nullptr;
 };
 
 // A captured step holds the addresses of the weights and of the workspace as they were at capture time: whatever
 // frees or replaces one of them drops the graph, and the next graph run captures again.  Replays of it may still be under
 // way (no call waits for them): they are waited for first.
-static void drop_graph(yscv_hip_decoder *d) {
-  if (d->graph_exec) {
+static void drop_captured(hipGraph_t *graph, hipGraphExec_t *exec) {
+  if (*exec) {
     (void)hipDeviceSynchronize();
-    (void)hipGraphExecDestroy(d->graph_exec);
+    (void)hipGraphExecDestroy(*exec);
   }
-  if (d->graph) (void)hipGraphDestroy(d->graph);
-  d->graph_exec = nullptr;
-  d->graph = nullptr;
+  if (*graph) (void)hipGraphDestroy(*graph);
+  *exec = nullptr;
+  *graph = nullptr;
+}
+static void drop_graph(yscv_hip_decoder *d) {
+  drop_captured(&d->graph, &d->graph_exec);
+  drop_captured(&d->l_graph, &d->l_graph_exec);
   d->graph_batch = 0;
 }
 
@@ -248,6 +265,10 @@ static void decoder_free(yscv_hip_decoder *d) {
   (void)hipFree(d->p_exch);
   (void)hipFree(d->p_abort);
   (void)hipFree(d->p_trace);
+  (void)hipFree(d->l_table);
+  (void)hipFree(d->l_exch);
+  (void)hipFree(d->l_count);
+  (void)hipHostFree(d->l_give_up);
   if (d->end_event) (void)hipEventDestroy(d->end_event);
   delete d;
 }
@@ -475,6 +496,81 @@ static int32_t alloc_runtime(yscv_hip_decoder *d) {
   return YSCV_HIP_OK;
 }
 
+static int32_t layers_setup(yscv_hip_decoder *d) {
+  const Context *ctx = nullptr;
+  YSCV_TRY(ensure_context(&ctx));
+  const auto &c = d->cfg;
+  if (d->kv_dtype != YSCV_HIP_KV_F16 || !layers_supported(c, ctx->num_cus)) return YSCV_HIP_OK;
+  LayersModel &m = d->lm;
+  m.n_layers = c.n_layers;
+  m.d = c.d_model;
+  m.heads = c.n_heads;
+  m.kv_heads = c.n_kv_heads;
+  m.ff = c.d_ff;
+  m.vocab = c.vocab;
+  m.max_ctx = c.max_ctx;
+  m.G = c.d_model / 16;
+  m.theta = c.rope_theta;
+  m.eps = c.rms_eps;
+  m.emb = d->emb;
+  m.tokens = d->tokens;
+  m.pos = d->pos;
+  m.h = d->h;
+  size_t entries[5], total = 0, at[5];
+  layers_exchange_entries(c, entries);
+  for (int i = 0; i < 5; i++) {
+    at[i] = total;
+    total += round_up(entries[i], 32);  // every buffer 256-byte aligned
+  }
+  if (total >= (1ull << 31)) return YSCV_HIP_OK;  // offsets are 32-bit
+  DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->l_exch), total * 8));
+  DEC_HIP(hipMemset(d->l_exch, 0, total * 8));
+  d->l_exch_entries = total;
+  DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->l_count), 4));
+  DEC_HIP(hipMemset(d->l_count, 0, 4));
+  DEC_HIP(hipHostMalloc(reinterpret_cast<void **>(&d->l_give_up), 4, hipHostMallocDefault));
+  *d->l_give_up = 0;
+  DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->l_table), c.n_layers * sizeof(LayersLayer)));
+  m.x = d->l_exch;
+  m.at_attn = (int)at[0];
+  m.at_ffn = (int)at[1];
+  m.at_qkv = (int)at[2];
+  m.at_act = (int)at[3];
+  m.at_part = (int)at[4];
+  m.steps = d->l_count;
+  m.give_up = d->l_give_up;
+  m.layers = reinterpret_cast<decltype(m.layers)>(reinterpret_cast<uintptr_t>(d->l_table));
+  return YSCV_HIP_OK;
+}
+
+// the weights, caches and biases as they are now
+static int32_t layers_fill_table(yscv_hip_decoder *d) {
+  d->layers_ok = false;
+  if (!d->l_table) return YSCV_HIP_OK;
+  std::vector<LayersLayer> t(d->layers.size());
+  bool usable = true;
+  for (size_t l = 0; l < t.size(); l++) {
+    auto &L = d->layers[l];
+    const yscv_hip_int4_weight *w[4] = {L.wqkv, L.wo, L.wgu, L.wdown};
+    for (int i = 0; i < 4; i++) {
+      if (!w[i]->tiled || w[i]->gm != 0 || w[i]->scale_dtype != YSCV_HIP_F16 || w[i]->has_zp || w[i]->chunks != w[i]->ktp ||
+          (l > 0 && (int)w[i]->ktp != d->lm.ktp[i]))
+        usable = false;
+      d->lm.ktp[i] = (int)w[i]->ktp;
+      t[l].tiles[i] = w[i]->tiles;
+      t[l].scales[i] = static_cast<const _Float16 *>(w[i]->tscales);
+    }
+    t[l].gamma[0] = L.attn_norm;
+    t[l].gamma[1] = L.ffn_norm;
+    t[l].kc = L.kc;
+    t[l].vc = L.vc;
+    t[l].qkv_bias = L.qkv_bias;
+  }
+  DEC_HIP(hipMemcpy(d->l_table, t.data(), t.size() * sizeof(LayersLayer), hipMemcpyHostToDevice));
+  d->layers_ok = usable;
+  return YSCV_HIP_OK;
+}
+
 static int32_t finish_setup(yscv_hip_decoder *d) {
   drop_graph(d);
   // workspace: the largest any projection needs at the maximum batch
@@ -533,7 +629,38 @@ static int32_t finish_setup(yscv_hip_decoder *d) {
     ok = ok && direct(d->lm_head);
     d->fold_norm = ok;
   }
+  YSCV_TRY(layers_fill_table(d));
   d->finalized = true;
+  return YSCV_HIP_OK;
+}
+
+// the launches of a step whose layers run in one
+static int32_t enqueue_layers_step(yscv_hip_decoder *d, hipStream_t s) {
+  const auto &c = d->cfg;
+  YSCV_TRY(launch_decode_layers(d->lm, s));
+  YSCV_TRY(launch_rmsnorm(d->h, d->final_norm, 1, c.d_model, c.rms_eps, d->xn, s));
+  YSCV_TRY(int4_run_ws(d->lm_head, d->xn, YSCV_HIP_F16, d->logits, YSCV_HIP_F32, 1, 1, EPI_STORE, d->ws, d->ws_bytes, s));
+  YSCV_TRY(launch_argmax(d->logits, 1, c.vocab, d->tokens, d->history, d->step, c.max_steps, s));
+  YSCV_TRY(launch_advance(d->pos, d->step, s));
+  return YSCV_HIP_OK;
+}
+
+// captures what `enqueue` launches on the stream it is given
+template <typename F>
+static int32_t capture_step(F enqueue, hipGraph_t *graph, hipGraphExec_t *exec) {
+  hipStream_t cs = nullptr;
+  DEC_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
+  hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
+  int32_t st = YSCV_HIP_OK;
+  if (e == hipSuccess) {
+    st = enqueue(cs);
+    hipError_t e2 = hipStreamEndCapture(cs, graph);
+    if (st == YSCV_HIP_OK && e2 != hipSuccess) e = e2;
+  }
+  if (st == YSCV_HIP_OK && e == hipSuccess) e = hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0);
+  (void)hipStreamDestroy(cs);
+  if (st != YSCV_HIP_OK) return st;
+  if (e != hipSuccess) return set_error(YSCV_HIP_ERR_DEVICE, "graph capture failed: %s", hipGetErrorString(e));
   return YSCV_HIP_OK;
 }
 
@@ -643,6 +770,10 @@ static int32_t enqueue_step(yscv_hip_decoder *d, int batch, hipStream_t s) {
 }
 
 static int32_t check_persist_abort(yscv_hip_decoder *d) {
+  if (d->l_give_up && *d->l_give_up) {  // (the device has been waited for)
+    *d->l_give_up = 0;
+    return set_error(YSCV_HIP_ERR_DEVICE, "the decode step gave up waiting for a stage of a layer (bounded wait expired)");
+  }
   if (!d->persist_ok) return YSCV_HIP_OK;
   uint32_t flag = 0;
   DEC_HIP(hipMemcpy(&flag, d->p_abort, 4, hipMemcpyDeviceToHost));
@@ -730,6 +861,7 @@ int32_t yscv_hip_decoder_create_kv(const yscv_hip_decoder_config *cfg, int32_t k
     if (e != hipSuccess) st = set_error(YSCV_HIP_ERR_DEVICE, "setup failed: %s", hipGetErrorString(e));
   }
   if (st == YSCV_HIP_OK && c.max_batch >= 1) st = persist_setup(d);
+  if (st == YSCV_HIP_OK) st = layers_setup(d);
   if (st != YSCV_HIP_OK) {
     decoder_free(d);
     return st;
@@ -1002,7 +1134,9 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
                d->cfg.max_ctx);
   YSCV_REQUIRE(step + n_steps <= d->cfg.max_steps, "token history overflow: %d + %d > max_steps %d", step, n_steps,
                d->cfg.max_steps);
-  if (use_graph == YSCV_HIP_DECODE_AUTO)  // the fastest path this decoder has for its batch
+  // the fastest path this decoder has for its batch; the layers of a small model in one launch are part of a graph too
+  const bool layers = use_graph == YSCV_HIP_DECODE_AUTO && d->batch == 1 && d->layers_ok;
+  if (use_graph == YSCV_HIP_DECODE_AUTO)
     use_graph = (d->batch == 1 && d->persist_ok && !d->has_bias && d->kv_dtype == YSCV_HIP_KV_F16) ? 2 : 1;
   d->last_path = use_graph == 2 ? 2 : (use_graph ? 1 : 0);
   if (use_graph == 2) {
@@ -1035,6 +1169,28 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
     return YSCV_HIP_OK;
   }
   DEC_HIP(call.enter());
+  if (layers) {
+    // tags count steps: before they wrap, the entries are cleared and the count starts again
+    const uint32_t most = (uint32_t)(0xFFFFFFFEull / ((uint64_t)d->cfg.n_layers + 1)) - 1;
+    if (d->l_steps >= most - (uint32_t)n_steps) {
+      hipLaunchKernelGGL(fill_i32_kernel, dim3(grid_for(d->l_exch_entries * 2)), dim3(256), 0, s,
+                         reinterpret_cast<int32_t *>(d->l_exch), d->l_exch_entries * 2, 0);
+      hipLaunchKernelGGL(fill_i32_kernel, dim3(1), dim3(256), 0, s, reinterpret_cast<int32_t *>(d->l_count), (size_t)1, 0);
+      DEC_HIP(hipGetLastError());
+      d->l_steps = 0;
+    }
+    if (!d->l_graph_exec)
+      YSCV_TRY(capture_step([&](hipStream_t cs) { return enqueue_layers_step(d, cs); }, &d->l_graph, &d->l_graph_exec));
+    for (int i = 0; i < n_steps; i++) {
+      DEC_HIP(hipGraphLaunch(d->l_graph_exec, s));
+      d->pos_host++;
+      d->step_host++;
+      d->l_steps++;
+      d->l_last_pos = d->pos_host - 1;
+    }
+    return YSCV_HIP_OK;
+  }
+  d->l_last_pos = -1;
   if (!use_graph) {
     for (int i = 0; i < n_steps; i++) {
       YSCV_TRY(enqueue_step(d, d->batch, s));
@@ -1044,20 +1200,8 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
     return YSCV_HIP_OK;
   }
   if (!d->graph_exec || d->graph_batch != d->batch) {
-    drop_graph(d);
-    hipStream_t cs = nullptr;
-    DEC_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
-    hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
-    int32_t st = YSCV_HIP_OK;
-    if (e == hipSuccess) {
-      st = enqueue_step(d, d->batch, cs);
-      hipError_t e2 = hipStreamEndCapture(cs, &d->graph);
-      if (st == YSCV_HIP_OK && e2 != hipSuccess) e = e2;
-    }
-    if (st == YSCV_HIP_OK && e == hipSuccess) e = hipGraphInstantiate(&d->graph_exec, d->graph, nullptr, nullptr, 0);
-    (void)hipStreamDestroy(cs);
-    if (st != YSCV_HIP_OK) return st;
-    if (e != hipSuccess) return set_error(YSCV_HIP_ERR_DEVICE, "graph capture failed: %s", hipGetErrorString(e));
+    drop_captured(&d->graph, &d->graph_exec);
+    YSCV_TRY(capture_step([&](hipStream_t cs) { return enqueue_step(d, d->batch, cs); }, &d->graph, &d->graph_exec));
     d->graph_batch = d->batch;
   }
   for (int i = 0; i < n_steps; i++) {
@@ -1077,6 +1221,7 @@ int32_t yscv_hip_decoder_run_projections(yscv_hip_decoder *d, int32_t n_steps, v
   if (!stream_capturing(s)) DEC_HIP(call.enter());  // (a graph of them is ordered by whoever replays it)
   const int batch = d->batch;
   const auto &c = d->cfg;
+  d->l_last_pos = -1;
   for (int i = 0; i < n_steps; i++) {
     // the same calls as in a real step, folded norms included (their partial sums are whatever the buffers hold)
     int cur = 0, cnt = 1;
@@ -1167,6 +1312,10 @@ int32_t yscv_hip_decoder_read_activation(yscv_hip_decoder *d, int32_t which, flo
   }
   YSCV_REQUIRE(capacity >= elems, "output holds %zu values, the buffer has %zu", capacity, elems);
   DEC_HIP(hipDeviceSynchronize());
+  if (d->l_last_pos >= 0) {
+    YSCV_TRY(launch_layers_report(d->lm, d->l_last_pos, d->qkv, d->qrot, d->ao, d->act, nullptr));
+    DEC_HIP(hipDeviceSynchronize());
+  }
   if (!half) {
     DEC_HIP(hipMemcpy(out_host, src, elems * 4, hipMemcpyDeviceToHost));
     return YSCV_HIP_OK;
@@ -1180,7 +1329,7 @@ int32_t yscv_hip_decoder_read_activation(yscv_hip_decoder *d, int32_t which, flo
       DEC_HIP(hipMemcpy(tmp.data() + b * qkv_n, d->qrot + b * qn, qn * 2, hipMemcpyDeviceToHost));
   }
   for (size_t i = 0; i < elems; i++) out_host[i] = (float)tmp[i];
-  if (which == YSCV_HIP_DEC_ACT_NORMED && d->fold_norm && d->last_ss_count > 0) {
+  if (which == YSCV_HIP_DEC_ACT_NORMED && d->fold_norm && d->last_ss_count > 0 && d->l_last_pos < 0) {
     // folded norm: the buffer holds fp16(h * gamma * pre[row]); what the consumer multiplied by its weights is that
     // times the row factor it worked out from the partial sums of squares and pre[row]
     std::vector<float> ss((size_t)B * d->ss_stride), pre(B);
@@ -1215,6 +1364,11 @@ __attribute__((visibility("default"))) int32_t yscv_hip_debug_persist_trace(yscv
 int32_t yscv_hip_decoder_debug_set_tag_epoch(yscv_hip_decoder *d, uint32_t epoch) {
   YSCV_REQUIRE(d != nullptr && epoch >= 1, "null decoder or epoch 0");
   d->epoch = epoch;
+  if (d->l_count) {
+    DEC_HIP(hipDeviceSynchronize());
+    DEC_HIP(hipMemcpy(d->l_count, &epoch, 4, hipMemcpyHostToDevice));
+    d->l_steps = epoch;
+  }
   return YSCV_HIP_OK;
 }
 
@@ -1249,6 +1403,7 @@ int32_t yscv_hip_decoder_set_qkv_bias(yscv_hip_decoder *d, int32_t layer, const 
   }
   d->has_bias = false;
   for (auto &l : d->layers) d->has_bias = d->has_bias || l.qkv_bias != nullptr;
+  if (d->finalized) YSCV_TRY(layers_fill_table(d));
   return YSCV_HIP_OK;
 }
 
