@@ -150,6 +150,8 @@ struct yscv_hip_decoder {
   void *ws = nullptr;
   size_t ws_bytes = 0;
   int32_t *tokens = nullptr, *history = nullptr, *pos = nullptr, *step = nullptr;
+  PickPart *pick = nullptr;       // what the greedy pick kept of every chunk of the last logits
+  uint32_t *cand = nullptr;       // pinned: flag, counts and entries of launch_top_candidates, allocated by the first call for them
   int batch = 0;
   // what *pos and *step hold once everything enqueued so far has run: every call knows how far it moves them, so the
   // bounds checks of a run need no read-back
@@ -254,6 +256,8 @@ static void decoder_free(yscv_hip_decoder *d) {
   (void)hipFree(d->prompt);
   (void)hipFree(d->tokens);
   (void)hipFree(d->history);
+  (void)hipFree(d->pick);
+  (void)hipHostFree(d->cand);
   (void)hipFree(d->pos);
   (void)hipFree(d->step);
   (void)hipFree(d->p_stream);
@@ -487,6 +491,7 @@ static int32_t alloc_runtime(yscv_hip_decoder *d) {
   }
   DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->tokens), B * 4));
   DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->history), B * (size_t)c.max_steps * 4));
+  DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->pick), B * (size_t)pick_chunks(c.vocab) * sizeof(PickPart)));
   DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->pos), 4));
   DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->step), 4));
   DEC_HIP(hipMemset(d->tokens, 0, B * 4));
@@ -640,8 +645,7 @@ static int32_t enqueue_layers_step(yscv_hip_decoder *d, hipStream_t s) {
   YSCV_TRY(launch_decode_layers(d->lm, s));
   YSCV_TRY(launch_rmsnorm(d->h, d->final_norm, 1, c.d_model, c.rms_eps, d->xn, s));
   YSCV_TRY(int4_run_ws(d->lm_head, d->xn, YSCV_HIP_F16, d->logits, YSCV_HIP_F32, 1, 1, EPI_STORE, d->ws, d->ws_bytes, s));
-  YSCV_TRY(launch_argmax(d->logits, 1, c.vocab, d->tokens, d->history, d->step, c.max_steps, s));
-  YSCV_TRY(launch_advance(d->pos, d->step, s));
+  YSCV_TRY(launch_pick(d->logits, 1, c.vocab, d->pick, d->tokens, d->history, d->pos, d->step, c.max_steps, s));
   return YSCV_HIP_OK;
 }
 
@@ -764,8 +768,7 @@ static int32_t enqueue_step(yscv_hip_decoder *d, int batch, hipStream_t s) {
     YSCV_TRY(launch_rmsnorm(d->h, d->final_norm, batch, D, c.rms_eps, d->xn, s));
     YSCV_TRY(int4_run_ws(d->lm_head, d->xn, YSCV_HIP_F16, d->logits, YSCV_HIP_F32, batch, 1, EPI_STORE, d->ws, d->ws_bytes, s));
   }
-  YSCV_TRY(launch_argmax(d->logits, batch, c.vocab, d->tokens, d->history, d->step, c.max_steps, s));
-  YSCV_TRY(launch_advance(d->pos, d->step, s));
+  YSCV_TRY(launch_pick(d->logits, batch, c.vocab, d->pick, d->tokens, d->history, d->pos, d->step, c.max_steps, s));
   return YSCV_HIP_OK;
 }
 
@@ -1293,6 +1296,42 @@ int32_t yscv_hip_decoder_read_logits(yscv_hip_decoder *d, float *out_host) {
   return YSCV_HIP_OK;
 }
 
+}  // extern "C"
+
+namespace yscv {
+// The logits of the last step that top-k sampling with their values times `scale` can keep, in index order; *whole when the
+// caller has to look at all of them (k outside 1 .. chunks, a NaN or an infinity among them).  Waits for the device.
+int32_t decoder_top_candidates(yscv_hip_decoder *d, size_t k, float scale, std::vector<float> &values, std::vector<uint32_t> &indices,
+                               bool *whole) {
+  const int vocab = d->cfg.vocab, chunks = pick_chunks(vocab);
+  *whole = true;
+  if (k < 1 || k > (size_t)chunks || chunks > 1024) return YSCV_HIP_OK;
+  InOrder call(d, nullptr);
+  DEC_HIP(call.enter());
+  const size_t at_entries = round_up((size_t)(1 + chunks) * 4, 64);
+  if (!d->cand)
+    DEC_HIP(hipHostMalloc(reinterpret_cast<void **>(&d->cand), at_entries + (size_t)chunks * kPickChunk * sizeof(TopCandidate), hipHostMallocDefault));
+  d->cand[0] = 0;
+  TopCandidate *entries = reinterpret_cast<TopCandidate *>(reinterpret_cast<char *>(d->cand) + at_entries);
+  if (d->last_path == 2) YSCV_TRY(launch_pick_chunks(d->logits, 1, vocab, d->pick, nullptr));  // that kernel picks by itself
+  YSCV_TRY(launch_top_candidates(d->logits, vocab, d->pick, (int)k, scale, d->cand + 1, entries, d->cand, nullptr));
+  DEC_HIP(hipDeviceSynchronize());
+  YSCV_TRY(check_persist_abort(d));
+  if (d->cand[0]) return YSCV_HIP_OK;
+  values.clear();
+  indices.clear();
+  for (int c = 0; c < chunks; c++)
+    for (uint32_t i = 0; i < d->cand[1 + c]; i++) {
+      values.push_back(entries[(size_t)c * kPickChunk + i].value);
+      indices.push_back(entries[(size_t)c * kPickChunk + i].index);
+    }
+  *whole = false;
+  return YSCV_HIP_OK;
+}
+}  // namespace yscv
+
+extern "C" {
+
 int32_t yscv_hip_decoder_read_activation(yscv_hip_decoder *d, int32_t which, float *out_host, size_t capacity) {
   YSCV_REQUIRE(d && out_host, "null argument");
   YSCV_REQUIRE(d->batch >= 1, "call yscv_hip_decoder_reset first");
@@ -1520,8 +1559,7 @@ int32_t yscv_hip_decoder_prefill(yscv_hip_decoder *d, const int32_t *tokens_host
   DEC_HIP(hipGetLastError());
   d->pos_host = start_pos + n_tokens - 1;
   d->step_host = 0;
-  YSCV_TRY(launch_argmax(d->logits, 1, c.vocab, d->tokens, d->history, d->step, c.max_steps, s));
-  YSCV_TRY(launch_advance(d->pos, d->step, s));
+  YSCV_TRY(launch_pick(d->logits, 1, c.vocab, d->pick, d->tokens, d->history, d->pos, d->step, c.max_steps, s));
   d->pos_host = start_pos + n_tokens;
   d->step_host = 1;
   d->last_path = 1;

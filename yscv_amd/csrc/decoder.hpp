@@ -45,9 +45,26 @@ int32_t launch_attention_fused_i8(const _Float16 *qkv, int8_t *kc, float *ks, in
                                   int batch, int hq, int hkv, int hd, float theta, int max_ctx, float *part, _Float16 *qrot,
                                   _Float16 *out, hipStream_t s);
 int32_t launch_kv_random_fill_i8(int8_t *buf, size_t n, float *scales, size_t n_scales, float scale, uint64_t seed, hipStream_t s);
-int32_t launch_argmax(const float *logits, int batch, int vocab, int32_t *tokens, int32_t *history,
-                      int32_t *step_ptr, int max_steps, hipStream_t s);
-int32_t launch_advance(int32_t *pos_ptr, int32_t *step_ptr, hipStream_t s);
+// greedy pick per row of logits, tokens and history recorded, *pos and *step advanced; `parts` keeps what the chunks of 1024
+// logits gave: pick_chunks(vocab) per row
+constexpr int kPickChunk = 1024;
+inline int pick_chunks(int vocab) { return (vocab + kPickChunk - 1) / kPickChunk; }
+struct PickPart {
+  float best;
+  int idx;
+  float top;  // largest value that is no NaN
+  int flags;  // 1: a NaN, 2: a NaN or +inf
+};
+int32_t launch_pick_chunks(const float *logits, int batch, int vocab, PickPart *parts, hipStream_t s);
+int32_t launch_pick(const float *logits, int batch, int vocab, PickPart *parts, int32_t *tokens, int32_t *history, int32_t *pos_ptr,
+                    int32_t *step_ptr, int max_steps, hipStream_t s);
+struct TopCandidate {
+  float value;
+  uint32_t index;
+};
+// row 0's logits that can be among the k largest (decoder_kernels.hip); counts, out and odd are pinned host memory
+int32_t launch_top_candidates(const float *logits, int vocab, const PickPart *parts, int k, float scale, uint32_t *counts, TopCandidate *out,
+                              uint32_t *odd, hipStream_t s);
 int32_t launch_kv_random_fill(_Float16 *buf, size_t n, uint64_t seed, hipStream_t s);
 
 // glue_ops.hip: the general attention kernel over the fp16 cache (any head width that is a multiple of 32 up to 128,

@@ -223,20 +223,29 @@ uint32_t sample_selected(float *logits, size_t vocab_size, size_t top_k, float t
   return kept[best];
 }
 
+// xorshift64 draw (generate.rs:188-192); `u64 as f32` rounds to nearest, u64::MAX as f32 is 2^64
+float draw(uint64_t *rng) {
+  uint64_t x = *rng;
+  x ^= x << 13;
+  x ^= x >> 7;
+  x ^= x << 17;
+  *rng = x;
+  return (float)x / 18446744073709551616.0f;
+}
+
 }  // namespace
+
+namespace yscv {
+int32_t decoder_top_candidates(yscv_hip_decoder *d, size_t k, float scale, std::vector<float> &values, std::vector<uint32_t> &indices,
+                               bool *whole);
+}
 
 extern "C" {
 
 int32_t yscv_hip_sample_token(float *logits, size_t vocab_size, size_t top_k, float top_p, uint64_t *rng, uint32_t *token_out) {
   YSCV_REQUIRE(logits && rng && token_out, "null argument");
   YSCV_REQUIRE(vocab_size > 0, "empty vocabulary");
-  // xorshift64 draw (generate.rs:188-192); `u64 as f32` rounds to nearest, u64::MAX as f32 is 2^64
-  uint64_t x = *rng;
-  x ^= x << 13;
-  x ^= x >> 7;
-  x ^= x << 17;
-  *rng = x;
-  const float u = (float)x / 18446744073709551616.0f;
+  const float u = draw(rng);
   int odd = 0, finite = 0;  // a NaN or +inf anywhere; anything above -inf anywhere
   for (size_t i = 0; i < vocab_size; i++) {
     odd |= !(logits[i] <= FLT_MAX);
@@ -269,9 +278,24 @@ int32_t yscv_hip_decoder_generate(yscv_hip_decoder *d, const uint32_t *input_ids
     YSCV_REQUIRE(n_input < ((size_t)1 << 31), "prompt too long");
     YSCV_TRY(yscv_hip_decoder_prefill(d, prompt.data(), (int32_t)n_input, 0, nullptr));
   }
+  const bool scaled = cfg->temperature != 1.0f && cfg->temperature > 0.0f;
+  const float inv_temp = scaled ? 1.0f / cfg->temperature : 1.0f;
+  std::vector<float> cand;
+  std::vector<uint32_t> cand_index;
   for (size_t g = 0; g < cfg->max_tokens; g++) {
-    YSCV_TRY(yscv_hip_decoder_read_logits(d, logits.data()));
-    if (cfg->repetition_penalty != 1.0f) {  // generate.rs:80-92
+    // Without a repetition penalty the device sends the few logits that top-k can keep (multiplied by 1 / temperature there,
+    // the same f32 product): everything below the k-th largest has probability 0 in sample_token, so the sampler gives the
+    // same token on those alone.  A sampled token of a 151936-token vocabulary beside prompt and decode steps: 100 -> 3 us.
+    bool whole = true;
+    uint32_t next = 0;
+    if (cfg->repetition_penalty == 1.0f && inv_temp > 0.0f && inv_temp <= FLT_MAX && cfg->top_k < vocab)
+      YSCV_TRY(decoder_top_candidates(d, cfg->top_k, inv_temp, cand, cand_index, &whole));
+    if (!whole) {
+      const float u = draw(&rng_state);
+      next = cand_index[sample_selected(cand.data(), cand.size(), cfg->top_k, cfg->top_p, u)];
+    }
+    if (whole) YSCV_TRY(yscv_hip_decoder_read_logits(d, logits.data()));
+    if (whole && cfg->repetition_penalty != 1.0f) {  // generate.rs:80-92
       for (uint32_t t : tokens) {
         if (t < logits.size()) {
           if (logits[t] > 0.0f) logits[t] /= cfg->repetition_penalty;
@@ -279,12 +303,10 @@ int32_t yscv_hip_decoder_generate(yscv_hip_decoder *d, const uint32_t *input_ids
         }
       }
     }
-    if (cfg->temperature != 1.0f && cfg->temperature > 0.0f) {  // generate.rs:95-100
-      const float inv_temp = 1.0f / cfg->temperature;
+    if (whole && scaled) {  // generate.rs:95-100
       for (float &v : logits) v *= inv_temp;
     }
-    uint32_t next = 0;
-    YSCV_TRY(yscv_hip_sample_token(logits.data(), vocab, cfg->top_k, cfg->top_p, &rng_state, &next));
+    if (whole) YSCV_TRY(yscv_hip_sample_token(logits.data(), vocab, cfg->top_k, cfg->top_p, &rng_state, &next));
     if (cfg->has_eos && cfg->eos_token_id == next) break;
     generated_out[(*n_generated)++] = next;
     tokens.push_back(next);
