@@ -13,6 +13,11 @@ CASES = [
     (257, 32768, 128, 128, "f16", False), (300, 32761, 192, 64, "f16", True), (512, 32700, 96, 32, "f16", False),
     (511, 32768, 320, 32, "f32", True), (600, 16384, 64, 64, "f32", False), (1000, 16383, 256, 256, "f16", True),
     (520, 33000, 160, 32, "f16", True), (1024, 20000, 384, 128, "f32", True), (2048, 8192, 1024, 64, "f16", False),
+    # tiles of 224 and 192 columns: one round is 28672 / 24576 columns at two row tiles, 14336 / 12288 at four
+    (512, 28672, 128, 128, "f16", False), (300, 28661, 192, 64, "f16", True), (1000, 14330, 320, 32, "f16", False),
+    (513, 14300, 256, 128, "f32", True), (700, 14336, 160, 32, "f16", True),
+    (512, 24576, 128, 128, "f16", True), (257, 24561, 192, 64, "f32", False), (1024, 12280, 320, 32, "f16", True),
+    (2048, 6144, 192, 32, "f16", False),
 ]
 
 

@@ -594,7 +594,7 @@ bool int4_gemm_ring_eligible(const yscv_hip_int4_weight *w, const _Float16 *xh, 
 namespace {
 
 // Tile shapes: 0 = 128 x 128, 1 = 128 x 256, 2 = 256 x 128 (m > 128), 3 = 32 x 128 (m <= 32), 4 = 64 x 128 (m <= 64),
-// 5 = 256 x 256 (m > 256, int4_gemm_wide.hip)
+// 5, 6, 7 = 256 x 256, 256 x 224, 256 x 192 (m > 256, int4_gemm_wide.hip)
 struct RingPlan {
   int one;           // shape of the launch, or of the first of two launches
   int second;        // < 0: one launch; else the shape of the launch that takes the columns from split_col on
@@ -630,8 +630,9 @@ RingPlan ring_plan(size_t m, size_t n, size_t kt, size_t cus) {
     // would leave idle (512 rows against N 4096: 256 tiles instead of 128).
     // The 256 x 256 tile of int4_gemm_wide.hip takes 110 us where two rounds of 256 x 128 tiles take 138 (weights without
     // zero points; with them its gain depends on the clock, see its header).
-    const Shape shapes[5] = {{128, 128, 100, 0}, {128, 256, 172, 1}, {256, 128, 163, 2}, {256, 256, 280, 5}, {64, 128, 75, 4}};
-    auto allowed = [&](const Shape &sh) { return sh.code == 2 ? m > 128 : (sh.code == 5 ? m > 256 : true); };
+    const Shape shapes[7] = {{128, 128, 100, 0}, {128, 256, 172, 1}, {256, 128, 163, 2}, {256, 256, 280, 5}, {256, 224, 250, 6}, {256, 192, 225, 7},
+                             {64, 128, 75, 4}};
+    auto allowed = [&](const Shape &sh) { return sh.code == 2 ? m > 128 : (sh.code >= 5 ? m > 256 : true); };
     // best single shape for columns [c0, n): cost of its rounds over the CUs
     auto best_single = [&](size_t c0, int *which, size_t *tiles_out) {
       size_t best = (size_t)-1;
@@ -649,7 +650,7 @@ RingPlan ring_plan(size_t m, size_t n, size_t kt, size_t cus) {
     };
     size_t best = best_single(0, &pl.one, &tiles);
     const size_t launch_cost = 10;  // a second launch: about a tenth of a tile time
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < 6; i++) {
       if (!allowed(shapes[i])) continue;
       const size_t tm = ceil_div(m, shapes[i].bm), tn = ceil_div(n, shapes[i].bn);
       const size_t rounds = tm * tn / cus;    // whole rounds
@@ -741,7 +742,9 @@ int32_t launch_int4_gemm_ring(const yscv_hip_int4_weight *w, const _Float16 *xh,
   }
   auto launch_shape = [&](int which, const RingArgs &r) {
     switch (which) {
-      case 5: return launch_int4_gemm_wide(w, xh, row_scale, k_pad, y, y_dtype, m, (size_t)r.col0, (size_t)r.n, s, epi);
+      case 5:
+      case 6:
+      case 7: return launch_int4_gemm_wide(w, xh, row_scale, k_pad, y, y_dtype, m, (size_t)r.col0, (size_t)r.n, 16 - 2 * (which - 5), s, epi);
       case 4: return ring_launch_gm<2, 4, 2, 6, 8>(r, w->gm, sf16, s);
       case 3: return ring_launch_gm<1, 4, 2, 6, 4>(r, w->gm, sf16, s);
       case 2: return ring_launch_gm<8, 4, 2, 4, 4>(r, w->gm, sf16, s);

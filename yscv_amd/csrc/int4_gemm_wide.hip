@@ -16,6 +16,10 @@
 // 28672 x 4096 525 -> 472 | 456 -> 408, 700 x 24000 x 2048 95 -> 84 | 90 -> 79.  With zero points (two more instructions per
 // pair of weights, and the bf16 rows prepared first: 9 us of it) the decode takes back most of it: 2048 x 14336 x 4096 in
 // 128-groups 254 -> 266 | 242 -> 233: slower while the clock is still coming up behind an idle stretch, faster once it is there.
+// Tiles of 14 and 12 column blocks (224, 192 columns) where they fill the CUs in whole rounds and 256 columns leave the last
+// one short: 2048 x 7168 x 4096 101 us (a round of 256 columns 113), 2048 x 6144 x 4096 105 -> 91, with zero points 103 -> 96;
+// 2048 x 14336 x 4096 with zero points 220 -> 207, without 207 -> 202, 2048 x 28672 x 4096 no change (settled clock: CUs left
+// idle by a short round leave the others a higher clock, so a round saved is worth less than its share).
 // A stage takes 1.43 us (1.09 without the decode) where its MFMAs take 1.05 at the rate a registers-only loop reaches.
 #include <mutex>
 #include <type_traits>
@@ -27,10 +31,10 @@ namespace yscv {
 
 namespace {
 
-constexpr int WG_MT = 8, WG_NT = 4, WG_WM = 2, WG_WN = 4;  // MFMA tiles of a wave, waves of a workgroup
-constexpr int WG_BM = 16 * WG_MT * WG_WM, WG_BN = 16 * WG_NT * WG_WN, WG_THREADS = 64 * WG_WM * WG_WN;
+constexpr int WG_MT = 8, WG_NT = 4, WG_WM = 2, WG_WN = 4;  // MFMA tiles of a wave (the widest tile), waves of a workgroup
+constexpr int WG_BM = 16 * WG_MT * WG_WM, WG_BLOCKS = WG_NT * WG_WN, WG_THREADS = 64 * WG_WM * WG_WN;
 constexpr int WG_XSLOT = WG_BM * 128, WG_XSLOTS = 3;  // activations of 64 k
-constexpr int WG_WSLOT = WG_BN * 64;                  // packed weights of 128 k, two slots
+constexpr int WG_WSLOT = WG_BLOCKS * 1024;            // packed weights of 128 k, two slots
 constexpr int WG_RS = 16 * WG_NT + 4;                 // floats per row of the epilogue's LDS tile
 constexpr int WG_ERED = 8 * WG_MT * WG_RS * 4;        // a wave's LDS there: half of its rows
 
@@ -66,21 +70,16 @@ __device__ __forceinline__ void wide_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-template <int GM, bool SF16, bool HAS_ZP>
-__global__ void __launch_bounds__(WG_THREADS, 2) int4_gemm_wide_kernel(WideArgs p, int tiles_m, int tiles_n) {
+// One wave's share of a tile: 128 rows of the half wave & 1, the NT column blocks from block OFF + NT (wave / 2) of the tile's on.
+template <int GM, bool SF16, bool HAS_ZP, int NT, int OFF>
+__device__ __forceinline__ void wide_wave(const WideArgs &p, int m0, int n0) {
   using S = WideScale<GM, SF16, HAS_ZP>;
-  constexpr int MT = WG_MT, NT = WG_NT, XL = WG_BM / 64, WL = WG_BN / 16 / 8, SL = S::LOADS + S::ZLOADS;  // loads per wave
+  constexpr int MT = WG_MT, XL = WG_BM / 64, WL = WG_BLOCKS / 8, SL = S::LOADS + S::ZLOADS;  // loads per wave
   extern __shared__ __attribute__((aligned(1024))) uint8_t wide_lds[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 15, c = lane >> 4, wm = wave & 1, wn = wave >> 1;
-  // Tiles are numbered down bands of eight row tiles, column by column; an XCD (workgroup ids equal modulo 8) takes an eighth
-  // of them in a row: 32 neighbours share row and column panels in its L2, and no XCD has more than its share (super-blocks of
-  // 32 tiles gave four XCDs a second one at three row tiles x 85 columns: 700 x 24000 x 2048 140 us against 98)
-  const int tiles = tiles_m * tiles_n, share = (tiles + 7) >> 3, t = (int)(blockIdx.x & 7) * share + (int)(blockIdx.x >> 3);
-  if (t >= tiles) return;
-  const int band = t / (8 * tiles_n), in_band = t - band * 8 * tiles_n, rows = min(8, tiles_m - 8 * band);
-  const int tn = in_band / rows, tm = 8 * band + in_band % rows;
-  const int m0 = tm * WG_BM, n0 = p.col0 + tn * WG_BN, nb0 = n0 / 16;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // (offsets shared by the two forms of a 14-block tile would be kept beside the accumulators)
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, c = lane >> 4, wm = wave & 1, first = OFF + NT * (wave >> 1), nb0 = n0 / 16;
   NibbleConsts nc;
   nc.init();
 
@@ -107,12 +106,12 @@ __global__ void __launch_bounds__(WG_THREADS, 2) int4_gemm_wide_kernel(WideArgs 
   uint32_t scoff[S::LOADS], zpoff[S::ZLOADS > 0 ? S::ZLOADS : 1];
 #pragma unroll
   for (int u = 0; u < S::LOADS; u++) {
-    const int byte = (u * 256 + lane * 4) % (NT * S::BLOCK), blk = min(nb0 + wn * NT + byte / S::BLOCK, p.nt - 1);
+    const int byte = (u * 256 + lane * 4) % (NT * S::BLOCK), blk = min(nb0 + first + byte / S::BLOCK, p.nt - 1);
     scoff[u] = (uint32_t)blk * (uint32_t)(p.chunks * S::BLOCK) + (uint32_t)(byte % S::BLOCK);
   }
 #pragma unroll
   for (int u = 0; u < S::ZLOADS; u++) {
-    const int byte = (u * 256 + lane * 4) % (NT * S::ZBLOCK), blk = min(nb0 + wn * NT + byte / S::ZBLOCK, p.nt - 1);
+    const int byte = (u * 256 + lane * 4) % (NT * S::ZBLOCK), blk = min(nb0 + first + byte / S::ZBLOCK, p.nt - 1);
     zpoff[u] = (uint32_t)blk * (uint32_t)(p.chunks * S::ZBLOCK) + (uint32_t)(byte % S::ZBLOCK);
   }
   auto load_w = [&](int kt) {
@@ -144,7 +143,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) int4_gemm_wide_kernel(WideArgs 
   scale_t sv[NT];  // (f32 scales are rounded as the weights are)
   uint32_t zv[HAS_ZP ? NT : 1];
   auto read_w = [&](int kt, int half) {
-    const uint8_t *src = w_lds + (kt & 1) * WG_WSLOT + wn * NT * 1024 + lane * 16 + half * 8;
+    const uint8_t *src = w_lds + (kt & 1) * WG_WSLOT + first * 1024 + lane * 16 + half * 8;
 #pragma unroll
     for (int j = 0; j < NT; j++) wq[j] = *reinterpret_cast<const word_pair_t *>(src + j * 1024);
     if (half == 1) return;
@@ -269,7 +268,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) int4_gemm_wide_kernel(WideArgs 
   // copy of the store code per half, not one per MFMA tile)
   float *red = reinterpret_cast<float *>(wide_lds) + wave * WG_ERED / 4;
   const bool vec = (p.ldy & 3) == 0;
-  const int col = n0 + wn * NT * 16 + 4 * r;
+  const int col = n0 + first * 16 + 4 * r;
 #pragma unroll
   for (int i0 = 0; i0 < MT; i0 += MT / 2) {
 #pragma unroll
@@ -281,7 +280,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) int4_gemm_wide_kernel(WideArgs 
 #pragma unroll 4
     for (int q = 0; q < 2 * MT; q++) {
       const int row = row0 + 4 * q;
-      if (row < p.m && col < p.n) {
+      if (row < p.m && col < p.n && r < 4 * NT) {
         float4_t v = *reinterpret_cast<const float4_t *>(red + (4 * q + c) * WG_RS + 4 * r);
         if (p.row_scale) v = v * p.row_scale[row];
         store_cols4(p.y, p.y_dtype, p.epi, p.ldy, p.n, row, col, vec, v);
@@ -291,31 +290,62 @@ __global__ void __launch_bounds__(WG_THREADS, 2) int4_gemm_wide_kernel(WideArgs 
   }
 }
 
-template <int GM, bool SF16, bool HAS_ZP>
+// NB: column blocks of a tile, 16, 14 or 12.  Waves w and w + 4 share a SIMD: with 14 blocks the column quarters are 4, 4, 3 and
+// 3 blocks wide and every SIMD has one wave of each kind.
+template <int GM, bool SF16, bool HAS_ZP, int NB>
+__global__ void __launch_bounds__(WG_THREADS, 2) int4_gemm_wide_kernel(WideArgs p, int tiles_m, int tiles_n) {
+  // Tiles are numbered down bands of eight row tiles, column by column; an XCD (workgroup ids equal modulo 8) takes an eighth
+  // of them in a row: 32 neighbours share row and column panels in its L2, and no XCD has more than its share (super-blocks of
+  // 32 tiles gave four XCDs a second one at three row tiles x 85 columns: 700 x 24000 x 2048 140 us against 98)
+  const int tiles = tiles_m * tiles_n, share = (tiles + 7) >> 3, t = (int)(blockIdx.x & 7) * share + (int)(blockIdx.x >> 3);
+  if (t >= tiles) return;
+  const int band = t / (8 * tiles_n), in_band = t - band * 8 * tiles_n, rows = min(8, tiles_m - 8 * band);
+  const int tn = in_band / rows, tm = 8 * band + in_band % rows;
+  const int m0 = tm * WG_BM, n0 = p.col0 + tn * 16 * NB;
+  if constexpr (NB == 16) {
+    wide_wave<GM, SF16, HAS_ZP, 4, 0>(p, m0, n0);
+  } else if constexpr (NB == 12) {
+    wide_wave<GM, SF16, HAS_ZP, 3, 0>(p, m0, n0);
+  } else {
+    static_assert(NB == 14, "column blocks of a tile");
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256) wide_wave<GM, SF16, HAS_ZP, 3, 2>(p, m0, n0);
+    else wide_wave<GM, SF16, HAS_ZP, 4, 0>(p, m0, n0);
+  }
+}
+
+template <int GM, bool SF16, bool HAS_ZP, int NB>
 int32_t wide_launch_one(const WideArgs &a, hipStream_t s) {
   constexpr int LOOP = WG_XSLOTS * WG_XSLOT + 2 * WG_WSLOT + 16 * WideScale<GM, SF16, HAS_ZP>::BYTES;
   constexpr int LDS = LOOP > 8 * WG_ERED ? LOOP : 8 * WG_ERED;
   static_assert(LDS <= 160 * 1024, "LDS of a CU");
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  auto kern = int4_gemm_wide_kernel<GM, SF16, HAS_ZP>;
+  auto kern = int4_gemm_wide_kernel<GM, SF16, HAS_ZP, NB>;
   std::call_once(once, [&] { attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS); });
   if (attr_err != hipSuccess) return set_error(YSCV_HIP_ERR_DEVICE, "cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(attr_err));
-  const int tiles_m = (a.m + WG_BM - 1) / WG_BM, tiles_n = (a.n - a.col0 + WG_BN - 1) / WG_BN;
+  const int tiles_m = (a.m + WG_BM - 1) / WG_BM, tiles_n = (a.n - a.col0 + 16 * NB - 1) / (16 * NB);
   hipLaunchKernelGGL(kern, dim3((unsigned)((tiles_m * tiles_n + 7) / 8 * 8)), dim3(WG_THREADS), LDS, s, a, tiles_m, tiles_n);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
 
+template <int GM, bool SF16, bool HAS_ZP>
+int32_t wide_launch_nb(const WideArgs &a, int blocks, hipStream_t s) {
+  // (with zero points and a scale per 32 k the 14-block form needs one register more than there are: 16 blocks then)
+  if constexpr (!(GM == GM32 && HAS_ZP))
+    if (blocks == 14) return wide_launch_one<GM, SF16, HAS_ZP, 14>(a, s);
+  if (blocks == 12) return wide_launch_one<GM, SF16, HAS_ZP, 12>(a, s);
+  return wide_launch_one<GM, SF16, HAS_ZP, 16>(a, s);
+}
 template <int GM, bool SF16>
-int32_t wide_launch_zp(const WideArgs &a, hipStream_t s) {
-  return a.tzps ? wide_launch_one<GM, SF16, true>(a, s) : wide_launch_one<GM, SF16, false>(a, s);
+int32_t wide_launch_zp(const WideArgs &a, int blocks, hipStream_t s) {
+  return a.tzps ? wide_launch_nb<GM, SF16, true>(a, blocks, s) : wide_launch_nb<GM, SF16, false>(a, blocks, s);
 }
 
 }  // namespace
 
 int32_t launch_int4_gemm_wide(const yscv_hip_int4_weight *w, const _Float16 *xh, const float *row_scale, size_t ldx, void *y, int y_dtype,
-                              size_t m, size_t col0, size_t col1, hipStream_t s, int epi) {
+                              size_t m, size_t col0, size_t col1, int blocks, hipStream_t s, int epi) {
   WideArgs a;
   a.tiles = w->tiles;
   a.tscales = w->tscales;
@@ -337,9 +367,9 @@ int32_t launch_int4_gemm_wide(const yscv_hip_int4_weight *w, const _Float16 *xh,
   a.y_dtype = y_dtype;
   a.epi = epi;
   const bool sf16 = w->scale_dtype == YSCV_HIP_F16;
-  if (w->gm == GM32) return sf16 ? wide_launch_zp<GM32, true>(a, s) : wide_launch_zp<GM32, false>(a, s);
-  if (w->gm == GM64) return sf16 ? wide_launch_zp<GM64, true>(a, s) : wide_launch_zp<GM64, false>(a, s);
-  return sf16 ? wide_launch_zp<GM128, true>(a, s) : wide_launch_zp<GM128, false>(a, s);
+  if (w->gm == GM32) return sf16 ? wide_launch_zp<GM32, true>(a, blocks, s) : wide_launch_zp<GM32, false>(a, blocks, s);
+  if (w->gm == GM64) return sf16 ? wide_launch_zp<GM64, true>(a, blocks, s) : wide_launch_zp<GM64, false>(a, blocks, s);
+  return sf16 ? wide_launch_zp<GM128, true>(a, blocks, s) : wide_launch_zp<GM128, false>(a, blocks, s);
 }
 
 }  // namespace yscv
