@@ -32,6 +32,10 @@ def _reference(q, k, v, hq, hkv):
     (4, 520, 140, 32, 8, 32),     # 256 rows per workgroup, the last one part full
     (4, 512, 33, 32, 8, 96),
     (1, 17, 31, 2, 1, 128),
+    # keys and values prepared in front: 64, 128 and 256 rows, ragged rows and keys, keys split over the grid
+    (1, 512, 511, 32, 8, 128), (4, 300, 515, 8, 8, 32), (2, 130, 1999, 8, 2, 96), (1, 200, 2000, 32, 8, 128), (1, 90, 1290, 16, 2, 64),
+    (1, 1000, 1111, 32, 8, 128), (1, 1024, 1025, 32, 8, 64), (2, 515, 1201, 32, 8, 96), (1, 1023, 1500, 32, 8, 32),
+    (4, 1000, 1111, 32, 8, 64), (4, 520, 1057, 32, 8, 128), (4, 513, 800, 32, 8, 96), (4, 600, 300, 32, 8, 32),
 ])
 def test_operator_against_float32(B, Sq, Sk, hq, hkv, d):
     import torch
@@ -68,14 +72,15 @@ def test_more_rows_or_problems_than_one_launch_takes(B, Sq, hq, hkv):
     assert bool(((got - want).abs() <= 17 * 2.0**-24 * want.abs()).all())
 
 
-def test_values_on_four_byte_alignment():
+@pytest.mark.parametrize("sq,sk", [(40, 50), (600, 1300)])
+def test_values_on_four_byte_alignment(sq, sk):
     import torch
 
     from yscv_amd import onnx_ops as ops
 
-    q, k = torch.randn(1, 40, 8 * 64, device="cuda"), torch.randn(1, 50, 2 * 64, device="cuda")
-    buf = torch.randn(50 * 128 + 1, device="cuda")
-    v = buf[1:].view(1, 50, 128)
+    q, k = torch.randn(1, sq, 8 * 64, device="cuda"), torch.randn(1, sk, 2 * 64, device="cuda")
+    buf = torch.randn(sk * 128 + 1, device="cuda")
+    v = buf[1:].view(1, sk, 128)
     want = ops.exec_grouped_query_attention(q, k, v.clone(), 8, 2)
     assert torch.equal(ops.exec_grouped_query_attention(q, k, v, 8, 2), want)
 

@@ -520,25 +520,30 @@ int32_t gqa_launch_fused_decode(const GqaArgs &a, int hd, hipStream_t s) {
 // single decode position of four heads fills one row tile instead of four.  A workgroup of eight waves is RW row waves
 // (16 QT rows each) times KS = 8 / RW key groups; a key group streams its stages of KB keys through LDS, converted to
 // fp16 on the way in and V transposed into slabs of eight positions per channel, where all its row waves read them.
-// What bounds it is the f32 K / V every workgroup has to take in (512 KB for 512 keys of 128 channels, 115 GB/s per CU
+// What bounds that is the f32 K / V every workgroup has to take in (512 KB for 512 keys of 128 channels, 115 GB/s per CU
 // from L2), so a workgroup gets as many rows as still leave one workgroup per CU, the waves left over split the keys
 // and are merged through LDS, and where even that leaves CUs idle (decode: 8 workgroups) the keys are split over the
-// grid too, with the partial results merged by a second kernel.  512 queries x 512 keys, 32 heads over 8 of 128: 21 us,
-// against 88 for the kernel before (one wave per 32 rows of one head, V gathered by single values); one query x 2048
-// keys: 9.5 + 5.7 us against 70.  Of the 21 us, 5 pass before the first stage is in LDS, 12 are four rounds of stages
-// (2 048 cycles each for the f32 K / V alone at 64 bytes per cycle and CU), 3 the merge and the stores.
+// grid too, with the partial results merged by a second kernel: one query x 2048 keys 9.5 + 5.7 us.
+// PRE: where several workgroups share a kv head, its stages are converted once by a kernel in front (3.2 us for 512 keys of 8
+// heads), travel to LDS by LDS-direct loads ahead of their use, and sixteen waves of one row tile each work on them: 512 queries
+// x 512 keys, 32 heads over 8 of 128: 18.3 -> 14.0 us in all.  Its 10 us: 1.9 until the first stage and q are there, 6.5 of stages,
+// 1.7 the merge and the stores.
 // QT: row tiles per wave; RW 1 is the form for few rows (wave-private stages: no barrier in the loop).
-template <int HD, int RW, int QT>
+template <int HD, int RW, int QT, bool PRE = false>
 struct FlatCfg {
-  static constexpr int KS = 8 / RW, T = 64 * RW;        // key groups, threads of one
-  static constexpr int KB = RW <= 2 ? 32 : 16 * RW;     // keys per stage: the same registers per thread whatever RW
-  static constexpr int NBUF = RW == 1 ? 1 : 2;
+  static constexpr int WAVES = PRE && QT == 1 ? 16 : 8, THREADS = 64 * WAVES;
+  static constexpr int KS = WAVES / RW, T = 64 * RW;             // key groups, threads of one
+  static constexpr int KB = PRE || RW <= 2 ? 32 : 16 * RW;       // keys per stage: the same registers per thread whatever RW
+  static constexpr int NBUF = PRE ? (KS > 2 ? 2 : 4) : (RW == 1 ? 1 : 2);
   static constexpr int PITCH = HD > 64 ? 16 : (HD > 32 ? 8 : 4);  // K row pitch in 16-byte pieces
   static constexpr int K_BYTES = KB * PITCH * 16, V_BYTES = (KB / 8) * HD * 16, ST_BYTES = K_BYTES + V_BYTES;
   static constexpr int ROWS = RW * 16 * QT;
   static constexpr int OP = HD + 4;                      // floats per row of the merge buffer
   static constexpr int MERGE_BYTES = KS > 1 ? KS * ROWS * (OP + 2) * 4 : 0;
-  static constexpr int LDS = KS * NBUF * ST_BYTES > MERGE_BYTES ? KS * NBUF * ST_BYTES : MERGE_BYTES;
+  static constexpr int Q_AT = KS * NBUF * ST_BYTES;      // PRE: where q changes to operand order
+  static constexpr int LOOP_BYTES = Q_AT + (PRE ? ROWS * HD * 2 : 0);
+  static constexpr int LDS = LOOP_BYTES > MERGE_BYTES ? LOOP_BYTES : MERGE_BYTES;
+  static_assert(LDS <= 160 * 1024, "LDS of a CU");
 };
 
 struct FlatArgs {
@@ -546,16 +551,66 @@ struct FlatArgs {
   float *out, *part;       // part: [b * Hkv][gs][R][HD + 2] when gs > 1 (un-normalised output, maximum, sum)
   int Sq, Sk, Hq, Hkv, group, R, gs;  // Sq: query positions from one sequence to the next; R: rows of this launch
   int v16;                 // v is 16-byte aligned
+  const uint8_t *pre;      // PRE: the stages of every (sequence, kv head) as they lie in LDS
   uint32_t magic;          // ceil(2^32 / group): row / group = the high half of row * magic (0: divide)
   float scale;             // log2(e) / sqrt(head width)
 };
 
-template <int HD, int RW, int QT>
-__global__ void __launch_bounds__(512) gqa_flat_kernel(FlatArgs p) {
-  using C = FlatCfg<HD, RW, QT>;
+// Where the 16-byte piece (row, piece) of a stage's K lies in LDS
+template <typename C>
+__device__ __forceinline__ int flat_k_at(int row, int piece) {
+  return (row * C::PITCH + (piece ^ ((((row >> 3) & 3) * 4 + (row & 3)) / (16 / C::PITCH)))) * 16;
+}
+
+// The stages of every (sequence, kv head) once, as gqa_flat_kernel has them in LDS: fp16, K swizzled, V in slabs of eight
+// positions per channel (positions past the end 0).  What that kernel would do once per workgroup: with 32 workgroups to a
+// kv head (512 queries of four heads, 64 rows each) 32 times.
+template <int HD>
+__global__ void __launch_bounds__(256) gqa_flat_prepare_kernel(FlatArgs p, uint8_t *__restrict__ pre) {
+  using C = FlatCfg<HD, 4, 1, true>;  // (a stage is the same in all forms)
+  constexpr int KB = C::KB, CPR = HD / 8, K_PIECES = KB * CPR, V_UNITS = (KB / 8) * (HD / 4), BLOCKS = (K_PIECES + V_UNITS + 255) / 256;
+  const int nb = blockIdx.x, b = nb / p.Hkv, kvh = nb % p.Hkv, st = blockIdx.y / BLOCKS, idx = (int)(blockIdx.y % BLOCKS) * 256 + (int)threadIdx.x;
+  const size_t kv_s = (size_t)p.Hkv * HD, base = (size_t)b * p.Sk * kv_s + (size_t)kvh * HD;
+  const int stages = (int)gridDim.y / BLOCKS, left = min(KB, p.Sk - st * KB);
+  uint8_t *dst = pre + ((size_t)nb * stages + st) * C::ST_BYTES;
+  if (idx < K_PIECES) {
+    const int row = idx / CPR, piece = idx % CPR;
+    const float *src = p.k + base + (size_t)(st * KB + min(row, left - 1)) * kv_s + piece * 8;
+    *reinterpret_cast<half8_t *>(dst + flat_k_at<C>(row, piece)) = load8<float>(src);
+  } else if (idx < K_PIECES + V_UNITS) {
+    const int u = idx - K_PIECES, pos = u / (HD / 4) * 8, ch = u % (HD / 4) * 4;
+    float v[8][4];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const float *src = p.v + base + (size_t)(st * KB + min(pos + e, left - 1)) * kv_s + ch;
+      if (p.v16) {
+        const float4_t q = *reinterpret_cast<const float4_t *>(src);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[e][i] = q[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[e][i] = src[i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      half8_t h;
+#pragma unroll
+      for (int e = 0; e < 8; e++) h[e] = pos + e < left ? (_Float16)v[e][i] : (_Float16)0.0f;
+      *reinterpret_cast<half8_t *>(dst + C::K_BYTES + (u * 4 + i) * 16) = h;
+    }
+  }
+}
+
+template <int HD, int RW, int QT, bool PRE>
+__global__ void __launch_bounds__((FlatCfg<HD, RW, QT, PRE>::THREADS)) gqa_flat_kernel(FlatArgs p) {
+  using C = FlatCfg<HD, RW, QT, PRE>;
+  static_assert(!PRE || C::ST_BYTES % 1024 == 0, "a stage travels in KiB");
   constexpr int KK = HD / 32, DT = HD / 16, KB = C::KB, PITCH = C::PITCH, RPW = 16 / PITCH, CPR = HD / 8, T = C::T, KS = C::KS;
   constexpr int K_PIECES = KB * CPR, V_UNITS = (KB / 8) * (HD / 4);  // V unit: eight positions x four channels
   constexpr int K_LD = (K_PIECES + T - 1) / T, V_LD = (V_UNITS + T - 1) / T;
+  // the values are read behind the scores' MFMAs and arrive during the softmax, where registers allow it
+  constexpr bool V_EARLY = PRE && QT == 1;
   extern __shared__ __attribute__((aligned(16))) uint8_t flat_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, c = lane >> 4;
@@ -647,7 +702,7 @@ __global__ void __launch_bounds__(512) gqa_flat_kernel(FlatArgs p) {
         half8_t h;
 #pragma unroll
         for (int e = 0; e < 8; e++) h[e] = (_Float16)kr[j][e >> 2][e & 3];
-        *reinterpret_cast<half8_t *>(base + (row * PITCH + (piece ^ ((((row >> 3) & 3) * 4 + (row & 3)) / RPW))) * 16) = h;
+        *reinterpret_cast<half8_t *>(base + flat_k_at<C>(row, piece)) = h;
       }
     }
 #pragma unroll
@@ -670,17 +725,63 @@ __global__ void __launch_bounds__(512) gqa_flat_kernel(FlatArgs p) {
     }
   };
 
+  // PRE: a stage is one run of bytes and goes to LDS as it is; a wave moves every RW-th KiB of its group's, the last one again
+  // where they do not come out even, and stages past the end repeat the last one: every wave has COPIES loads per stage
+  constexpr int KIB = C::ST_BYTES / 1024, COPIES = (KIB + RW - 1) / RW;
+  const uint32_t lds_at = (uint32_t)(size_t)lds, lane16 = lane * 16;
+  auto copy = [&](int buf, int stage) {
+    const uint8_t *src = p.pre + (size_t)__builtin_amdgcn_readfirstlane(nb * stages + min(stage, st_hi - 1)) * C::ST_BYTES;
+#pragma unroll
+    for (int j = 0; j < COPIES; j++) {
+      const int kib = min(rw + RW * j, KIB - 1);
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_at + (uint32_t)(buf * C::ST_BYTES + kib * 1024))),
+                   "v"(lane16), "s"(src + kib * 1024)
+                   : "memory");
+    }
+  };
+
   int st = st_lo + kg;
   const bool any = st < st_hi;
-  if (any) fetch(st);
+  if constexpr (PRE) copy(0, st);
+  else if (any) fetch(st);
 
   half8_t qf[QT][KK];
+  if constexpr (PRE) {
+    // The workgroup's rows come once, whole lines, and change to operand order through LDS.  (Every wave for itself, in pieces
+    // of 32 bytes, the key groups all the same rows: 256 load instructions of 16 lines each, 3.2 us until the first stage
+    // could start.)
+    constexpr int Q_ALL = C::ROWS * (HD / 4), Q_LD = (Q_ALL + C::THREADS - 1) / C::THREADS;  // threads past the end repeat the last piece
+    uint8_t *qs = flat_lds + C::Q_AT;
+    float4_t qr[Q_LD];
 #pragma unroll
-  for (int u = 0; u < QT; u++) {
-    const int row = min(row0 + 16 * u + r, p.R - 1);  // rows past the end repeat the last one and are not stored
-    const float *qrow = p.q + row_offset(row);
+    for (int j = 0; j < Q_LD; j++) {
+      const int idx = min(tid + C::THREADS * j, Q_ALL - 1), row = min((int)blockIdx.y * C::ROWS + idx / (HD / 4), p.R - 1);  // rows past the end repeat the last one
+      qr[j] = *reinterpret_cast<const float4_t *>(p.q + row_offset(row) + idx % (HD / 4) * 4);
+    }
 #pragma unroll
-    for (int kk = 0; kk < KK; kk++) qf[u][kk] = load8<float>(qrow + 32 * kk + 8 * c);
+    for (int i = 1; i < C::NBUF - 1; i++) copy(i, st + i * KS);
+    constexpr int QX = HD == 128 ? 15 : (HD == 64 ? 7 : 3);  // the 16-byte pieces of a row change places so that 16 rows meet different banks
+#pragma unroll
+    for (int j = 0; j < Q_LD; j++) {
+      const int idx = min(tid + C::THREADS * j, Q_ALL - 1), row = idx / (HD / 4), ch = idx % (HD / 4);
+      *reinterpret_cast<half4_t *>(qs + row * HD * 2 + (((ch >> 1) ^ (row & QX)) * 16) + (ch & 1) * 8) =
+          half4_t{(_Float16)qr[j][0], (_Float16)qr[j][1], (_Float16)qr[j][2], (_Float16)qr[j][3]};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < QT; u++) {
+      const int row = rw * 16 * QT + 16 * u + r;
+#pragma unroll
+      for (int kk = 0; kk < KK; kk++) qf[u][kk] = *reinterpret_cast<const half8_t *>(qs + row * HD * 2 + ((4 * kk + c) ^ (row & QX)) * 16);
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < QT; u++) {
+      const int row = min(row0 + 16 * u + r, p.R - 1);  // rows past the end repeat the last one and are not stored
+      const float *qrow = p.q + row_offset(row);
+#pragma unroll
+      for (int kk = 0; kk < KK; kk++) qf[u][kk] = load8<float>(qrow + 32 * kk + 8 * c);
+    }
   }
   float m_run[QT], l_run[QT];
   float4_t o_acc[QT][DT];
@@ -696,7 +797,11 @@ __global__ void __launch_bounds__(512) gqa_flat_kernel(FlatArgs p) {
   // 32 keys of a stage; layout and arithmetic as in gqa_shared_kv_kernel.  The scores of all row tiles come first and V
   // is read behind them: K and V fragments together would not fit beside the next stage's loads in flight.
   auto compute32 = [&](const uint8_t *base, int sub, int p0) {
-    half8_t pf[QT];
+    half8_t pf[QT], vv[DT];
+    auto read_v = [&]() {
+#pragma unroll
+      for (int t = 0; t < DT; t++) vv[t] = *reinterpret_cast<const half8_t *>(base + C::K_BYTES + ((sub * 4 + c) * HD + 16 * t + r) * 16);
+    };
     {
       half8_t kf[2][KK];
 #pragma unroll
@@ -714,6 +819,11 @@ __global__ void __launch_bounds__(512) gqa_flat_kernel(FlatArgs p) {
         for (int kk = 0; kk < KK; kk++) {
           s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[0][kk], qf[u][kk], s0, 0, 0, 0);
           s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[1][kk], qf[u][kk], s1, 0, 0, 0);
+        }
+        if constexpr (V_EARLY) {
+          __builtin_amdgcn_sched_barrier(0);
+          read_v();
+          __builtin_amdgcn_sched_barrier(0);
         }
         // softmax in powers of two: the scale (log2(e) in it) and the maximum go into one fma per score
         float sv[8], mx = -INFINITY, pe[8], sum = 0.0f;
@@ -745,10 +855,10 @@ __global__ void __launch_bounds__(512) gqa_flat_kernel(FlatArgs p) {
         }
       }
     }
-    __builtin_amdgcn_sched_barrier(0);
-    half8_t vv[DT];
-#pragma unroll
-    for (int t = 0; t < DT; t++) vv[t] = *reinterpret_cast<const half8_t *>(base + C::K_BYTES + ((sub * 4 + c) * HD + 16 * t + r) * 16);
+    if constexpr (!V_EARLY) {
+      __builtin_amdgcn_sched_barrier(0);
+      read_v();
+    }
 #pragma unroll
     for (int u = 0; u < QT; u++)
 #pragma unroll
@@ -772,6 +882,16 @@ __global__ void __launch_bounds__(512) gqa_flat_kernel(FlatArgs p) {
       compute(st, 0);
       asm volatile("" ::: "memory");
     }
+  } else if constexpr (PRE) {
+    int buf = 0;
+    for (int it = 0; it < iters; it++, st += KS) {  // uniform in the workgroup
+      // this wave's part of the stage has landed and its reads of the last one have returned; then everyone's
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((C::NBUF - 2) * COPIES) : "memory");
+      copy(buf == 0 ? C::NBUF - 1 : buf - 1, st + (C::NBUF - 1) * KS);
+      if (st < st_hi) compute(st, buf);
+      buf = buf + 1 == C::NBUF ? 0 : buf + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing is in flight to LDS any more
   } else {
     if (any) stash(0, st);
     __syncthreads();
@@ -827,7 +947,7 @@ __global__ void __launch_bounds__(512) gqa_flat_kernel(FlatArgs p) {
       }
     }
     __syncthreads();
-    for (int idx = tid; idx < C::ROWS * (HD / 4); idx += 512) {
+    for (int idx = tid; idx < C::ROWS * (HD / 4); idx += C::THREADS) {
       const int lr = idx / (HD / 4), d4 = idx % (HD / 4) * 4, row = (int)blockIdx.y * C::ROWS + lr;
       if (row >= p.R) continue;
       float M = -INFINITY, L = 0.0f;
@@ -876,47 +996,93 @@ __global__ void __launch_bounds__(256) gqa_flat_merge_kernel(FlatArgs p, int hd,
       L > 0.0f ? o / L : 0.0f;
 }
 
-template <int HD, int RW, int QT>
+template <int HD, int RW, int QT, bool PRE>
 int32_t gqa_flat_go(const FlatArgs &p, int nbs, hipStream_t s) {
-  using C = FlatCfg<HD, RW, QT>;
+  using C = FlatCfg<HD, RW, QT, PRE>;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  std::call_once(once, [] {
-    attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(gqa_flat_kernel<HD, RW, QT>), hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
-  });
+  auto kern = gqa_flat_kernel<HD, RW, QT, PRE>;
+  std::call_once(once, [&] { attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS); });
   YSCV_HIP_TRY(attr_err);
-  hipLaunchKernelGGL((gqa_flat_kernel<HD, RW, QT>), dim3((unsigned)nbs, (unsigned)((p.R + C::ROWS - 1) / C::ROWS), (unsigned)p.gs), dim3(512),
-                     C::LDS, s, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)nbs, (unsigned)((p.R + C::ROWS - 1) / C::ROWS), (unsigned)p.gs), dim3(C::THREADS), C::LDS, s, p);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
+}
+
+// Which form takes a problem of R rows x Sk keys per (sequence, kv head), by estimated time in units of 0.1 us: rounds of
+// workgroups over the CUs x (start and merge + steps of keys), and what runs in front or behind.  The prepared forms take
+// 32 keys of each of their 16-wave key groups in 1.6 us at 128 channels whatever their rows; the form for few rows takes 256
+// keys in 2.9, bound by the f32 K / V that every 16 rows take in again.  Measured (us): 512 x 512, 32 heads over 8 of 128: 18.3 in
+// 64 rows converting for themselves, 14.0 prepared; 1000 x 1111 42 -> 34.5 in 128 rows; 4 x 300 x 2000, 8 over 8: 79 in 16
+// rows, 43 in 64; 200 x 2000, 32 over 8: 47 -> 28.6, keys in two parts; 4 x 1024 x 2048, 32 over 8 of 64: 151 -> 133 in 256 rows.
+// In 256 rows the preparation is paid back late: 4 x 512 x 512 at 128 channels 35 as it was, 38 prepared, 2 x 1024 x 1024 57 and 58.
+struct FlatPlan {
+  int rows;  // 16, 64, 128 or 256
+  bool pre;
+  int gs;    // parts the keys are split into over the grid
+};
+FlatPlan flat_plan(int nbs, int R, int Sk, int hd, int num_cus, bool may_prepare) {
+  auto wgs = [&](int rows) { return (long long)nbs * ((R + rows - 1) / rows); };
+  auto rounds = [&](long long n) { return (n + num_cus - 1) / num_cus; };
+  auto ceil_of = [](long long n, long long d) { return (n + d - 1) / d; };
+  // without a prepared copy: the most rows that still give every CU a workgroup; 16 rows and a split of the keys over the grid
+  // where no choice does.  A split pays where it takes whole rounds of stages off the longest workgroup.
+  FlatPlan best{wgs(256) >= num_cus ? 256 : (wgs(128) >= num_cus ? 128 : (wgs(64) >= num_cus ? 64 : 16)), false, 1};
+  if (best.rows == 16) {
+    const long long steps = ceil_of(Sk, 32 * 8), room = num_cus / wgs(16);
+    const long long gs = steps < room ? steps : room;
+    if (gs >= 2) best.gs = (int)(gs > 64 ? 64 : gs);
+  }
+  if (!may_prepare || (best.rows == 256 && Sk <= 8 * hd)) return best;
+  const long long step = 8 + 8 * hd / 128, prep = 30 + (long long)nbs * Sk * hd * 8 / 330000;
+  long long cost;
+  if (best.rows == 16) cost = rounds(wgs(16) * best.gs) * (30 + 29 * hd / 128 * ceil_of(ceil_of(Sk, 256), best.gs)) + (best.gs > 1 ? 50 : 0);
+  else cost = rounds(wgs(best.rows)) * (80 + (step + 4) * ceil_of(Sk, 8192 / best.rows));
+  for (int rows : {64, 128, 256})
+    for (int gs : {1, 2, 4}) {
+      const long long steps = ceil_of(Sk, 8192 / rows);  // 4, 2, 1 key groups
+      if ((R + rows - 1) / rows > 65535) continue;  // a grid's y
+      if (gs > 1 && (rows > 64 || wgs(rows) * gs > num_cus || steps < 4 * gs)) continue;
+      const long long c = prep + rounds(wgs(rows) * gs) * (50 + step * ceil_of(steps, gs)) + (gs > 1 ? 50 : 0);
+      if (c < cost) {
+        cost = c;
+        best = FlatPlan{rows, true, gs};
+      }
+    }
+  return best;
 }
 
 template <int HD>
 int32_t gqa_flat_launch(FlatArgs p, int B, int num_cus, hipStream_t s) {
   const int nbs = B * p.Hkv;
-  // Rows per workgroup: the most that still give every CU a workgroup (K / V are taken in once per workgroup); 16 rows
-  // and a split of the keys over the grid where no choice does.
-  auto wgs = [&](int rows) { return nbs * ((p.R + rows - 1) / rows); };
-  const int rw = wgs(256) >= num_cus ? 8 : (wgs(128) >= num_cus ? 4 : (wgs(64) >= num_cus ? 2 : 1));
-  p.gs = 1;
-  Scratch part;
-  if (rw == 1) {
-    // a split pays where it takes whole rounds of stages off the longest workgroup (a stage: about 1 us; the second
-    // kernel about 4): at least two rounds of the eight key groups each
-    const int rounds = (p.Sk + 32 * 8 - 1) / (32 * 8), room = num_cus / wgs(16);
-    int gs = rounds < room ? rounds : room;
-    if (gs >= 2 && rounds >= 2) {
-      if (gs > 64) gs = 64;
-      p.gs = gs;
-      YSCV_TRY(part.take((size_t)nbs * gs * p.R * (HD + 2) * sizeof(float), s));
-      p.part = part.as<float>();
-    }
+  using C = FlatCfg<HD, 4, 1, true>;
+  constexpr unsigned BLOCKS = (C::KB * (HD / 8) + C::KB / 8 * (HD / 4) + 255) / 256;  // of the preparation, per stage
+  const size_t stages = ceil_div((size_t)p.Sk, (size_t)C::KB), pre_bytes = (size_t)nbs * stages * C::ST_BYTES;
+  auto part_bytes = [&](const FlatPlan &f) { return f.gs > 1 ? (size_t)nbs * f.gs * p.R * (HD + 2) * sizeof(float) : 0; };
+  FlatPlan f = flat_plan(nbs, p.R, p.Sk, HD, num_cus, pre_bytes <= ((size_t)64 << 20) && stages * BLOCKS <= 65535);
+  Scratch scratch;
+  if (f.pre && scratch.take(pre_bytes + part_bytes(f), s) != YSCV_HIP_OK) {
+    (void)hipGetLastError();  // no memory for the copy: the forms that need none
+    f = flat_plan(nbs, p.R, p.Sk, HD, num_cus, false);
   }
-  switch (rw) {
-    case 8: YSCV_TRY((gqa_flat_go<HD, 8, 2>(p, nbs, s))); break;
-    case 4: YSCV_TRY((gqa_flat_go<HD, 4, 2>(p, nbs, s))); break;
-    case 2: YSCV_TRY((gqa_flat_go<HD, 2, 2>(p, nbs, s))); break;
-    default: YSCV_TRY((gqa_flat_go<HD, 1, 1>(p, nbs, s))); break;
+  p.gs = f.gs;
+  if (f.pre) {
+    hipLaunchKernelGGL((gqa_flat_prepare_kernel<HD>), dim3((unsigned)nbs, (unsigned)stages * BLOCKS), dim3(256), 0, s, p, scratch.as<uint8_t>());
+    YSCV_HIP_TRY(hipGetLastError());
+    p.pre = scratch.as<uint8_t>();
+    p.part = scratch.as<float>(pre_bytes);
+    if (f.rows == 64) YSCV_TRY((gqa_flat_go<HD, 4, 1, true>(p, nbs, s)));
+    else if (f.rows == 128) YSCV_TRY((gqa_flat_go<HD, 8, 1, true>(p, nbs, s)));
+    else YSCV_TRY((gqa_flat_go<HD, 16, 1, true>(p, nbs, s)));
+  } else {
+    if (f.gs > 1) {
+      YSCV_TRY(scratch.take(part_bytes(f), s));
+      p.part = scratch.as<float>();
+    }
+    if (f.rows == 256) YSCV_TRY((gqa_flat_go<HD, 8, 2, false>(p, nbs, s)));
+    else if (f.rows == 128) YSCV_TRY((gqa_flat_go<HD, 4, 2, false>(p, nbs, s)));
+    else if (f.rows == 64) YSCV_TRY((gqa_flat_go<HD, 2, 2, false>(p, nbs, s)));
+    else YSCV_TRY((gqa_flat_go<HD, 1, 1, false>(p, nbs, s)));
   }
   if (p.gs > 1) {
     const size_t total = (size_t)nbs * p.R * HD;
