@@ -1,0 +1,59 @@
+"""One activation row of each type: every group form with and without zero points, waves that share a block of rows (one to
+eight, and slices behind the eighth), K that ends inside a slice, rows that end inside a block or a group of blocks, and several
+groups per workgroup.  Reference: the dequantised product in float64."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CASES = [(n, k, g, scales, zp) for (n, k) in [(1, 256), (17, 768), (1000, 1280), (129, 2816), (50, 4864), (200, 13056)]
+         for (g, scales, zp) in [(32, "f32", False), (64, "f16", True), (128, "f16", False), (256, "f32", True), (32, "f16", True)]]
+CASES += [(33, 32, 32, "f16", False), (100, 96, 32, "f32", True), (77, 2880, 64, "f32", False),
+          (70001, 96, 32, "f32", False), (33100, 2400, 32, "f16", True), (33100, 2112, 64, "f32", False),
+          (65700, 2080, 32, "f16", False)]
+
+
+def _problem(n, k, g, act, scales, zp):
+    """the weight, its dense form and the activations"""
+    import torch
+
+    from yscv_amd import kernels as K
+
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    q = torch.randint(0, 16, (n, k), generator=gen, device="cuda", dtype=torch.uint8)
+    sc = (torch.rand(n, k // g, generator=gen, device="cuda") * 0.015 + 0.005).to({"f16": torch.float16, "f32": torch.float32}[scales])
+    z = torch.full((n, k // g + (k // g) % 2), 8, device="cuda", dtype=torch.uint8)
+    if zp:
+        z[:, :k // g] = torch.randint(0, 16, (n, k // g), generator=gen, device="cuda", dtype=torch.uint8)
+    w = K.PackedInt4Weight((q[:, 0::2] | (q[:, 1::2] << 4)).cpu().numpy(), sc.cpu().numpy(), g, n, k,
+                           zero_points=(z[:, 0::2] | (z[:, 1::2] << 4)).cpu().numpy() if zp else None, nibble_format=K.NIBBLE_UNSIGNED)
+    dense = (q.double() - z[:, :k // g].double().repeat_interleave(g, 1)) * sc.double().repeat_interleave(g, 1)
+    x = torch.randn(1, k, generator=gen, device="cuda").to({"f16": torch.float16, "f32": torch.float32, "bf16": torch.bfloat16}[act])
+    return w, dense, x
+
+
+@pytest.mark.parametrize("act", ["f16", "f32", "bf16"])
+@pytest.mark.parametrize("n,k,g,scales,zp", CASES)
+def test_one_row(n, k, g, scales, zp, act):
+    import torch
+
+    w, dense, x = _problem(n, k, g, act, scales, zp)
+    got = w.matmul(x, out_dtype=torch.float32)
+    # products hold 22 bits of an f32 x (all of a 16-bit one) and the weight exactly; a zero point is subtracted behind the sum of
+    # 32 products (up to 15 times their size); then come four additions and the rounding of the result: every rounding is at
+    # most 2^-23 of a sum of magnitudes
+    bound = 2.0 ** -23 * ((32 if zp else 4) + 5) * (x.double().abs() @ (dense.abs() + (dense.abs().mean() if zp else 0)).t())
+    assert bool(((got.double() - x.double() @ dense.t()).abs() <= bound).all())
+    for dt in (torch.float16, torch.bfloat16):
+        assert torch.equal(w.matmul(x, out_dtype=dt), got.to(dt))
+
+
+def test_magnitudes():
+    """f32 rows far from one keep their relative accuracy, zeros give zeros."""
+    import torch
+
+    w, dense, x = _problem(300, 1536, 32, "f32", "f32", True)
+    want = x.double() @ dense.t()
+    for e in (-100, -30, 40):
+        got = w.matmul(x * 2.0 ** e, out_dtype=torch.float32).double() * 2.0 ** -e
+        assert float((got - want).norm() / want.norm()) < 2e-7  # about 1e-7 at one
+    assert float(w.matmul(x * 0, out_dtype=torch.float32).abs().max()) == 0.0

@@ -644,7 +644,7 @@ static int32_t enqueue_layers_step(yscv_hip_decoder *d, hipStream_t s) {
   const auto &c = d->cfg;
   YSCV_TRY(launch_decode_layers(d->lm, s));
   YSCV_TRY(launch_rmsnorm(d->h, d->final_norm, 1, c.d_model, c.rms_eps, d->xn, s));
-  YSCV_TRY(int4_run_ws(d->lm_head, d->xn, YSCV_HIP_F16, d->logits, YSCV_HIP_F32, 1, 1, EPI_STORE, d->ws, d->ws_bytes, s));
+  YSCV_TRY(int4_run_ws(d->lm_head, d->xn, YSCV_HIP_F16, d->logits, YSCV_HIP_F32, 1, 0, EPI_STORE, d->ws, d->ws_bytes, s));
   YSCV_TRY(launch_pick(d->logits, 1, c.vocab, d->pick, d->tokens, d->history, d->pos, d->step, c.max_steps, s));
   return YSCV_HIP_OK;
 }
