@@ -57,3 +57,27 @@ def test_magnitudes():
         got = w.matmul(x * 2.0 ** e, out_dtype=torch.float32).double() * 2.0 ** -e
         assert float((got - want).norm() / want.norm()) < 2e-7  # about 1e-7 at one
     assert float(w.matmul(x * 0, out_dtype=torch.float32).abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("n,k", [(40, 96), (1002, 1056), (520, 8736), (33100, 2400)])
+@pytest.mark.parametrize("act", ["f16", "f32"])
+def test_epilogues(n, k, act):
+    """residual update and SwiGLU against the plain product of the same kernel, and a workspace that is too small"""
+    import torch
+
+    from yscv_amd import kernels as K
+
+    w, _, x = _problem(n, k, 32, act, "f16", False)
+    v = w.matmul(x, out_dtype=torch.float32)
+    h = torch.randn(1, n, device="cuda")
+    y = h.clone()
+    w.matmul_fused(x, y, K.EPILOGUE_ADD_F32)
+    assert torch.equal(y, h + v)
+    out = torch.empty(1, n // 2, device="cuda", dtype=torch.float16)
+    w.matmul_fused(x, out, K.EPILOGUE_SWIGLU)
+    ref = torch.nn.functional.silu(v[:, 0::2].double()) * v[:, 1::2].double()
+    # one rounding to fp16 behind a silu whose exponential is good to a few units of 2^-22
+    assert float(((out.double() - ref).abs() - (2.0 ** -11 + 2.0 ** -19) * ref.abs()).max()) <= 2.0 ** -24
+    if k > 4096:  # (the kernel needs no workspace; the advertised size is for the others and still asked for)
+        with pytest.raises(Exception, match="workspace"):
+            w.matmul(x, out_dtype=torch.float32, workspace=torch.empty(256, dtype=torch.uint8, device="cuda"))

@@ -99,7 +99,8 @@ int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan
                            const NormFold *nf = nullptr);
 // one activation row (int4_gemv.hip)
 bool int4_gemv_takes(const yscv_hip_int4_weight *w, const void *x, int x_dtype, size_t m);
-int32_t launch_int4_gemv(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y, int y_dtype, int num_cus, hipStream_t s);
+int32_t launch_int4_gemv(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y, int y_dtype, int epi, const NormFold *nf,
+                         int num_cus, hipStream_t s);
 int32_t launch_int4_generic(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y,
                             int y_dtype, size_t m, hipStream_t s);
 int32_t launch_int4_gemm(const yscv_hip_int4_weight *w, const _Float16 *xh, const _Float16 *xl,
