@@ -529,9 +529,11 @@ int32_t yscv_hip_decoder_reset(yscv_hip_decoder *d, int32_t batch, int32_t start
 /* Run n_steps decode steps (asynchronously on `stream`).  use_graph = 0 launches the kernels of a step one
  * by one, 1 replays one captured HIP graph per step, 2 runs all n_steps in ONE cooperative launch of the
  * persistent decode kernel (batch 1 only; YSCV_HIP_ERR_UNSUPPORTED with the reason in the error text when
- * the model shape or the device cannot run it), YSCV_HIP_DECODE_AUTO picks 2 where it applies (batch 1, fp16
- * cache, supported shape) and 1 otherwise; for batch 1 of a small model (head width 64, d_model at most 1024, groups of
- * 32, fp16 cache) the step it captures holds all layers as one kernel.  Paths 0 and 1 run the same kernels and give the same
+ * the model shape or the device cannot run it), YSCV_HIP_DECODE_AUTO picks the fastest for
+ * the shape.  At batch 1 with an fp16 cache and groups of 32 that is a captured step that holds all layers as one kernel (path 1),
+ * for a small model (head width 64, d_model at most 1024) and for a large one (head width 128, up to four query heads per kv
+ * head, d_model a multiple of 512 with more than half a CU and at most one CU per 16 of it, d_ff at most 3.5 d_model); else, at
+ * batch 1, 2 where it applies; else 1.  Paths 0 and 1 run the same kernels and give the same
  * bits; path 2 and AUTO round their fp16 activations at other points, so their logits agree to about 1e-4 .. 5e-3 of max|logit|
  * (each path is within the float bar of the int4 kernels against the reference arithmetic) and a greedy pick can
  * differ where two logits are that close.  A caller that needs one arithmetic for every batch size names the path
@@ -578,8 +580,8 @@ int32_t yscv_hip_decoder_read_logits(yscv_hip_decoder *d, float *out_host);
 /* Inspection aid for parity tests: the activation buffers of the multi-kernel path (use_graph 0 or 1) as the last
  * step left them, widened to f32, [batch][width]: the residual stream after the last layer, the final RMSNorm's
  * output (the LM head's input), and the last layer's q|k|v (q and k rotated), attention output and SwiGLU output.
- * The single-launch path keeps these in registers and exchange records and does not fill them; behind a step of a small
- * model (YSCV_HIP_DECODE_AUTO) they are read from that step's exchange records.  No counterpart in
+ * The single-launch path keeps these in registers and exchange records and does not fill them; behind a step whose
+ * layers are one kernel (YSCV_HIP_DECODE_AUTO) they are read from that step's exchange records.  No counterpart in
  * the reference (its runner keeps every intermediate tensor in the TensorEnv by name). */
 #define YSCV_HIP_DEC_ACT_RESIDUAL 0 /* [batch][d_model] */
 #define YSCV_HIP_DEC_ACT_NORMED 1   /* [batch][d_model] */

@@ -14,9 +14,9 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hi
          "-Xclang", "-packed-fp32-ops", "-S", "--cuda-device-only"]
 # the sources with asm loads or hand-counted waits, and their extra flags in the Makefile
 SOURCES = {"int4_gemm_ring.hip": [], "decode_persistent.hip": [], "i8_gemm.hip": ["-ffp-contract=off"], "int4_gemm_wide.hip": [],
-           "int4_ksplit.hip": [], "i8_ksplit.hip": ["-ffp-contract=off"], "glue_ops.hip": [], "decode_layers.hip": []}
+           "int4_ksplit.hip": [], "i8_ksplit.hip": ["-ffp-contract=off"], "glue_ops.hip": [], "decode_layers.hip": [], "decode_wide.hip": []}
 # kernels whose pipeline counts on every value staying in registers
-PIPELINED = ("gemm_ring_kernel", "gemm_wide_kernel", "int4_ksplit_kernel", "i8_ksplit_kernel", "gqa_flat_kernel", "decode_layers_kernel")
+PIPELINED = ("gemm_ring_kernel", "gemm_wide_kernel", "int4_ksplit_kernel", "i8_ksplit_kernel", "gqa_flat_kernel", "decode_layers_kernel", "decode_wide_kernel")
 
 
 def test_checker_sees_a_copy_between_load_and_wait():

@@ -1,4 +1,5 @@
-// Interface of the kernel that takes one token through all layers of a small decoder in one launch (decode_layers.hip).
+// Interface of the kernels that take one token through all layers of a decoder in one launch (decode_layers.hip: head width 64,
+// decode_wide.hip: head width 128).
 #pragma once
 
 #include "common.hpp"
@@ -12,7 +13,7 @@ struct LayersLayer {
   const _Float16 *scales[4];
   const float *gamma[2];
   _Float16 *kc, *vc;
-  const _Float16 *qkv_bias;  // null or [(heads + 2 kv_heads) * 64]
+  const _Float16 *qkv_bias;  // null or [(heads + 2 kv_heads) * head width]
 };
 
 struct LayersModel {
@@ -27,13 +28,13 @@ struct LayersModel {
   // exchange buffer of 8-byte {payload, tag} entries: residual before each norm (f32), q/k/v and SwiGLU output (two fp16
   // each), attention partials.  No 128-byte line is written by two workgroups.
   unsigned long long *x;
-  int at_attn, at_ffn, at_qkv, at_act, at_part;
+  int at_attn, at_ffn, at_qkv, at_act, at_part, at_ao;  // (at_ao: decode_wide.hip only)
   uint32_t *steps;    // steps since the entries were cleared
   uint32_t *give_up;  // pinned host memory: a wait gave up
 };
 
 constexpr int kLayersChunk = 256;     // cached positions of one attention work item
-constexpr int kLayersActSlots = 32;   // entries a workgroup has for its SwiGLU output (at most 24 used)
+constexpr int kLayersActSlots = 32;   // entries a workgroup has for its SwiGLU output (at most 28 used)
 inline __host__ __device__ int layers_chunks(int max_ctx) { return (max_ctx + kLayersChunk - 1) / kLayersChunk; }
 constexpr int kLayersHeadRec = 80;    // entries of one head's partials of a chunk: o[64], max, sum; whole lines
 
@@ -42,5 +43,11 @@ bool layers_supported(const yscv_hip_decoder_config &c, int num_cus);
 void layers_exchange_entries(const yscv_hip_decoder_config &c, size_t out[5]);
 int32_t launch_decode_layers(const LayersModel &m, hipStream_t s);
 int32_t launch_layers_report(const LayersModel &m, int pos, _Float16 *qkv, _Float16 *qrot, _Float16 *ao, _Float16 *act, hipStream_t s);
+
+// the same for head width 128
+bool wide_supported(const yscv_hip_decoder_config &c, int num_cus);
+void wide_exchange_entries(const yscv_hip_decoder_config &c, size_t out[6]);
+int32_t launch_decode_wide(const LayersModel &m, hipStream_t s);
+int32_t launch_wide_report(const LayersModel &m, int pos, _Float16 *qkv, _Float16 *qrot, _Float16 *ao, _Float16 *act, hipStream_t s);
 
 }  // namespace yscv

@@ -5,6 +5,8 @@
 // memory, so the step is captured once into a HIP graph and replayed for every token.
 #include <algorithm>
 #include <cmath>
+#include <map>
+#include <mutex>
 #include <vector>
 
 #include "decode_layers.hpp"
@@ -187,6 +189,7 @@ struct yscv_hip_decoder {
   uint32_t epoch = 1;          // tag epoch of the next persistent step; tags are 24 bits wide: see yscv_hip_decoder_run
   unsigned long long *p_trace = nullptr;  // stage timestamps (builds with YSCV_PERSIST_TRACE only)
   // small models at batch 1, YSCV_HIP_DECODE_AUTO: all layers of a step in one launch (decode_layers.hip), a graph of its own
+  bool l_wide = false;         // decode_wide.hip, not decode_layers.hip
   bool layers_ok = false;      // the shape is supported, the buffers exist and the weights are laid out as it reads them
   LayersModel lm{};
   LayersLayer *l_table = nullptr;
@@ -217,6 +220,8 @@ static void drop_graph(yscv_hip_decoder *d) {
   drop_captured(&d->l_graph, &d->l_graph_exec);
   d->graph_batch = 0;
 }
+
+static void resident_forget(const yscv_hip_decoder *d);
 
 static void decoder_free(yscv_hip_decoder *d) {
   if (!d) return;
@@ -274,6 +279,7 @@ static void decoder_free(yscv_hip_decoder *d) {
   (void)hipFree(d->l_count);
   (void)hipHostFree(d->l_give_up);
   if (d->end_event) (void)hipEventDestroy(d->end_event);
+  resident_forget(d);
   delete d;
 }
 
@@ -319,6 +325,54 @@ struct InOrder {
     if (before >= 0) (void)hipSetDevice(before);
   }
 };
+
+// Launches whose workgroups wait for each other have to be on the chip as a whole.  Two of them that got half of it each would
+// both wait until they give up, so one decoder's are enqueued at a time, and another decoder's wait for them on the device.
+// Nothing is recorded while one decoder has the turn on the default stream.
+struct Resident {
+  struct Turn {
+    std::mutex mu;
+    const yscv_hip_decoder *last = nullptr;  // whose launches came last, on the default stream or in front of `end`
+    bool on_default = false;
+    hipEvent_t end = nullptr;
+  };
+  static Turn &of(int device) {
+    static std::mutex mu;
+    static std::map<int, Turn> turns;  // one entry and one event per device
+    std::lock_guard<std::mutex> hold(mu);
+    return turns[device];
+  }
+  Turn &t;
+  std::unique_lock<std::mutex> hold;
+  yscv_hip_decoder *d;
+  hipStream_t s;
+  bool entered = false;
+  Resident(yscv_hip_decoder *dec, hipStream_t stream) : t(of(dec->device)), hold(t.mu), d(dec), s(stream) {}
+  Resident(const Resident &) = delete;
+  Resident &operator=(const Resident &) = delete;
+  hipError_t enter() {
+    hipError_t e = t.end ? hipSuccess : hipEventCreateWithFlags(&t.end, hipEventDisableTiming);
+    if (e == hipSuccess && t.last && t.last != d && !(t.on_default && s == nullptr)) {
+      if (t.on_default) e = hipEventRecord(t.end, nullptr);
+      if (e == hipSuccess) e = hipStreamWaitEvent(s, t.end, 0);
+    }
+    entered = e == hipSuccess;
+    return e;
+  }
+  ~Resident() {
+    if (!entered) return;
+    if (s != nullptr && hipEventRecord(t.end, s) != hipSuccess) (void)hipStreamSynchronize(s);
+    t.last = d;
+    t.on_default = s == nullptr;
+  }
+};
+
+// (its work has been waited for)
+static void resident_forget(const yscv_hip_decoder *d) {
+  Resident::Turn &t = Resident::of(d->device);
+  std::lock_guard<std::mutex> hold(t.mu);
+  if (t.last == d) t.last = nullptr;
+}
 
 // The host keeps the position and the step the decoder is at and passes them, and a prompt's tokens, with the call: a graph
 // would replay the numbers of the call that was captured.
@@ -505,7 +559,8 @@ static int32_t layers_setup(yscv_hip_decoder *d) {
   const Context *ctx = nullptr;
   YSCV_TRY(ensure_context(&ctx));
   const auto &c = d->cfg;
-  if (d->kv_dtype != YSCV_HIP_KV_F16 || !layers_supported(c, ctx->num_cus)) return YSCV_HIP_OK;
+  d->l_wide = wide_supported(c, ctx->num_cus);
+  if (d->kv_dtype != YSCV_HIP_KV_F16 || !(d->l_wide || layers_supported(c, ctx->num_cus))) return YSCV_HIP_OK;
   LayersModel &m = d->lm;
   m.n_layers = c.n_layers;
   m.d = c.d_model;
@@ -521,9 +576,10 @@ static int32_t layers_setup(yscv_hip_decoder *d) {
   m.tokens = d->tokens;
   m.pos = d->pos;
   m.h = d->h;
-  size_t entries[5], total = 0, at[5];
-  layers_exchange_entries(c, entries);
-  for (int i = 0; i < 5; i++) {
+  size_t entries[6] = {}, total = 0, at[6];
+  if (d->l_wide) wide_exchange_entries(c, entries);
+  else layers_exchange_entries(c, entries);
+  for (int i = 0; i < 6; i++) {
     at[i] = total;
     total += round_up(entries[i], 32);  // every buffer 256-byte aligned
   }
@@ -542,6 +598,7 @@ static int32_t layers_setup(yscv_hip_decoder *d) {
   m.at_qkv = (int)at[2];
   m.at_act = (int)at[3];
   m.at_part = (int)at[4];
+  m.at_ao = (int)at[5];
   m.steps = d->l_count;
   m.give_up = d->l_give_up;
   m.layers = reinterpret_cast<decltype(m.layers)>(reinterpret_cast<uintptr_t>(d->l_table));
@@ -642,7 +699,7 @@ static int32_t finish_setup(yscv_hip_decoder *d) {
 // the launches of a step whose layers run in one
 static int32_t enqueue_layers_step(yscv_hip_decoder *d, hipStream_t s) {
   const auto &c = d->cfg;
-  YSCV_TRY(launch_decode_layers(d->lm, s));
+  YSCV_TRY(d->l_wide ? launch_decode_wide(d->lm, s) : launch_decode_layers(d->lm, s));
   YSCV_TRY(launch_rmsnorm(d->h, d->final_norm, 1, c.d_model, c.rms_eps, d->xn, s));
   YSCV_TRY(int4_run_ws(d->lm_head, d->xn, YSCV_HIP_F16, d->logits, YSCV_HIP_F32, 1, 0, EPI_STORE, d->ws, d->ws_bytes, s));
   YSCV_TRY(launch_pick(d->logits, 1, c.vocab, d->pick, d->tokens, d->history, d->pos, d->step, c.max_steps, s));
@@ -1140,7 +1197,7 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
   // the fastest path this decoder has for its batch; the layers of a small model in one launch are part of a graph too
   const bool layers = use_graph == YSCV_HIP_DECODE_AUTO && d->batch == 1 && d->layers_ok;
   if (use_graph == YSCV_HIP_DECODE_AUTO)
-    use_graph = (d->batch == 1 && d->persist_ok && !d->has_bias && d->kv_dtype == YSCV_HIP_KV_F16) ? 2 : 1;
+    use_graph = (!layers && d->batch == 1 && d->persist_ok && !d->has_bias && d->kv_dtype == YSCV_HIP_KV_F16) ? 2 : 1;
   d->last_path = use_graph == 2 ? 2 : (use_graph ? 1 : 0);
   if (use_graph == 2) {
     if (d->kv_dtype != YSCV_HIP_KV_F16)
@@ -1151,6 +1208,8 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
     if (d->batch != 1) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "the single-launch decode path runs batch 1 only");
     if (n_steps == 0) return YSCV_HIP_OK;
     DEC_HIP(call.enter());
+    Resident turn(d, s);
+    DEC_HIP(turn.enter());
     // A tag is ((epoch + step) * (layers + 2) + 1 + layer) modulo 2^24.  Before the tag space wraps, the exchange
     // buffers are cleared and the epoch starts again, so an entry left from half a million steps ago can never be taken
     // for a fresh one.
@@ -1173,6 +1232,8 @@ int32_t yscv_hip_decoder_run(yscv_hip_decoder *d, int32_t n_steps, int32_t use_g
   }
   DEC_HIP(call.enter());
   if (layers) {
+    Resident turn(d, s);
+    DEC_HIP(turn.enter());
     // tags count steps: before they wrap, the entries are cleared and the count starts again
     const uint32_t most = (uint32_t)(0xFFFFFFFEull / ((uint64_t)d->cfg.n_layers + 1)) - 1;
     if (d->l_steps >= most - (uint32_t)n_steps) {
@@ -1352,7 +1413,7 @@ int32_t yscv_hip_decoder_read_activation(yscv_hip_decoder *d, int32_t which, flo
   YSCV_REQUIRE(capacity >= elems, "output holds %zu values, the buffer has %zu", capacity, elems);
   DEC_HIP(hipDeviceSynchronize());
   if (d->l_last_pos >= 0) {
-    YSCV_TRY(launch_layers_report(d->lm, d->l_last_pos, d->qkv, d->qrot, d->ao, d->act, nullptr));
+    YSCV_TRY((d->l_wide ? launch_wide_report : launch_layers_report)(d->lm, d->l_last_pos, d->qkv, d->qrot, d->ao, d->act, nullptr));
     DEC_HIP(hipDeviceSynchronize());
   }
   if (!half) {

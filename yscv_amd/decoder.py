@@ -92,8 +92,8 @@ class Decoder:
 
     def run(self, n_steps, use_graph=True, stream=None, persistent=False, auto=False):
         """use_graph: replay one captured HIP graph per step; persistent: run all steps inside one
-        cooperative launch (batch 1, shapes the single-launch kernel supports); auto: the fastest of the two
-        that applies (YSCV_HIP_DECODE_AUTO, what generate() uses)."""
+        cooperative launch (batch 1, shapes the single-launch kernel supports); auto: the fastest way
+        for the shape, which may be a graph of its own with all layers in one kernel (YSCV_HIP_DECODE_AUTO, what generate() uses)."""
         mode = 3 if auto else (2 if persistent else int(bool(use_graph)))
         lib().decoder_run(self._h, int(n_steps), mode, C.c_void_p(stream) if stream else None)
 
