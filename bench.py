@@ -33,7 +33,7 @@ MFMA_I8_PEAK = 5000.0       # TOP/s dense
 # plain 256 MiB copy gives for FETCH_SIZE on this GPU, + write 38 KiB x 1.0): profiles/int4_skinny_decode7b_graph_path.md
 SKINNY_TRAFFIC_BYTES = 31_385_000
 # HBM bytes per decode step of the single-launch kernel from the same kind of counter runs (None until measured)
-PERSIST_TRAFFIC_BYTES_PER_STEP = 4_429_000_000  # fetch 4.337 GB (x2.0 scale) + write 0.092 GB: profiles/decode_persistent_7b.md
+WIDE_TRAFFIC_BYTES_PER_STEP = 4_462_000_000  # layers: fetch 4.358 GB (x2.0 scale) + write 0.030; LM head 0.074: profiles/decode_wide_7b.md
 
 CFG7B = dict(n_layers=32, d_model=4096, n_heads=32, n_kv_heads=8, head_dim=128, d_ff=14336, vocab=32000,
              group_size=32, max_batch=16, max_ctx=2048 + 512, max_steps=1024, rope_theta=10000.0, rms_eps=1e-5)
@@ -58,18 +58,18 @@ def event_time_ms(fn, torch):
     return s.elapsed_time(e)
 
 
-def bench_decode(dec, torch, batch, steps, warmup, stream_ptr, persistent=False):
-    """Wall time of `steps` decode steps after `warmup` untimed ones.  persistent: every run() call is ONE
-    cooperative launch that executes all its steps on the device; otherwise one HIP-graph replay per step."""
+def bench_decode(dec, torch, batch, steps, warmup, stream_ptr, auto=False):
+    """Wall time of `steps` decode steps after `warmup` untimed ones.  auto: the path the decoder picks for its shape, as
+    generate() does; otherwise one HIP-graph replay of the multi-kernel step per step."""
     import numpy as np
 
     dec.reset(np.arange(1, batch + 1, dtype=np.int32), PREFILL)
-    dec.run(warmup, use_graph=True, stream=stream_ptr, persistent=persistent)
+    dec.run(warmup, use_graph=True, stream=stream_ptr, auto=auto)
     torch.cuda.synchronize()
     s_ev, e_ev = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     t0 = time.perf_counter()
     s_ev.record()
-    dec.run(steps, use_graph=True, stream=stream_ptr, persistent=persistent)
+    dec.run(steps, use_graph=True, stream=stream_ptr, auto=auto)
     e_ev.record()
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
@@ -78,8 +78,8 @@ def bench_decode(dec, torch, batch, steps, warmup, stream_ptr, persistent=False)
     return dt, s_ev.elapsed_time(e_ev) * 1e-3
 
 
-def check_single_launch(dec, torch, steps=8):
-    """The single-launch kernel against the multi-kernel path from the benchmark's own start state: the last step's
+def check_auto(dec, torch, steps=8):
+    """The path the decoder picks against the multi-kernel path from the benchmark's own start state: the last step's
     logits agree to 2e-2 of max|logit| (two implementations with different fp16 rounding points) and a token differs
     only where the other path's logits of the two picks are within that difference.  Raises if not."""
     import numpy as np
@@ -89,11 +89,11 @@ def check_single_launch(dec, torch, steps=8):
     dec.run(steps, use_graph=True)
     tg, lg = dec.tokens(0, steps)[:, 0].copy(), dec.logits()[0].copy()
     dec.reset(start, PREFILL)
-    dec.run(steps, persistent=True)
+    dec.run(steps, auto=True)
     tp, lp = dec.tokens(0, steps)[:, 0].copy(), dec.logits()[0].copy()
     same = bool(np.array_equal(tg, tp))
     rel = float(np.abs(lg - lp).max() / np.abs(lg).max())
-    assert np.isfinite(lp).all() and (same or rel < 2e-2), "single-launch decode disagrees with the multi-kernel path"
+    assert np.isfinite(lp).all() and (same or rel < 2e-2), "decode disagrees with the multi-kernel path"
     assert not same or rel < 2e-2, "same tokens but logits differ by %g of max|logit|" % rel
     return {"steps": steps, "tokens_equal_multi_kernel_path": same, "max_rel_logit_diff_last_step": round(rel, 6)}
 
@@ -580,22 +580,21 @@ def main():
         print(json.dumps({"extra": {"prefill_%d_tokens" % n: bench_prefill(dec, torch, cfg, n, params) for n in args.prefill_tokens}}))
         return
 
-    persistent = args.batch == 1 and not args.graph_path
-    check = check_single_launch(dec, torch) if persistent and not args.no_check else None
-    dt, dt_events = bench_decode(dec, torch, args.batch, args.steps, args.warmup, stream_ptr, persistent=persistent)
+    auto = args.batch == 1 and not args.graph_path
+    check = check_auto(dec, torch) if auto and not args.no_check else None
+    dt, dt_events = bench_decode(dec, torch, args.batch, args.steps, args.warmup, stream_ptr, auto=auto)
+    single = dec.last_path() == 2
     tok_s = args.batch * args.steps / dt
     kv_row_bytes = 2 * cfg["n_layers"] * cfg["n_kv_heads"] * cfg["head_dim"] * 2  # K + V bytes one cached position adds
     kv_bytes_per_seq = kv_row_bytes * PREFILL
     ideal_step_s = (w_bytes + args.batch * kv_bytes_per_seq) / (HBM_PEAK_GBS * 1e9)
-    if persistent:
-        # dominant kernel = the single-launch decode kernel: one launch runs all timed steps.  Algorithmic bytes
-        # per launch = per step, the packed weights + scales (read once) + the KV cache rows attended to.
+    if auto:
+        # algorithmic bytes per step = the packed weights + scales (read once) + the KV cache rows attended to
         first = PREFILL + args.warmup
-        kv_bytes = sum(kv_row_bytes * (first + i) for i in range(args.steps))
-        bytes_per_launch = w_bytes * args.steps + kv_bytes
-        launch_s, launches = dt_events, 1
-        kernel = "decode_persistent_kernel (one launch = %d decode steps)" % args.steps
-        traffic = PERSIST_TRAFFIC_BYTES_PER_STEP * args.steps if PERSIST_TRAFFIC_BYTES_PER_STEP else None
+        bytes_per_launch = w_bytes + sum(kv_row_bytes * (first + i) for i in range(args.steps)) / args.steps
+        launch_s, launches = dt_events / args.steps, args.steps
+        kernel = "a whole decode step: decode_wide_kernel (all layers) and the LM head" if not single else "a step of decode_persistent_kernel"
+        traffic = WIDE_TRAFFIC_BYTES_PER_STEP if not single else None
     else:
         launch_s, launches = bench_projections(dec, torch, args.batch, stream_ptr)
         n_proj = 4 * cfg["n_layers"] + 1
@@ -620,7 +619,8 @@ def main():
         "config": {"workload": "BASELINE configs[3]: Llama-style decoder 32L d4096 32q/8kv hd128 ffn14336 vocab32000, "
                                "int4 g32 fp16 scales, fp16 KV ctx %d, greedy decode" % PREFILL,
                    "batch": args.batch, "tokens_per_step": args.batch,
-                   "path": "single cooperative launch for all steps" if persistent else "one HIP-graph replay per step",
+                   "path": "single cooperative launch for all steps" if auto and single else
+                   "one HIP-graph replay per step, all layers in one kernel" if auto else "one HIP-graph replay per step",
                    "arithmetic": "int4 weights (exact in fp16) x fp16 activations on v_mfma_f32_16x16x32_f16, fp32 accumulate"},
         "roofline": {
             "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -638,12 +638,12 @@ def main():
     extra = {}
     if not args.no_extra:
         n_proj = 4 * cfg["n_layers"] + 1
-        if persistent:
+        if auto:
             dtg, _ = bench_decode(dec, torch, 1, min(args.steps, 64), 4, stream_ptr)
             avg1, _ = bench_projections(dec, torch, 1, stream_ptr)
             extra["decode_batch1_graph_path"] = {"tok/s": round(min(args.steps, 64) / dtg, 1),
                                                  "ms_per_step": round(dtg / min(args.steps, 64) * 1e3, 4),
-                                                 "skinny_kernel_GB/s": round(w_bytes / n_proj / avg1 / 1e9, 1)}
+                                                 "projection_kernel_GB/s": round(w_bytes / n_proj / avg1 / 1e9, 1)}
         if args.batch != 16:
             dt16, _ = bench_decode(dec, torch, 16, min(args.steps, 64), 4, stream_ptr)
             avg16, _ = bench_projections(dec, torch, 16, stream_ptr, reps=3)
