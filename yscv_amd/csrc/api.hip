@@ -197,12 +197,12 @@ int32_t int4_run_ws(const yscv_hip_int4_weight *w, const void *x, int x_dtype, v
   }
   note_int4_fast();
   Int4Scratch L = int4_scratch_layout(w, x, x_dtype, y, y_dtype, m, force, ctx->num_cus);
-  if (force <= 1 && int4_gemv_takes(w, x, x_dtype, m)) {  // needs no scratch; a workspace that is passed is still checked
+  if (force <= 1 && int4_gemv_takes(w, x, m, ctx->num_cus)) {  // needs no scratch; a workspace that is passed is still checked
     if (ws) {
       YSCV_REQUIRE(ws_bytes >= L.total + L.opt_bytes, "workspace too small: %zu < %zu bytes", ws_bytes, L.total + L.opt_bytes);
       YSCV_REQUIRE(L.total + L.opt_bytes == 0 || (reinterpret_cast<uintptr_t>(ws) & 255) == 0, "workspace must be 256-byte aligned");
     }
-    return launch_int4_gemv(w, x, x_dtype, y, y_dtype, epi, nf, ctx->num_cus, s);
+    return launch_int4_gemv(w, x, x_dtype, y, y_dtype, m, epi, nf, ctx->num_cus, s);
   }
   // above 16 rows the LDS-ring GEMM (16-bit activations) has the add and SwiGLU epilogues; the exact-scale kernel has none
   if (!L.skinny && epi != EPI_STORE && !(x_dtype != YSCV_HIP_F32 && nf == nullptr))

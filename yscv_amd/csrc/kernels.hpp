@@ -97,10 +97,10 @@ int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan
                            const _Float16 *xl, const void *xraw, const float *row_scale, size_t ldx, int split,
                            void *y, int y_dtype, size_t m, float *partial, int epi, hipStream_t s,
                            const NormFold *nf = nullptr);
-// one activation row (int4_gemv.hip)
-bool int4_gemv_takes(const yscv_hip_int4_weight *w, const void *x, int x_dtype, size_t m);
-int32_t launch_int4_gemv(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y, int y_dtype, int epi, const NormFold *nf,
-                         int num_cus, hipStream_t s);
+// one activation row, or up to four where that pays (int4_gemv.hip)
+bool int4_gemv_takes(const yscv_hip_int4_weight *w, const void *x, size_t m, int num_cus);
+int32_t launch_int4_gemv(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y, int y_dtype, size_t m, int epi,
+                         const NormFold *nf, int num_cus, hipStream_t s);
 int32_t launch_int4_generic(const yscv_hip_int4_weight *w, const void *x, int x_dtype, void *y,
                             int y_dtype, size_t m, hipStream_t s);
 int32_t launch_int4_gemm(const yscv_hip_int4_weight *w, const _Float16 *xh, const _Float16 *xl,
