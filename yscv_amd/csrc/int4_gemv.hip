@@ -12,7 +12,7 @@
 // eight waves 8.9 us, with sixteen 7.8).  Residual updates, SwiGLU and a folded norm (NormFold in kernels.hpp) are done by the threads
 // that hold the sums, with their operands requested ahead of the weights.
 // Bound: below a few MB of weights the launch and one round trip to memory each for arguments, loads and sums (4096 x 4096 f32 8.6
-// -> 4.5 us, fp16 4.95 -> 4.15, bf16 6.3 -> 4.2; 4096 x 14336 f32 25 -> 9.5; 16384 x 1024 with zero points 8.4 -> 4.5; the weights
+// -> 4.5 us, fp16 4.95 -> 4.0, bf16 6.3 -> 4.0; 4096 x 14336 f32 25 -> 9.5; 16384 x 1024 with zero points 8.4 -> 4.5; the weights
 // alone are 1 - 4 us of HBM); above that the 4.5 - 5 TB/s that loads of this kind reach behind decode and MFMA (151936 x 1024
 // fp16 27.7 -> 16.5, f32 42.0 -> 18.7; 128256 x 4096 51 - 53 and 58.5 - 59 in both).  All captured, weights from HBM, the skinny
 // kernel -> this one.  A graph step of the 7B-shape decoder at batch 1: 1619 -> 1376 us (q/k/v 7.3 -> 5.5, o 6.2 -> 4.7, gate/up 14.5 ->
@@ -61,15 +61,22 @@ struct GemvRowArgs {
 };
 
 // XD: type of the activations; f32 takes two MFMA operands, the others one.
+// EPI: residual update, SwiGLU or a folded norm; a plain one-row product leaves that code out (4096 x 4096 fp16 4.0 instead of 4.2 us,
+// 3000 x 704 f32 3.25 instead of 3.5: less to fetch at the start).
 // KEEP: a wave has one slice of K (K <= 4096).  Its activations stay in registers while the workgroup goes through its groups of
 // rows; without it a workgroup has one group and the waves go through their slices.
 // waves of a workgroup, and those a SIMD has to hold
 constexpr int gemv_waves(int m, bool keep) { return keep || m > 1 ? 8 : 16; }
 constexpr int gemv_per_simd(int m, int xd, bool zp, bool keep) { return m == 4 || (m == 2 && (!keep || (zp && xd == YSCV_HIP_F32))) ? 2 : 4; }
 
-template <int M, int XD, int GM, bool SF16, bool HAS_ZP, bool KEEP>
+template <int M, int XD, int GM, bool SF16, bool HAS_ZP, bool KEEP, bool EPI>
 __global__ void __launch_bounds__((64 * gemv_waves(M, KEEP)), (gemv_per_simd(M, XD, HAS_ZP, KEEP))) int4_gemv_kernel(GemvRowArgs p) {
   constexpr int WAVES = gemv_waves(M, KEEP);
+  if constexpr (!EPI) {
+    p.epi = EPI_STORE;
+    p.ss_in = nullptr;
+    p.xg = nullptr;
+  }
   constexpr int SPT = GM == GM32 ? 4 : (GM == GM64 ? 2 : 1);
   constexpr bool F32 = XD == YSCV_HIP_F32;
   typedef typename std::conditional<SF16, _Float16, float>::type elem_t;
@@ -329,21 +336,29 @@ __global__ void __launch_bounds__((64 * gemv_waves(M, KEEP)), (gemv_per_simd(M, 
   }
 }
 
-template <int M, int XD, int GM, bool SF16>
+template <int M, int XD, int GM, bool SF16, bool EPI>
 int32_t gemv_go(const GemvRowArgs &a, unsigned grid, hipStream_t s) {
   const bool keep = a.slices <= 8;
-  if (keep && a.tzps) hipLaunchKernelGGL((int4_gemv_kernel<M, XD, GM, SF16, true, true>), dim3(grid), dim3(512), 0, s, a);
-  else if (keep) hipLaunchKernelGGL((int4_gemv_kernel<M, XD, GM, SF16, false, true>), dim3(grid), dim3(512), 0, s, a);
-  else if (a.tzps) hipLaunchKernelGGL((int4_gemv_kernel<M, XD, GM, SF16, true, false>), dim3(grid), dim3(64 * gemv_waves(M, false)), 0, s, a);
-  else hipLaunchKernelGGL((int4_gemv_kernel<M, XD, GM, SF16, false, false>), dim3(grid), dim3(64 * gemv_waves(M, false)), 0, s, a);
+  const dim3 threads(64 * gemv_waves(M, keep));
+  if (keep && a.tzps) hipLaunchKernelGGL((int4_gemv_kernel<M, XD, GM, SF16, true, true, EPI>), dim3(grid), threads, 0, s, a);
+  else if (keep) hipLaunchKernelGGL((int4_gemv_kernel<M, XD, GM, SF16, false, true, EPI>), dim3(grid), threads, 0, s, a);
+  else if (a.tzps) hipLaunchKernelGGL((int4_gemv_kernel<M, XD, GM, SF16, true, false, EPI>), dim3(grid), threads, 0, s, a);
+  else hipLaunchKernelGGL((int4_gemv_kernel<M, XD, GM, SF16, false, false, EPI>), dim3(grid), threads, 0, s, a);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
+template <int M, int XD, int GM, bool SF16>
+int32_t gemv_epi(const GemvRowArgs &a, unsigned grid, hipStream_t s) {
+  if constexpr (M == 1) {
+    if (a.epi == EPI_STORE && !a.ss_in) return gemv_go<M, XD, GM, SF16, false>(a, grid, s);
+  }
+  return gemv_go<M, XD, GM, SF16, true>(a, grid, s);
+}
 template <int M, int XD>
 int32_t gemv_gm(const GemvRowArgs &a, unsigned grid, int gm, bool sf16, hipStream_t s) {
-  if (gm == GM32) return sf16 ? gemv_go<M, XD, GM32, true>(a, grid, s) : gemv_go<M, XD, GM32, false>(a, grid, s);
-  if (gm == GM64) return sf16 ? gemv_go<M, XD, GM64, true>(a, grid, s) : gemv_go<M, XD, GM64, false>(a, grid, s);
-  return sf16 ? gemv_go<M, XD, GM128, true>(a, grid, s) : gemv_go<M, XD, GM128, false>(a, grid, s);
+  if (gm == GM32) return sf16 ? gemv_epi<M, XD, GM32, true>(a, grid, s) : gemv_epi<M, XD, GM32, false>(a, grid, s);
+  if (gm == GM64) return sf16 ? gemv_epi<M, XD, GM64, true>(a, grid, s) : gemv_epi<M, XD, GM64, false>(a, grid, s);
+  return sf16 ? gemv_epi<M, XD, GM128, true>(a, grid, s) : gemv_epi<M, XD, GM128, false>(a, grid, s);
 }
 template <int M>
 int32_t gemv_xd(const GemvRowArgs &a, unsigned grid, int x_dtype, int gm, bool sf16, hipStream_t s) {
