@@ -3,9 +3,10 @@
 //
 // A layer of such a model is 6 MB of weights, a microsecond of memory time, cut into five dependent stages (q/k/v, attention,
 // o, gate/up, down).  As kernels of a graph each stage costs 2.5-5 us whatever it moves; here the workgroups stay resident
-// and hand small vectors to each other.  24 layers of d_model 1024, 16 heads over 2, d_ff 2816: a step 690 -> 314 us at position
-// 64, 945 -> 345 at 1024, 2715 -> 483 at 8128, 11155 -> 1270 at 32704 (the other path's attention has one workgroup per head):
-// there is no context at which the other path is the faster one.
+// and hand small vectors to each other.  24 layers of d_model 1024, 16 heads over 2, d_ff 2816: a step 690 -> 305 us at position
+// 64, 945 -> 331 at 1000; 2715 -> 483 at 8128, 11155 -> 1270 at 32704 (these two with the LM head on the skinny kernel, 10 us more;
+// the other path's attention has one workgroup per head).  With its norms folded and the one-row kernel in its projections the
+// other path takes 500 at 100: there is no context at which it is the faster one.
 //   * G = d_model / 16 workgroups of eight waves.  Workgroup w owns 16-row blocks of every projection, its eight waves split K
 //     in tiles of 128, one 1 KiB load per (block, tile) in the layout the other int4 kernels use.  A wave's weights for a whole
 //     layer fit its registers (2 + 1 + 6 + 3 tiles of 4 registers, and scales): the tiles of a stage are requested one or two
