@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(const float *__restrict__ 
       if ((u * 256 + (int)threadIdx.x) * 4 < d) ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
     }
   } else {
-    for (int i = threadIdx.x * 4; i < d; i += blockDim.x * 4) {
+    for (int i = threadIdx.x * 4; i < d; i += 256 * 4) {
       float4_t v = *reinterpret_cast<const float4_t *>(row + i);
       ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
     }
@@ -143,7 +143,7 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(const float *__restrict__ 
     }
     return;
   }
-  for (int i = threadIdx.x * 4; i < d; i += blockDim.x * 4) {
+  for (int i = threadIdx.x * 4; i < d; i += 256 * 4) {
     float4_t v = *reinterpret_cast<const float4_t *>(row + i);
     float4_t g = *reinterpret_cast<const float4_t *>(gamma + i);
     half4_t o;

@@ -566,12 +566,12 @@ __device__ __forceinline__ int flat_k_at(int row, int piece) {
 // positions per channel (positions past the end 0).  What that kernel would do once per workgroup: with 32 workgroups to a
 // kv head (512 queries of four heads, 64 rows each) 32 times.
 template <int HD>
-__global__ void __launch_bounds__(256) gqa_flat_prepare_kernel(FlatArgs p, uint8_t *__restrict__ pre) {
+__global__ void __launch_bounds__(256) gqa_flat_prepare_kernel(FlatArgs p, uint8_t *__restrict__ pre, int stages) {
   using C = FlatCfg<HD, 4, 1, true>;  // (a stage is the same in all forms)
   constexpr int KB = C::KB, CPR = HD / 8, K_PIECES = KB * CPR, V_UNITS = (KB / 8) * (HD / 4), BLOCKS = (K_PIECES + V_UNITS + 255) / 256;
   const int nb = blockIdx.x, b = nb / p.Hkv, kvh = nb % p.Hkv, st = blockIdx.y / BLOCKS, idx = (int)(blockIdx.y % BLOCKS) * 256 + (int)threadIdx.x;
   const size_t kv_s = (size_t)p.Hkv * HD, base = (size_t)b * p.Sk * kv_s + (size_t)kvh * HD;
-  const int stages = (int)gridDim.y / BLOCKS, left = min(KB, p.Sk - st * KB);
+  const int left = min(KB, p.Sk - st * KB);
   uint8_t *dst = pre + ((size_t)nb * stages + st) * C::ST_BYTES;
   if (idx < K_PIECES) {
     const int row = idx / CPR, piece = idx % CPR;
@@ -1067,7 +1067,7 @@ int32_t gqa_flat_launch(FlatArgs p, int B, int num_cus, hipStream_t s) {
   }
   p.gs = f.gs;
   if (f.pre) {
-    hipLaunchKernelGGL((gqa_flat_prepare_kernel<HD>), dim3((unsigned)nbs, (unsigned)stages * BLOCKS), dim3(256), 0, s, p, scratch.as<uint8_t>());
+    hipLaunchKernelGGL((gqa_flat_prepare_kernel<HD>), dim3((unsigned)nbs, (unsigned)stages * BLOCKS), dim3(256), 0, s, p, scratch.as<uint8_t>(), (int)stages);
     YSCV_HIP_TRY(hipGetLastError());
     p.pre = scratch.as<uint8_t>();
     p.part = scratch.as<float>(pre_bytes);
@@ -1158,7 +1158,7 @@ __global__ void __launch_bounds__(64) rope_f32_kernel(float *__restrict__ x, int
 // whole slab is new.
 __global__ void __launch_bounds__(256) prefill_rope_append_kernel(_Float16 *__restrict__ qkv, int rows, int start_pos, int hq, int hkv,
                                                                   int hd, float theta, int max_ctx, _Float16 *__restrict__ kc,
-                                                                  _Float16 *__restrict__ vc) {
+                                                                  _Float16 *__restrict__ vc, int parts) {
   const int tid = threadIdx.x;
   const int slab = start_pos / 8 + (int)blockIdx.x;
   const int p_lo = max(start_pos, slab * 8), p_hi = min(start_pos + rows, slab * 8 + 8);  // positions [p_lo, p_hi)
@@ -1175,8 +1175,8 @@ __global__ void __launch_bounds__(256) prefill_rope_append_kernel(_Float16 *__re
   __syncthreads();
   const int slots = hq + hkv, vecs = half_d / 8;  // eight pairs per item: 16-byte loads and stores
 #pragma unroll 2
-  // blockIdx.y takes every gridDim.y-th item of the slab (short prompts have few slabs and would leave the CUs idle)
-  for (int item = tid + 256 * (int)blockIdx.y; item < n_pos * slots * vecs; item += 256 * (int)gridDim.y) {
+  // blockIdx.y takes every parts-th item of the slab (short prompts have few slabs and would leave the CUs idle)
+  for (int item = tid + 256 * (int)blockIdx.y; item < n_pos * slots * vecs; item += 256 * parts) {
     const int i0 = (item % vecs) * 8, slot = (item / vecs) % slots, e = item / (vecs * slots);
     const int pos = p_lo + e;
     _Float16 *src = qkv + (size_t)(pos - start_pos) * row_elems + (size_t)slot * hd;
@@ -1198,7 +1198,7 @@ __global__ void __launch_bounds__(256) prefill_rope_append_kernel(_Float16 *__re
   // v: channel ch of kv head kvh at the slab's positions
   const _Float16 *vsrc = qkv + (size_t)(hq + hkv) * hd;
   const bool whole = p_hi - p_lo == 8;
-  for (int idx = tid + 256 * (int)blockIdx.y; idx < hkv * hd; idx += 256 * (int)gridDim.y) {
+  for (int idx = tid + 256 * (int)blockIdx.y; idx < hkv * hd; idx += 256 * parts) {
     const int kvh = idx / hd, ch = idx % hd;
     _Float16 *dst = vc + (((size_t)kvh * (max_ctx / 8) + slab) * hd + ch) * 8;
     if (whole) {
@@ -1231,7 +1231,7 @@ int32_t launch_prefill_rope_append(_Float16 *qkv, int rows, int start_pos, int h
   int parts = 512 / slabs;  // about two workgroups per CU
   parts = parts < 1 ? 1 : (parts > 16 ? 16 : parts);
   hipLaunchKernelGGL(prefill_rope_append_kernel, dim3(slabs, parts), dim3(256), 0, s, qkv, rows, start_pos, hq, hkv, hd, theta, max_ctx,
-                     kc, vc);
+                     kc, vc, parts);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }

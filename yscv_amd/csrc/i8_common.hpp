@@ -50,7 +50,7 @@ struct I8Args {
   const int32_t *corr;
   const float *composite_v;
   float composite, y_zp, dq_scale;
-  int round_mode, lo, hi, mode;  // as I8Epilogue::mode
+  int16_t round_mode, lo, hi, mode;  // as I8Epilogue; 16 bits each for kCheapArgs
   int m, n, k;
   int lda;          // row stride of a in bytes (k, or kp for a padded copy)
   int ksteps;       // kp / 64
@@ -58,6 +58,8 @@ struct I8Args {
   int zp_mul;       // multiplies col_sum in the epilogue
   const float *a_zp_dev;  // null, or the uint8 zero point of A as an f32 in device memory (then zp_mul = 128 - that)
 };
+
+static_assert(sizeof(I8Args) + 2 * sizeof(int) <= kCheapArgs, "arguments of a launch");
 
 // Shapes whose tiles leave the ring kernel's grid short of the CUs (i8_ksplit.hip): 16-byte aligned a with an lda that is a
 // multiple of 64, m * lda below 2 GiB.

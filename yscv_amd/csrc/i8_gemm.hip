@@ -591,9 +591,9 @@ int32_t launch_i8_gemm(const void *a, int a_is_u8, int a_zp, const yscv_hip_i8_w
   p.composite_v = ep.composite_v;
   p.composite = ep.composite;
   p.y_zp = ep.y_zp;
-  p.round_mode = ep.round_mode;
-  p.lo = ep.lo;
-  p.hi = ep.hi;
+  p.round_mode = (int16_t)ep.round_mode;
+  p.lo = (int16_t)ep.lo;
+  p.hi = (int16_t)ep.hi;
   p.mode = ep.mode;
   p.dq_scale = ep.dq_scale;
   p.m = (int)m;

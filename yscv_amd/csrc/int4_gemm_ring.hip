@@ -43,17 +43,18 @@ struct RingArgs {
   void *y;
   int m, n;        // rows; end of the column range of this launch
   int col0, ldy;   // first column of this launch (a multiple of the tile width); row stride of y
-  int nt, kt, ktp;
+  int kt;          // 128-k tiles; a block's are stored in a multiple of four
   int chunks, chunk_div;
   int ldx;         // row stride of xh
   int stages;      // 64-k stages that hold data; the rows of xh reach to the end of the last one
-  int y_dtype;
-  int epi;         // EPI_STORE, EPI_ADD_F32 (y f32, y += product) or EPI_SWIGLU (y [m][n / 2] = silu(gate) * up, columns 2i / 2i+1)
+  int16_t y_dtype;
+  int16_t epi;     // EPI_STORE, EPI_ADD_F32 (y f32, y += product) or EPI_SWIGLU (y [m][n / 2] = silu(gate) * up, columns 2i / 2i+1)
   // K split (shapes with fewer tiles than CUs): the workgroups of split j multiply 128-k tiles j * kt_per .. and
   // stores its f32 products to partial[j][m][n]; ring_finalize_kernel adds the splits in order and applies `epi`
   float *partial;  // null: no split
   int kt_per, splits;  // splits == 1 and kt_per == kt without a split
 };
+static_assert(sizeof(RingArgs) + 2 * sizeof(int) <= kCheapArgs, "arguments of a launch");
 
 template <int N>
 __device__ __forceinline__ void g4_wait_vm() {
@@ -260,8 +261,8 @@ __global__ void __launch_bounds__(256 + 64 * NP) int4_gemm_ring_kernel(RingArgs 
     const uint8_t *wbase[WT], *sbase[WT], *zbase[WT];
 #pragma unroll
     for (int u = 0; u < WT; u++) {
-      const int nt = min(n0 / 16 + pw * WT + u, p.nt - 1);
-      wbase[u] = p.tiles + (size_t)nt * p.ktp * kTileBytes;
+      const int nt = min(n0 / 16 + pw * WT + u, (p.ldy + 15) / 16 - 1);
+      wbase[u] = p.tiles + (size_t)nt * ((p.kt + 3) & ~3) * kTileBytes;
       sbase[u] = reinterpret_cast<const uint8_t *>(p.tscales) + (size_t)nt * p.chunks * 16 * SC::SC_BYTES;
       zbase[u] = has_zp ? p.tzps + (size_t)nt * p.chunks * 16 * SC::ZP_BYTES : sbase[u];  // keeps the load count uniform
     }
@@ -511,10 +512,10 @@ __global__ void __launch_bounds__(256 + 64 * NP) int4_gemm_ring_kernel(RingArgs 
 
 // Adds the K splits of a launch in a fixed order and applies the epilogue: four columns per thread.
 __global__ void __launch_bounds__(256) ring_finalize_kernel(const float *__restrict__ partial, int splits, int m, int n, void *y,
-                                                            int y_dtype, int epi, int ldy) {
+                                                            int y_dtype, int epi, int ldy, int threads) {
   const int chunks = (n + 3) / 4;
   const size_t total = (size_t)m * chunks;
-  for (size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x; idx < total; idx += (size_t)gridDim.x * blockDim.x) {
+  for (size_t idx = blockIdx.x * (size_t)256 + threadIdx.x; idx < total; idx += threads) {
     const int row = (int)(idx / chunks), col = (int)(idx % chunks) * 4;
     const bool whole = col + 4 <= n && (n & 3) == 0;
     float4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -577,7 +578,7 @@ int32_t ring_launch_gm(const RingArgs &a, int gm, bool sf16, hipStream_t s) {
 int32_t launch_int4_partial_sum(const float *partial, int splits, int m, int n, void *y, int y_dtype, int epi, hipStream_t s) {
   const size_t work = (size_t)m * ((n + 3) / 4);
   const unsigned fb = (unsigned)std::min<size_t>((work + 255) / 256, 4096);
-  hipLaunchKernelGGL(ring_finalize_kernel, dim3(fb), dim3(256), 0, s, partial, splits, m, n, y, y_dtype, epi, n);
+  hipLaunchKernelGGL(ring_finalize_kernel, dim3(fb), dim3(256), 0, s, partial, splits, m, n, y, y_dtype, epi, n, (int)(fb * 256));
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
@@ -614,9 +615,7 @@ int32_t launch_int4_gemm_ring(const yscv_hip_int4_weight *w, const _Float16 *xh,
   a.n = (int)w->n;
   a.col0 = 0;
   a.ldy = (int)w->n;
-  a.nt = (int)w->nt;
   a.kt = (int)w->kt;
-  a.ktp = (int)w->ktp;
   a.chunks = (int)w->chunks;
   a.chunk_div = w->gm == GM128 ? (int)(w->g / 128) : 1;
   a.ldx = (int)k_pad;

@@ -42,16 +42,20 @@ __device__ __forceinline__ double sum_xor16_xor32(double v) {  // v + v[lane ^ 1
   return __hiloint2double(__float_as_int(xh), __float_as_int(xl)) + __hiloint2double(__float_as_int(yh), __float_as_int(yl));
 }
 
-struct GemvRowArgs {
+struct GemvPlainArgs {
   const uint8_t *tiles;
   const void *tscales;
   const uint8_t *tzps;
   const void *x;
   void *y;
   int m, n, k, nt, ktp, chunks, chunk_div;
-  int groups;              // groups of rows, waves / split blocks of 16 each
+  int groups, wgs;         // groups of rows, waves / split blocks of 16 each; workgroups that share them
   int slices, split_log2;  // 512-k slices of K; waves of a workgroup that share a block of 16 rows (1, 2, 4, 8 or 16)
   int y_dtype, epi;
+};
+static_assert(sizeof(GemvPlainArgs) <= kCheapArgs, "arguments of a launch");
+
+struct GemvRowArgs : GemvPlainArgs {
   // a norm folded into this call (NormFold in kernels.hpp); null / 0 when unused
   const float *gamma_next, *pre;
   _Float16 *xg;
@@ -63,7 +67,7 @@ struct GemvRowArgs {
 };
 
 // XD: type of the activations; f32 takes two MFMA operands, the others one.
-// EPI: residual update, SwiGLU or a folded norm; a plain one-row product leaves that code out (4096 x 4096 fp16 4.0 instead of 4.2 us,
+// EPI: residual update, SwiGLU or a folded norm; a plain product leaves that code and its arguments out (one row, 4096 x 4096 fp16 4.0 instead of 4.2 us,
 // 3000 x 704 f32 3.25 instead of 3.5: less to fetch at the start).
 // KEEP: a wave has one slice of K (K <= 4096).  Its activations stay in registers while the workgroup goes through its groups of
 // rows; without it a workgroup has one group and the waves go through their slices.
@@ -71,7 +75,11 @@ struct GemvRowArgs {
 constexpr int gemv_per_simd(int m, int xd, bool zp, bool keep) { return m == 4 || (m == 2 && (!keep || (zp && xd == YSCV_HIP_F32))) ? 2 : 4; }
 
 template <int M, int XD, int GM, bool SF16, bool HAS_ZP, bool KEEP, bool EPI>
-__global__ void __launch_bounds__((64 * gemv_waves(M, KEEP)), (gemv_per_simd(M, XD, HAS_ZP, KEEP))) int4_gemv_kernel(GemvRowArgs p) {
+__global__ void __launch_bounds__((64 * gemv_waves(M, KEEP)), (gemv_per_simd(M, XD, HAS_ZP, KEEP)))
+int4_gemv_kernel(typename std::conditional<EPI, GemvRowArgs, GemvPlainArgs>::type args) {
+  GemvRowArgs p;
+  if constexpr (EPI) p = args;
+  else static_cast<GemvPlainArgs &>(p) = args;
   constexpr int WAVES = gemv_waves(M, KEEP);
   if constexpr (!EPI) {
     p.epi = EPI_STORE;
@@ -300,7 +308,7 @@ __global__ void __launch_bounds__((64 * gemv_waves(M, KEEP)), (gemv_per_simd(M, 
   for (int i = 0; i < M; i++) nothing.v[i] = 0.0;
 
   if constexpr (KEEP) {  // two buffers: a wave past the barrier of group i + 1 has read the sums of group i
-    const int sl = min(ks, p.slices - 1), step = (int)gridDim.x;
+    const int sl = min(ks, p.slices - 1), step = p.wgs;
     const bool in = ks < p.slices;
     int group = (int)blockIdx.x, buf = 0;
     const Raw xr = load_x(sl);
@@ -338,7 +346,8 @@ __global__ void __launch_bounds__((64 * gemv_waves(M, KEEP)), (gemv_per_simd(M, 
 }
 
 template <int M, int XD, int GM, bool SF16, bool EPI>
-int32_t gemv_go(const GemvRowArgs &a, unsigned grid, hipStream_t s) {
+int32_t gemv_go(const GemvRowArgs &all, unsigned grid, hipStream_t s) {
+  const typename std::conditional<EPI, GemvRowArgs, GemvPlainArgs>::type &a = all;
   const bool keep = a.slices <= 8;
   const dim3 threads(64 * gemv_waves(M, keep));
   if (keep && a.tzps) hipLaunchKernelGGL((int4_gemv_kernel<M, XD, GM, SF16, true, true, EPI>), dim3(grid), threads, 0, s, a);
@@ -350,9 +359,7 @@ int32_t gemv_go(const GemvRowArgs &a, unsigned grid, hipStream_t s) {
 }
 template <int M, int XD, int GM, bool SF16>
 int32_t gemv_epi(const GemvRowArgs &a, unsigned grid, hipStream_t s) {
-  if constexpr (M == 1) {
-    if (a.epi == EPI_STORE && !a.ss_in) return gemv_go<M, XD, GM, SF16, false>(a, grid, s);
-  }
+  if (a.epi == EPI_STORE && !a.ss_in) return gemv_go<M, XD, GM, SF16, false>(a, grid, s);
   return gemv_go<M, XD, GM, SF16, true>(a, grid, s);
 }
 template <int M, int XD>
@@ -432,6 +439,7 @@ int32_t launch_int4_gemv(const yscv_hip_int4_weight *w, const void *x, int x_dty
                                                 : (x_dtype == YSCV_HIP_F32 && a.groups > 4 * num_cus ? 2 : 1);
     grid = (unsigned)((a.groups + rounds - 1) / rounds);
   }
+  a.wgs = (int)grid;
   const bool sf16 = w->scale_dtype == YSCV_HIP_F16;
   if (m == 1) return gemv_xd<1>(a, grid, x_dtype, w->gm, sf16, s);
   if (m == 2) return gemv_xd<2>(a, grid, x_dtype, w->gm, sf16, s);

@@ -35,10 +35,12 @@ struct KsArgs {
   const float *row_scale;  // null: 1
   void *y;
   float *partial;  // [parts][m][n] when K is also split over workgroups, else null
-  int m, n, nt, ktp, chunks, chunk_div, ldx, y_dtype, epi;
+  int m, n, nt, ktp, chunks, chunk_div, ldx;
+  int16_t y_dtype, epi;
   int kt, ksteps;  // 128-k tiles and 32-k steps that hold data
   int tiles_m, tiles_n, parts, kt_per;
 };
+static_assert(sizeof(KsArgs) <= kCheapArgs, "arguments of a launch");
 
 template <int GM, bool SF16>
 struct KsScale {

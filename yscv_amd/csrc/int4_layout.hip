@@ -168,12 +168,12 @@ template <bool VEC>
 __global__ void __launch_bounds__(1024) x_prep_kernel(const void *__restrict__ x, int x_dtype, size_t k,
                                                       size_t k_pad, int split, _Float16 *__restrict__ xh,
                                                       _Float16 *__restrict__ xl,
-                                                      float *__restrict__ row_scale) {
+                                                      float *__restrict__ row_scale, int threads) {
   __shared__ float red[16];
   const size_t row = blockIdx.x;
   const size_t base = row * k;
   const size_t chunks = k_pad / 8;
-  // pass 1: abs-max of the row.  The first sweep's values stay in registers for pass 2 (a row of up to 8 blockDim
+  // pass 1: abs-max of the row.  The first sweep's values stay in registers for pass 2 (a row of up to 8 threads
   // elements is read from memory once); longer rows re-read the rest.
   float amax = 0.0f;
   float v0[8];
@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(1024) x_prep_kernel(const void *__restrict__ x
   }
 #pragma unroll
   for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(v0[i]));  // NaN is ignored here, kept in the values
-  for (size_t ch = ch0 + blockDim.x; ch < chunks; ch += blockDim.x) {
+  for (size_t ch = ch0 + threads; ch < chunks; ch += threads) {
     if (ch * 8 < k) {
       float v[8];
       load8<VEC>(x, base + ch * 8, x_dtype, base + k, v);
@@ -199,7 +199,7 @@ __global__ void __launch_bounds__(1024) x_prep_kernel(const void *__restrict__ x
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
   __syncthreads();
   amax = 0.0f;
-  for (unsigned w = 0; w < (blockDim.x >> 6); w++) amax = fmaxf(amax, red[w]);
+  for (unsigned w = 0; w < ((unsigned)threads >> 6); w++) amax = fmaxf(amax, red[w]);
   int e = 14;
   if (amax > 0.0f && amax < 3.0e38f) {
     (void)frexpf(amax, &e);  // amax = f * 2^e, f in [0.5, 1)
@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(1024) x_prep_kernel(const void *__restrict__ x
   const float up = ldexpf(1.0f, shift);
   if (threadIdx.x == 0) row_scale[row] = ldexpf(1.0f, -shift);
   const size_t obase = row * k_pad;
-  for (size_t ch = ch0; ch < chunks; ch += blockDim.x) {
+  for (size_t ch = ch0; ch < chunks; ch += threads) {
     float v[8];
     if (ch == ch0) {
 #pragma unroll
@@ -308,10 +308,10 @@ int32_t launch_x_prep(const void *x, int x_dtype, size_t m, size_t k, size_t k_p
   unsigned threads = chunks >= 1024 ? 1024 : (unsigned)round_up(chunks < 64 ? 64 : chunks, 64);
   if (vec)
     hipLaunchKernelGGL(x_prep_kernel<true>, dim3((unsigned)m), dim3(threads), 0, s, x, x_dtype, k, k_pad, split,
-                       xh, xl, row_scale);
+                       xh, xl, row_scale, (int)threads);
   else
     hipLaunchKernelGGL(x_prep_kernel<false>, dim3((unsigned)m), dim3(threads), 0, s, x, x_dtype, k, k_pad,
-                       split, xh, xl, row_scale);
+                       split, xh, xl, row_scale, (int)threads);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }

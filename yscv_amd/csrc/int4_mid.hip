@@ -35,7 +35,9 @@ struct MidArgs {
   void *y;
   float *partial;  // [parts][m][n] when K is cut into parts, else null
   int m, n, nt, ktp, chunks, chunk_div, k, ldx, y_dtype, epi, ldy;
+  int wgs;  // workgroups of a part
 };
+static_assert(sizeof(MidArgs) <= kCheapArgs, "arguments of a launch");
 
 template <int GM, bool SF16>
 struct MidScale {
@@ -78,9 +80,9 @@ __global__ void __launch_bounds__(512, 1) int4_mid_kernel(MidArgs a) {
   NibbleConsts nc;
   nc.init();
 
-  // ---- weight stream of this wave: block `it` of the workgroup is 16-column block blockIdx.x + it * gridDim.x.  Tiles
+  // ---- weight stream of this wave: block `it` of the workgroup is 16-column block blockIdx.x + it * wgs.  Tiles
   // past the stored ones repeat the last one (their activations are zero), requests past the last block repeat it
-  const int stride = gridDim.x;
+  const int stride = a.wgs;
   const int iters = (a.nt - (int)blockIdx.x + stride - 1) / stride;  // >= 1, uniform in the workgroup
   int tl[TPWM], ch[TPWM];
 #pragma unroll
@@ -212,7 +214,7 @@ __global__ void __launch_bounds__(512, 1) int4_mid_kernel(MidArgs a) {
 }
 
 template <int RT, int TPWM, int GM, bool SF16, bool HAS_ZP, int P>
-int32_t mid_launch_one(const MidArgs &a, int parts, int cus, hipStream_t s) {
+int32_t mid_launch_one(MidArgs a, int parts, int cus, hipStream_t s) {
   constexpr int LDS = 2 * 8 * RT * 64 * 16;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
@@ -224,6 +226,7 @@ int32_t mid_launch_one(const MidArgs &a, int parts, int cus, hipStream_t s) {
     return set_error(YSCV_HIP_ERR_DEVICE, "cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(attr_err));
   int nparts = cus / parts;
   nparts = nparts < 1 ? 1 : (nparts > a.nt ? a.nt : nparts);
+  a.wgs = nparts;
   hipLaunchKernelGGL(kern, dim3((unsigned)nparts, (unsigned)parts), dim3(512), LDS, s, a);
   YSCV_HIP_TRY(hipGetLastError());
   if (a.partial != nullptr) return launch_int4_partial_sum(a.partial, parts, a.m, a.n, a.y, a.y_dtype, a.epi, s);

@@ -45,11 +45,9 @@ constexpr int TPW = 4;  // 128-k tiles per wave: 512 k of activations live in 64
 struct SkinnyArgs {
   const uint8_t *tiles;
   const void *tscales;
-  const uint8_t *tzps;  // null: zero point 8 everywhere
-  const _Float16 *xh;
-  const _Float16 *xl;
-  const float *xf;     // raw f32 activations for the kernels that split them themselves, else null
-  const uint16_t *xb;  // raw bf16 activations, else null
+  const uint8_t *tzps;     // null: zero point 8 everywhere
+  const void *x;           // fp16; XM 1: raw f32, XM 2: raw bf16
+  const _Float16 *xl;      // low parts of prepared f32
   const float *row_scale;
   void *y;
   float *partial;  // [ksg][m][n] when ksg > 1
@@ -58,11 +56,15 @@ struct SkinnyArgs {
   int chunks;      // scale chunks per 16-row block
   int chunk_div;   // GM128: tiles per scale chunk (group_size / 128)
   int k, ldx;      // K (a multiple of 32) and the row stride of the activations; the weights hold zeros behind K
-  int y_dtype;
+  int wgs;         // workgroups of a k-split slice
+  uint8_t y_dtype, epi;  // epi: EPI_STORE / EPI_ADD_F32 / EPI_SWIGLU
+  uint8_t waves;
   int ksg;
-  int epi;         // EPI_STORE / EPI_ADD_F32 / EPI_SWIGLU
-  int slices;      // ktp / TPW: number of wave-sized k slices that exist
-  // RMSNorm folded into the projections around it (NormFold in kernels.hpp); all null / 0 when unused
+};
+static_assert(sizeof(SkinnyArgs) <= kCheapArgs, "arguments of a launch");
+
+// RMSNorm folded into the projections around it (NormFold in kernels.hpp); all null / 0 when unused
+struct SkinnyFold {
   const float *gamma_next;  // producer: scale vector of the norm that follows the residual update
   const float *pre;         // producer: power of two per row, [m]
   _Float16 *xg;             // producer: fp16(h_new * gamma_next * pre[row]), [m][n]
@@ -119,8 +121,9 @@ constexpr int kStageRow = 512 * 2 + 64, kStageWave = 2 * 4 * kStageRow;
 constexpr int skinny_ub(int ni, int p) { return p % 4 == 0 ? 4 : (p % 2 == 0 && ni > 1 ? 2 : 1); }
 
 // XM: where the activations come from -- 0 prepared fp16 (hi [+ lo]), 1 raw f32 (split into hi + lo here), 2 raw bf16
-template <int SPLIT, int NI, int GM, bool SF16, bool HAS_ZP, int P, int XM>
-__global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
+// FOLD: a norm is folded into this call; other calls leave that code out
+template <int SPLIT, int NI, int GM, bool SF16, bool HAS_ZP, int P, int XM, bool FOLD>
+__device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
   constexpr bool RAWX = XM != 0;
   static_assert(XM != 1 || SPLIT == 2, "raw f32 activations are split into hi + lo");
   static_assert(XM != 2 || SPLIT == 1, "bf16 activations fit one fp16 operand exactly");
@@ -134,11 +137,14 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
   extern __shared__ float red[];  // [2][waves][UB][NI][64]
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int waves = blockDim.x >> 6;
+  const int waves = a.waves;
+  const float *xf = static_cast<const float *>(a.x);
+  const uint16_t *xb = static_cast<const uint16_t *>(a.x);
+  const _Float16 *xh = static_cast<const _Float16 *>(a.x);
   const int r = lane & 15;
   const int c = lane >> 4;
   const int slice = blockIdx.y * waves + wave;     // this wave's 512-k slice
-  const bool wave_active = slice < a.slices;       // trailing waves of the last k-split may be idle
+  const bool wave_active = slice < a.ktp / TPW;       // trailing waves of the last k-split may be idle
   const int t0 = (wave_active ? slice : 0) * TPW;  // first 128-k tile of the slice
   NibbleConsts nc;
   nc.init();
@@ -151,14 +157,14 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
   if constexpr (SPLIT == 2 && NI == 4) {
     const int r0 = (int)blockIdx.z * 16;
     a.m = min(16, a.m - r0);
-    if (a.xf) a.xf += (size_t)r0 * a.ldx;
-    a.xh += (size_t)r0 * a.ldx;
+    xf += (size_t)r0 * a.ldx;
+    xh += (size_t)r0 * a.ldx;
     a.xl += (size_t)r0 * a.ldx;
     if (a.row_scale) a.row_scale += r0;
     if (a.partial) a.partial += (size_t)r0 * a.n;
     a.y = static_cast<char *>(a.y) + (size_t)r0 * a.n * (a.y_dtype == YSCV_HIP_F32 ? 4 : 2);
   }
-  const int stride = gridDim.x;
+  const int stride = a.wgs;
   const size_t w_step = (size_t)stride * a.ktp * kTileBytes;
   const size_t s_step = (size_t)stride * a.chunks * 16 * SC_BYTES;
   const size_t z_step = (size_t)stride * a.chunks * 16 * SPT;
@@ -208,15 +214,15 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
   constexpr int kSsRowsPerWave = 4;  // rows wave, wave + waves, ...: the launcher checks that four per wave cover m
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   float ss_pre[kSsRowsPerWave][4], ss_scale[kSsRowsPerWave];
-  if (a.ss_in) {
+  if (FOLD && f.ss_in) {
 #pragma unroll
     for (int u = 0; u < kSsRowsPerWave; u++) {
       const int row = wave_u + u * waves;
-      ss_scale[u] = a.pre_in[min(row, a.m - 1)];
+      ss_scale[u] = f.pre_in[min(row, a.m - 1)];
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int j = 4 * lane + e;
-        ss_pre[u][e] = (row < a.m && j < a.ss_in_count) ? a.ss_in[(size_t)row * a.ss_in_stride + j] : 0.0f;
+        ss_pre[u][e] = (row < a.m && j < f.ss_in_count) ? f.ss_in[(size_t)row * f.ss_in_stride + j] : 0.0f;
       }
     }
   }
@@ -225,9 +231,9 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
   // reduction will need, requested now (their round trip would otherwise sit at the end of a one-block kernel)
   // (only in the instantiations with a ring of one or two blocks, where a residual update of a decode step lands and
   // registers are to spare)
-  constexpr bool PREFETCH_H = P <= 2;
+  constexpr bool PREFETCH_H = FOLD && P <= 2;
   float h_pre[2] = {0.0f, 0.0f}, g_pre[2] = {0.0f, 0.0f}, p_pre[2] = {0.0f, 0.0f};
-  if (PREFETCH_H && a.xg) {
+  if (PREFETCH_H && f.xg) {
 #pragma unroll
     for (int sl = 0; sl < 2; sl++) {
       const int q = wave_u + sl * waves;
@@ -235,10 +241,10 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
         const int u = q / NI, i = q % NI;
         const int col = ((int)blockIdx.x + u * stride) * 16 + r;
         const int mrow = c * NI + i;
-        if (col < a.n) g_pre[sl] = a.gamma_next[col];
+        if (col < a.n) g_pre[sl] = f.gamma_next[col];
         if (mrow < a.m && col < a.n) {
           h_pre[sl] = reinterpret_cast<const float *>(a.y)[(size_t)mrow * a.n + col];
-          p_pre[sl] = a.pre[mrow];
+          p_pre[sl] = f.pre[mrow];
         }
       }
     }
@@ -263,7 +269,7 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
       // bf16 activations straight from the caller: the wave scales its own 512-k slice of every row by a power of
       // two (abs-max to [2^14, 2^15)), which makes every bf16 value an exact fp16 one (8 significant bits; only
       // values below 2^-29 of the slice maximum are lost); the power of two is undone on the wave's partial sums.
-      const uint16_t *src = a.xb + (size_t)(valid ? mrow : 0) * a.ldx + c * 8;
+      const uint16_t *src = xb + (size_t)(valid ? mrow : 0) * a.ldx + c * 8;
       uint4_t raw[TPW][4];
       if (whole) {
         src += (size_t)t0 * 128;
@@ -328,7 +334,7 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
       const int srow = lane >> 4, q = lane & 15;
       const bool svalid = wave_active && srow < a.m;
       const bool k_in = t0 * 128 + q * 32 < a.k;
-      const float *src = a.xf + (size_t)(svalid ? srow : 0) * a.ldx + (k_in ? t0 * 128 + q * 32 : 0);
+      const float *src = xf + (size_t)(svalid ? srow : 0) * a.ldx + (k_in ? t0 * 128 + q * 32 : 0);
       float4_t raw[8];
 #pragma unroll
       for (int e = 0; e < 8; e++) raw[e] = *reinterpret_cast<const float4_t *>(src + 4 * e);
@@ -387,7 +393,7 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
       // Idle lanes read row 0 and discard it: every load is unconditional, so all of them are in flight together
       // instead of one round trip per guarded load.
       // (K a multiple of 512: the launcher checks)
-      const float *src = a.xf + (size_t)(valid ? mrow : 0) * a.ldx + (size_t)t0 * 128 + c * 8;
+      const float *src = xf + (size_t)(valid ? mrow : 0) * a.ldx + (size_t)t0 * 128 + c * 8;
       float amax = 0.0f;
 #pragma unroll
       for (int t = 0; t < TPW; t++)
@@ -440,7 +446,7 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
 #pragma unroll
           for (int j = 0; j < 4; j++) {
             const size_t off = row_off + (size_t)(t0 + t) * 128 + j * 32;
-            xa[t][j][0] = *reinterpret_cast<const half8_t *>(a.xh + off);
+            xa[t][j][0] = *reinterpret_cast<const half8_t *>(xh + off);
             if constexpr (SPLIT == 2) xa[t][j][1] = *reinterpret_cast<const half8_t *>(a.xl + off);
           }
       } else {
@@ -449,7 +455,7 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
 #pragma unroll
           for (int j = 0; j < 4; j++) {
             const size_t off = row_off + block_k(t, j);
-            xa[t][j][0] = *reinterpret_cast<const half8_t *>(a.xh + off);
+            xa[t][j][0] = *reinterpret_cast<const half8_t *>(xh + off);
             if constexpr (SPLIT == 2) xa[t][j][1] = *reinterpret_cast<const half8_t *>(a.xl + off);
           }
 #pragma unroll
@@ -479,17 +485,17 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
   // then a fixed tree of DPP moves and lane swaps: the same order in every run); the sixteen factors meet in LDS
   // behind the barrier of the first reduction, which every use of them follows.
   float *rs_lds = red + (size_t)2 * waves * (UB * NI) * 64;
-  if (a.ss_in) {
+  if (FOLD && f.ss_in) {
 #pragma unroll
     for (int u = 0; u < kSsRowsPerWave; u++) {
       const int row = wave_u + u * waves;
       if (row < a.m) {  // uniform in the wave
         const float t = wave_sum((ss_pre[u][0] + ss_pre[u][1]) + (ss_pre[u][2] + ss_pre[u][3]));
-        const float inv_rms = 1.0f / sqrtf(t * a.ss_inv_d + a.ss_eps);
+        const float inv_rms = 1.0f / sqrtf(t * f.ss_inv_d + f.ss_eps);
         if (lane == 0) {
           rs_lds[row] = inv_rms / ss_scale[u];
           // one workgroup leaves the scale of the next residual update behind (every workgroup holds the same bits)
-          if (a.pre_next && blockIdx.x == 0 && blockIdx.y == 0) a.pre_next[row] = norm_fold_prescale(inv_rms);
+          if (f.pre_next && blockIdx.x == 0 && blockIdx.y == 0) f.pre_next[row] = norm_fold_prescale(inv_rms);
         }
       }
     }
@@ -654,9 +660,9 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
         float rsv = rs[0];
 #pragma unroll
         for (int ii = 1; ii < NI; ii++) rsv = (i == ii) ? rs[ii] : rsv;
-        if (a.ss_in) rsv = rs_lds[min(mrow, a.m - 1)];
+        if (FOLD && f.ss_in) rsv = rs_lds[min(mrow, a.m - 1)];
         v *= rsv;
-        if (a.epi == EPI_ADD_F32 && a.xg) {
+        if (FOLD && a.epi == EPI_ADD_F32 && f.xg) {
           // residual update that also feeds the next norm: h_new, its fp16 image times gamma and the row's power of
           // two, and the sum of h_new^2 over the sixteen columns of this block (the lanes r = 0..15 of a lane group),
           // one per row
@@ -665,15 +671,15 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
             float *hp = reinterpret_cast<float *>(a.y) + (size_t)mrow * a.n + col;
             const bool pre = PREFETCH_H && ex == 0 && slot >= 0 && slot < 2;  // requested at the start of the kernel
             const float hold = pre ? (slot == 0 ? h_pre[0] : h_pre[1]) : *hp;
-            const float gam = pre ? (slot == 0 ? g_pre[0] : g_pre[1]) : a.gamma_next[col];
-            const float pw = pre ? (slot == 0 ? p_pre[0] : p_pre[1]) : a.pre[mrow];
+            const float gam = pre ? (slot == 0 ? g_pre[0] : g_pre[1]) : f.gamma_next[col];
+            const float pw = pre ? (slot == 0 ? p_pre[0] : p_pre[1]) : f.pre[mrow];
             hn = hold + v;
             *hp = hn;
             const float gx = fminf(fmaxf(hn * gam * pw, -65504.0f), 65504.0f);
-            a.xg[(size_t)mrow * a.n + col] = (_Float16)gx;
+            f.xg[(size_t)mrow * a.n + col] = (_Float16)gx;
           }
           const float sq = row_sum16(hn * hn);
-          if (r == 0 && mrow < a.m && (nt0 + u * stride) < a.nt) a.ss_out[(size_t)mrow * a.ss_out_stride + (nt0 + u * stride)] = sq;
+          if (r == 0 && mrow < a.m && (nt0 + u * stride) < a.nt) f.ss_out[(size_t)mrow * f.ss_out_stride + (nt0 + u * stride)] = sq;
           return;
         }
         if (a.epi == EPI_SWIGLU) {
@@ -784,14 +790,22 @@ __global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
   }
 }
 
+template <int SPLIT, int NI, int GM, bool SF16, bool HAS_ZP, int P, int XM>
+__global__ void __launch_bounds__(512, 1) int4_skinny_kernel(SkinnyArgs a) {
+  skinny_body<SPLIT, NI, GM, SF16, HAS_ZP, P, XM, false>(a, SkinnyFold{});
+}
+template <int NI, int GM, int P>
+__global__ void __launch_bounds__(512, 1) int4_skinny_fold_kernel(SkinnyArgs a, SkinnyFold f) {
+  skinny_body<1, NI, GM, true, false, P, 0, true>(a, f);
+}
+
 // partial [ksg][m][n] -> y, fixed summation order, same epilogues as the fused path
-__global__ void int4_skinny_finalize_kernel(const float *__restrict__ partial, int ksg, int m, int n,
-                                            const float *__restrict__ row_scale, void *y, int y_dtype, int epi) {
+__global__ void __launch_bounds__(256) int4_skinny_finalize_kernel(const float *__restrict__ partial, int ksg, int m, int n,
+                                            const float *__restrict__ row_scale, void *y, int y_dtype, int epi, int threads) {
   const size_t total = (size_t)m * n;
   if (epi == EPI_SWIGLU) {
     const size_t half_n = (size_t)(n >> 1);
-    for (size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x; idx < (size_t)m * half_n;
-         idx += (size_t)gridDim.x * blockDim.x) {
+    for (size_t idx = blockIdx.x * (size_t)256 + threadIdx.x; idx < (size_t)m * half_n; idx += threads) {
       const size_t row = idx / half_n, j = idx % half_n;
       float g = 0.0f, u = 0.0f;
       for (int s = 0; s < ksg; s++) {
@@ -806,8 +820,7 @@ __global__ void int4_skinny_finalize_kernel(const float *__restrict__ partial, i
     }
     return;
   }
-  for (size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (size_t)gridDim.x * blockDim.x) {
+  for (size_t idx = blockIdx.x * (size_t)256 + threadIdx.x; idx < total; idx += threads) {
     // issue the loads of this element together (one memory round trip), the residual it is added to included, then
     // add in slice order
     float p[8];
@@ -886,11 +899,11 @@ static unsigned skinny_groups(const SkinnyArgs &a) {
 }
 
 template <int SPLIT, int NI, int GM, bool SF16, bool HAS_ZP, int P>
-static int32_t launch_p(const SkinnyArgs &a, const SkinnyPlan &plan, hipStream_t s) {
+static int32_t launch_p(const SkinnyArgs &a, const SkinnyPlan &plan, bool xraw, const SkinnyFold *fold, hipStream_t s) {
   constexpr int UB = skinny_ub(NI, P);
   const size_t lds = (size_t)2 * plan.waves * UB * NI * 64 * sizeof(float) + 64;  // + the sixteen row factors of a folded norm
   if constexpr (SPLIT == 2) {
-    if (a.xf != nullptr) {
+    if (xraw) {
       const size_t stage = NI == 1 ? (size_t)plan.waves * kStageWave : 0;
       if (stage > 0) {  // 8 waves: 68 KB, above the default dynamic-LDS limit
         static std::once_flag once;
@@ -908,11 +921,18 @@ static int32_t launch_p(const SkinnyArgs &a, const SkinnyPlan &plan, hipStream_t
       return YSCV_HIP_OK;
     }
   } else {
-    if (a.xb != nullptr) {
+    if (xraw) {
       hipLaunchKernelGGL((int4_skinny_kernel<SPLIT, NI, GM, SF16, HAS_ZP, P, 2>), dim3(plan.grid_x, plan.ksg, skinny_groups<SPLIT, NI>(a)),
                          dim3(plan.waves * 64), lds, s, a);
       YSCV_HIP_TRY(hipGetLastError());
       return YSCV_HIP_OK;
+    }
+    if constexpr (SF16 && !HAS_ZP) {
+      if (fold) {
+        hipLaunchKernelGGL((int4_skinny_fold_kernel<NI, GM, P>), dim3(plan.grid_x, plan.ksg), dim3(plan.waves * 64), lds, s, a, *fold);
+        YSCV_HIP_TRY(hipGetLastError());
+        return YSCV_HIP_OK;
+      }
     }
   }
   hipLaunchKernelGGL((int4_skinny_kernel<SPLIT, NI, GM, SF16, HAS_ZP, P, 0>), dim3(plan.grid_x, plan.ksg, skinny_groups<SPLIT, NI>(a)),
@@ -922,13 +942,13 @@ static int32_t launch_p(const SkinnyArgs &a, const SkinnyPlan &plan, hipStream_t
 }
 
 template <int SPLIT, int NI, int GM, bool SF16, bool HAS_ZP>
-static int32_t launch_one(const SkinnyArgs &a, const SkinnyPlan &plan, hipStream_t s) {
+static int32_t launch_one(const SkinnyArgs &a, const SkinnyPlan &plan, bool xraw, const SkinnyFold *fold, hipStream_t s) {
   // ring depth: bounded by the VGPR budget (activations: 64 per split, ring: ~26 per slot)
   if constexpr (SPLIT == 2 && NI == 1) {
     // two slots fit only with a few spilled registers, whose cost a workgroup recovers over sixteen or more blocks
     const int blocks_per_wg = (a.nt + plan.grid_x - 1) / plan.grid_x;
-    if (blocks_per_wg < 16) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 1>(a, plan, s);
-    return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 2>(a, plan, s);
+    if (blocks_per_wg < 16) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 1>(a, plan, xraw, fold, s);
+    return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 2>(a, plan, xraw, fold, s);
   } else {
     constexpr int P = SPLIT == 2 ? 1 : (SF16 && !HAS_ZP ? 4 : 3);
     if constexpr (SPLIT == 1) {
@@ -937,25 +957,25 @@ static int32_t launch_one(const SkinnyArgs &a, const SkinnyPlan &plan, hipStream
       // CU's memory pipeline for sixteen cycles whatever it asks for, and with one block three quarters of the ring
       // fill would be such fillers (2 of the 8 us of an output projection at m = 16).
       const int blocks_per_wg = (a.nt + plan.grid_x - 1) / plan.grid_x;
-      if (blocks_per_wg == 1) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 1>(a, plan, s);
-      if (blocks_per_wg == 2) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 2>(a, plan, s);
+      if (blocks_per_wg == 1) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 1>(a, plan, xraw, fold, s);
+      if (blocks_per_wg == 2) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 2>(a, plan, xraw, fold, s);
     }
-    return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, P>(a, plan, s);
+    return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, P>(a, plan, xraw, fold, s);
   }
 }
 
 template <int SPLIT, int NI, int GM>
-static int32_t launch_sz(const SkinnyArgs &a, const SkinnyPlan &plan, bool sf16, bool has_zp, hipStream_t s) {
+static int32_t launch_sz(const SkinnyArgs &a, const SkinnyPlan &plan, bool sf16, bool has_zp, bool xraw, const SkinnyFold *fold, hipStream_t s) {
   if (sf16)
-    return has_zp ? launch_one<SPLIT, NI, GM, true, true>(a, plan, s) : launch_one<SPLIT, NI, GM, true, false>(a, plan, s);
-  return has_zp ? launch_one<SPLIT, NI, GM, false, true>(a, plan, s) : launch_one<SPLIT, NI, GM, false, false>(a, plan, s);
+    return has_zp ? launch_one<SPLIT, NI, GM, true, true>(a, plan, xraw, fold, s) : launch_one<SPLIT, NI, GM, true, false>(a, plan, xraw, fold, s);
+  return has_zp ? launch_one<SPLIT, NI, GM, false, true>(a, plan, xraw, fold, s) : launch_one<SPLIT, NI, GM, false, false>(a, plan, xraw, fold, s);
 }
 
 template <int SPLIT, int NI>
-static int32_t launch_gm(const SkinnyArgs &a, const SkinnyPlan &plan, int gm, bool sf16, bool has_zp, hipStream_t s) {
-  if (gm == GM32) return launch_sz<SPLIT, NI, GM32>(a, plan, sf16, has_zp, s);
-  if (gm == GM64) return launch_sz<SPLIT, NI, GM64>(a, plan, sf16, has_zp, s);
-  return launch_sz<SPLIT, NI, GM128>(a, plan, sf16, has_zp, s);
+static int32_t launch_gm(const SkinnyArgs &a, const SkinnyPlan &plan, int gm, bool sf16, bool has_zp, bool xraw, const SkinnyFold *fold, hipStream_t s) {
+  if (gm == GM32) return launch_sz<SPLIT, NI, GM32>(a, plan, sf16, has_zp, xraw, fold, s);
+  if (gm == GM64) return launch_sz<SPLIT, NI, GM64>(a, plan, sf16, has_zp, xraw, fold, s);
+  return launch_sz<SPLIT, NI, GM128>(a, plan, sf16, has_zp, xraw, fold, s);
 }
 
 int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan, const _Float16 *xh,
@@ -971,10 +991,8 @@ int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan
   a.tiles = w->tiles;
   a.tscales = w->tscales;
   a.tzps = w->has_zp ? w->tzps : nullptr;
-  a.xh = xh;
+  a.x = xraw ? xraw : xh;
   a.xl = xl;
-  a.xf = split == 2 ? static_cast<const float *>(xraw) : nullptr;
-  a.xb = split == 1 ? static_cast<const uint16_t *>(xraw) : nullptr;
   a.row_scale = row_scale;
   a.y = y;
   a.partial = partial;
@@ -986,35 +1004,32 @@ int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan
   a.chunk_div = w->gm == GM128 ? (int)(w->g / 128) : 1;
   a.k = (int)w->k;
   a.ldx = (int)ldx;
-  a.y_dtype = y_dtype;
+  a.y_dtype = (uint8_t)y_dtype;
   a.ksg = plan.ksg;
-  a.epi = epi;
-  a.slices = (int)(w->ktp / TPW);
-  a.gamma_next = nullptr;
-  a.xg = nullptr;
-  a.pre = a.pre_in = nullptr;
-  a.pre_next = nullptr;
-  a.ss_out = nullptr;
-  a.ss_out_stride = 0;
-  a.ss_in = nullptr;
-  a.ss_in_count = a.ss_in_stride = 0;
-  a.ss_inv_d = a.ss_eps = 0.0f;
+  a.epi = (uint8_t)epi;
+  a.wgs = plan.grid_x;
+  a.waves = (uint8_t)plan.waves;
+  SkinnyFold f = {};
+  const SkinnyFold *fold = nullptr;
   const bool produce = nf && nf->xg != nullptr;
   if (produce && row_scale) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "folded norm: the producing call takes activations as they are");
   if (nf) {
+    if (w->has_zp || w->scale_dtype != YSCV_HIP_F16)
+      return set_error(YSCV_HIP_ERR_UNSUPPORTED, "folded norm: weights with fp16 scales and no zero points, as a decoder's are");
     if (nf->ss_in) {
       if (plan.ksg > 1) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "folded norm: the consuming projection must not be K-split");
       if (m > (size_t)4 * plan.waves || nf->ss_in_count > 256)
         return set_error(YSCV_HIP_ERR_UNSUPPORTED, "folded norm: %zu rows on %d waves, %d partial sums per row", m, plan.waves, nf->ss_in_count);
       if (split != 1 || xraw) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "folded norm: fp16 activations only");
       if (!nf->pre_in) return set_error(YSCV_HIP_ERR_INVALID_ARG, "folded norm: the row scales of the activations are missing");
-      a.ss_in = nf->ss_in;
-      a.pre_in = nf->pre_in;
-      a.pre_next = nf->pre_next;
-      a.ss_in_count = nf->ss_in_count;
-      a.ss_in_stride = nf->ss_in_stride;
-      a.ss_inv_d = nf->inv_d;
-      a.ss_eps = nf->eps;
+      fold = &f;
+      f.ss_in = nf->ss_in;
+      f.pre_in = nf->pre_in;
+      f.pre_next = nf->pre_next;
+      f.ss_in_count = nf->ss_in_count;
+      f.ss_in_stride = nf->ss_in_stride;
+      f.ss_inv_d = nf->inv_d;
+      f.ss_eps = nf->eps;
     }
     if (produce) {
       if (epi != EPI_ADD_F32 || !nf->gamma_next || !nf->ss_out || !nf->ss_out_count || !nf->pre)
@@ -1025,11 +1040,12 @@ int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan
         *nf->ss_out_count = (int)(w->n / 256);
       } else {
         if (nf->ss_out_stride < (int)w->nt) return set_error(YSCV_HIP_ERR_INVALID_ARG, "folded norm: room for %zu partial sums per row", w->nt);
-        a.gamma_next = nf->gamma_next;
-        a.pre = nf->pre;
-        a.xg = nf->xg;
-        a.ss_out = nf->ss_out;
-        a.ss_out_stride = nf->ss_out_stride;
+        fold = &f;
+        f.gamma_next = nf->gamma_next;
+        f.pre = nf->pre;
+        f.xg = nf->xg;
+        f.ss_out = nf->ss_out;
+        f.ss_out_stride = nf->ss_out_stride;
         *nf->ss_out_count = (int)w->nt;
       }
     }
@@ -1041,11 +1057,11 @@ int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan
   const bool small = m <= 4;
   int32_t st;
   if (split == 2)
-    st = small ? launch_gm<2, 1>(a, plan, w->gm, sf16, w->has_zp, s) : launch_gm<2, 4>(a, plan, w->gm, sf16, w->has_zp, s);
+    st = small ? launch_gm<2, 1>(a, plan, w->gm, sf16, w->has_zp, xraw != nullptr, fold, s) : launch_gm<2, 4>(a, plan, w->gm, sf16, w->has_zp, xraw != nullptr, fold, s);
   else if (m > 4 && m <= 8)  // two accumulators per lane: half the scale FMAs and half the exchange of the 16-row form
-    st = launch_gm<1, 2>(a, plan, w->gm, sf16, w->has_zp, s);
+    st = launch_gm<1, 2>(a, plan, w->gm, sf16, w->has_zp, xraw != nullptr, fold, s);
   else
-    st = small ? launch_gm<1, 1>(a, plan, w->gm, sf16, w->has_zp, s) : launch_gm<1, 4>(a, plan, w->gm, sf16, w->has_zp, s);
+    st = small ? launch_gm<1, 1>(a, plan, w->gm, sf16, w->has_zp, xraw != nullptr, fold, s) : launch_gm<1, 4>(a, plan, w->gm, sf16, w->has_zp, xraw != nullptr, fold, s);
   YSCV_TRY(st);
   if (plan.ksg > 1 && produce) {
     hipLaunchKernelGGL(int4_skinny_finalize_norm_kernel, dim3((unsigned)(m * (w->n / 256))), dim3(256), 0, s, partial, plan.ksg,
@@ -1058,7 +1074,7 @@ int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan
     int blocks = (int)ceil_div(total, (size_t)256);
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(int4_skinny_finalize_kernel, dim3(blocks), dim3(256), 0, s, partial, plan.ksg,
-                       (int)m, (int)w->n, row_scale, y, y_dtype, epi);
+                       (int)m, (int)w->n, row_scale, y, y_dtype, epi, blocks * 256);
     YSCV_HIP_TRY(hipGetLastError());
   }
   return YSCV_HIP_OK;

@@ -118,8 +118,8 @@ constexpr int DQL_BLOCKS = 1024;
 
 // the values of x this thread takes, f(index, value) for each of them, in batches of four loads
 template <bool VEC, typename F>
-__device__ __forceinline__ void dql_each(const float *__restrict__ x, size_t len, F f) {
-  const size_t step = (size_t)gridDim.x * blockDim.x, first = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+__device__ __forceinline__ void dql_each(const float *__restrict__ x, size_t len, int blocks, F f) {
+  const size_t step = (size_t)blocks * 256, first = blockIdx.x * (size_t)256 + threadIdx.x;
   if constexpr (VEC) {
     const size_t n4 = len / 4;
     for (size_t i = first; i < n4; i += 4 * step) {
@@ -137,14 +137,14 @@ __device__ __forceinline__ void dql_each(const float *__restrict__ x, size_t len
 
 template <bool VEC>
 __global__ void __launch_bounds__(256) dql_minmax_kernel(const float *__restrict__ x, size_t len,
-                                                         float *__restrict__ minmax) {
+                                                         float *__restrict__ minmax, int blocks) {
   __shared__ float smin[4], smax[4];
   float mn = 3.40282347e+38f, mx = -3.40282347e+38f;
   auto take = [&](float v) {
     if (v < mn) mn = v;  // comparisons, not fmin: NaN never wins, as in misc.rs:250-256
     if (v > mx) mx = v;
   };
-  dql_each<VEC>(x, len, [&](size_t, const auto &v) {
+  dql_each<VEC>(x, len, blocks, [&](size_t, const auto &v) {
     if constexpr (VEC) {
 #pragma unroll
       for (int e = 0; e < 4; e++) take(v[e]);
@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(256) dql_quantize_kernel(const float *__restri
                                                            float *__restrict__ zp_out) {
   __shared__ float smin[4], smax[4];
   float mn = 3.40282347e+38f, mx = -3.40282347e+38f;
-  for (int i = threadIdx.x; i < nparts; i += blockDim.x) {
+  for (int i = threadIdx.x; i < nparts; i += 256) {
     float a = minmax[2 * i], b = minmax[2 * i + 1];
     if (a < mn) mn = a;
     if (b > mx) mx = b;
@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(256) dql_quantize_kernel(const float *__restri
     *zp_out = zp;
   }
   auto one = [&](float v) { return (uint8_t)clamp_cast(round_half_away_f(__fadd_rn(__fdiv_rn(v, scale), zp)), 0.0f, 255.0f); };
-  dql_each<VEC>(x, len, [&](size_t i, const auto &v) {
+  dql_each<VEC>(x, len, nparts, [&](size_t i, const auto &v) {
     if constexpr (VEC) {
       typedef T vec4 __attribute__((ext_vector_type(4)));
       reinterpret_cast<vec4 *>(y)[i] = vec4{(T)one(v[0]), (T)one(v[1]), (T)one(v[2]), (T)one(v[3])};
@@ -238,7 +238,7 @@ int32_t launch_dynamic_quantize_linear(const float *x, size_t len, void *y, bool
   const bool vec = len % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
   auto go = [&](auto VEC) -> int32_t {
     constexpr bool V = decltype(VEC)::value;
-    hipLaunchKernelGGL(dql_minmax_kernel<V>, dim3(blocks), dim3(256), 0, s, x, len, partial);
+    hipLaunchKernelGGL(dql_minmax_kernel<V>, dim3(blocks), dim3(256), 0, s, x, len, partial, blocks);
     YSCV_HIP_TRY(hipGetLastError());
     if (y_f32)
       hipLaunchKernelGGL((dql_quantize_kernel<float, V>), dim3(blocks), dim3(256), 0, s, x, len, partial, blocks, static_cast<float *>(y), scale_out, zp_out);
