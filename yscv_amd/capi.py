@@ -170,6 +170,9 @@ _SPECIAL = {
     "yscv_hip_should_prepack_i8_b": ([_sz, _sz], _i32),
 }
 
+# what _calls.so (csrc/calls.cpp) calls without ctypes, in the order of its bind()
+_DIRECT_CALLS = ("int4_matmul", "int8_matmul", "int8_matmul_requant", "exec_dql_matmul_integer", "rms_norm_dev", "gqa_attention_dev")
+
 EXPORTED_SYMBOLS = sorted(list(_SIGNATURES) + list(_SPECIAL))
 
 _lib = None
@@ -202,12 +205,16 @@ class _Checked:
             fn.restype = restype
             setattr(self, name[len("yscv_hip_"):], fn)
 
+    def fail(self, st):
+        """Raises what a status other than 0 stands for (the text is the calling thread's)."""
+        msg = self._cdll.yscv_hip_last_error()
+        raise YscvHipError(st, msg.decode() if msg else "")
+
     def _wrap(self, fn):
         def call(*args):
             st = fn(*args)
             if st != 0:
-                msg = self._cdll.yscv_hip_last_error()
-                raise YscvHipError(st, msg.decode() if msg else "")
+                self.fail(st)
             return st
 
         call.raw = fn
@@ -226,5 +233,9 @@ def lib() -> _Checked:
         # only one, and torch's must be the one that is loaded first or torch loses the GPU.
         import torch  # noqa: F401
 
-        _lib = _Checked(C.CDLL(_LIB_PATH))
+        from . import _calls
+
+        checked = _Checked(C.CDLL(_LIB_PATH))
+        _calls.bind(*(C.cast(getattr(checked, name).raw, _vp).value for name in _DIRECT_CALLS))
+        _lib = checked
     return _lib

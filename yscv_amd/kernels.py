@@ -12,7 +12,7 @@ import ctypes as C
 import numpy as np
 import torch
 
-from . import capi
+from . import _calls, capi
 from .capi import (BF16, EPILOGUE_ADD_F32, EPILOGUE_STORE, EPILOGUE_SWIGLU, F16, F32, NIBBLE_SIGNED, NIBBLE_UNSIGNED,
                    ROUND_HALF_AWAY, ROUND_TIES_EVEN, lib, stream_ptr)
 
@@ -250,7 +250,11 @@ class PackedInt4Weight:
         x.shape[:-1] + [m_w], like exec_matmul's int4 branch (runner/linear.rs:269-270).  With `workspace` (a CUDA
         uint8 tensor of at least workspace_bytes(m, x.dtype), 256-byte aligned) the call allocates nothing
         (yscv_hip_int4_matmul_ws, mode auto only)."""
-        # (pointers and sizes go to ctypes as plain integers: at decode sizes the call is as long as its host side)
+        # (at decode sizes the call is as long as its host side: the usual one is a single native step)
+        if out is None and out_dtype is None and workspace is None and mode == "auto":
+            y = _calls.int4_matmul(self._h, x, self.k, self.m_w)
+            if y is not None:
+                return y if y.__class__ is not int else lib().fail(y)
         shape = x.shape
         assert x.is_cuda and shape[-1] == self.k
         x = x.contiguous()
@@ -331,6 +335,10 @@ class PackedI8B:
 
     def matmul(self, a, a_zp: int = 0, out=None):
         """a: CUDA tensor [m][k] int8 or uint8 -> int32 [m][n] (exact)."""
+        if out is None:
+            y = _calls.int8_matmul(self._h, a, self._k, self._n, a_zp)
+            if y is not None:
+                return y if y.__class__ is not int else lib().fail(y)
         assert a.is_cuda and a.dim() == 2 and a.shape[1] == self._k and a.dtype in (torch.int8, torch.uint8)
         a = a.contiguous()
         m = a.shape[0]
@@ -341,6 +349,10 @@ class PackedI8B:
 
     def matmul_requant(self, a, a_zp, composite, y_zp, round_mode, clamp_lo, clamp_hi, corr=None, out=None):
         """Fused GEMM + requantize.  composite: float or CUDA f32 tensor [n]; corr: CUDA i32 [n] or None."""
+        if out is None and corr is None:
+            y = _calls.int8_requant(self._h, a, self._k, self._n, a_zp, composite, y_zp, round_mode, clamp_lo, clamp_hi)
+            if y is not None:
+                return y if y.__class__ is not int else lib().fail(y)
         assert a.is_cuda and a.dim() == 2 and a.shape[1] == self._k and a.dtype in (torch.int8, torch.uint8)
         a = a.contiguous()
         m = a.shape[0]

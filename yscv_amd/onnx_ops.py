@@ -13,6 +13,7 @@ from dataclasses import dataclass
 
 import torch
 
+from . import _calls
 from .capi import PATH_FALLBACK_EXACT, PATH_FALLBACK_F32, PATH_FAST, QuantStats, lib, stream_ptr  # noqa: F401
 
 _sz = C.c_size_t
@@ -141,6 +142,9 @@ def exec_qdq_matmul(x, a_scale, prepacked: PrepackedI8B, b_scale, y_scale, y_zp:
 
 def exec_dql_matmul_integer(x, prepacked: PrepackedI8B):
     """DynamicQuantizeLinear -> MatMulInteger (b_zero_point 0) in one call.  Returns (out [m][n] f32, y_scale [1], y_zp [1])."""
+    y = _calls.dql_matmul(prepacked.handle, x, prepacked.k, prepacked.n)
+    if y is not None:
+        return y if y.__class__ is not int else lib().fail(y)
     x = _dev_f32(x, "x")
     if x.dim() != 2 or int(x.shape[1]) != prepacked.k:
         raise ValueError("x must be [m][k] with k matching the prepacked weight")
@@ -255,6 +259,9 @@ def exec_dynamic_quantize_linear(x):
 # ---- the operators between the MatMuls of an LLM graph (device tensors in, device tensors out) ----------------------
 def rms_norm(x, gamma, eps: float):
     """rms_norm_last_dim (crates/yscv-kernels/src/ops/norm.rs:1431-1518) over the last axis of a CUDA f32 tensor."""
+    y = _calls.rms_norm(x, gamma, eps)
+    if y is not None:
+        return y if y.__class__ is not int else lib().fail(y)
     x = _dev_f32(x, "x")
     gamma = _dev_f32(gamma, "gamma")
     d = x.shape[-1]
@@ -279,8 +286,11 @@ def apply_rotary_embedding(q, k, num_q_heads: int, num_kv_heads: int, d_head: in
 def exec_grouped_query_attention(q, k, v, num_heads: int, kv_num_heads: int | None = None):
     """exec_grouped_query_attention (crates/yscv-onnx/src/runner/linear.rs:552-646): q [B][Sq][Hq d], k / v [B][Sk][Hkv d]
     CUDA f32 tensors -> [B][Sq][Hq d]."""
-    q, k, v = _dev_f32(q, "q"), _dev_f32(k, "k"), _dev_f32(v, "v")
     kv_num_heads = num_heads if kv_num_heads is None else kv_num_heads
+    y = _calls.gqa(q, k, v, num_heads, kv_num_heads)
+    if y is not None:
+        return y if y.__class__ is not int else lib().fail(y)
+    q, k, v = _dev_f32(q, "q"), _dev_f32(k, "k"), _dev_f32(v, "v")
     B, Sq, Sk = q.shape[0], q.shape[1], k.shape[1]
     d_head = q.shape[2] // num_heads
     if k.shape != (B, Sk, kv_num_heads * d_head) or v.shape != k.shape or q.shape[2] != num_heads * d_head:
