@@ -1,0 +1,55 @@
+"""Attention of a decode step over the fp16 cache (csrc/decode_attention.hip) where it can go wrong: one share, the edges of shares and of
+blocks of 32, merges over several levels, more than sixteen query heads per kv head; against a float64 softmax over the cache rows and the
+rotated q that the decoder itself reports."""
+import math
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _decoder(heads, batch, max_ctx):
+    from yscv_amd.decoder import Decoder
+
+    nh, nkv, hd = heads
+    dec = Decoder(n_layers=1, d_model=256, n_heads=nh, n_kv_heads=nkv, head_dim=hd, d_ff=256, vocab=512, group_size=32, max_batch=batch,
+                  max_ctx=max_ctx, max_steps=8, rope_theta=10000.0, rms_eps=1e-5)
+    dec.init_random(seed=3, nibbles=(1, 15))
+    dec.finalize()
+    return dec
+
+
+@pytest.mark.parametrize("heads,batch,max_ctx,positions", [
+    ((16, 4, 128), 16, 2176, (0, 31, 32, 511, 512, 1023, 1024, 1100, 2170)),  # 64 pairs: up to four shares
+    ((32, 8, 128), 16, 2176, (511, 512, 2100)),                               # two shares, the 7B head layout
+    ((16, 2, 64), 3, 4224, (5, 512, 700, 1600, 4200)),                        # eight shares
+    ((36, 2, 32), 2, 1152, (40, 600, 1150)),                                  # eighteen query heads per kv head: two blocks of them
+    ((12, 4, 96), 5, 1152, (63, 1025)),
+], ids=["16q4kv-hd128", "32q8kv-hd128", "16q2kv-hd64", "36q2kv-hd32", "12q4kv-hd96"])
+def test_against_float64(heads, batch, max_ctx, positions):
+    nh, nkv, hd = heads
+    dec = _decoder(heads, batch, max_ctx)
+    rng = np.random.default_rng(17)
+    k = rng.standard_normal((batch, max_ctx - 8, nkv, hd)).astype(np.float16)
+    v = rng.standard_normal((batch, max_ctx - 8, nkv, hd)).astype(np.float16)
+    tokens = (np.arange(batch) * 7 + 3).astype(np.int32)
+    for pos in positions:
+        k[:, pos:], v[:, pos:] = np.nan, np.nan  # what lies behind the context must not be seen
+        dec.set_kv(0, k, v)
+        outs = []
+        for use_graph in (False, True, True):  # the slots of the merge are empty again behind every launch
+            dec.reset(tokens, pos)
+            dec.run(1, use_graph=use_graph)
+            outs.append(dec.activation("attn_out"))
+        assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+        q = dec.activation("qkv")[:, : nh * hd].reshape(batch, nkv, nh // nkv, hd).astype(np.float64)
+        kc, vc = (a.astype(np.float64).transpose(0, 2, 1, 3) for a in dec.get_kv(0, batch, 0, pos + 1))
+        s = q @ kc.transpose(0, 1, 3, 2) / math.sqrt(hd)
+        p = np.exp(s - s.max(-1, keepdims=True))
+        want = (p @ vc / p.sum(-1, keepdims=True)).reshape(batch, nh * hd)
+        # weights and result are rounded to fp16 (2^-11 each), v is exact; scores to 2^-22 of a few hundred
+        assert np.abs(outs[0] - want).max() <= 2.0 ** -10 * np.abs(vc).max() * 1.1, (pos, np.abs(outs[0] - want).max())
+        k = np.nan_to_num(k)
+        v = np.nan_to_num(v)
+    dec.close()

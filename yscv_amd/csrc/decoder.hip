@@ -139,7 +139,8 @@ struct yscv_hip_decoder {
   _Float16 *xn = nullptr, *qkv = nullptr, *ao = nullptr, *act = nullptr;
   _Float16 *qrot = nullptr;       // rotated query heads of the last fused attention launch (diagnostics)
   bool fused_attn = true;         // rope + append inside the attention kernel
-  bool generic_attn = false;      // head width other than 128 or more than 4 query heads per kv head: the general kernel
+  uint64_t *attn_meet = nullptr;  // launch_attention_decode, like the angles of the step's position
+  float *angles = nullptr;
   bool has_bias = false;          // a layer has a q / k / v bias (the single-launch kernel has none)
   // RMSNorm folded into the projections around it (NormFold, kernels.hpp): two buffers of partial sums of squares,
   // written and read in turn, each with the power of two per row that xn's rows were multiplied by
@@ -249,6 +250,8 @@ static void decoder_free(yscv_hip_decoder *d) {
   (void)hipFree(d->h);
   (void)hipFree(d->logits);
   (void)hipFree(d->attn_part);
+  (void)hipFree(d->attn_meet);
+  (void)hipFree(d->angles);
   (void)hipFree(d->qrot);
   (void)hipFree(d->ss[0]);
   (void)hipFree(d->ss[1]);
@@ -545,8 +548,15 @@ static int32_t alloc_runtime(yscv_hip_decoder *d) {
   DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->qkv), B * qkv_n * 2));
   DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->ao), B * (size_t)c.n_heads * c.head_dim * 2));
   DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->act), B * (size_t)c.d_ff * 2));
-  const size_t chunks = c.max_ctx / 128;
-  DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->attn_part), B * c.n_heads * chunks * (c.head_dim + 2) * 4));
+  const Context *ctx = nullptr;
+  YSCV_TRY(ensure_context(&ctx));
+  DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->attn_part), B * c.n_heads * (size_t)(c.max_ctx / 128) * (c.head_dim + 2) * 4));
+  if (d->kv_dtype == YSCV_HIP_KV_F16) {
+    const size_t meet = attention_decode_meet_bytes(c.max_batch, c.n_heads, c.n_kv_heads, c.head_dim, c.max_ctx, ctx->num_cus);
+    DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->attn_meet), meet));
+    DEC_HIP(hipMemset(d->attn_meet, 0xff, meet));
+    DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->angles), c.head_dim * 4));
+  }
   DEC_HIP(hipMalloc(reinterpret_cast<void **>(&d->qrot), B * (size_t)c.n_heads * c.head_dim * 2));
   DEC_HIP(hipMemset(d->qrot, 0, B * (size_t)c.n_heads * c.head_dim * 2));
   d->ss_stride = c.d_model / 16;
@@ -747,11 +757,20 @@ static int32_t capture_step(F enqueue, hipGraph_t *graph, hipGraphExec_t *exec) 
   return YSCV_HIP_OK;
 }
 
+// Chunks of 128 positions and a merge launch, or the kernel of decode_attention.hip (times of both in its header): the line is a
+// quarter of the CUs, from where on a pair's positions need no more than four workgroups.
+static bool chunked_attention(const yscv_hip_decoder *d, int batch) {
+  const auto &c = d->cfg;
+  return c.head_dim == 128 && c.n_heads / c.n_kv_heads <= 4 && batch * c.n_kv_heads < 64;
+}
+
 // every launch of one decode step, in order, on stream s
 static int32_t enqueue_step(yscv_hip_decoder *d, int batch, hipStream_t s) {
   const auto &c = d->cfg;
   const int D = c.d_model;
   const bool fold = d->fold_norm;
+  const Context *ctx = nullptr;
+  YSCV_TRY(ensure_context(&ctx));
   // folded norms: `cur` is the buffer of partial sums the next consumer reads, `cnt` how many partials a row has there
   int cur = 0, cnt = 0;
   // `feeds_update`: a residual update follows this norm's projection and takes its row scales from it
@@ -772,13 +791,18 @@ static int32_t enqueue_step(yscv_hip_decoder *d, int batch, hipStream_t s) {
     nf.ss_out_stride = d->ss_stride;
     nf.ss_out_count = count_out;
   };
+  RopeTable rope;
+  rope.pos = d->pos;
+  rope.angles = d->angles;
+  rope.hd = c.head_dim;
+  rope.theta = c.rope_theta;
   if (fold) {
     YSCV_TRY(launch_embed_norm(d->tokens, d->emb, batch, D, c.vocab, c.rms_eps, d->h, d->layers[0].attn_norm, d->xn, d->ss[0],
-                               d->ss_stride, d->pre[0], s));
+                               d->ss_stride, d->pre[0], s, rope));
     cur = 0;
     cnt = 1;
   } else {
-    YSCV_TRY(launch_embed(d->tokens, d->emb, batch, D, c.vocab, d->h, s));
+    YSCV_TRY(launch_embed(d->tokens, d->emb, batch, D, c.vocab, d->h, s, rope));
   }
   for (size_t li = 0; li < d->layers.size(); li++) {
     auto &L = d->layers[li];
@@ -792,14 +816,7 @@ static int32_t enqueue_step(yscv_hip_decoder *d, int batch, hipStream_t s) {
     }
     const int qkv_n = (c.n_heads + 2 * c.n_kv_heads) * c.head_dim;
     if (L.qkv_bias) YSCV_TRY(launch_bias_add_f16(d->qkv, L.qkv_bias, (size_t)batch, (size_t)qkv_n, s));
-    if (d->generic_attn && d->fused_attn) {
-      YSCV_TRY(launch_gqa_cache(d->qkv, L.kc, L.vc, d->pos, batch, 0, c.n_heads, c.n_kv_heads, c.head_dim, c.max_ctx, d->ao, s,
-                                c.rope_theta, d->qrot));
-    } else if (d->generic_attn) {
-      YSCV_TRY(launch_rope_append(d->qkv, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta, c.max_ctx,
-                                  L.kc, L.vc, s));
-      YSCV_TRY(launch_gqa_cache(d->qkv, L.kc, L.vc, d->pos, batch, 0, c.n_heads, c.n_kv_heads, c.head_dim, c.max_ctx, d->ao, s));
-    } else if (d->kv_dtype == YSCV_HIP_KV_I8 && d->fused_attn) {
+    if (d->kv_dtype == YSCV_HIP_KV_I8 && d->fused_attn) {
       YSCV_TRY(launch_attention_fused_i8(d->qkv, L.kc8, L.ks, L.vc8, L.vs, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim,
                                          c.rope_theta, c.max_ctx, d->attn_part, d->qrot, d->ao, s));
     } else if (d->kv_dtype == YSCV_HIP_KV_I8) {
@@ -807,14 +824,16 @@ static int32_t enqueue_step(yscv_hip_decoder *d, int batch, hipStream_t s) {
                                      L.kc8, L.ks, L.vc8, L.vs, s));
       YSCV_TRY(launch_attention_i8(d->qkv, L.kc8, L.ks, L.vc8, L.vs, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim,
                                    c.max_ctx, d->attn_part, d->ao, s));
-    } else if (d->fused_attn) {
-      YSCV_TRY(launch_attention_fused(d->qkv, L.kc, L.vc, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta,
-                                      c.max_ctx, d->attn_part, d->qrot, d->ao, s));
     } else {
-      YSCV_TRY(launch_rope_append(d->qkv, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta, c.max_ctx,
-                                  L.kc, L.vc, s));
-      YSCV_TRY(launch_attention(d->qkv, L.kc, L.vc, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim, c.max_ctx,
-                                d->attn_part, d->ao, s));
+      _Float16 *qrot = d->fused_attn ? d->qrot : nullptr;
+      if (!d->fused_attn)
+        YSCV_TRY(launch_rope_append(d->qkv, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta, c.max_ctx, L.kc, L.vc, s));
+      if (chunked_attention(d, batch))
+        YSCV_TRY(launch_attention_chunks(d->qkv, L.kc, L.vc, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim, d->angles, c.max_ctx,
+                                         d->attn_part, qrot, d->ao, s));
+      else
+        YSCV_TRY(launch_attention_decode(d->qkv, L.kc, L.vc, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim, d->angles, c.max_ctx,
+                                         ctx->num_cus, d->attn_meet, qrot, d->ao, s));
     }
     if (fold) {
       // o: h += W ao, and the ffn norm's inputs; gate/up reads them; down: h += W act, and the next norm's inputs
@@ -889,8 +908,7 @@ int32_t yscv_hip_decoder_create_kv(const yscv_hip_decoder_config *cfg, int32_t k
   YSCV_REQUIRE(c.head_dim == 32 || c.head_dim == 64 || c.head_dim == 96 || c.head_dim == 128,
                "head_dim must be 32, 64, 96 or 128 (got %d)", c.head_dim);
   YSCV_REQUIRE(c.n_heads % c.n_kv_heads == 0, "the kv heads must divide the query heads (%d over %d)", c.n_heads, c.n_kv_heads);
-  const bool generic_attn = c.head_dim != 128 || c.n_heads / c.n_kv_heads > 4;
-  if (generic_attn && kv_dtype == YSCV_HIP_KV_I8)
+  if ((c.head_dim != 128 || c.n_heads / c.n_kv_heads > 4) && kv_dtype == YSCV_HIP_KV_I8)
     return set_error(YSCV_HIP_ERR_UNSUPPORTED, "the int8 cache exists for head_dim 128 with 1..4 query heads per kv head");
   YSCV_REQUIRE(c.d_model % 128 == 0 && c.d_ff % 128 == 0 && (c.n_heads * c.head_dim) % 128 == 0,
                "d_model, d_ff and n_heads*head_dim must be multiples of 128");
@@ -902,7 +920,6 @@ int32_t yscv_hip_decoder_create_kv(const yscv_hip_decoder_config *cfg, int32_t k
   auto *d = new yscv_hip_decoder();
   d->cfg = c;
   d->kv_dtype = kv_dtype;
-  d->generic_attn = generic_attn;
   (void)hipGetDevice(&d->device);
   d->layers.resize(c.n_layers);
   int32_t st = alloc_runtime(d);
@@ -1595,12 +1612,12 @@ static int32_t prefill_chunk(yscv_hip_decoder *d, const int32_t *tokens_dev, int
       // the quantised append, and attention over what the int8 cache returns for every position so far (fp16 scratch)
       YSCV_TRY(launch_prefill_rope_append_i8(qkv, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta,
                                              c.max_ctx, L.kc8, L.ks, L.vc8, L.vs, t_ctx, tk, tv, s));
-      YSCV_TRY(launch_gqa_cache(qkv, tk, tv, nullptr, rows, start_pos, c.n_heads,
+      YSCV_TRY(launch_gqa_cache(qkv, tk, tv, rows, start_pos, c.n_heads,
                                 c.n_kv_heads, c.head_dim, t_ctx, ao, s));
     } else {
       YSCV_TRY(launch_prefill_rope_append(qkv, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta,
                                           c.max_ctx, L.kc, L.vc, s));
-      YSCV_TRY(launch_gqa_cache(qkv, L.kc, L.vc, nullptr, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim,
+      YSCV_TRY(launch_gqa_cache(qkv, L.kc, L.vc, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim,
                                 c.max_ctx, ao, s));
     }
     // the residual update and SwiGLU ride on the projections' epilogues (both kernels have them: the skinny kernel up to

@@ -19,16 +19,29 @@
 #include "decoder.hpp"
 #include "int4_common.hpp"
 #include "kernels.hpp"
+#include "rope.hpp"
 
 namespace yscv {
 
 // ---- embedding: h[b][:] = table[token[b]][:] (fp16 -> f32 residual stream) ----------------------
-__global__ void embed_kernel(const int32_t *__restrict__ tokens, const _Float16 *__restrict__ table, int d,
-                             int vocab, float *__restrict__ h) {
+// the angles of the step's position, once for all layers (powf and sincosf in every attention workgroup were a third of that
+// kernel's code)
+__device__ __forceinline__ void leave_angles(const RopeTable &rope) {
+  const int half_d = rope.hd / 2;
+  if (rope.angles && blockIdx.x == 0 && (int)threadIdx.x < half_d) {
+    const SinCos sc = rope_sincos(rope.theta, (int)threadIdx.x, rope.hd, *rope.pos);
+    rope.angles[threadIdx.x] = sc.cs;
+    rope.angles[half_d + threadIdx.x] = sc.sn;
+  }
+}
+
+__global__ void __launch_bounds__(256) embed_kernel(const int32_t *__restrict__ tokens, const _Float16 *__restrict__ table, int d,
+                                                    int vocab, float *__restrict__ h, RopeTable rope) {
   const int b = blockIdx.x;
+  leave_angles(rope);
   int tok = tokens[b];
   tok = tok < 0 ? 0 : (tok >= vocab ? vocab - 1 : tok);
-  for (int i = threadIdx.x; i < d; i += blockDim.x) h[(size_t)b * d + i] = (float)table[(size_t)tok * d + i];
+  for (int i = threadIdx.x; i < d; i += 256) h[(size_t)b * d + i] = (float)table[(size_t)tok * d + i];
 }
 
 // embedding lookup that also feeds the first norm in its folded form (NormFold, kernels.hpp): the row stays in
@@ -37,7 +50,7 @@ __global__ void embed_kernel(const int32_t *__restrict__ tokens, const _Float16 
 __global__ void __launch_bounds__(256) embed_norm_kernel(const int32_t *__restrict__ tokens, const _Float16 *__restrict__ table,
                                                          int d, int vocab, float eps, float *__restrict__ h,
                                                          const float *__restrict__ gamma, _Float16 *__restrict__ xg,
-                                                         float *__restrict__ ss_out, int ss_stride, float *__restrict__ pre) {
+                                                         float *__restrict__ ss_out, int ss_stride, float *__restrict__ pre, RopeTable rope) {
   __shared__ float red4[4];
   const int b = blockIdx.x;
   int tok = tokens[b];
@@ -92,6 +105,7 @@ __global__ void __launch_bounds__(256) embed_norm_kernel(const int32_t *__restri
     ss_out[(size_t)b * ss_stride] = total;
     pre[b] = scale;
   }
+  leave_angles(rope);
 }
 
 // ---- RMSNorm: f32 residual -> fp16 normalised activations -----------------------------------------
@@ -151,36 +165,6 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(const float *__restrict__ 
     for (int e = 0; e < 4; e++) o[e] = (_Float16)(v[e] * inv * g[e]);
     *reinterpret_cast<half4_t *>(out + (size_t)b * d + i) = o;
   }
-}
-
-// sin and cos of the angle of pair i at position pos: inv_freq[i] = 1 / theta^(2i / d)
-struct SinCos {
-  float sn, cs;
-};
-__device__ __forceinline__ SinCos rope_sincos(float theta, int i, int d, int pos) {
-  const float inv_freq = 1.0f / powf(theta, (float)(2 * i) / (float)d);
-  SinCos r;
-  sincosf(inv_freq * (float)pos, &r.sn, &r.cs);
-  return r;
-}
-
-// rotate-half of one pair, written with explicit fused multiply-adds so that every kernel that rotates rounds alike
-__device__ __forceinline__ void rope_pair_f32(float x0, float x1, float cs, float sn, float &y0, float &y1) {
-  y0 = fmaf(x0, cs, -(x1 * sn));
-  y1 = fmaf(x0, sn, x1 * cs);
-}
-// f32 -> fp16 of a value that exists as an f32 first.  Without the empty asm the compiler may merge the conversion
-// into the multiply-add that produced the value (a mixed-precision fma that rounds once, straight to fp16), in one
-// kernel and not in another: one rotated q element in a few thousand then differs by an fp16 ulp between them.
-__device__ __forceinline__ _Float16 f16_of_f32(float v) {
-  asm volatile("" : "+v"(v));
-  return (_Float16)v;
-}
-__device__ __forceinline__ void rope_pair(float x0, float x1, float cs, float sn, _Float16 &y0, _Float16 &y1) {
-  float f0, f1;
-  rope_pair_f32(x0, x1, cs, sn, f0, f1);
-  y0 = f16_of_f32(f0);
-  y1 = f16_of_f32(f1);
 }
 
 // ---- RoPE on q (in place) and k, then append k / v to the cache -------------------------------------
@@ -285,10 +269,9 @@ __device__ __forceinline__ float v_scale_pow2(float v0, float v1, bool live0, bo
   return ldexpf(1.0f, e);
 }
 
-template <bool KV8>
-__global__ void __launch_bounds__(256) attn_partial_kernel(const _Float16 *__restrict__ qkv,
-                                                           const void *__restrict__ kc_v,
-                                                           const void *__restrict__ vc_v,
+__global__ void __launch_bounds__(256) attn_partial_i8_kernel(const _Float16 *__restrict__ qkv,
+                                                           const int8_t *__restrict__ kc,
+                                                           const int8_t *__restrict__ vc,
                                                            const float *__restrict__ ks, const float *__restrict__ vs,
                                                            const int32_t *__restrict__ pos_ptr, int hq, int hkv,
                                                            int max_ctx, int max_chunks, float scale,
@@ -326,41 +309,27 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const _Float16 *__res
     }
     const size_t k_off = (((size_t)b * hkv + kvh) * max_ctx + p0) * HD;
     const size_t v_off = ((((size_t)b * hkv + kvh) * (max_ctx / 8) + p0 / 8) * HD) * 8;
-    // issue every load of this wave up front: 8 KiB of K, 8 KiB of V (half of that from an int8 cache)
+    // issue every load of this wave up front: 4 KiB of K, 4 KiB of V
     half8_t kf[2][4], vf[8];
-    float k_scale[2] = {1.0f, 1.0f}, v_scale[2] = {1.0f, 1.0f};  // of position p0 + 16 pb + r
-    if constexpr (KV8) {
-      const int8_t *kbase = static_cast<const int8_t *>(kc_v) + k_off;
-      const int8_t *vbase = static_cast<const int8_t *>(vc_v) + v_off;
-      int2_t kraw[2][4], vraw[8];
+    float k_scale[2], v_scale[2];  // of position p0 + 16 pb + r
+    const int8_t *kbase = kc + k_off, *vbase = vc + v_off;
+    int2_t kraw[2][4], vraw[8];
 #pragma unroll
-      for (int pb = 0; pb < 2; pb++) {
-        k_scale[pb] = ks[(size_t)b * max_ctx + p0 + pb * 16 + r];
-        v_scale[pb] = vs[(size_t)b * max_ctx + p0 + pb * 16 + r];
+    for (int pb = 0; pb < 2; pb++) {
+      k_scale[pb] = ks[(size_t)b * max_ctx + p0 + pb * 16 + r];
+      v_scale[pb] = vs[(size_t)b * max_ctx + p0 + pb * 16 + r];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-          kraw[pb][j] = *reinterpret_cast<const int2_t *>(kbase + (size_t)(pb * 16 + r) * HD + 32 * c + 8 * j);
-      }
-#pragma unroll
-      for (int t = 0; t < 8; t++) vraw[t] = *reinterpret_cast<const int2_t *>(vbase + ((size_t)c * HD + t * 16 + r) * 8);
-#pragma unroll
-      for (int pb = 0; pb < 2; pb++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) kf[pb][j] = i8x8_to_half8(kraw[pb][j]);
-#pragma unroll
-      for (int t = 0; t < 8; t++) vf[t] = i8x8_to_half8(vraw[t]);
-    } else {
-      const _Float16 *kbase = static_cast<const _Float16 *>(kc_v) + k_off;
-      const _Float16 *vbase = static_cast<const _Float16 *>(vc_v) + v_off;
-#pragma unroll
-      for (int pb = 0; pb < 2; pb++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          kf[pb][j] = *reinterpret_cast<const half8_t *>(kbase + (size_t)(pb * 16 + r) * HD + 32 * c + 8 * j);
-#pragma unroll
-      for (int t = 0; t < 8; t++)
-        vf[t] = *reinterpret_cast<const half8_t *>(vbase + ((size_t)c * HD + t * 16 + r) * 8);
+      for (int j = 0; j < 4; j++)
+        kraw[pb][j] = *reinterpret_cast<const int2_t *>(kbase + (size_t)(pb * 16 + r) * HD + 32 * c + 8 * j);
     }
+#pragma unroll
+    for (int t = 0; t < 8; t++) vraw[t] = *reinterpret_cast<const int2_t *>(vbase + ((size_t)c * HD + t * 16 + r) * 8);
+#pragma unroll
+    for (int pb = 0; pb < 2; pb++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) kf[pb][j] = i8x8_to_half8(kraw[pb][j]);
+#pragma unroll
+    for (int t = 0; t < 8; t++) vf[t] = i8x8_to_half8(vraw[t]);
 
     float s[2];
 #pragma unroll
@@ -378,12 +347,12 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const _Float16 *__res
     const float sum = row_sum16(e0 + e1);
     m_h = mx;
     l_h = sum;
-    float vS = 1.0f, vS_inv = 1.0f;
-    if constexpr (KV8) vS = v_scale_pow2(v_scale[0], v_scale[1], p0 + r < n_ctx, p0 + 16 + r < n_ctx, &vS_inv);
+    float vS_inv = 1.0f;
+    const float vS = v_scale_pow2(v_scale[0], v_scale[1], p0 + r < n_ctx, p0 + 16 + r < n_ctx, &vS_inv);
     if (c < 4) {
-      // int8 cache: the V scale of the position rides on its weight (a dead position has weight 0 whatever its scale)
-      p_lds[wave][c][r] = KV8 ? (e0 == 0.0f ? (_Float16)0.0f : (_Float16)(e0 * (v_scale[0] * vS_inv))) : (_Float16)e0;
-      p_lds[wave][c][16 + r] = KV8 ? (e1 == 0.0f ? (_Float16)0.0f : (_Float16)(e1 * (v_scale[1] * vS_inv))) : (_Float16)e1;
+      // the V scale of the position rides on its weight (a dead position has weight 0 whatever its scale)
+      p_lds[wave][c][r] = e0 == 0.0f ? (_Float16)0.0f : (_Float16)(e0 * (v_scale[0] * vS_inv));
+      p_lds[wave][c][16 + r] = e1 == 0.0f ? (_Float16)0.0f : (_Float16)(e1 * (v_scale[1] * vS_inv));
     }
     __builtin_amdgcn_wave_barrier();  // LDS is in order per wave: the reads below see the writes above
     // P operand: MFMA row 4*h = head h, lane (r, c) holds positions 8c .. 8c+7 of this wave's 32
@@ -402,7 +371,7 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const _Float16 *__res
       }
       float4_t d = {0.0f, 0.0f, 0.0f, 0.0f};
       d = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, vv, d, 0, 0, 0);
-      o_acc[t] = KV8 ? d[0] * vS : d[0];  // lane (r, c): o of head c at d = 16 t + r
+      o_acc[t] = d[0] * vS;  // lane (r, c): o of head c at d = 16 t + r
     }
   }
 
@@ -510,19 +479,19 @@ __global__ void __launch_bounds__(128) attn_combine_kernel(const float *__restri
 }
 
 // ---- rotary embedding + cache append + attention partials in ONE launch (fp16 cache) ------------------------------
-// Same arithmetic as rope_append_kernel -> attn_partial_kernel<false>, without the kernel boundary between them:
+// The arithmetic of rope_append_kernel and of attention over the cache, without a kernel boundary between them:
 //   * every workgroup rotates the query heads of its kv head itself (one (i, i + 64) pair per thread, through LDS)
 //     while its K / V loads are in flight; the rotated q is never written back (the workgroups of the other chunks
 //     read the unrotated one at the same time), only the workgroup of chunk 0 leaves a copy in `qrot` for diagnostics;
 //   * the workgroup whose chunk holds the current position rotates k, appends k and v to the cache and patches the
 //     new row into the registers of the wave that owns the position (the loads issued up front saw the old bytes).
-// attn_combine_kernel follows as a launch of its own.  (Merging the chunks in the same launch as well -- partials
-// through agent-scope stores, an arrival counter per (batch row, kv head), the last workgroup merges -- computed the
-// same values but was slower than the separate launch: 36.9 against 29.2 + 4.7 us at batch 16, context 2048; with an
-// acquire-release counter, whose cache write-back every workgroup pays, 113 us.)
-__global__ void __launch_bounds__(256) attn_fused_kernel(const _Float16 *__restrict__ qkv, _Float16 *kc, _Float16 *vc,
+// attn_combine_kernel follows as a launch of its own.  For decoders with few (sequence, kv head) pairs, whose positions have to be
+// spread over many CUs; decode_attention.hip takes the others (the line is in enqueue_step, decoder.hip).  (Merging the chunks in
+// this launch -- partials through agent-scope stores, an arrival counter, the last workgroup merges -- was slower than
+// the separate launch: 36.9 against 29.2 + 4.7 us at batch 16, context 2048.)
+__global__ void __launch_bounds__(256) attn_chunk_kernel(const _Float16 *__restrict__ qkv, _Float16 *kc, _Float16 *vc,
                                                          const int32_t *__restrict__ pos_ptr, int hq, int hkv, int max_ctx,
-                                                         int max_chunks, float scale, float theta,
+                                                         int max_chunks, float scale, const float *__restrict__ angles,
                                                          float *__restrict__ part, _Float16 *__restrict__ qrot) {
   constexpr int HD = 128;
   __shared__ __attribute__((aligned(16))) _Float16 q_lds[4][HD];
@@ -543,9 +512,19 @@ __global__ void __launch_bounds__(256) attn_fused_kernel(const _Float16 *__restr
   const int p0 = chunk * ATT_CHUNK + wave * ATT_POS_PER_WAVE;
   const int row_elems = (hq + 2 * hkv) * HD;
   const bool wave_live = p0 < n_ctx;
-  const bool owner = (pos / ATT_CHUNK) == chunk;  // this workgroup's positions include the current token
+  const bool fused = qrot != nullptr;  // else qkv holds the rotated q, and the cache the row of the token
+  const bool owner = fused && (pos / ATT_CHUNK) == chunk;  // this workgroup's positions include the current token
 
-  // ---- K / V of this wave's 32 positions: requested before anything else ----
+  // ---- what this thread rotates or copies, requested first: loads return in order, and this is needed while K and V are on
+  // their way
+  const int rh = tid >> 6, ri = tid & 63;
+  const float cs = angles[ri], sn = angles[HD / 2 + ri];
+  const _Float16 *qrow = qkv + (size_t)b * row_elems;
+  const _Float16 *qsrc = qrow + (size_t)(kvh * group + min(rh, group - 1)) * HD, *ksrc = qrow + (size_t)(hq + kvh) * HD;
+  const float qx0 = (float)qsrc[ri], qx1 = (float)qsrc[ri + HD / 2], kx0 = (float)ksrc[ri], kx1 = (float)ksrc[ri + HD / 2];
+  const _Float16 vx = qrow[(size_t)(hq + hkv + kvh) * HD + (rh == 2 ? 64 : 0) + ri];
+
+  // ---- K / V of this wave's 32 positions ----
   const size_t k_off = (((size_t)b * hkv + kvh) * max_ctx + p0) * HD;
   const size_t v_off = ((((size_t)b * hkv + kvh) * (max_ctx / 8) + p0 / 8) * HD) * 8;
   half8_t kf[2][4], vf[8];
@@ -567,28 +546,22 @@ __global__ void __launch_bounds__(256) attn_fused_kernel(const _Float16 *__restr
 
   // ---- rotary embedding: thread (h = tid / 64, i = tid % 64) turns the pair (i, i + 64) of query head h ----
   {
-    const int h = tid >> 6, i = tid & 63;
-    const SinCos sc = rope_sincos(theta, i, HD, pos);
-    const float sn = sc.sn, cs = sc.cs;
+    const int h = rh, i = ri;
     if (h < group) {
       const int head = kvh * group + h;
-      const _Float16 *src = qkv + (size_t)b * row_elems + (size_t)head * HD;
-      const float x0 = (float)src[i], x1 = (float)src[i + HD / 2];
       _Float16 y0, y1;
-      rope_pair(x0, x1, cs, sn, y0, y1);
-      q_lds[h][i] = y0;
-      q_lds[h][i + HD / 2] = y1;
-      if (chunk == 0) {
+      rope_pair(qx0, qx1, cs, sn, y0, y1);
+      q_lds[h][i] = fused ? y0 : (_Float16)qx0;
+      q_lds[h][i + HD / 2] = fused ? y1 : (_Float16)qx1;
+      if (fused && chunk == 0) {
         qrot[((size_t)b * hq + head) * HD + i] = y0;
         qrot[((size_t)b * hq + head) * HD + i + HD / 2] = y1;
       }
     }
     if (owner) {
       if (h == 0) {
-        const _Float16 *src = qkv + (size_t)b * row_elems + (size_t)(hq + kvh) * HD;
-        const float x0 = (float)src[i], x1 = (float)src[i + HD / 2];
         _Float16 y0, y1;
-      rope_pair(x0, x1, cs, sn, y0, y1);
+        rope_pair(kx0, kx1, cs, sn, y0, y1);
         knew[i] = y0;
         knew[i + HD / 2] = y1;
         _Float16 *dst = kc + (((size_t)b * hkv + kvh) * max_ctx + pos) * HD;
@@ -596,13 +569,12 @@ __global__ void __launch_bounds__(256) attn_fused_kernel(const _Float16 *__restr
         dst[i + HD / 2] = y1;
       } else if (h == 1 || h == 2) {
         const int dd = (h - 1) * 64 + i;
-        const _Float16 v = qkv[(size_t)b * row_elems + (size_t)(hq + hkv + kvh) * HD + dd];
-        vnew[dd] = v;
-        vc[((((size_t)b * hkv + kvh) * (max_ctx / 8) + pos / 8) * HD + dd) * 8 + (pos & 7)] = v;
+        vnew[dd] = vx;
+        vc[((((size_t)b * hkv + kvh) * (max_ctx / 8) + pos / 8) * HD + dd) * 8 + (pos & 7)] = vx;
       }
     }
   }
-  __syncthreads();
+  lds_barrier();  // (K and V stay in flight)
 
   float m_h = -INFINITY, l_h = 0.0f;
   float o_acc[8];
@@ -687,7 +659,7 @@ __global__ void __launch_bounds__(256) attn_fused_kernel(const _Float16 *__restr
     for (int t = 0; t < 8; t++) w_o[wave][c][t * 16 + r] = o_acc[t];
   }
   __syncthreads();
-  for (int idx = tid; idx < group * HD; idx += blockDim.x) {
+  for (int idx = tid; idx < group * HD; idx += 256) {
     const int h = idx / HD, dd = idx % HD;
     float mx = -INFINITY;
 #pragma unroll
@@ -1043,7 +1015,7 @@ __global__ void __launch_bounds__(256) kv_dequant_i8_kernel(const int8_t *__rest
 }
 
 // ---- rotary embedding + int8 cache append + attention partials in ONE launch (int8 cache) ---------------------------
-// rope_append_i8_kernel -> attn_partial_kernel<true> without the kernel boundary, as attn_fused_kernel does it for the
+// rope_append_i8_kernel -> attn_partial_i8_kernel without the kernel boundary, as attn_chunk_kernel does it for the
 // fp16 cache.  The scale of an int8 row spans all kv heads of the position, so each of the Hkv workgroups whose chunk
 // holds the current position rotates the whole k row (Hkv * 64 pairs) and scans the whole v row to get the two scales
 // (all of them write the same two values), then quantises and appends its own head's 128 + 128 values and patches
@@ -1316,18 +1288,19 @@ __global__ void fill_const_f32_kernel(float *p, size_t n, float v) {
 }
 
 // ---- launchers -------------------------------------------------------------------------------------------
-int32_t launch_embed(const int32_t *tokens, const _Float16 *table, int batch, int d, int vocab, float *h,
-                     hipStream_t s) {
-  hipLaunchKernelGGL(embed_kernel, dim3(batch), dim3(256), 0, s, tokens, table, d, vocab, h);
+int32_t launch_embed(const int32_t *tokens, const _Float16 *table, int batch, int d, int vocab, float *h, hipStream_t s,
+                     const RopeTable &rope) {
+  hipLaunchKernelGGL(embed_kernel, dim3(batch), dim3(256), 0, s, tokens, table, d, vocab, h, rope);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
 
 int32_t launch_embed_norm(const int32_t *tokens, const _Float16 *table, int batch, int d, int vocab, float eps, float *h,
-                          const float *gamma, _Float16 *xg, float *ss_out, int ss_stride, float *pre, hipStream_t s) {
+                          const float *gamma, _Float16 *xg, float *ss_out, int ss_stride, float *pre, hipStream_t s,
+                          const RopeTable &rope) {
   if (d > 4096 || d % 8 != 0) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "embedding with a folded norm: rows of at most 4096 values, a multiple of 8");
   hipLaunchKernelGGL(embed_norm_kernel, dim3(batch), dim3(256), 0, s, tokens, table, d, vocab, eps, h, gamma, xg, ss_out, ss_stride,
-                     pre);
+                     pre, rope);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
@@ -1359,32 +1332,15 @@ int32_t launch_kv_relayout(const _Float16 *k_nat, const _Float16 *v_nat, int bat
   return YSCV_HIP_OK;
 }
 
-int32_t launch_attention(const _Float16 *qkv, const _Float16 *kc, const _Float16 *vc, const int32_t *pos_ptr,
-                         int batch, int hq, int hkv, int hd, int max_ctx, float *part, _Float16 *out,
-                         hipStream_t s) {
+int32_t launch_attention_chunks(const _Float16 *qkv, _Float16 *kc, _Float16 *vc, const int32_t *pos_ptr, int batch, int hq, int hkv,
+                                int hd, const float *angles, int max_ctx, float *part, _Float16 *qrot, _Float16 *out, hipStream_t s) {
   if (hd != 128) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention kernel is built for head_dim 128, got %d", hd);
   if (hq % hkv != 0 || hq / hkv > 4)
     return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention kernel handles 1..4 query heads per kv head");
   const int max_chunks = max_ctx / ATT_CHUNK;
   const float scale = 1.0f / sqrtf((float)hd);
-  hipLaunchKernelGGL(attn_partial_kernel<false>, dim3(max_chunks, hkv, batch), dim3(256), 0, s, qkv, kc, vc, nullptr, nullptr,
-                     pos_ptr, hq, hkv, max_ctx, max_chunks, scale, part);
-  YSCV_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(attn_combine_kernel, dim3(hq, batch), dim3(128), 0, s, part, pos_ptr, hq, max_chunks, out);
-  YSCV_HIP_TRY(hipGetLastError());
-  return YSCV_HIP_OK;
-}
-
-int32_t launch_attention_fused(const _Float16 *qkv, _Float16 *kc, _Float16 *vc, const int32_t *pos_ptr, int batch, int hq,
-                               int hkv, int hd, float theta, int max_ctx, float *part, _Float16 *qrot, _Float16 *out,
-                               hipStream_t s) {
-  if (hd != 128) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention kernel is built for head_dim 128, got %d", hd);
-  if (hq % hkv != 0 || hq / hkv > 4)
-    return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention kernel handles 1..4 query heads per kv head");
-  const int max_chunks = max_ctx / ATT_CHUNK;
-  const float scale = 1.0f / sqrtf((float)hd);
-  hipLaunchKernelGGL(attn_fused_kernel, dim3(hkv, batch, max_chunks), dim3(256), 0, s, qkv, kc, vc, pos_ptr, hq, hkv, max_ctx,
-                     max_chunks, scale, theta, part, qrot);
+  hipLaunchKernelGGL(attn_chunk_kernel, dim3(hkv, batch, max_chunks), dim3(256), 0, s, qkv, kc, vc, pos_ptr, hq, hkv, max_ctx,
+                     max_chunks, scale, angles, part, qrot);
   YSCV_HIP_TRY(hipGetLastError());
   hipLaunchKernelGGL(attn_combine_kernel, dim3(hq, batch), dim3(128), 0, s, part, pos_ptr, hq, max_chunks, out);
   YSCV_HIP_TRY(hipGetLastError());
@@ -1399,7 +1355,7 @@ int32_t launch_attention_i8(const _Float16 *qkv, const int8_t *kc, const float *
     return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention kernel handles 1..4 query heads per kv head");
   const int max_chunks = max_ctx / ATT_CHUNK;
   const float scale = 1.0f / sqrtf((float)hd);
-  hipLaunchKernelGGL(attn_partial_kernel<true>, dim3(max_chunks, hkv, batch), dim3(256), 0, s, qkv, kc, vc, ks, vs, pos_ptr, hq,
+  hipLaunchKernelGGL(attn_partial_i8_kernel, dim3(max_chunks, hkv, batch), dim3(256), 0, s, qkv, kc, vc, ks, vs, pos_ptr, hq,
                      hkv, max_ctx, max_chunks, scale, part);
   YSCV_HIP_TRY(hipGetLastError());
   hipLaunchKernelGGL(attn_combine_kernel, dim3(hq, batch), dim3(128), 0, s, part, pos_ptr, hq, max_chunks, out);
