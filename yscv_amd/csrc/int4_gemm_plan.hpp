@@ -8,16 +8,18 @@ namespace yscv {
 
 constexpr size_t plan_ceil_div(size_t a, size_t b) { return (a + b - 1) / b; }
 
-// Column blocks of 16 of the 256-row tile shapes 5, 6, 7 below, and whether int4_gemm_wide.hip has the tile for a kind of weight.
-// With zero points and a scale per 32 k the 14-block form needs one register more than there are.  (Planned all the same and then
-// run as 256 x 256, 2048 x 28672 x 4096 of that kind took 441 us; planned without it, 414.)
+// Tiles of int4_gemm_wide.hip, rows x columns; a plan names them kWide + tile
+enum : int { WIDE_256x256 = 0, WIDE_256x192, WIDE_128x256, WIDE_128x192, WIDE_TILES };
+constexpr int kWide = 16;
+
+// Column blocks of 16 of the 256-row tile shapes 5, 6, 7 below, and for which kinds of weight ring_plan counts with them.
 constexpr int wide_tile_blocks(int shape) { return 16 - 2 * (shape - 5); }
 constexpr bool wide_tile_built(int gm, bool has_zp, int blocks) {
   return blocks == 16 || blocks == 12 || (blocks == 14 && !(gm == 0 && has_zp));
 }
 
 // Tile shapes: 0 = 128 x 128, 1 = 128 x 256, 2 = 256 x 128 (m > 128), 3 = 32 x 128 (m <= 32), 4 = 64 x 128 (m <= 64),
-// 5, 6, 7 = 256 x 256, 256 x 224, 256 x 192 (m > 256, int4_gemm_wide.hip)
+// 5, 6, 7 = 256 x 256, 256 x 224, 256 x 192 (m > 256): the work is one for the tiles of int4_gemm_wide.hip, which int4_plan deals out
 struct RingPlan {
   int one;           // shape of the launch, or of the first of two launches
   int second;        // < 0: one launch; else the shape of the launch that takes the columns from split_col on
@@ -122,6 +124,70 @@ inline RingPlan ring_plan(size_t m, size_t n, size_t kt, size_t cus, int gm, boo
       pl.kt_per = (int)plan_ceil_div(kt, best_ks);
       pl.splits = (int)plan_ceil_div(kt, (size_t)pl.kt_per);
     }
+  }
+  return pl;
+}
+
+// us that rounds of one kind of tile take over the CUs, `kt` 128-k tiles deep: whole rounds at the clock that all CUs busy leave, a
+// last round that fills a part of them at a higher one (the card holds its power, not its clock: 64 stages of a 256 x 256 tile take
+// 91 us on 256 CUs, 68 on 32), but never below what one tile takes.
+struct TileTime {
+  size_t bm, bn;
+  double full_fixed, full_kt, fast_fixed, fast_kt;
+};
+inline double tile_rounds_us(const TileTime &t, size_t tiles, size_t kt, size_t cus) {
+  const double full = t.full_fixed + t.full_kt * (double)kt, fast = t.fast_fixed + t.fast_kt * (double)kt;
+  const size_t rest = tiles % cus;
+  const double last = rest == 0 ? 0.0 : (full * (double)rest / (double)cus > fast ? full * (double)rest / (double)cus : fast);
+  return (double)(tiles / cus) * full + last;
+}
+// fitted to 128 .. 2048 rows, N 2049 .. 28672, K 1024 and 4096, fp16 rows, groups of 32; the ring kernel's tiles for comparison
+constexpr TileTime kWideTime[WIDE_TILES] = {
+    {256, 256, 8.0, 2.90, 5.5, 2.12}, {256, 192, 5.5, 2.34, 4.5, 1.74}, {128, 256, 5.5, 1.56, 4.5, 1.25}, {128, 192, 4.8, 1.52, 4.2, 1.06}};
+constexpr TileTime kRingTime[5] = {
+    {128, 128, 1.5, 1.06, 1.5, 1.06}, {128, 256, 8.0, 2.0, 8.0, 2.0}, {256, 128, 8.0, 1.9, 8.0, 1.9}, {32, 128, 1.5, 0.6, 1.5, 0.6}, {64, 128, 1.5, 0.76, 1.5, 0.76}};
+
+// The plan of a launch: ring_plan's, or tiles of int4_gemm_wide.hip where their estimated time is shorter.  From 65 rows on (a
+// 128-row tile decodes a weight once for all of them; the 64-row ring tile is half of one).  us of the op, ring plan -> this one, fp16
+// rows, groups of 32: 2048 x 4096 x 4096 71 -> 58, 2048 x 8192 x 4096 108 -> 100, 512 x 14336 x 4096 66 -> 53, 150 x 28672 x 4096 64 ->
+// 53, 700 x 5632 x 4096 56 -> 42; 128 x 28672 x 4096 43 -> 39.
+inline RingPlan int4_plan(size_t m, size_t n, size_t kt, size_t cus, int gm, bool has_zp) {
+  RingPlan ring = ring_plan(m, n, kt, cus, gm, has_zp);
+  if (m <= 64) return ring;
+  constexpr double kSecondLaunch = 1.0, kSumLaunch = 5.5;  // us
+  auto tiles_of = [&](const TileTime &t, size_t cols) { return plan_ceil_div(m, t.bm) * plan_ceil_div(cols, t.bn); };
+  auto sum_us = [&](size_t parts) { return kSumLaunch + (double)(parts * m * n * 8) / 4e6; };  // partial products out and in
+  double best = 1e30;
+  if (ring.one < 5 && ring.second < 5) {
+    if (ring.splits > 1) best = tile_rounds_us(kRingTime[ring.one], tiles_of(kRingTime[ring.one], n) * ring.splits, (size_t)ring.kt_per, cus) + sum_us((size_t)ring.splits);
+    else if (ring.second < 0) best = tile_rounds_us(kRingTime[ring.one], tiles_of(kRingTime[ring.one], n), kt, cus);
+    else
+      best = tile_rounds_us(kRingTime[ring.one], tiles_of(kRingTime[ring.one], ring.split_col), kt, cus) +
+             tile_rounds_us(kRingTime[ring.second], tiles_of(kRingTime[ring.second], n - ring.split_col), kt, cus) + kSecondLaunch;
+  }
+  RingPlan pl = ring;
+  const size_t x_bytes = m * kt * 128 * 2, cap = x_bytes >= ((size_t)31 << 20) ? 0 : (((size_t)31 << 20) - x_bytes < ((size_t)16 << 20) ? ((size_t)31 << 20) - x_bytes : (size_t)16 << 20);
+  for (int i = 0; i < WIDE_TILES; i++) {
+    const TileTime &t = kWideTime[i];
+    const size_t tiles = tiles_of(t, n);
+    auto take = [&](double us, const RingPlan &p) {
+      if (us < best) {
+        best = us;
+        pl = p;
+      }
+    };
+    take(tile_rounds_us(t, tiles, kt, cus), RingPlan{kWide + i, -1, 0, 1, (int)kt});
+    // K cut over workgroups: under a round of tiles, parts of at least four 128-k tiles, the same bounds on scratch as the ring plan's
+    for (size_t parts = 2; tiles < cus && parts <= 16 && parts <= kt / 4 && parts * m * n * sizeof(float) <= cap; parts++) {
+      const size_t per = plan_ceil_div(kt, parts), used = plan_ceil_div(kt, per);
+      if (used == parts) take(tile_rounds_us(t, tiles * parts, per, cus) + sum_us(parts), RingPlan{kWide + i, -1, 0, (int)parts, (int)per});
+    }
+    // the columns of whole rounds, and the rest in the tiles that suit it
+    const size_t tm = plan_ceil_div(m, t.bm), cols = tiles / cus * cus / tm;
+    if (cols == 0 || cols * t.bn >= n) continue;
+    const double whole = tile_rounds_us(t, tm * cols, kt, cus) + kSecondLaunch;
+    for (int j = 0; j < WIDE_TILES; j++)
+      take(whole + tile_rounds_us(kWideTime[j], tiles_of(kWideTime[j], n - cols * t.bn), kt, cus), RingPlan{kWide + i, kWide + j, cols * t.bn, 1, (int)kt});
   }
   return pl;
 }

@@ -513,20 +513,32 @@ __global__ void __launch_bounds__(256 + 64 * NP) int4_gemm_ring_kernel(RingArgs 
 // Adds the K splits of a launch in a fixed order and applies the epilogue: four columns per thread.
 __global__ void __launch_bounds__(256) ring_finalize_kernel(const float *__restrict__ partial, int splits, int m, int n, void *y,
                                                             int y_dtype, int epi, int ldy, int threads) {
+  typedef float4_t loose4_t __attribute__((aligned(4)));  // (rows of odd widths: a load needs no alignment beyond the element's)
+  typedef half4_t loose_half4_t __attribute__((aligned(2)));
   const int chunks = (n + 3) / 4;
   const size_t total = (size_t)m * chunks;
   for (size_t idx = blockIdx.x * (size_t)256 + threadIdx.x; idx < total; idx += threads) {
     const int row = (int)(idx / chunks), col = (int)(idx % chunks) * 4;
-    const bool whole = col + 4 <= n && (n & 3) == 0;
+    const bool whole = col + 4 <= n;
     float4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int j = 0; j < splits; j++) {
-      const float *src = partial + ((size_t)j * m + row) * n + col;
-      if (whole) {
-        v += *reinterpret_cast<const float4_t *>(src);
-      } else {
+    const float *src = partial + (size_t)row * n + col;
+    const size_t part = (size_t)m * n;
+    if (whole) {
+      int j = 0;
+      for (; j + 4 <= splits; j += 4) {  // four parts on their way at once, added in order
+        const float4_t a = *reinterpret_cast<const loose4_t *>(src), b = *reinterpret_cast<const loose4_t *>(src + part),
+                       c = *reinterpret_cast<const loose4_t *>(src + 2 * part), d = *reinterpret_cast<const loose4_t *>(src + 3 * part);
+        v += a;
+        v += b;
+        v += c;
+        v += d;
+        src += 4 * part;
+      }
+      for (; j < splits; j++, src += part) v += *reinterpret_cast<const loose4_t *>(src);
+    } else {
+      for (int j = 0; j < splits; j++, src += part)
         for (int e = 0; e < 4; e++)
           if (col + e < n) v[e] += src[e];
-      }
     }
     const size_t o = (size_t)row * ldy + col;
     if (epi == EPI_SWIGLU) {
@@ -535,8 +547,14 @@ __global__ void __launch_bounds__(256) ring_finalize_kernel(const float *__restr
       if (col + 2 < n) store_out(y, oh + 1, silu(v[2]) * v[3], y_dtype);
     } else if (epi == EPI_ADD_F32) {
       float *dst = reinterpret_cast<float *>(y) + o;
-      for (int e = 0; e < 4; e++)
-        if (col + e < n) dst[e] += v[e];
+      if (whole) *reinterpret_cast<loose4_t *>(dst) = *reinterpret_cast<const loose4_t *>(dst) + v;
+      else
+        for (int e = 0; e < 4; e++)
+          if (col + e < n) dst[e] += v[e];
+    } else if (whole && y_dtype == YSCV_HIP_F32) {
+      *reinterpret_cast<loose4_t *>(reinterpret_cast<float *>(y) + o) = v;
+    } else if (whole && y_dtype == YSCV_HIP_F16) {
+      *reinterpret_cast<loose_half4_t *>(reinterpret_cast<_Float16 *>(y) + o) = half4_t{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
     } else {
       for (int e = 0; e < 4; e++)
         if (col + e < n) store_out(y, o + e, v[e], y_dtype);
@@ -595,7 +613,7 @@ bool int4_gemm_ring_eligible(const yscv_hip_int4_weight *w, const _Float16 *xh, 
 
 size_t int4_gemm_ring_partial_bytes(const yscv_hip_int4_weight *w, size_t m, int num_cus) {
   if (!w->tiled || m <= 16) return 0;
-  const RingPlan pl = ring_plan(m, w->n, w->kt, (size_t)(num_cus > 0 ? num_cus : 256), w->gm, w->has_zp);
+  const RingPlan pl = int4_plan(m, w->n, w->kt, (size_t)(num_cus > 0 ? num_cus : 256), w->gm, w->has_zp);
   return pl.splits > 1 ? (size_t)pl.splits * m * w->n * sizeof(float) : 0;
 }
 
@@ -627,7 +645,7 @@ int32_t launch_int4_gemm_ring(const yscv_hip_int4_weight *w, const _Float16 *xh,
   const bool sf16 = w->scale_dtype == YSCV_HIP_F16;
   const Context *ctx = nullptr;
   YSCV_TRY(ensure_context(&ctx));
-  const RingPlan pl = ring_plan(m, w->n, w->kt, (size_t)(ctx->num_cus > 0 ? ctx->num_cus : 256), w->gm, w->has_zp);
+  const RingPlan pl = int4_plan(m, w->n, w->kt, (size_t)(ctx->num_cus > 0 ? ctx->num_cus : 256), w->gm, w->has_zp);
   if (pl.splits > 1 && partial != nullptr && partial_bytes >= (size_t)pl.splits * m * w->n * sizeof(float) &&
       (reinterpret_cast<uintptr_t>(partial) & 15) == 0) {
     a.partial = partial;
@@ -635,10 +653,9 @@ int32_t launch_int4_gemm_ring(const yscv_hip_int4_weight *w, const _Float16 *xh,
     a.splits = pl.splits;
   }
   auto launch_shape = [&](int which, const RingArgs &r) {
+    if (which >= kWide)
+      return launch_int4_gemm_wide(w, xh, row_scale, k_pad, y, y_dtype, m, (size_t)r.col0, (size_t)r.n, which - kWide, s, epi, r.splits, r.kt_per, r.partial);
     switch (which) {
-      case 5:
-      case 6:
-      case 7: return launch_int4_gemm_wide(w, xh, row_scale, k_pad, y, y_dtype, m, (size_t)r.col0, (size_t)r.n, wide_tile_blocks(which), s, epi);
       case 4: return ring_launch_gm<2, 4, 2, 6, 8>(r, w->gm, sf16, s);
       case 3: return ring_launch_gm<1, 4, 2, 6, 4>(r, w->gm, sf16, s);
       case 2: return ring_launch_gm<8, 4, 2, 4, 4>(r, w->gm, sf16, s);

@@ -120,10 +120,11 @@ int32_t launch_int4_gemm_ring(const yscv_hip_int4_weight *w, const _Float16 *xh,
                               size_t partial_bytes = 0);
 size_t int4_gemm_ring_partial_bytes(const yscv_hip_int4_weight *w, size_t m, int num_cus);
 
-// The same product in tiles of 256 rows x 16, 14 or 12 column blocks of 16 for columns col0 .. col1 - 1 (multiples of 16, or col1 = n), same conditions
-// (int4_gemm_wide.hip); launch_int4_gemm_ring plans with it.
+// The same product in one of the tiles of int4_gemm_wide.hip (WIDE_*) for columns col0 .. col1 - 1 (multiples of 16, or col1 = n), same
+// conditions; launch_int4_gemm_ring plans with it.  parts > 1: K in parts of kt_per 128-k tiles, all columns, through `partial`.
 int32_t launch_int4_gemm_wide(const yscv_hip_int4_weight *w, const _Float16 *xh, const float *row_scale, size_t ldx, void *y, int y_dtype,
-                              size_t m, size_t col0, size_t col1, int blocks, hipStream_t s, int epi);
+                              size_t m, size_t col0, size_t col1, int tile, hipStream_t s, int epi, int parts = 1, int kt_per = 0,
+                              float *partial = nullptr);
 
 // A few dozen to a few hundred rows of fp16-prepared activations (int4_ksplit.hip): taken while its tiles fit the CUs at once.
 // A launch that is also split over K needs int4_ksplit_partial_bytes() of scratch (at most kKsplitPartialCap; without it the
