@@ -1,4 +1,8 @@
 """The native form of the short Python calls (csrc/calls.cpp) against the general way through ctypes, and what it does not take."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -110,3 +114,13 @@ def test_modes_and_streams_are_seen():
         assert torch.equal(z, y)
     with pytest.raises(RuntimeError):  # a batched tensor has no storage
         torch.vmap(w.matmul)(x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", ["O.rms_norm(x, g, 1e-5)", "O.exec_grouped_query_attention(x, x, x, 1, 1)"])
+def test_the_first_call_of_a_process(call):
+    """Nothing has loaded the library yet: the call goes the general way."""
+    code = ("import torch; from yscv_amd import onnx_ops as O; x, g = torch.ones(1, 4, 64, device='cuda'), torch.ones(64, device='cuda'); "
+            "y = " + call + "; z = " + call + "; torch.cuda.synchronize(); assert bool(((y - 1).abs() < 1e-3).all()) and bool((y == z).all())")
+    run = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), timeout=100)
+    assert run.returncode == 0

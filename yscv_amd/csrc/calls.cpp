@@ -2,8 +2,8 @@
 //
 // A call of one kernel took 6.6 us through ctypes, of which the launch is 2.8, the C ABI 0.4, torch's new_empty from Python 1.5
 // and the rest argument checks and conversions; here the same call takes 4.1.  Every function returns None for a call that it does not
-// take (anything but plain contiguous CUDA tensors of the expected types and shapes, or a torch mode that wants to see the
-// allocation); the Python method then goes its general way, which also raises what there is to raise.  A status other than 0
+// take (anything but plain contiguous CUDA tensors of the expected types and shapes, a torch mode that wants to see the
+// allocation, or no library loaded yet); the Python method then goes its general way, which also raises what there is to raise.  A status other than 0
 // comes back as an int.
 // The entry points are handed over by address (bind), so that this module works on whichever build of the library is loaded.
 #include <ATen/TensorSubclassLikeUtils.h>
@@ -28,7 +28,8 @@ decltype(&yscv_hip_gqa_attention_dev) p_gqa = nullptr;
 
 PyObject *value_name = nullptr;
 
-bool modes_active() { return at::impl::torch_function_mode_enabled() || c10::impl::dispatch_mode_enabled(); }
+// a call from before the library was loaded (the general way loads and binds it), or a torch mode
+bool not_taken() { return p_gqa == nullptr || at::impl::torch_function_mode_enabled() || c10::impl::dispatch_mode_enabled(); }
 
 // the tensor of a plain CUDA argument, else null
 const at::Tensor *plain(PyObject *o) {
@@ -80,7 +81,7 @@ PyObject *result(int32_t st, at::Tensor out) { return st == 0 ? THPVariable_Wrap
 PyObject *int4_matmul(PyObject *, PyObject *const *a, Py_ssize_t na) {
   HANDLE_TH_ERRORS
   int64_t k, n;
-  if (na != 4 || modes_active() || !as_size(a[2], k) || !as_size(a[3], n)) Py_RETURN_NONE;
+  if (na != 4 || not_taken() || !as_size(a[2], k) || !as_size(a[3], n)) Py_RETURN_NONE;
   const at::Tensor *x = plain(a[1]);
   void *w = handle(a[0]);
   if (!x || !w || x->dim() < 1 || x->size(-1) != k) Py_RETURN_NONE;
@@ -111,7 +112,7 @@ PyObject *int8_matmul(PyObject *, PyObject *const *a, Py_ssize_t na) {
   HANDLE_TH_ERRORS
   int64_t k, n;
   void *w;
-  if (na != 5 || modes_active() || !PyLong_CheckExact(a[4])) Py_RETURN_NONE;
+  if (na != 5 || not_taken() || !PyLong_CheckExact(a[4])) Py_RETURN_NONE;
   const at::Tensor *t = int8_rows(a, w, k, n);
   const long zp = PyLong_AsLong(a[4]);
   if (PyErr_Occurred()) PyErr_Clear();
@@ -132,7 +133,7 @@ PyObject *int8_requant(PyObject *, PyObject *const *a, Py_ssize_t na) {
   HANDLE_TH_ERRORS
   int64_t k, n;
   void *w;
-  if (na != 10 || modes_active()) Py_RETURN_NONE;
+  if (na != 10 || not_taken()) Py_RETURN_NONE;
   long v[4];
   const int at_arg[4] = {4, 7, 8, 9};
   for (int i = 0; i < 4; i++) {
@@ -163,7 +164,7 @@ PyObject *int8_requant(PyObject *, PyObject *const *a, Py_ssize_t na) {
 PyObject *dql_matmul(PyObject *, PyObject *const *a, Py_ssize_t na) {
   HANDLE_TH_ERRORS
   int64_t k, n;
-  if (na != 4 || modes_active() || !as_size(a[2], k) || !as_size(a[3], n)) Py_RETURN_NONE;
+  if (na != 4 || not_taken() || !as_size(a[2], k) || !as_size(a[3], n)) Py_RETURN_NONE;
   const at::Tensor *x = plain_f32(a[1]);
   void *w = handle(a[0]);
   if (!x || !w || x->dim() != 2 || x->size(1) != k) Py_RETURN_NONE;
@@ -184,7 +185,7 @@ PyObject *dql_matmul(PyObject *, PyObject *const *a, Py_ssize_t na) {
 // rms_norm(x, gamma, eps)
 PyObject *rms_norm(PyObject *, PyObject *const *a, Py_ssize_t na) {
   HANDLE_TH_ERRORS
-  if (na != 3 || modes_active() || !PyFloat_CheckExact(a[2])) Py_RETURN_NONE;
+  if (na != 3 || not_taken() || !PyFloat_CheckExact(a[2])) Py_RETURN_NONE;
   const at::Tensor *x = plain_f32(a[0]), *g = plain_f32(a[1]);
   if (!x || !g || x->dim() < 1 || g->dim() != 1 || g->size(0) != x->size(-1)) Py_RETURN_NONE;
   const float eps = (float)PyFloat_AS_DOUBLE(a[2]);
@@ -202,7 +203,7 @@ PyObject *rms_norm(PyObject *, PyObject *const *a, Py_ssize_t na) {
 PyObject *gqa(PyObject *, PyObject *const *a, Py_ssize_t na) {
   HANDLE_TH_ERRORS
   int64_t hq, hkv;
-  if (na != 5 || modes_active() || !as_size(a[3], hq) || !as_size(a[4], hkv)) Py_RETURN_NONE;
+  if (na != 5 || not_taken() || !as_size(a[3], hq) || !as_size(a[4], hkv)) Py_RETURN_NONE;
   const at::Tensor *q = plain_f32(a[0]), *k = plain_f32(a[1]), *v = plain_f32(a[2]);
   if (!q || !k || !v || q->dim() != 3 || k->dim() != 3 || v->sizes() != k->sizes()) Py_RETURN_NONE;
   const int64_t B = q->size(0), sq = q->size(1), sk = k->size(1), d = q->size(2) / hq;
