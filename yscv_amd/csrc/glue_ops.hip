@@ -197,41 +197,86 @@ __global__ void __launch_bounds__(64 * GQA_WAVES) gqa_generic_kernel(GqaArgs p) 
   }
 }
 
-// Prompt pass over the decoder's fp16 cache: the four waves of a workgroup take the same key range -- query heads
-// that share a kv head (as many of them as divide four), else neighbouring 32-query ranges of one head -- so a
-// stage of 32 cache positions is fetched once per workgroup into LDS (K rows with their 16-byte pieces XOR-swizzled
+// One step of a running softmax in powers of two over 32 positions for QT row tiles: lane (r, c) has the scores of positions 8 c .. 8 c + 7
+// against row r of tile u, scale2 is the scale with log2(e) in it.  Leaves the weights as fp16 (the B operand of the product with V).  The row
+// tiles' chains are independent and run side by side.  The lanes of a row agree on a new maximum, and the output is rescaled, only in
+// steps where some score passes the running one (weights that stay within 1 .. 2^8 of an older maximum would need that less often, but
+// the largest weight is then no longer exact in fp16: 4 % more error at 512 keys).  l_run is the lane's own part of the sum; the lanes of
+// a row meet behind the last step.
+template <int QT, int DT>
+__device__ __forceinline__ void softmax_step(const float4_t (&sc)[QT][2], float scale2, float (&m_run)[QT], float (&l_run)[QT], float4_t (&o_acc)[QT][DT],
+                                             half8_t (&pf)[QT]) {
+  float mx[QT];
+  bool grows = false;
+#pragma unroll
+  for (int u = 0; u < QT; u++) {
+    mx[u] = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 8; e++) mx[u] = fmaxf(mx[u], sc[u][e >> 2][e & 3]);
+    mx[u] *= scale2;
+    grows = grows || mx[u] > m_run[u];
+  }
+  if (__builtin_amdgcn_ballot_w64(grows) != 0) {
+#pragma unroll
+    for (int u = 0; u < QT; u++) {
+      const float m_new = fmaxf(m_run[u], max_xor16_xor32(mx[u]));
+      const float alpha = m_run[u] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run[u] - m_new);
+      l_run[u] *= alpha;
+      m_run[u] = m_new;
+#pragma unroll
+      for (int t = 0; t < DT; t++) o_acc[u][t] = o_acc[u][t] * alpha;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < QT; u++) {
+    const float m_sub = m_run[u] == -INFINITY ? 0.0f : m_run[u];
+    float pe[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) pe[e] = __builtin_amdgcn_exp2f(fmaf(sc[u][e >> 2][e & 3], scale2, -m_sub));
+    l_run[u] += ((pe[0] + pe[1]) + (pe[2] + pe[3])) + ((pe[4] + pe[5]) + (pe[6] + pe[7]));
+    pf[u] = half8_t{(_Float16)pe[0], (_Float16)pe[1], (_Float16)pe[2], (_Float16)pe[3], (_Float16)pe[4], (_Float16)pe[5], (_Float16)pe[6], (_Float16)pe[7]};
+  }
+}
+
+// Prompt pass over the decoder's fp16 cache: four waves of a workgroup take the same key range -- query heads
+// that share a kv head (as many of them as divide four), else neighbouring query ranges of one head -- so a
+// stage of cache positions is fetched once per workgroup into LDS (K rows with their 16-byte pieces XOR-swizzled
 // so that the 16 rows a fragment read touches fall into 16 different bank groups; V as its slabs lie in memory) and
 // read from there by all four: a quarter of the L2 traffic of waves that fetch for themselves, which bounds such a
-// kernel at prompt lengths in the thousands.  Two stage buffers: the next stage's pieces are requested into registers before
-// this stage's arithmetic and written to the other buffer behind it, one barrier per stage.  Arithmetic per
-// (query, position) as in gqa_generic_kernel; the running output is rescaled only where some query's maximum moved
-// (a factor of exactly one otherwise).
-template <int HD>
-__global__ void __launch_bounds__(64 * GQA_WAVES, 2) gqa_shared_kv_kernel(GqaArgs p, int hw_log2) {
+// kernel at prompt lengths in the thousands.  Two such groups of waves take the halves of a 64-position stage and meet through LDS
+// at the end: with one group the time was that of the last query range's chain of stages, one wave per SIMD, on CUs whose other
+// workgroup was long done.  Two stage buffers: the next stage's pieces are requested into registers before
+// this stage's arithmetic and written to the other buffer behind it, one barrier per stage.  Bound by the chain scores ->
+// softmax -> product of a step, two waves per SIMD.
+// us a launch, one group and a chain per row tile -> this: 2048 queries, 32 heads over 8 of 128 84 -> 59, 700 queries, 16 heads over 2 of
+// 64 21.0 -> 10.6, 150 queries, 32 heads over 8 of 128 11.1 -> 7.8.
+constexpr int SHARED_KG = 2;  // key groups of a workgroup
+template <int HD, int QT>
+__global__ void __launch_bounds__(64 * GQA_WAVES * SHARED_KG, QT == 1 && HD <= 64 ? 4 : 2) gqa_shared_kv_kernel(GqaArgs p, int hw_log2) {
   static_assert(HD % 32 == 0 && HD >= 32 && HD <= 128, "head width");
-  constexpr int KK = HD / 32, DT = HD / 16, QT = 2, KB = 32;  // KB: cache positions per stage
+  constexpr int KK = HD / 32, DT = HD / 16, KB = 32 * SHARED_KG;  // KB: cache positions per stage
   constexpr int CPR = HD / 8;                                  // 16-byte pieces of a K row
   constexpr int PITCH = HD > 64 ? 16 : (HD > 32 ? 8 : 4);      // row pitch in pieces (a power of two)
   constexpr int RPW = 16 / PITCH;                              // rows per 256 bytes
   constexpr int K_BYTES = KB * PITCH * 16, V_BYTES = (KB / 8) * HD * 16, ST_BYTES = K_BYTES + V_BYTES;
   constexpr int K_PIECES = KB * CPR, V_PIECES = (KB / 8) * HD;
-  constexpr int THREADS = 64 * GQA_WAVES;
+  constexpr int THREADS = 64 * GQA_WAVES * SHARED_KG;
   constexpr int K_LD = (K_PIECES + THREADS - 1) / THREADS, V_LD = (V_PIECES + THREADS - 1) / THREADS;
-  __shared__ __attribute__((aligned(16))) uint8_t stage[2 * ST_BYTES];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int MERGE = GQA_WAVES * DT * 1024;  // one row tile of every wave of a key group
+  __shared__ __attribute__((aligned(16))) uint8_t stage[2 * ST_BYTES > MERGE ? 2 * ST_BYTES : MERGE];
+  __shared__ float ml_s[GQA_WAVES][QT][16][2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6 & (GQA_WAVES - 1), kg = tid >> 8;
   const int r = lane & 15, c = lane >> 4;
   const int hw = 1 << hw_log2, qw = GQA_WAVES >> hw_log2;  // heads x query ranges of a workgroup
   const int group = p.Hq / p.Hkv, chunks = group >> hw_log2;
   const int kvh = (int)blockIdx.x / chunks, b = blockIdx.z;
   const int h = kvh * group + ((int)blockIdx.x % chunks) * hw + (wave & (hw - 1));
-  // Workgroups start in the order of blockIdx.y.  The first half takes the late query ranges (most positions), the
-  // second half the early ones in rising order: two workgroups that start half a grid apart, and so tend to share
-  // a CU, carry about the same work together as any other such pair.
-  const int T = gridDim.y, first_half = (T + 1) / 2;
-  const int tile = (int)blockIdx.y < first_half ? T - 1 - (int)blockIdx.y : (int)blockIdx.y - first_half;
+  // Workgroups start in the order of blockIdx.y: the late query ranges (most positions) first, what is left fills the gaps
+  const int tile = (int)(gridDim.y - 1 - blockIdx.y);
   const int q0 = (tile * qw + (wave >> hw_log2)) * 16 * QT;
   const bool active = q0 < p.Sq;
   const int Sk = p.Sk;
+  const float scale2 = p.scale * 1.44269504088896341f;
   int qi[QT], lim_q[QT];
   half8_t qf[QT][KK];
 #pragma unroll
@@ -296,76 +341,52 @@ __global__ void __launch_bounds__(64 * GQA_WAVES, 2) gqa_shared_kv_kernel(GqaArg
   };
   auto compute = [&](int st) {
     const uint8_t *base = stage + (st & 1) * ST_BYTES;
-    const int p0 = st * KB;
+    const int p0 = st * KB + 32 * kg;
     if (active && p0 <= lim_wave) {  // uniform in the wave
       // Two S^T tiles per stage.  Row rho of tile j is stage position 8 (rho / 4) + 4 j + rho % 4, so lane (r, c)
       // ends up with the weights of positions 8c .. 8c+7 (tile 0: the first four, tile 1: the last four): one 16-byte
       // slab piece of V^T per channel, and the B operand of one 32-deep MFMA.
-      half8_t kf[2][KK], vv[DT];
+      half8_t vv[DT], pf[QT];
+      float4_t sc[QT][2];
+      {
+        half8_t kf[2][KK];
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
-        const int row = 8 * (r >> 2) + 4 * j + (r & 3);
+        for (int j = 0; j < 2; j++) {
+          const int row = 8 * (r >> 2) + 4 * j + (r & 3);
+#pragma unroll
+          for (int kk = 0; kk < KK; kk++)
+            kf[j][kk] = *reinterpret_cast<const half8_t *>(base + ((32 * kg + row) * PITCH + ((4 * kk + c) ^ (r / RPW))) * 16);
+        }
+#pragma unroll
+        for (int u = 0; u < QT; u++) sc[u][0] = sc[u][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int kk = 0; kk < KK; kk++)
-          kf[j][kk] = *reinterpret_cast<const half8_t *>(base + (row * PITCH + ((4 * kk + c) ^ (r / RPW))) * 16);
+#pragma unroll
+          for (int u = 0; u < QT; u++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) sc[u][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[j][kk], qf[u][kk], sc[u][j], 0, 0, 0);
       }
 #pragma unroll
-      for (int t = 0; t < DT; t++) vv[t] = *reinterpret_cast<const half8_t *>(base + K_BYTES + (c * HD + 16 * t + r) * 16);
-      if (p0 + KB > Sk) {  // 0 * NaN would poison the sum: positions past the context are blanked
+      for (int t = 0; t < DT; t++) vv[t] = *reinterpret_cast<const half8_t *>(base + K_BYTES + ((4 * kg + c) * HD + 16 * t + r) * 16);
+      if (p0 + 32 > Sk) {  // 0 * NaN would poison the sum: positions past the context are blanked
 #pragma unroll
         for (int t = 0; t < DT; t++)
 #pragma unroll
           for (int e = 0; e < 8; e++)
             if (p0 + 8 * c + e >= Sk) vv[t][e] = (_Float16)0.0f;
       }
+      if (p0 + 31 > lim_first) {  // uniform in the wave: some query does not see the whole stage
 #pragma unroll
-      for (int u = 0; u < QT; u++) {
-        float4_t s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int u = 0; u < QT; u++)
 #pragma unroll
-        for (int kk = 0; kk < KK; kk++) {
-          s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[0][kk], qf[u][kk], s0, 0, 0, 0);
-          s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[1][kk], qf[u][kk], s1, 0, 0, 0);
-        }
-        float sv[8], mx = -INFINITY, pe[8], sum = 0.0f, m_new;
-        if (p0 + KB - 1 <= lim_first) {  // uniform in the wave: every query of the wave sees the whole stage
-#pragma unroll
-          for (int e = 0; e < 8; e++) {
-            sv[e] = (e < 4 ? s0[e & 3] : s1[e & 3]) * p.scale;
-            mx = fmaxf(mx, sv[e]);
-          }
-          m_new = fmaxf(m_run[u], max_xor16_xor32(mx));
-#pragma unroll
-          for (int e = 0; e < 8; e++) {
-            pe[e] = __expf(sv[e] - m_new);
-            sum += pe[e];
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; e++) {
-            const float raw = (e < 4 ? s0[e & 3] : s1[e & 3]) * p.scale;
-            sv[e] = (p0 + 8 * c + e <= lim_q[u]) ? raw : -INFINITY;
-            mx = fmaxf(mx, sv[e]);
-          }
-          m_new = fmaxf(m_run[u], max_xor16_xor32(mx));
-#pragma unroll
-          for (int e = 0; e < 8; e++) {
-            pe[e] = (sv[e] == -INFINITY) ? 0.0f : __expf(sv[e] - m_new);
-            sum += pe[e];
-          }
-        }
-        sum = sum_xor16_xor32(sum);
-        const float alpha = (m_run[u] == -INFINITY) ? 0.0f : __expf(m_run[u] - m_new);
-        l_run[u] = l_run[u] * alpha + sum;
-        m_run[u] = m_new;
-        const half8_t pf = {(_Float16)pe[0], (_Float16)pe[1], (_Float16)pe[2], (_Float16)pe[3],
-                            (_Float16)pe[4], (_Float16)pe[5], (_Float16)pe[6], (_Float16)pe[7]};
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-#pragma unroll
-          for (int t = 0; t < DT; t++) o_acc[u][t] = o_acc[u][t] * alpha;
-        }
-#pragma unroll
-        for (int t = 0; t < DT; t++) o_acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[t], pf, o_acc[u][t], 0, 0, 0);
+          for (int e = 0; e < 8; e++)
+            if (p0 + 8 * c + e > lim_q[u]) sc[u][e >> 2][e & 3] = -INFINITY;
       }
+      softmax_step<QT, DT>(sc, scale2, m_run, l_run, o_acc, pf);
+#pragma unroll
+      for (int t = 0; t < DT; t++)
+#pragma unroll
+        for (int u = 0; u < QT; u++) o_acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[t], pf[u], o_acc[u][t], 0, 0, 0);
     }
   };
   uint4_t kr[K_LD], vr[V_LD];
@@ -379,16 +400,36 @@ __global__ void __launch_bounds__(64 * GQA_WAVES, 2) gqa_shared_kv_kernel(GqaArg
     if (more) stash((st + 1) & 1, kr, vr);
     __syncthreads();
   }
-  if (!active) return;
+#pragma unroll
+  for (int u = 0; u < QT; u++) l_run[u] = sum_xor16_xor32(l_run[u]);
+  // the second key group's part meets the first one's, a row tile at a time, lane by lane
+  const float4_t *o_other = reinterpret_cast<const float4_t *>(stage) + wave * DT * 64 + lane;
   _Float16 *obase = static_cast<_Float16 *>(p.out) + (size_t)b * p.o_b + (size_t)h * HD;
+  if (kg == 1 && c == 0) {
+#pragma unroll
+    for (int u = 0; u < QT; u++) {
+      ml_s[wave][u][r][0] = m_run[u];
+      ml_s[wave][u][r][1] = l_run[u];
+    }
+  }
 #pragma unroll
   for (int u = 0; u < QT; u++) {
-    if (q0 + 16 * u + r >= p.Sq) continue;
-    const float inv = l_run[u] > 0.0f ? 1.0f / l_run[u] : 0.0f;
+    if (u > 0) __syncthreads();
+    if (kg == 1) {
+#pragma unroll
+      for (int t = 0; t < DT; t++) const_cast<float4_t *>(o_other)[t * 64] = o_acc[u][t];
+    }
+    __syncthreads();
+    if (kg == 1 || !active || q0 + 16 * u + r >= p.Sq) continue;
+    const float m1 = ml_s[wave][u][r][0], l1 = ml_s[wave][u][r][1], m = fmaxf(m_run[u], m1), m_sub = m == -INFINITY ? 0.0f : m;
+    const float f0 = __builtin_amdgcn_exp2f(m_run[u] - m_sub), f1 = __builtin_amdgcn_exp2f(m1 - m_sub), l = l_run[u] * f0 + l1 * f1;
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     _Float16 *orow = obase + (size_t)(q0 + 16 * u + r) * p.o_s;
 #pragma unroll
-    for (int t = 0; t < DT; t++)
-      store4<_Float16>(orow + 16 * t + 4 * c, o_acc[u][t][0] * inv, o_acc[u][t][1] * inv, o_acc[u][t][2] * inv, o_acc[u][t][3] * inv);
+    for (int t = 0; t < DT; t++) {
+      const float4_t o = (o_acc[u][t] * f0 + o_other[t * 64] * f1) * inv;
+      store4<_Float16>(orow + 16 * t + 4 * c, o[0], o[1], o[2], o[3]);
+    }
   }
 }
 
@@ -397,15 +438,24 @@ inline int shared_kv_hw_log2(int group) { return group % 4 == 0 ? 2 : (group % 2
 
 int32_t gqa_launch_shared_kv(const GqaArgs &a, int hd, hipStream_t s) {
   const int hw_log2 = shared_kv_hw_log2(a.Hq / a.Hkv);
-  const int q_per_wg = 32 * (GQA_WAVES >> hw_log2);
-  const dim3 grid((unsigned)(a.Hq >> hw_log2), (unsigned)((a.Sq + q_per_wg - 1) / q_per_wg), (unsigned)a.B), block(64 * GQA_WAVES);
+  // 32 queries per wave where that fills the CUs, else 16: twice the workgroups, shorter steps (700 queries, 16 heads over 2 of 64:
+  // 88 workgroups of 32)
+  const unsigned heads = (unsigned)(a.Hq >> hw_log2) * (unsigned)a.B, waves_q = (unsigned)(GQA_WAVES >> hw_log2);
+  const bool two = heads * ((a.Sq + 32 * waves_q - 1) / (32 * waves_q)) >= 256;
+  const unsigned q_per_wg = (two ? 32 : 16) * waves_q;
+  const dim3 grid((unsigned)(a.Hq >> hw_log2), (a.Sq + q_per_wg - 1) / q_per_wg, (unsigned)a.B), block(64 * GQA_WAVES * SHARED_KG);
+#define YSCV_SHARED_KV(HD)                                                                      \
+  if (two) hipLaunchKernelGGL((gqa_shared_kv_kernel<HD, 2>), grid, block, 0, s, a, hw_log2);    \
+  else hipLaunchKernelGGL((gqa_shared_kv_kernel<HD, 1>), grid, block, 0, s, a, hw_log2);        \
+  break
   switch (hd) {
-    case 32: hipLaunchKernelGGL((gqa_shared_kv_kernel<32>), grid, block, 0, s, a, hw_log2); break;
-    case 64: hipLaunchKernelGGL((gqa_shared_kv_kernel<64>), grid, block, 0, s, a, hw_log2); break;
-    case 96: hipLaunchKernelGGL((gqa_shared_kv_kernel<96>), grid, block, 0, s, a, hw_log2); break;
-    case 128: hipLaunchKernelGGL((gqa_shared_kv_kernel<128>), grid, block, 0, s, a, hw_log2); break;
+    case 32: YSCV_SHARED_KV(32);
+    case 64: YSCV_SHARED_KV(64);
+    case 96: YSCV_SHARED_KV(96);
+    case 128: YSCV_SHARED_KV(128);
     default: return set_error(YSCV_HIP_ERR_UNSUPPORTED, "attention: head width %d (supported: 32, 64, 96, 128)", hd);
   }
+#undef YSCV_SHARED_KV
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
@@ -436,8 +486,8 @@ int32_t gqa_launch_cache(const GqaArgs &a, int hd, hipStream_t s) {
 // grid too, with the partial results merged by a second kernel: one query x 2048 keys 9.5 + 5.7 us.
 // PRE: where several workgroups share a kv head, its stages are converted once by a kernel in front (3.2 us for 512 keys of 8
 // heads), travel to LDS by LDS-direct loads ahead of their use, and sixteen waves of one row tile each work on them: 512 queries
-// x 512 keys, 32 heads over 8 of 128: 18.3 -> 14.0 us in all.  Its 10 us: 1.9 until the first stage and q are there, 6.5 of stages,
-// 1.7 the merge and the stores.
+// x 512 keys, 32 heads over 8 of 128: 18.3 -> 14.0 us in all, 13.0 with the row tiles' softmax side by side and no rescaling in steps
+// that need none.  Its 10 us: 1.9 until the first stage and q are there, 6 of stages, 1.7 the merge and the stores.
 // QT: row tiles per wave; RW 1 is the form for few rows (wave-private stages: no barrier in the loop).
 template <int HD, int RW, int QT, bool PRE = false>
 struct FlatCfg {
@@ -712,6 +762,7 @@ __global__ void __launch_bounds__((FlatCfg<HD, RW, QT, PRE>::THREADS)) gqa_flat_
 #pragma unroll
       for (int t = 0; t < DT; t++) vv[t] = *reinterpret_cast<const half8_t *>(base + C::K_BYTES + ((sub * 4 + c) * HD + 16 * t + r) * 16);
     };
+    float4_t sc[QT][2];
     {
       half8_t kf[2][KK];
 #pragma unroll
@@ -721,58 +772,36 @@ __global__ void __launch_bounds__((FlatCfg<HD, RW, QT, PRE>::THREADS)) gqa_flat_
         for (int kk = 0; kk < KK; kk++)
           kf[j][kk] = *reinterpret_cast<const half8_t *>(base + ((sub * 32 + row) * PITCH + ((4 * kk + c) ^ (r / RPW))) * 16);
       }
-      const bool tail = p0 + 32 > p.Sk;  // uniform
 #pragma unroll
-      for (int u = 0; u < QT; u++) {
-        float4_t s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int u = 0; u < QT; u++) sc[u][0] = sc[u][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int kk = 0; kk < KK; kk++) {
-          s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[0][kk], qf[u][kk], s0, 0, 0, 0);
-          s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[1][kk], qf[u][kk], s1, 0, 0, 0);
-        }
-        if constexpr (V_EARLY) {
-          __builtin_amdgcn_sched_barrier(0);
-          read_v();
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        // softmax in powers of two: the scale (log2(e) in it) and the maximum go into one fma per score
-        float sv[8], mx = -INFINITY, pe[8], sum = 0.0f;
+      for (int kk = 0; kk < KK; kk++)
 #pragma unroll
-        for (int e = 0; e < 8; e++) sv[e] = e < 4 ? s0[e & 3] : s1[e & 3];
-        if (tail) {
+        for (int u = 0; u < QT; u++)
 #pragma unroll
-          for (int e = 0; e < 8; e++)
-            if (p0 + 8 * c + e >= p.Sk) sv[e] = -INFINITY;  // (an existing key's scores repeated)
-        }
-#pragma unroll
-        for (int e = 0; e < 8; e++) mx = fmaxf(mx, sv[e]);
-        const float m_new = fmaxf(m_run[u], max_xor16_xor32(mx) * p.scale);
-        const float m_sub = m_new == -INFINITY ? 0.0f : m_new;
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          pe[e] = __builtin_amdgcn_exp2f(fmaf(sv[e], p.scale, -m_sub));
-          sum += pe[e];
-        }
-        sum = sum_xor16_xor32(sum);
-        const float alpha = __builtin_amdgcn_exp2f(m_run[u] - m_sub);
-        l_run[u] = l_run[u] * alpha + sum;
-        m_run[u] = m_new;
-        pf[u] = half8_t{(_Float16)pe[0], (_Float16)pe[1], (_Float16)pe[2], (_Float16)pe[3],
-                        (_Float16)pe[4], (_Float16)pe[5], (_Float16)pe[6], (_Float16)pe[7]};
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-#pragma unroll
-          for (int t = 0; t < DT; t++) o_acc[u][t] = o_acc[u][t] * alpha;
-        }
-      }
+          for (int j = 0; j < 2; j++) sc[u][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[j][kk], qf[u][kk], sc[u][j], 0, 0, 0);
     }
+    if constexpr (V_EARLY) {
+      __builtin_amdgcn_sched_barrier(0);
+      read_v();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (p0 + 32 > p.Sk) {  // uniform
+#pragma unroll
+      for (int u = 0; u < QT; u++)
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          if (p0 + 8 * c + e >= p.Sk) sc[u][e >> 2][e & 3] = -INFINITY;  // (an existing key's scores repeated)
+    }
+    softmax_step<QT, DT>(sc, p.scale, m_run, l_run, o_acc, pf);
     if constexpr (!V_EARLY) {
       __builtin_amdgcn_sched_barrier(0);
       read_v();
     }
 #pragma unroll
-    for (int u = 0; u < QT; u++)
+    for (int t = 0; t < DT; t++)
 #pragma unroll
-      for (int t = 0; t < DT; t++) o_acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[t], pf[u], o_acc[u][t], 0, 0, 0);
+      for (int u = 0; u < QT; u++) o_acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[t], pf[u], o_acc[u][t], 0, 0, 0);
   };
   auto compute = [&](int stage_index, int buf) {
     if (!active) return;
@@ -814,6 +843,8 @@ __global__ void __launch_bounds__((FlatCfg<HD, RW, QT, PRE>::THREADS)) gqa_flat_
     }
   }
 
+#pragma unroll
+  for (int u = 0; u < QT; u++) l_run[u] = sum_xor16_xor32(l_run[u]);
   // lane (r, c) holds O^T[16 t + 4c + e][row r]
   const size_t part_row0 = ((size_t)nb * p.gs + gs) * p.R;
   if constexpr (KS == 1) {
