@@ -879,13 +879,17 @@ SkinnyPlan plan_int4_skinny(const yscv_hip_int4_weight *w, size_t m, int split, 
   (void)split;
   SkinnyPlan p;
   p.tpw = TPW;
-  const int max_waves = 8;  // 8 waves x <= 256 VGPRs: one workgroup per CU
+  const int max_waves = 8;  // of a CU, x <= 256 VGPRs
   const int slices = (int)(w->ktp / TPW);
   p.ksg = (int)ceil_div((size_t)slices, (size_t)max_waves);
   p.waves = (int)ceil_div((size_t)slices, (size_t)p.ksg);
   int gx = (int)w->nt;
-  const int cap = num_cus > 0 ? num_cus : 256;
-  // one resident workgroup per CU and k-split slice; more blocks than that loop inside the kernel
+  // One resident workgroup per CU and k-split slice; more blocks than that loop inside the kernel.  Workgroups of one or two waves (K up
+  // to 1024) come as eight waves to a CU, two per SIMD at up to 256 VGPRs, less what groups of 16 rows side by side bring: 151936 x 1024,
+  // 6 f32 rows 65 -> 28 us, 114181 x 896, 13 rows 37 -> 19.5, 5632 x 1024, 16 rows 6.4 -> 5.3.  With three or four waves a second workgroup
+  // repeats the set-up of the first: 7774 x 1920, 15 rows 7.5 -> 8.7, 9000 x 1312, 16 rows 8.7 -> 9.2, 40000 x 2048, 8 rows no change.
+  const int side_by_side = (int)ceil_div(m, (size_t)16) * (p.waves <= 2 ? p.waves : max_waves);
+  const int cap = (num_cus > 0 ? num_cus : 256) * std::max(1, max_waves / side_by_side);
   int per = cap / p.ksg;
   if (per < 1) per = 1;
   if (gx > per) {
