@@ -19,7 +19,8 @@ constexpr bool wide_tile_built(int gm, bool has_zp, int blocks) {
 }
 
 // Tile shapes: 0 = 128 x 128, 1 = 128 x 256, 2 = 256 x 128 (m > 128), 3 = 32 x 128 (m <= 32), 4 = 64 x 128 (m <= 64),
-// 5, 6, 7 = 256 x 256, 256 x 224, 256 x 192 (m > 256): the work is one for the tiles of int4_gemm_wide.hip, which int4_plan deals out
+// 5, 6, 7 = 256 x 256, 256 x 224, 256 x 192 (m > 256).  The ring kernel has 0, 3 and 4; where the others are the cheapest, int4_plan names
+// tiles of int4_gemm_wide.hip
 struct RingPlan {
   int one;           // shape of the launch, or of the first of two launches
   int second;        // < 0: one launch; else the shape of the launch that takes the columns from split_col on
@@ -141,11 +142,11 @@ inline double tile_rounds_us(const TileTime &t, size_t tiles, size_t kt, size_t 
   const double last = rest == 0 ? 0.0 : (full * (double)rest / (double)cus > fast ? full * (double)rest / (double)cus : fast);
   return (double)(tiles / cus) * full + last;
 }
-// fitted to 128 .. 2048 rows, N 2049 .. 28672, K 1024 and 4096, fp16 rows, groups of 32; the ring kernel's tiles for comparison
+// fitted to 128 .. 2048 rows, N 2049 .. 28672, K 1024 and 4096, fp16 rows, groups of 32; the ring kernel's tiles of 128 and 64 rows for
+// comparison
 constexpr TileTime kWideTime[WIDE_TILES] = {
     {256, 256, 8.0, 2.90, 5.5, 2.12}, {256, 192, 5.5, 2.34, 4.5, 1.74}, {128, 256, 5.5, 1.56, 4.5, 1.25}, {128, 192, 4.8, 1.52, 4.2, 1.06}};
-constexpr TileTime kRingTime[5] = {
-    {128, 128, 1.5, 1.06, 1.5, 1.06}, {128, 256, 8.0, 2.0, 8.0, 2.0}, {256, 128, 8.0, 1.9, 8.0, 1.9}, {32, 128, 1.5, 0.6, 1.5, 0.6}, {64, 128, 1.5, 0.76, 1.5, 0.76}};
+constexpr TileTime kRingTime[2] = {{128, 128, 1.5, 1.06, 1.5, 1.06}, {64, 128, 1.5, 0.76, 1.5, 0.76}};
 
 // The plan of a launch: ring_plan's, or tiles of int4_gemm_wide.hip where their estimated time is shorter.  From 65 rows on (a
 // 128-row tile decodes a weight once for all of them; the 64-row ring tile is half of one).  us of the op, ring plan -> this one, fp16
@@ -158,12 +159,10 @@ inline RingPlan int4_plan(size_t m, size_t n, size_t kt, size_t cus, int gm, boo
   auto tiles_of = [&](const TileTime &t, size_t cols) { return plan_ceil_div(m, t.bm) * plan_ceil_div(cols, t.bn); };
   auto sum_us = [&](size_t parts) { return kSumLaunch + (double)(parts * m * n * 8) / 4e6; };  // partial products out and in
   double best = 1e30;
-  if (ring.one < 5 && ring.second < 5) {
-    if (ring.splits > 1) best = tile_rounds_us(kRingTime[ring.one], tiles_of(kRingTime[ring.one], n) * ring.splits, (size_t)ring.kt_per, cus) + sum_us((size_t)ring.splits);
-    else if (ring.second < 0) best = tile_rounds_us(kRingTime[ring.one], tiles_of(kRingTime[ring.one], n), kt, cus);
-    else
-      best = tile_rounds_us(kRingTime[ring.one], tiles_of(kRingTime[ring.one], ring.split_col), kt, cus) +
-             tile_rounds_us(kRingTime[ring.second], tiles_of(kRingTime[ring.second], n - ring.split_col), kt, cus) + kSecondLaunch;
+  // (its larger tiles and its second launches never beat these)
+  if ((ring.one == 0 || ring.one == 4) && ring.second < 0) {
+    const TileTime &t = ring.one == 0 ? kRingTime[0] : kRingTime[1];
+    best = tile_rounds_us(t, tiles_of(t, n) * (size_t)ring.splits, (size_t)ring.kt_per, cus) + (ring.splits > 1 ? sum_us((size_t)ring.splits) : 0.0);
   }
   RingPlan pl = ring;
   const size_t x_bytes = m * kt * 128 * 2, cap = x_bytes >= ((size_t)31 << 20) ? 0 : (((size_t)31 << 20) - x_bytes < ((size_t)16 << 20) ? ((size_t)31 << 20) - x_bytes : (size_t)16 << 20);

@@ -1,8 +1,8 @@
 // Wide-M packed-int4 matmul for fp16 / bf16 activations: y[m][n] = sum_k x[m][k] * W[n][k], MFMA-bound design.
 // Replaces packed_int4_gemm_dispatch (crates/yscv-kernels/src/ops/int4_matmul.rs:548-605) for prefill-sized m.
 //
-// A workgroup owns a (32 MT) x (32 NT) tile of y: 32, 64 or 128 rows by 128 columns by m, or 128 x 256 / 256 x 128
-// where such tiles still fill the CUs in whole rounds.  It has four MMA waves (2 x 2, MT x NT MFMA tiles each) and NP producer waves.  Per stage of KS k-steps (32 k each) the producers
+// A workgroup owns a (32 MT) x (32 NT) tile of y: 32, 64 or 128 rows by 128 columns, by m (larger tiles: int4_gemm_wide.hip).
+// It has four MMA waves (2 x 2, MT x NT MFMA tiles each) and NP producer waves.  Per stage of KS k-steps (32 k each) the producers
 //   * fetch the activation rows (fp16, prepared by x_prep) with LDS-direct loads, one 16-byte piece per lane: an
 //     instruction takes eight whole 128-byte lines (eight rows x both k-steps of the stage), and a per-row XOR of
 //     the chunk index makes the later fragment reads conflict-free, so the row-major -> MFMA-fragment
@@ -658,9 +658,8 @@ int32_t launch_int4_gemm_ring(const yscv_hip_int4_weight *w, const _Float16 *xh,
     switch (which) {
       case 4: return ring_launch_gm<2, 4, 2, 6, 8>(r, w->gm, sf16, s);
       case 3: return ring_launch_gm<1, 4, 2, 6, 4>(r, w->gm, sf16, s);
-      case 2: return ring_launch_gm<8, 4, 2, 4, 4>(r, w->gm, sf16, s);
-      case 1: return ring_launch_gm<4, 8, 2, 4, 4>(r, w->gm, sf16, s);
-      default: return ring_launch_gm<4, 4, 2, 6, 8>(r, w->gm, sf16, s);
+      case 0: return ring_launch_gm<4, 4, 2, 6, 8>(r, w->gm, sf16, s);
+      default: return set_error(YSCV_HIP_ERR_INVALID_ARG, "no tile of shape %d", which);
     }
   };
   if (pl.second < 0) return launch_shape(pl.one, a);
