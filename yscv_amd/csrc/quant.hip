@@ -115,19 +115,22 @@ int32_t launch_requant(const int32_t *acc, size_t len, size_t c, const int32_t *
 // Both passes take four values per load where x allows it, four loads ahead (VEC): a loop of single values waits for each of
 // them in turn.  With the GEMM behind them, 1024 x 4096 values 41.5 -> 37.7 us, 1000 x 8192 107.6 -> 98.5.
 constexpr int DQL_BLOCKS = 1024;
+// values that a workgroup goes through for itself: with the GEMM behind it, 18 000 values 10.5 -> 9.4 and
+// 11.4 -> 10.8 us, 37 000 11.7 -> 11.8
+constexpr size_t kDqlOwn = 24576;
 
 // the values of x this thread takes, f(index, value) for each of them, in batches of four loads
-template <bool VEC, typename F>
-__device__ __forceinline__ void dql_each(const float *__restrict__ x, size_t len, int blocks, F f) {
-  const size_t step = (size_t)blocks * 256, first = blockIdx.x * (size_t)256 + threadIdx.x;
+template <bool VEC, int BATCH = 4, typename F>
+__device__ __forceinline__ void dql_each(const float *__restrict__ x, size_t len, int block, int blocks, F f) {
+  const size_t step = (size_t)blocks * 256, first = block * (size_t)256 + threadIdx.x;
   if constexpr (VEC) {
     const size_t n4 = len / 4;
-    for (size_t i = first; i < n4; i += 4 * step) {
-      float4_t v[4];
+    for (size_t i = first; i < n4; i += BATCH * step) {
+      float4_t v[BATCH];
 #pragma unroll
-      for (int u = 0; u < 4; u++) v[u] = reinterpret_cast<const float4_t *>(x)[min(i + u * step, n4 - 1)];
+      for (int u = 0; u < BATCH; u++) v[u] = reinterpret_cast<const float4_t *>(x)[min(i + u * step, n4 - 1)];
 #pragma unroll
-      for (int u = 0; u < 4; u++)
+      for (int u = 0; u < BATCH; u++)
         if (i + u * step < n4) f(i + u * step, v[u]);
     }
   } else {
@@ -144,7 +147,7 @@ __global__ void __launch_bounds__(256) dql_minmax_kernel(const float *__restrict
     if (v < mn) mn = v;  // comparisons, not fmin: NaN never wins, as in misc.rs:250-256
     if (v > mx) mx = v;
   };
-  dql_each<VEC>(x, len, blocks, [&](size_t, const auto &v) {
+  dql_each<VEC>(x, len, (int)blockIdx.x, blocks, [&](size_t, const auto &v) {
     if constexpr (VEC) {
 #pragma unroll
       for (int e = 0; e < 4; e++) take(v[e]);
@@ -172,17 +175,28 @@ __global__ void __launch_bounds__(256) dql_minmax_kernel(const float *__restrict
   }
 }
 
-template <typename T, bool VEC>
+// OWN: few values (kDqlOwn): every workgroup takes the minimum and maximum of all of them itself, from L2, instead of a launch in front
+template <typename T, bool VEC, bool OWN>
 __global__ void __launch_bounds__(256) dql_quantize_kernel(const float *__restrict__ x, size_t len,
                                                            const float *__restrict__ minmax, int nparts,
                                                            T *__restrict__ y, float *__restrict__ scale_out,
                                                            float *__restrict__ zp_out) {
   __shared__ float smin[4], smax[4];
   float mn = 3.40282347e+38f, mx = -3.40282347e+38f;
-  for (int i = threadIdx.x; i < nparts; i += 256) {
-    float a = minmax[2 * i], b = minmax[2 * i + 1];
-    if (a < mn) mn = a;
-    if (b > mx) mx = b;
+  if constexpr (OWN) {
+    dql_each<VEC, 8>(x, len, 0, 1, [&](size_t, const float4_t &v) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        if (v[e] < mn) mn = v[e];
+        if (v[e] > mx) mx = v[e];
+      }
+    });
+  } else {
+    for (int i = threadIdx.x; i < nparts; i += 256) {
+      float a = minmax[2 * i], b = minmax[2 * i + 1];
+      if (a < mn) mn = a;
+      if (b > mx) mx = b;
+    }
   }
   for (int off = 32; off > 0; off >>= 1) {
     float a = __shfl_xor(mn, off, 64), b = __shfl_xor(mx, off, 64);
@@ -211,7 +225,7 @@ __global__ void __launch_bounds__(256) dql_quantize_kernel(const float *__restri
     *zp_out = zp;
   }
   auto one = [&](float v) { return (uint8_t)clamp_cast(round_half_away_f(__fadd_rn(__fdiv_rn(v, scale), zp)), 0.0f, 255.0f); };
-  dql_each<VEC>(x, len, nparts, [&](size_t i, const auto &v) {
+  dql_each<VEC>(x, len, (int)blockIdx.x, nparts, [&](size_t i, const auto &v) {
     if constexpr (VEC) {
       typedef T vec4 __attribute__((ext_vector_type(4)));
       reinterpret_cast<vec4 *>(y)[i] = vec4{(T)one(v[0]), (T)one(v[1]), (T)one(v[2]), (T)one(v[3])};
@@ -236,18 +250,23 @@ int32_t launch_dynamic_quantize_linear(const float *x, size_t len, void *y, bool
     partial = own.as<float>();
   }
   const bool vec = len % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
-  auto go = [&](auto VEC) -> int32_t {
-    constexpr bool V = decltype(VEC)::value;
-    hipLaunchKernelGGL(dql_minmax_kernel<V>, dim3(blocks), dim3(256), 0, s, x, len, partial, blocks);
-    YSCV_HIP_TRY(hipGetLastError());
+  auto quantize = [&](auto VEC, auto OWN) -> int32_t {
+    constexpr bool V = decltype(VEC)::value, O = decltype(OWN)::value;
     if (y_f32)
-      hipLaunchKernelGGL((dql_quantize_kernel<float, V>), dim3(blocks), dim3(256), 0, s, x, len, partial, blocks, static_cast<float *>(y), scale_out, zp_out);
+      hipLaunchKernelGGL((dql_quantize_kernel<float, V, O>), dim3(blocks), dim3(256), 0, s, x, len, partial, blocks, static_cast<float *>(y), scale_out, zp_out);
     else
-      hipLaunchKernelGGL((dql_quantize_kernel<uint8_t, V>), dim3(blocks), dim3(256), 0, s, x, len, partial, blocks, static_cast<uint8_t *>(y), scale_out, zp_out);
+      hipLaunchKernelGGL((dql_quantize_kernel<uint8_t, V, O>), dim3(blocks), dim3(256), 0, s, x, len, partial, blocks, static_cast<uint8_t *>(y), scale_out, zp_out);
     YSCV_HIP_TRY(hipGetLastError());
     return YSCV_HIP_OK;
   };
-  return vec ? go(std::true_type()) : go(std::false_type());
+  // (one launch reads what another workgroup may already have written, were y to lie on x)
+  const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
+  const bool apart = ya + len * (y_f32 ? 4 : 1) <= xa || xa + len * 4 <= ya;
+  if (vec && apart && len > 0 && len <= kDqlOwn) return quantize(std::true_type(), std::true_type());
+  if (vec) hipLaunchKernelGGL(dql_minmax_kernel<true>, dim3(blocks), dim3(256), 0, s, x, len, partial, blocks);
+  else hipLaunchKernelGGL(dql_minmax_kernel<false>, dim3(blocks), dim3(256), 0, s, x, len, partial, blocks);
+  YSCV_HIP_TRY(hipGetLastError());
+  return vec ? quantize(std::true_type(), std::false_type()) : quantize(std::false_type(), std::false_type());
 }
 
 // ---- KV-cache int8 storage: per-row symmetric quantisation (crates/yscv-onnx/src/runner/kv_cache.rs:45-61) ----
