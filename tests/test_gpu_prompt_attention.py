@@ -1,5 +1,5 @@
 """Attention of long prompts: 32 queries per wave (a pass that fills the CUs with them) against 16 (the same prompt in shorter passes,
-which the checker's tests cover).  The second layer's cache rows depend on the first layer's attention at their position; both forms round
+which the oracle's tests cover).  The second layer's cache rows depend on the first layer's attention at their position; both forms round
 weights and outputs to fp16, so rows agree to a few of those."""
 import numpy as np
 import pytest
