@@ -53,3 +53,34 @@ def test_against_float64(heads, batch, max_ctx, positions):
         k = np.nan_to_num(k)
         v = np.nan_to_num(v)
     dec.close()
+
+
+def test_weights_of_shares_at_large_scores():
+    """Every key of a share is the same row or zero, so its weights are exactly 1 or 0 and only the meeting of the shares can round: with
+    values of +1 in one share and -1 in the other the result is (n0 - n1) / (n0 + n1) whatever the score, which reaches 1e5 here (a log
+    of the weights' sum in f32 would be off by 2^-8 there)."""
+    nh, nkv, hd = heads = (16, 2, 64)
+    batch, max_ctx, pos = 3, 4224, 1024
+    dec = _decoder(heads, batch, max_ctx)
+    tokens = (np.arange(batch) * 7 + 3).astype(np.int32)
+    dec.reset(tokens, pos)
+    dec.run(1)
+    q = dec.activation("qkv")[:, : nh * hd].reshape(batch, nkv, nh // nkv, hd).astype(np.float64)
+    # along the first head of each kv head, of a size that brings its score to 1e5
+    k0 = q[:, :, 0] / (q[:, :, 0] ** 2).sum(-1, keepdims=True) * 1e5 * math.sqrt(hd)
+    assert np.abs(k0).max() < 65504
+    k = np.repeat(k0.astype(np.float16)[:, None], max_ctx - 8, axis=1)
+    v = np.ones_like(k)
+    k[:, 300:512] = 0  # 300 keys that count against 512
+    v[:, 512:1024] = -1
+    dec.set_kv(0, k, v)
+    for use_graph in (False, True):
+        dec.reset(tokens, pos)
+        dec.run(1, use_graph=use_graph)
+        got = dec.activation("attn_out").reshape(batch, nkv, nh // nkv, hd).astype(np.float64)
+        scores = (q * k[:, 0].astype(np.float64)[:, :, None]).sum(-1) / math.sqrt(hd)
+        large = scores > 1000.0  # (the token's own key, and zero keys, have no weight there)
+        assert large[:, :, 0].all()
+        want = (300.0 - 512.0) / 812.0
+        assert np.abs(got[large] - want).max() <= 2.0 ** -11 * abs(want) * 1.01, np.abs(got[large] - want).max()  # one rounding to fp16
+    dec.close()

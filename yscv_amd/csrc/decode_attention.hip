@@ -8,10 +8,14 @@
 //   S^T = K Q^T   a block's K rows are the A operand; row i of tile u is position 8 (i / 4) + 4 u + i % 4, so that a lane ends
 //                 up with the weights of eight consecutive positions of one query head, which is
 //   O^T += V^T P^T  the B operand here; A is a slab piece of the cache as it lies (eight positions of a channel).
-// Shares of one kv head meet pairwise, element by element: a thread exchanges its {value, log of the weights' sum} with a slot; who
-// finds the slot empty leaves, who finds the partner's pair merges (always in the order of the positions), empties the slot and goes on
-// to the next level.  One trip to memory per level (1.1 us), nobody waits, and nothing but the words themselves has to be ordered.
-// (Partials through agent-scope stores, an arrival counter and a last workgroup that reads them back: three trips, 5 us.)
+// Shares of one kv head meet pairwise, two channels of a head at a time: a thread exchanges {maximum, sum of weights} with the first word of
+// a slot and, once that is there, its two sums of weighted values with the second.  Who finds the second word empty leaves; who finds it
+// full has the partner's first word, too, or finds it in the slot by now; it merges (always in the order of the positions), empties the
+// slot and goes on to the next level.  Nobody waits for another workgroup.  Two trips to memory per level (1.1 us each), the first of the
+// first level behind the merge of the waves; maximum and sum stay two f32, so that a share's weight is exact whatever the size of the
+// scores.  ({value, log of the weights' sum} in one word is one trip, a step of the 7B shape at 16 sequences 0.3 % shorter, and
+// weights that are off by |score| 2^-24.  Partials through agent-scope stores, an arrival counter and a last workgroup that reads them
+// back: three trips, 5 us.)
 // Chunks of 128 positions and a launch that merges them (attn_chunk_kernel) -> this: 32 heads over 8 of 128, 16 sequences of 2048
 // positions 27.2 + 4.8 -> 25.3 us (5.3 TB/s; a step of 32 layers 2757 -> 2571), 8 sequences 2205 -> 2117 a step.  With fewer than 64
 // (sequence, kv head) pairs a workgroup has to take in more than it can at 50 .. 60 GB/s, or the merge gets deep: 4 sequences of 1000
@@ -31,7 +35,14 @@ namespace {
 
 constexpr int AD_WAVES = 8, AD_THREADS = 64 * AD_WAVES, AD_Q = 16;
 constexpr int kAttMin = 512;  // positions below which a share is not cut further: two blocks per wave (256: 0.5 % slower, 1024: up to 10 %)
-constexpr uint64_t kEmpty = ~(uint64_t)0;  // a slot nobody has been to (no value is stored as this NaN)
+constexpr uint64_t kEmpty = ~(uint64_t)0;  // a word nobody has been to (no pair is stored with this NaN in it)
+
+typedef float float2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float2_t word_pair(uint64_t w) { return float2_t{__uint_as_float((uint32_t)w), __uint_as_float((uint32_t)(w >> 32))}; }
+__device__ __forceinline__ uint64_t swap_pair(uint64_t *slot, float x, float y) {
+  y = y == y ? y : __uint_as_float(0x7fc00000u);
+  return __hip_atomic_exchange(slot, ((uint64_t)__float_as_uint(y) << 32) | __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 struct AttnDecodeArgs {
   const _Float16 *qkv;  // [batch][(hq + 2 hkv) HD]
@@ -254,56 +265,86 @@ __global__ void __launch_bounds__(AD_THREADS, 2) attn_decode_kernel(AttnDecodeAr
     m_s[wave][r] = m_run;
     l_s[wave][r] = l_run;
   }
-  if (r < nq) {
-#pragma unroll
-    for (int t = 0; t < DT; t++) *reinterpret_cast<float4_t *>(&o_s[(wave * nq + r) * OP + 16 * t + 4 * c]) = o[t];
-  }
-  __syncthreads();
   const int pair = ((int)b * a.hkv + kvh) * qblocks + qb;
   uint64_t *nodes = a.meet + (size_t)pair * (size_t)a.splits * min(AD_Q, group) * HD;  // (the last block of heads may be smaller)
-  for (int idx = tid; idx < nq * HD; idx += AD_THREADS) {
-    const int h = idx / HD, d = idx % HD;
-    float m = -INFINITY, l = 0.0f, v = 0.0f;
+  const size_t node = (size_t)nq * HD;
+  const bool meets = live > 1 && (split ^ 1) < live;  // at the first level (the last share of an odd number goes on by itself)
+  // a thread's two channels of a head: the share's maximum and sum
+  float m, l, f[AD_WAVES];
+  auto sums = [&](int h) {
+    m = -INFINITY;
+    l = 0.0f;
 #pragma unroll
     for (int w = 0; w < AD_WAVES; w++) m = fmaxf(m, m_s[w][h]);
 #pragma unroll
     for (int w = 0; w < AD_WAVES; w++) {
-      const float f = m_s[w][h] == -INFINITY ? 0.0f : __expf(m_s[w][h] - m);
-      l += l_s[w][h] * f;
-      v += o_s[(w * nq + h) * OP + d] * f;
+      f[w] = m_s[w][h] == -INFINITY ? 0.0f : __expf(m_s[w][h] - m);
+      l += l_s[w][h] * f[w];
     }
-    v = l > 0.0f ? v / l : v * 0.0f;  // (a NaN stays one)
+  };
+  lds_barrier();
+  uint64_t ml = kEmpty;
+  if (tid < nq * HALF) {
+    sums(tid / HALF);
+    if (meets) ml = swap_pair(nodes + 2 * tid + (size_t)(split >> 1) * node, m, l);  // on its way while the waves' outputs are added up
+  }
+  if (r < nq) {
+#pragma unroll
+    for (int t = 0; t < DT; t++) *reinterpret_cast<float4_t *>(&o_s[(wave * nq + r) * OP + 16 * t + 4 * c]) = o[t];
+  }
+  lds_barrier();
+  for (int idx = tid; idx < nq * HALF; idx += AD_THREADS) {
+    const int h = idx / HALF, d = idx % HALF * 2;
+    uint64_t *level = nodes + 2 * idx;
+    if (idx != tid) {
+      sums(h);
+      if (meets) ml = swap_pair(level + (size_t)(split >> 1) * node, m, l);
+    }
+    float2_t o = {0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < AD_WAVES; w++) o += *reinterpret_cast<const float2_t *>(&o_s[(w * nq + h) * OP + d]) * f[w];
     bool top = true;
     if (live > 1) {
-      float lse = m + __logf(l);
-      v = v == v ? v : __uint_as_float(0x7fc00000u);
-      uint64_t *level = nodes + idx;
       int met = 0;  // bit i: merged at level i
       for (int at = split, count = live, width = a.splits, bit = 1; count > 1; at >>= 1, count = (count + 1) >> 1, width >>= 1, bit <<= 1) {
-        uint64_t *slot = level + (size_t)(at >> 1) * nq * HD;
-        level += (size_t)(width >> 1) * nq * HD;
-        if ((at ^ 1) >= count) continue;  // the last node of an odd level goes on by itself
-        const uint64_t other = __hip_atomic_exchange(slot, ((uint64_t)__float_as_uint(lse) << 32) | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (other == kEmpty) {
+        uint64_t *slot = level + (size_t)(at >> 1) * node;
+        level += (size_t)(width >> 1) * node;
+        if ((at ^ 1) >= count) continue;
+        if (bit > 1) ml = swap_pair(slot, m, l);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(ml)::"memory");  // the first word is there before the second one goes
+        const uint64_t ov = swap_pair(slot + 1, o[0], o[1]);
+        if (ov == kEmpty) {
           top = false;
           break;
         }
         met |= bit;
-        const float ov = __uint_as_float((uint32_t)other), ol = __uint_as_float((uint32_t)(other >> 32));
-        const float l0 = (at & 1) ? ol : lse, l1 = (at & 1) ? lse : ol, v0 = (at & 1) ? ov : v, v1 = (at & 1) ? v : ov;
-        const float mx = fmaxf(l0, l1), w0 = l0 == mx ? 1.0f : __expf(l0 - mx), w1 = l1 == mx ? 1.0f : __expf(l1 - mx), sum = w0 + w1;
-        v = (v0 * w0 + v1 * w1) / sum;
-        v = v == v ? v : __uint_as_float(0x7fc00000u);
-        lse = mx + __logf(sum);
+        // (found the first slot empty and the second one full: the partner's first word has taken this one's place since)
+        if (ml == kEmpty) ml = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const float2_t om = word_pair(ov), other = word_pair(ml);
+        const float mo = other[0], lo = other[1], mx = fmaxf(m, mo);
+        const float own = m == mx ? 1.0f : __expf(m - mx), theirs = mo == mx ? 1.0f : __expf(mo - mx);
+        const bool second = (at & 1) != 0;  // always added in the order of the positions
+        const float f0 = second ? theirs : own, f1 = second ? own : theirs;
+        const float2_t o0 = second ? om : o, o1 = second ? o : om;
+        l = (second ? lo : l) * f0 + (second ? l : lo) * f1;
+        o = o0 * f0 + o1 * f1;
+        m = mx;
       }
       // the slots are emptied at the end: a store in front of the next exchange would be waited for with it
-      level = nodes + idx;
+      level = nodes + 2 * idx;
       for (int at = split, width = a.splits; met != 0; at >>= 1, width >>= 1, met >>= 1) {
-        if (met & 1) __hip_atomic_store(level + (size_t)(at >> 1) * nq * HD, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        level += (size_t)(width >> 1) * nq * HD;
+        uint64_t *slot = level + (size_t)(at >> 1) * node;
+        if (met & 1) {
+          __hip_atomic_store(slot, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(slot + 1, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        level += (size_t)(width >> 1) * node;
       }
     }
-    if (top) a.out[((size_t)b * a.hq + head0 + h) * HD + d] = (_Float16)v;
+    if (top) {
+      const float2_t v = l > 0.0f ? float2_t{o[0] / l, o[1] / l} : o * 0.0f;  // (a NaN stays one)
+      *reinterpret_cast<half2_t *>(a.out + ((size_t)b * a.hq + head0 + h) * HD + d) = half2_t{(_Float16)v[0], (_Float16)v[1]};
+    }
   }
 }
 
