@@ -28,6 +28,30 @@ def test_calls_that_are_not_taken_go_the_general_way():
         _calls.bind(1)
 
 
+@pytest.mark.parametrize("module", ["None", "types.SimpleNamespace(torch_version=lambda: '0.0')"])
+def test_without_a_module_that_fits(module):
+    """Not built, or built for another torch: the package is there all the same, and every call goes the general way."""
+    code = f"""
+import sys, types, warnings
+warnings.simplefilter("ignore")
+import yscv_amd
+sys.modules["yscv_amd._calls"] = yscv_amd._calls = {module}
+if yscv_amd._calls is None: del yscv_amd._calls
+import torch
+from yscv_amd import kernels as K, onnx_ops as O, short_calls
+assert K.lib().abi_version() == 1 and short_calls.calls.rms_norm(1, 2, 3) is None
+host = torch.zeros(2, 64)
+for call, error in ((lambda: O.rms_norm(host, host[0], 1e-5), TypeError), (lambda: K.PackedI8B.matmul(types.SimpleNamespace(_h=None, _k=64, _n=2), host), AssertionError)):
+    try:
+        call()
+    except error:
+        continue
+    raise SystemExit("no error")
+"""
+    run = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), timeout=100)
+    assert run.returncode == 0
+
+
 @pytest.mark.gpu
 def test_same_results_as_the_general_way():
     import torch

@@ -233,9 +233,9 @@ def lib() -> _Checked:
         # only one, and torch's must be the one that is loaded first or torch loses the GPU.
         import torch  # noqa: F401
 
-        from . import _calls
+        from .short_calls import calls
 
         checked = _Checked(C.CDLL(_LIB_PATH))
-        _calls.bind(*(C.cast(getattr(checked, name).raw, _vp).value for name in _DIRECT_CALLS))
+        calls.bind(*(C.cast(getattr(checked, name).raw, _vp).value for name in _DIRECT_CALLS))
         _lib = checked
     return _lib

@@ -240,8 +240,11 @@ PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t na) {
   Py_RETURN_NONE;
 }
 
+// torch.__version__ of the torch whose headers this was built with
+PyObject *torch_version(PyObject *, PyObject *) { return PyUnicode_FromString(YSCV_TORCH_VERSION); }
+
 #define YSCV_CALL(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {YSCV_CALL(bind), YSCV_CALL(int4_matmul), YSCV_CALL(int8_matmul), YSCV_CALL(int8_requant),
+PyMethodDef methods[] = {YSCV_CALL(bind), {"torch_version", torch_version, METH_NOARGS, nullptr}, YSCV_CALL(int4_matmul), YSCV_CALL(int8_matmul), YSCV_CALL(int8_requant),
                          YSCV_CALL(dql_matmul), YSCV_CALL(rms_norm), YSCV_CALL(gqa), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", "The short calls of yscv_amd without ctypes", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

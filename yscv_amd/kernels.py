@@ -12,9 +12,10 @@ import ctypes as C
 import numpy as np
 import torch
 
-from . import _calls, capi
+from . import capi
 from .capi import (BF16, EPILOGUE_ADD_F32, EPILOGUE_STORE, EPILOGUE_SWIGLU, F16, F32, NIBBLE_SIGNED, NIBBLE_UNSIGNED,
                    ROUND_HALF_AWAY, ROUND_TIES_EVEN, lib, stream_ptr)
+from .short_calls import calls as _calls
 
 _sz = C.c_size_t
 

@@ -13,8 +13,8 @@ from dataclasses import dataclass
 
 import torch
 
-from . import _calls
 from .capi import PATH_FALLBACK_EXACT, PATH_FALLBACK_F32, PATH_FAST, QuantStats, lib, stream_ptr  # noqa: F401
+from .short_calls import calls as _calls
 
 _sz = C.c_size_t
 
