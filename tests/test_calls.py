@@ -101,6 +101,51 @@ def test_same_results_as_the_general_way():
 
 
 @pytest.mark.gpu
+def test_other_threads_run_while_the_output_is_allocated():
+    """Mapping memory for an output of 4 GiB takes 0.4 ms: a call that held the interpreter would stop the other thread for as long."""
+    import threading
+    import time
+
+    import torch
+
+    from yscv_amd import kernels as K
+
+    m, n, k = 1 << 17, 8192, 64
+    b = K.pack_i8_b_for_matmul(np.ones((k, n), np.int8), k, n)
+    a = torch.ones(m, k, dtype=torch.uint8, device="cuda")
+    b.matmul(a[:8])
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks.append(time.perf_counter())
+
+    shares, interval = [], sys.getswitchinterval()
+    sys.setswitchinterval(1e-5)  # (the time until the call has the interpreter back is no part of it)
+    for _ in range(3):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        ticks.clear()
+        stop.clear()
+        other = threading.Thread(target=tick)
+        other.start()
+        time.sleep(0.01)
+        t0 = time.perf_counter()
+        y = b.matmul(a)
+        t1 = time.perf_counter()
+        stop.set()
+        other.join()
+        inside = [t0] + [t for t in ticks if t0 < t < t1] + [t1]
+        gap = max(q - p for p, q in zip(inside, inside[1:]))
+        shares.append(gap / (t1 - t0))
+        print(f"call {1e3 * (t1 - t0):.2f} ms, longest stop of the other thread {1e3 * gap:.2f} ms", flush=True)
+        assert bool((y[-1] == k).all())
+        del y
+    sys.setswitchinterval(interval)
+    assert min(shares) < 0.4
+
+
+@pytest.mark.gpu
 def test_modes_and_streams_are_seen():
     import torch
     from torch.utils._python_dispatch import TorchDispatchMode

@@ -67,13 +67,17 @@ int dtype_code(at::ScalarType t) {
 // the stream of the current device, as torch.cuda.current_stream() names it
 void *stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
-template <typename F>
-int32_t without_gil(F f) {
-  PyThreadState *ts = PyEval_SaveThread();
-  const int32_t st = f();
-  PyEval_RestoreThread(ts);
-  return st;
-}
+// Other Python threads run meanwhile: the allocator may have to map memory, and the launch may have to wait for the queue.
+class NoGil {
+ public:
+  NoGil() : state_(PyEval_SaveThread()) {}
+  ~NoGil() { PyEval_RestoreThread(state_); }  // (an allocation may throw)
+  NoGil(const NoGil &) = delete;
+  NoGil &operator=(const NoGil &) = delete;
+
+ private:
+  PyThreadState *state_;
+};
 
 PyObject *result(int32_t st, at::Tensor out) { return st == 0 ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(st); }
 
@@ -89,11 +93,16 @@ PyObject *int4_matmul(PyObject *, PyObject *const *a, Py_ssize_t na) {
   if (dt < 0) Py_RETURN_NONE;
   c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
   shape.back() = n;
-  at::Tensor y = at::empty(shape, x->options());
   const void *xp = x->data_ptr();
-  void *yp = y.data_ptr(), *s = stream();
   const size_t m = (size_t)(x->numel() / k);
-  const int32_t st = without_gil([&] { return p_int4_matmul(static_cast<const yscv_hip_int4_weight *>(w), xp, dt, yp, dt, m, s); });
+  const at::TensorOptions like = x->options();
+  at::Tensor y;
+  int32_t st;
+  {
+    NoGil released;
+    y = at::empty(shape, like);
+    st = p_int4_matmul(static_cast<const yscv_hip_int4_weight *>(w), xp, dt, y.data_ptr(), dt, m, stream());
+  }
   return result(st, std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -117,13 +126,17 @@ PyObject *int8_matmul(PyObject *, PyObject *const *a, Py_ssize_t na) {
   const long zp = PyLong_AsLong(a[4]);
   if (PyErr_Occurred()) PyErr_Clear();
   if (!t || zp < -128 || zp > 255) Py_RETURN_NONE;
-  at::Tensor y = at::empty({t->size(0), n}, t->options().dtype(at::kInt));
   const void *ap = t->data_ptr();
-  int32_t *yp = y.data_ptr<int32_t>();
-  void *s = stream();
-  const size_t m = (size_t)t->size(0);
+  const int64_t m = t->size(0);
   const int u8 = t->scalar_type() == at::kByte;
-  const int32_t st = without_gil([&] { return p_int8_matmul(ap, u8, (int32_t)zp, static_cast<const yscv_hip_i8_weight *>(w), m, yp, s); });
+  const at::TensorOptions like = t->options().dtype(at::kInt);
+  at::Tensor y;
+  int32_t st;
+  {
+    NoGil released;
+    y = at::empty({m, n}, like);
+    st = p_int8_matmul(ap, u8, (int32_t)zp, static_cast<const yscv_hip_i8_weight *>(w), (size_t)m, y.data_ptr<int32_t>(), stream());
+  }
   return result(st, std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -146,16 +159,19 @@ PyObject *int8_requant(PyObject *, PyObject *const *a, Py_ssize_t na) {
   const float y_zp = (float)PyFloat_AS_DOUBLE(a[6]);
   const at::Tensor *t = int8_rows(a, w, k, n), *comp = plain_f32(a[5]);
   if (!t || !comp || comp->dim() != 1 || comp->size(0) != n) Py_RETURN_NONE;
-  at::Tensor y = at::empty({t->size(0), n}, t->options().dtype(v[2] < 0 ? at::kChar : at::kByte));
   const void *ap = t->data_ptr();
   const float *cp = comp->data_ptr<float>();
-  void *yp = y.data_ptr(), *s = stream();
-  const size_t m = (size_t)t->size(0);
+  const int64_t m = t->size(0);
   const int u8 = t->scalar_type() == at::kByte;
-  const int32_t st = without_gil([&] {
-    return p_int8_matmul_requant(ap, u8, (int32_t)v[0], static_cast<const yscv_hip_i8_weight *>(w), m, nullptr, cp, 0.0f, y_zp,
-                                 (int32_t)v[1], (int32_t)v[2], (int32_t)v[3], yp, s);
-  });
+  const at::TensorOptions like = t->options().dtype(v[2] < 0 ? at::kChar : at::kByte);
+  at::Tensor y;
+  int32_t st;
+  {
+    NoGil released;
+    y = at::empty({m, n}, like);
+    st = p_int8_matmul_requant(ap, u8, (int32_t)v[0], static_cast<const yscv_hip_i8_weight *>(w), (size_t)m, nullptr, cp, 0.0f, y_zp,
+                               (int32_t)v[1], (int32_t)v[2], (int32_t)v[3], y.data_ptr(), stream());
+  }
   return result(st, std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -168,12 +184,18 @@ PyObject *dql_matmul(PyObject *, PyObject *const *a, Py_ssize_t na) {
   const at::Tensor *x = plain_f32(a[1]);
   void *w = handle(a[0]);
   if (!x || !w || x->dim() != 2 || x->size(1) != k) Py_RETURN_NONE;
-  at::Tensor y = at::empty({x->size(0), n}, x->options()), scale = at::empty({1}, x->options()), zp = at::empty({1}, x->options());
   const float *xp = x->data_ptr<float>();
-  float *yp = y.data_ptr<float>(), *sp = scale.data_ptr<float>(), *zpp = zp.data_ptr<float>();
-  void *s = stream();
-  const size_t m = (size_t)x->size(0);
-  const int32_t st = without_gil([&] { return p_exec_dql(xp, m, static_cast<const yscv_hip_i8_weight *>(w), yp, sp, zpp, s); });
+  const int64_t m = x->size(0);
+  const at::TensorOptions like = x->options();
+  at::Tensor y, scale, zp;
+  int32_t st;
+  {
+    NoGil released;
+    y = at::empty({m, n}, like);
+    scale = at::empty({1}, like);
+    zp = at::empty({1}, like);
+    st = p_exec_dql(xp, (size_t)m, static_cast<const yscv_hip_i8_weight *>(w), y.data_ptr<float>(), scale.data_ptr<float>(), zp.data_ptr<float>(), stream());
+  }
   if (st != 0) return PyLong_FromLong(st);
   PyObject *t[3] = {THPVariable_Wrap(std::move(y)), THPVariable_Wrap(std::move(scale)), THPVariable_Wrap(std::move(zp))};
   PyObject *r = PyTuple_Pack(3, t[0], t[1], t[2]);
@@ -190,11 +212,16 @@ PyObject *rms_norm(PyObject *, PyObject *const *a, Py_ssize_t na) {
   if (!x || !g || x->dim() < 1 || g->dim() != 1 || g->size(0) != x->size(-1)) Py_RETURN_NONE;
   const float eps = (float)PyFloat_AS_DOUBLE(a[2]);
   const size_t d = (size_t)x->size(-1), rows = (size_t)x->numel() / d;
-  at::Tensor y = at::empty(x->sizes(), x->options());
   const float *xp = x->data_ptr<float>(), *gp = g->data_ptr<float>();
-  float *yp = y.data_ptr<float>();
-  void *s = stream();
-  const int32_t st = without_gil([&] { return p_rms_norm(xp, gp, rows, d, eps, yp, s); });
+  const c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
+  const at::TensorOptions like = x->options();
+  at::Tensor y;
+  int32_t st;
+  {
+    NoGil released;
+    y = at::empty(shape, like);
+    st = p_rms_norm(xp, gp, rows, d, eps, y.data_ptr<float>(), stream());
+  }
   return result(st, std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -208,11 +235,16 @@ PyObject *gqa(PyObject *, PyObject *const *a, Py_ssize_t na) {
   if (!q || !k || !v || q->dim() != 3 || k->dim() != 3 || v->sizes() != k->sizes()) Py_RETURN_NONE;
   const int64_t B = q->size(0), sq = q->size(1), sk = k->size(1), d = q->size(2) / hq;
   if (k->size(0) != B || k->size(2) != hkv * d || q->size(2) != hq * d) Py_RETURN_NONE;
-  at::Tensor y = at::empty(q->sizes(), q->options());
   const float *qp = q->data_ptr<float>(), *kp = k->data_ptr<float>(), *vp = v->data_ptr<float>();
-  float *yp = y.data_ptr<float>();
-  void *s = stream();
-  const int32_t st = without_gil([&] { return p_gqa(qp, kp, vp, (size_t)B, (size_t)sq, (size_t)sk, (size_t)hq, (size_t)hkv, (size_t)d, yp, s); });
+  const int64_t width = q->size(2);
+  const at::TensorOptions like = q->options();
+  at::Tensor y;
+  int32_t st;
+  {
+    NoGil released;
+    y = at::empty({B, sq, width}, like);
+    st = p_gqa(qp, kp, vp, (size_t)B, (size_t)sq, (size_t)sk, (size_t)hq, (size_t)hkv, (size_t)d, y.data_ptr<float>(), stream());
+  }
   return result(st, std::move(y));
   END_HANDLE_TH_ERRORS
 }
