@@ -708,12 +708,14 @@ static int32_t finish_setup(yscv_hip_decoder *d) {
   {
     const Context *ctx = nullptr;
     YSCV_TRY(ensure_context(&ctx));
-    // (a consuming projection adds up at most 256 partial sums per row: four rows per wave of 512 k, sixteen rows of up to 64)
+    // (a consuming projection adds up at most 256 partial sums per row, four rows per wave of 512 k.  Sixteen rows of up to 64 sums
+    // would fit a wave, 947 -> 858 us a step of 24 layers of d_model 1024 at batch 16; those batches have the norm in f32 with one rounding
+    // at its end, whatever a row's growth within an update, and unnormalised fp16 rows bound it)
     bool ok = d->cfg.d_model % 256 == 0 && d->cfg.d_model <= 4096 && d->fold_norm_wanted;
     auto consumes = [&](const yscv_hip_int4_weight *w) {
       if (!w->tiled) return false;
       const SkinnyPlan plan = plan_int4_skinny(w, d->cfg.max_batch, 1, ctx->num_cus);
-      return plan.ksg == 1 && d->cfg.max_batch <= (d->cfg.d_model <= 1024 ? 16 : 4) * plan.waves;
+      return plan.ksg == 1 && d->cfg.max_batch <= 4 * plan.waves;
     };
     for (auto &L : d->layers)
       for (auto *w : {L.wqkv, L.wgu}) ok = ok && consumes(w);

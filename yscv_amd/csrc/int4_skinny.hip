@@ -211,18 +211,16 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
   if constexpr (EARLY) fill_ring();
   // folded norm, consumer side: this wave's share of the partial sums of squares (see further down), requested
   // here so that their round trip overlaps the activations'
-  // Four loads of four partial sums per lane: a row of up to 256 sums takes the wave, of up to 64 sums sixteen lanes, so that a wave
-  // covers four rows or sixteen (a lane's sums past the end of its row are not counted, rows past the last repeat it)
+  // Rows wave, wave + waves, ...: the launcher checks that four per wave cover m.  Four partial sums per lane (those past the end of a row
+  // are not counted, rows past the last repeat it)
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const bool ss_narrow = FOLD && f.ss_in_count <= 64;
-  auto ss_row = [&](int u) { return ss_narrow ? wave_u + (4 * u + c) * waves : wave_u + u * waves; };
   float4_t ss_pre[4];
   float ss_scale[4];
   if (FOLD && f.ss_in) {
-    const int j = min(ss_narrow ? 4 * r : 4 * lane, f.ss_in_stride - 4);
+    const int j = min(4 * lane, f.ss_in_stride - 4);
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-      const int row = min(ss_row(u), a.m - 1);
+      const int row = min(wave_u + u * waves, a.m - 1);
       ss_scale[u] = f.pre_in[row];
       ss_pre[u] = *reinterpret_cast<const float4_t *>(f.ss_in + (size_t)row * f.ss_in_stride + j);
     }
@@ -489,15 +487,14 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
   if (FOLD && f.ss_in) {
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-      const int row = ss_row(u), j = ss_narrow ? 4 * r : 4 * lane;
-      if (wave_u + (ss_narrow ? 4 * u : u) * waves < a.m) {  // uniform in the wave
+      const int row = wave_u + u * waves;
+      if (row < a.m) {  // uniform in the wave
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          if (j + e >= f.ss_in_count) ss_pre[u][e] = 0.0f;
-        float t = row_sum16((ss_pre[u][0] + ss_pre[u][1]) + (ss_pre[u][2] + ss_pre[u][3]));
-        if (!ss_narrow) t = sum_xor16_xor32(t);
+          if (4 * lane + e >= f.ss_in_count) ss_pre[u][e] = 0.0f;
+        const float t = wave_sum((ss_pre[u][0] + ss_pre[u][1]) + (ss_pre[u][2] + ss_pre[u][3]));
         const float inv_rms = 1.0f / sqrtf(t * f.ss_inv_d + f.ss_eps);
-        if (row < a.m && (ss_narrow ? r : lane) == 0) {
+        if (lane == 0) {
           rs_lds[row] = inv_rms / ss_scale[u];
           // one workgroup leaves the scale of the next residual update behind (every workgroup holds the same bits)
           if (f.pre_next && blockIdx.x == 0 && blockIdx.y == 0) f.pre_next[row] = norm_fold_prescale(inv_rms);
@@ -1027,7 +1024,7 @@ int32_t launch_int4_skinny(const yscv_hip_int4_weight *w, const SkinnyPlan &plan
       return set_error(YSCV_HIP_ERR_UNSUPPORTED, "folded norm: weights with fp16 scales and no zero points, as a decoder's are");
     if (nf->ss_in) {
       if (plan.ksg > 1) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "folded norm: the consuming projection must not be K-split");
-      if (m > (size_t)(nf->ss_in_count <= 64 ? 16 : 4) * plan.waves || nf->ss_in_count > 256 || nf->ss_in_stride < 16 || nf->ss_in_stride % 4 != 0)
+      if (m > (size_t)4 * plan.waves || nf->ss_in_count > 256 || nf->ss_in_stride < 16 || nf->ss_in_stride % 4 != 0)
         return set_error(YSCV_HIP_ERR_UNSUPPORTED, "folded norm: %zu rows on %d waves, %d partial sums per row", m, plan.waves, nf->ss_in_count);
       if (split != 1 || xraw) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "folded norm: fp16 activations only");
       if (!nf->pre_in) return set_error(YSCV_HIP_ERR_INVALID_ARG, "folded norm: the row scales of the activations are missing");
