@@ -32,16 +32,20 @@ def test_steps_match_numpy(name, batch):
 @pytest.mark.parametrize("name,batch", [("k2816", 9), ("k2816", 16), ("k768", 16), ("one_slice", 5)])
 def test_more_rows_than_four_to_a_wave_grow_without_a_bound(name, batch):
     """Widths up to 1024 have two waves or fewer: such batches have their norms in f32.  An embedding far below sqrt(eps) and cached values of
-    2^12 .. 2^13 raise a row by 2^26 within the first update, past what an unnormalised fp16 row holds."""
+    some hundred raise a row from 2^-8 (eps in it) to 2^10 within the first update, and the norm behind it multiplies by 16: past what an
+    unnormalised fp16 row holds."""
     rng = np.random.default_rng(8100 + batch)
     cfg = dict(BASE, **SHAPES[name], max_batch=batch)
     dec, ref = _build(rng, cfg, symmetric=True, emb_scale=2.0 ** -13)
     shape = (batch, 40, cfg["n_kv_heads"], cfg["head_dim"])
     for layer in range(cfg["n_layers"]):
         k = rng.standard_normal(shape).astype(np.float16)
-        v = np.broadcast_to((rng.choice([-1.0, 1.0], (batch, 1) + shape[2:]) * rng.uniform(4096, 8192, (batch, 1) + shape[2:])), shape).astype(np.float16)
+        v = np.broadcast_to((rng.choice([-1.0, 1.0], (batch, 1) + shape[2:]) * rng.uniform(512, 1024, (batch, 1) + shape[2:])), shape).astype(np.float16)
         dec.set_kv(layer, k, v)
         ref.set_kv(layer, k.astype(np.float32), v.astype(np.float32))
+    ref.norms[(0, "ffn")] *= np.float32(16.0)
+    dec.set_norm(0, "ffn", ref.norms[(0, "ffn")])
+    dec.finalize()
     tok = rng.integers(0, cfg["vocab"], batch).astype(np.int32)
     dec.reset(tok, 40)
     dec.run(1)
