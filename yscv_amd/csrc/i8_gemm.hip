@@ -17,6 +17,7 @@
 // the reference uses for VNNI (int8_matmul.rs:1866-1868); the epilogue adds
 // (128 - a_zp) * colsum(b), the algebra of runner/conv/quantized.rs:119-147.
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "i8_common.hpp"
@@ -100,17 +101,17 @@ __global__ void __launch_bounds__(I8_THREADS) i8_gemm_kernel(I8Args p) {
       uint4_t v = {0, 0, 0, 0};
       if (gm < p.m) {
         if constexpr (VEC) {
-          if (gk + 16 <= p.k) {
-            v = *reinterpret_cast<const uint4_t *>(p.a + (size_t)gm * p.k + gk);
-          } else if (gk < p.k) {
+          if (gk + 16 <= p.lda) {
+            v = *reinterpret_cast<const uint4_t *>(p.a + (size_t)gm * p.lda + gk);
+          } else if (gk < p.lda) {
             uint8_t tmp[16];
-            for (int e = 0; e < 16; e++) tmp[e] = (gk + e < p.k) ? p.a[(size_t)gm * p.k + gk + e] : 0;
+            for (int e = 0; e < 16; e++) tmp[e] = (gk + e < p.lda) ? p.a[(size_t)gm * p.lda + gk + e] : 0;
             v = *reinterpret_cast<uint4_t *>(tmp);
           }
         } else {
           uint32_t wv[4] = {0, 0, 0, 0};
           for (int e = 0; e < 16; e++)
-            if (gk + e < p.k) wv[e >> 2] |= (uint32_t)p.a[(size_t)gm * p.k + gk + e] << (8 * (e & 3));
+            if (gk + e < p.lda) wv[e >> 2] |= (uint32_t)p.a[(size_t)gm * p.lda + gk + e] << (8 * (e & 3));
           v = uint4_t{wv[0], wv[1], wv[2], wv[3]};
         }
         // bytes beyond k must stay 0 *after* the xor: they meet zero-padded B, so any value is fine
@@ -185,16 +186,16 @@ __global__ void __launch_bounds__(I8_THREADS) i8_gemm_kernel(I8Args p) {
         if (row >= p.m) continue;
         const int32_t v = (int32_t)((uint32_t)acc[i][j][e] + (uint32_t)zc);
         const size_t o = (size_t)row * p.n + col;
-        if (p.mode == 0) {
+        if (p.mode() == 0) {
           reinterpret_cast<int32_t *>(p.out)[o] = v;
-        } else if (p.mode == 3) {
+        } else if (p.mode() == 3) {
           reinterpret_cast<float *>(p.out)[o] = (float)v;
-        } else if (p.mode == 2) {
-          reinterpret_cast<int32_t *>(p.out)[o] = requant_dequant_bits(v, corr, comp, p.y_zp, p.round_mode, lo, hi, p.dq_scale);
-        } else if (p.mode == 4) {
-          reinterpret_cast<int32_t *>(p.out)[o] = requant_f32_bits(v, corr, comp, p.y_zp, p.round_mode, lo, hi);
+        } else if (p.mode() == 2) {
+          reinterpret_cast<int32_t *>(p.out)[o] = requant_dequant_bits(v, corr, comp, p.y_zp, p.round_mode(), lo, hi, p.dq_scale);
+        } else if (p.mode() == 4) {
+          reinterpret_cast<int32_t *>(p.out)[o] = requant_f32_bits(v, corr, comp, p.y_zp, p.round_mode(), lo, hi);
         } else {
-          int q = requant_one(v, corr, comp, p.y_zp, p.round_mode, lo, hi);
+          int q = requant_one(v, corr, comp, p.y_zp, p.round_mode(), lo, hi);
           reinterpret_cast<uint8_t *>(p.out)[o] = (uint8_t)q;
         }
       }
@@ -435,7 +436,10 @@ __global__ void __launch_bounds__(I8R_THREADS) i8_gemm_ring_kernel(I8Args p, int
   __syncthreads();  // every wave is done with the ring
   const float lo = (float)p.lo, hi = (float)p.hi;
   const int zp_mul = p.a_zp_dev ? 128 - (int)p.a_zp_dev[0] : p.zp_mul;
-  if (wave < 4) {
+  // One form of the loops per mode: with the mode asked for each four values a wave of plain sums jumps over the code of the other forms,
+  // most of which then has to be fetched (512 x 4096 x 4096 to int32: 16.1 -> 15.7 us).
+  auto leave = [&](auto MODE) __attribute__((always_inline)) {
+    constexpr int mode = decltype(MODE)::value;
 #pragma unroll
     for (int j = 0; j < NT; j++) {
       const int lcol = wn * NT * 16 + j * 16 + c * 4;
@@ -450,37 +454,31 @@ __global__ void __launch_bounds__(I8R_THREADS) i8_gemm_ring_kernel(I8Args p, int
 #pragma unroll
       for (int i = 0; i < MT; i++) {
         const int lrow = wm * MT * 16 + i * 16 + r;
-        int32_t v[4];
+        int4_t f;
+        uint32_t packed = 0;
 #pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = (int32_t)((uint32_t)acc[i][j][e] + (uint32_t)zc[e]);
-        if (p.mode == 0) {
-          *reinterpret_cast<int4_t *>(i8_ring + lrow * RS32 + lcol * 4) = int4_t{v[0], v[1], v[2], v[3]};
-        } else if (p.mode == 3) {
-          *reinterpret_cast<int4_t *>(i8_ring + lrow * RS32 + lcol * 4) =
-              int4_t{__float_as_int((float)v[0]), __float_as_int((float)v[1]), __float_as_int((float)v[2]), __float_as_int((float)v[3])};
-        } else if (p.mode == 2) {
-          int4_t f;
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            f[e] = requant_dequant_bits(v[e], corr[e], comp[e], p.y_zp, p.round_mode, lo, hi, p.dq_scale);
-          *reinterpret_cast<int4_t *>(i8_ring + lrow * RS32 + lcol * 4) = f;
-        } else if (p.mode == 4) {
-          int4_t f;
-#pragma unroll
-          for (int e = 0; e < 4; e++) f[e] = requant_f32_bits(v[e], corr[e], comp[e], p.y_zp, p.round_mode, lo, hi);
-          *reinterpret_cast<int4_t *>(i8_ring + lrow * RS32 + lcol * 4) = f;
-        } else {
-          uint32_t packed = 0;
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            packed |= (uint32_t)(uint8_t)requant_one(v[e], corr[e], comp[e], p.y_zp, p.round_mode, lo, hi) << (8 * e);
-          *reinterpret_cast<uint32_t *>(i8_ring + lrow * RS8 + lcol) = packed;
+        for (int e = 0; e < 4; e++) {
+          const int32_t v = (int32_t)((uint32_t)acc[i][j][e] + (uint32_t)zc[e]);
+          if constexpr (mode == 0) f[e] = v;
+          else if constexpr (mode == 3) f[e] = __float_as_int((float)v);
+          else if constexpr (mode == 2) f[e] = requant_dequant_bits(v, corr[e], comp[e], p.y_zp, p.round_mode(), lo, hi, p.dq_scale);
+          else if constexpr (mode == 4) f[e] = requant_f32_bits(v, corr[e], comp[e], p.y_zp, p.round_mode(), lo, hi);
+          else packed |= (uint32_t)(uint8_t)requant_one(v, corr[e], comp[e], p.y_zp, p.round_mode(), lo, hi) << (8 * e);
         }
+        if constexpr (mode == 1) *reinterpret_cast<uint32_t *>(i8_ring + lrow * RS8 + lcol) = packed;
+        else *reinterpret_cast<int4_t *>(i8_ring + lrow * RS32 + lcol * 4) = f;
       }
     }
+  };
+  if (wave < 4) {
+    if (p.mode() == 0) leave(std::integral_constant<int, 0>{});
+    else if (p.mode() == 1) leave(std::integral_constant<int, 1>{});
+    else if (p.mode() == 2) leave(std::integral_constant<int, 2>{});
+    else if (p.mode() == 3) leave(std::integral_constant<int, 3>{});
+    else leave(std::integral_constant<int, 4>{});
   }
   __syncthreads();
-  if (p.mode != 1) {  // four-byte results: int32 sums or dequantised f32
+  if (p.mode() != 1) {  // four-byte results: int32 sums or dequantised f32
     constexpr int CPR = BN / 4;  // 16-byte chunks per row
     const bool vec = (p.n & 3) == 0;
     for (int q = tid; q < BM * CPR; q += I8R_THREADS) {
@@ -591,14 +589,12 @@ int32_t launch_i8_gemm(const void *a, int a_is_u8, int a_zp, const yscv_hip_i8_w
   p.composite_v = ep.composite_v;
   p.composite = ep.composite;
   p.y_zp = ep.y_zp;
-  p.round_mode = (int16_t)ep.round_mode;
-  p.lo = (int16_t)ep.lo;
-  p.hi = (int16_t)ep.hi;
-  p.mode = ep.mode;
+  p.lo = ep.lo;
+  p.hi = ep.hi;
+  p.how = ep.mode | ep.round_mode << 8;
   p.dq_scale = ep.dq_scale;
   p.m = (int)m;
   p.n = (int)b->n;
-  p.k = (int)b->k;
   p.ksteps = (int)(b->kp / 64);
   p.a_xor = a_is_u8 ? (int)0x80808080u : 0;
   p.zp_mul = a_is_u8 ? (128 - a_zp) : -a_zp;
@@ -626,7 +622,7 @@ int32_t launch_i8_gemm(const void *a, int a_is_u8, int a_zp, const yscv_hip_i8_w
         const size_t rows = m - r0 < step ? m - r0 : step;
         const size_t blocks = ceil_div(rows * b->kp / 16, (size_t)256);
         hipLaunchKernelGGL(i8_pad_rows_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, p.a + r0 * b->k, rows,
-                           p.k, (int)b->kp, static_cast<uint8_t *>(pad));
+                           (int)b->k, (int)b->kp, static_cast<uint8_t *>(pad));
         YSCV_HIP_TRY(hipGetLastError());
         piece.m = (int)rows;
         piece.out = static_cast<char *>(out) + r0 * out_row;

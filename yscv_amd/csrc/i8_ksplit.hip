@@ -27,10 +27,10 @@ __device__ __forceinline__ void iks_wait_vm() {
 
 // one column of the result through the epilogue, as the four bytes that modes 0, 2, 3 and 4 store
 __device__ __forceinline__ int32_t iks_word(const I8Args &p, int32_t v, int32_t corr, float comp, float lo, float hi) {
-  if (p.mode == 0) return v;
-  if (p.mode == 3) return __float_as_int((float)v);
-  if (p.mode == 2) return requant_dequant_bits(v, corr, comp, p.y_zp, p.round_mode, lo, hi, p.dq_scale);
-  return requant_f32_bits(v, corr, comp, p.y_zp, p.round_mode, lo, hi);
+  if (p.mode() == 0) return v;
+  if (p.mode() == 3) return __float_as_int((float)v);
+  if (p.mode() == 2) return requant_dequant_bits(v, corr, comp, p.y_zp, p.round_mode(), lo, hi, p.dq_scale);
+  return requant_f32_bits(v, corr, comp, p.y_zp, p.round_mode(), lo, hi);
 }
 
 constexpr int iks_row_ints(int nt) { return 16 * nt + 4; }  // 16 bytes of padding: rows fall into different banks
@@ -175,11 +175,11 @@ __global__ void __launch_bounds__(64 * WAVES) i8_ksplit_kernel(I8Args p, int til
 #pragma unroll
     for (int e = 0; e < 4; e++) v[e] = (int32_t)((uint32_t)v[e] + (uint32_t)zp_mul * (uint32_t)zc[e]);
     const size_t o = (size_t)row * p.n + col;
-    if (p.mode == 1) {
+    if (p.mode() == 1) {
       uint32_t packed = 0;
 #pragma unroll
       for (int e = 0; e < 4; e++)
-        packed |= (uint32_t)(uint8_t)requant_one(v[e], corr[e], comp[e], p.y_zp, p.round_mode, lo, hi) << (8 * e);
+        packed |= (uint32_t)(uint8_t)requant_one(v[e], corr[e], comp[e], p.y_zp, p.round_mode(), lo, hi) << (8 * e);
       uint8_t *out = reinterpret_cast<uint8_t *>(p.out) + o;
       if (vec) {
         *reinterpret_cast<uint32_t *>(out) = packed;
