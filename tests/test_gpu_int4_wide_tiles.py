@@ -15,6 +15,9 @@ CASES = [
     (1024, 24002, 576, 64, False),                                                           # whole rounds, then the rest
     (300, 4096, 4096, 32, False), (260, 2050, 8192, 128, True), (991, 469, 7520, 32, False),  # K in parts
     (66, 50001, 96, 32, False),
+    (147, 6085, 1952, 32, True), (66, 12518, 4672, 64, False),                               # K in parts: 128 x 192, 128 x 256
+    (1894, 257, 3200, 128, False), (925, 203, 4640, 32, True),                               # and the LDS-ring GEMM's 128 and 64 rows
+    (811, 22008, 96, 32, False), (415, 53494, 96, 32, True), (921, 21739, 192, 64, False),   # whole rounds, then the rest
 ]
 
 

@@ -84,14 +84,6 @@ __device__ __forceinline__ void g4_wait(G4Frags<MT, NT> &f) {
     asm volatile("s_waitcnt lgkmcnt(0)"
                  : "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.a[3]), "+v"(f.b[0]), "+v"(f.b[1]), "+v"(f.b[2]),
                    "+v"(f.b[3])::"memory");
-  } else if constexpr (MT == 4 && NT == 8) {
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.a[3]), "+v"(f.b[0]), "+v"(f.b[1]), "+v"(f.b[2]),
-                   "+v"(f.b[3]), "+v"(f.b[4]), "+v"(f.b[5]), "+v"(f.b[6]), "+v"(f.b[7])::"memory");
-  } else if constexpr (MT == 8 && NT == 4) {
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.a[3]), "+v"(f.a[4]), "+v"(f.a[5]), "+v"(f.a[6]),
-                   "+v"(f.a[7]), "+v"(f.b[0]), "+v"(f.b[1]), "+v"(f.b[2]), "+v"(f.b[3])::"memory");
   } else if constexpr (MT == 2 && NT == 4) {
     asm volatile("s_waitcnt lgkmcnt(0)"
                  : "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.b[0]), "+v"(f.b[1]), "+v"(f.b[2]), "+v"(f.b[3])::"memory");
@@ -613,7 +605,7 @@ bool int4_gemm_ring_eligible(const yscv_hip_int4_weight *w, const _Float16 *xh, 
 
 size_t int4_gemm_ring_partial_bytes(const yscv_hip_int4_weight *w, size_t m, int num_cus) {
   if (!w->tiled || m <= 16) return 0;
-  const RingPlan pl = int4_plan(m, w->n, w->kt, (size_t)(num_cus > 0 ? num_cus : 256), w->gm, w->has_zp);
+  const GemmPlan pl = int4_plan(m, w->n, w->kt, (size_t)(num_cus > 0 ? num_cus : 256));
   return pl.splits > 1 ? (size_t)pl.splits * m * w->n * sizeof(float) : 0;
 }
 
@@ -645,7 +637,7 @@ int32_t launch_int4_gemm_ring(const yscv_hip_int4_weight *w, const _Float16 *xh,
   const bool sf16 = w->scale_dtype == YSCV_HIP_F16;
   const Context *ctx = nullptr;
   YSCV_TRY(ensure_context(&ctx));
-  const RingPlan pl = int4_plan(m, w->n, w->kt, (size_t)(ctx->num_cus > 0 ? ctx->num_cus : 256), w->gm, w->has_zp);
+  const GemmPlan pl = int4_plan(m, w->n, w->kt, (size_t)(ctx->num_cus > 0 ? ctx->num_cus : 256));
   if (pl.splits > 1 && partial != nullptr && partial_bytes >= (size_t)pl.splits * m * w->n * sizeof(float) &&
       (reinterpret_cast<uintptr_t>(partial) & 15) == 0) {
     a.partial = partial;
@@ -656,10 +648,10 @@ int32_t launch_int4_gemm_ring(const yscv_hip_int4_weight *w, const _Float16 *xh,
     if (which >= kWide)
       return launch_int4_gemm_wide(w, xh, row_scale, k_pad, y, y_dtype, m, (size_t)r.col0, (size_t)r.n, which - kWide, s, epi, r.splits, r.kt_per, r.partial);
     switch (which) {
-      case 4: return ring_launch_gm<2, 4, 2, 6, 8>(r, w->gm, sf16, s);
-      case 3: return ring_launch_gm<1, 4, 2, 6, 4>(r, w->gm, sf16, s);
-      case 0: return ring_launch_gm<4, 4, 2, 6, 8>(r, w->gm, sf16, s);
-      default: return set_error(YSCV_HIP_ERR_INVALID_ARG, "no tile of shape %d", which);
+      case RING_64x128: return ring_launch_gm<2, 4, 2, 6, 8>(r, w->gm, sf16, s);
+      case RING_32x128: return ring_launch_gm<1, 4, 2, 6, 4>(r, w->gm, sf16, s);
+      case RING_128x128: return ring_launch_gm<4, 4, 2, 6, 8>(r, w->gm, sf16, s);
+      default: return set_error(YSCV_HIP_ERR_INVALID_ARG, "no tile %d", which);
     }
   };
   if (pl.second < 0) return launch_shape(pl.one, a);
