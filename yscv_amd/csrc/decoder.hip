@@ -9,6 +9,7 @@
 #include <mutex>
 #include <vector>
 
+#include "attention_plan.hpp"
 #include "decode_layers.hpp"
 #include "decoder.hpp"
 #include "int4_common.hpp"
@@ -758,13 +759,6 @@ static int32_t capture_step(F enqueue, hipGraph_t *graph, hipGraphExec_t *exec) 
   return YSCV_HIP_OK;
 }
 
-// Chunks of 128 positions and a merge launch, or the kernel of decode_attention.hip (times of both in its header): the line is a
-// quarter of the CUs, from where on a pair's positions need no more than four workgroups.
-static bool chunked_attention(const yscv_hip_decoder *d, int batch) {
-  const auto &c = d->cfg;
-  return c.head_dim == 128 && c.n_heads / c.n_kv_heads <= 4 && batch * c.n_kv_heads < 64;
-}
-
 // every launch of one decode step, in order, on stream s
 static int32_t enqueue_step(yscv_hip_decoder *d, int batch, hipStream_t s) {
   const auto &c = d->cfg;
@@ -829,7 +823,7 @@ static int32_t enqueue_step(yscv_hip_decoder *d, int batch, hipStream_t s) {
       _Float16 *qrot = d->fused_attn ? d->qrot : nullptr;
       if (!d->fused_attn)
         YSCV_TRY(launch_rope_append(d->qkv, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta, c.max_ctx, L.kc, L.vc, s));
-      if (chunked_attention(d, batch))
+      if (attention_in_chunks(batch, c.n_heads, c.n_kv_heads, c.head_dim, ctx->num_cus))
         YSCV_TRY(launch_attention_chunks(d->qkv, L.kc, L.vc, d->pos, batch, c.n_heads, c.n_kv_heads, c.head_dim, d->angles, c.max_ctx,
                                          d->attn_part, qrot, d->ao, s));
       else

@@ -29,6 +29,7 @@
 #include <cmath>
 #include <mutex>
 
+#include "attention_plan.hpp"
 #include "int4_common.hpp"
 #include "decoder.hpp"
 #include "kernels.hpp"
@@ -438,10 +439,10 @@ inline int shared_kv_hw_log2(int group) { return group % 4 == 0 ? 2 : (group % 2
 
 int32_t gqa_launch_shared_kv(const GqaArgs &a, int hd, hipStream_t s) {
   const int hw_log2 = shared_kv_hw_log2(a.Hq / a.Hkv);
-  // 32 queries per wave where that fills the CUs, else 16: twice the workgroups, shorter steps (700 queries, 16 heads over 2 of 64:
-  // 88 workgroups of 32)
+  const Context *ctx = nullptr;
+  YSCV_TRY(ensure_context(&ctx));
   const unsigned heads = (unsigned)(a.Hq >> hw_log2) * (unsigned)a.B, waves_q = (unsigned)(GQA_WAVES >> hw_log2);
-  const bool two = heads * ((a.Sq + 32 * waves_q - 1) / (32 * waves_q)) >= 256;
+  const bool two = prompt_row_tiles(heads, (unsigned)a.Sq, waves_q, ctx->num_cus) == 2;
   const unsigned q_per_wg = (two ? 32 : 16) * waves_q;
   const dim3 grid((unsigned)(a.Hq >> hw_log2), (a.Sq + q_per_wg - 1) / q_per_wg, (unsigned)a.B), block(64 * GQA_WAVES * SHARED_KG);
 #define YSCV_SHARED_KV(HD)                                                                      \
