@@ -33,3 +33,30 @@ def bf16_round(x):
     b = np.ascontiguousarray(x, np.float32).view(np.uint32)
     r = ((b + 0x7FFF + ((b >> 16) & 1)) >> 16).astype(np.uint32) << 16
     return r.view(np.float32)
+
+
+def attention_bound(p, v, want, score_err):
+    """What an attention kernel with fp16 weights may be off by, per element: p [.., keys] are the weights relative to the largest one,
+    v [.., keys, channels], want the result in 64 bits.  A weight is rounded by 2^-11 of itself (2^-25 where it is subnormal) and off by
+    score_err, as their sum is; f32 sums over the keys are off by keys * 2^-24 of the products' magnitudes; the result is rounded to fp16."""
+    total = p.sum(-1)[..., None]
+    mag = (p[..., None, :] @ np.abs(v))[..., 0, :] / total
+    tiny = 2.0 ** -25 * np.abs(v).sum(-2) / total
+    return (2.0 ** -11 + 2 * score_err + p.shape[-1] * 2.0 ** -24) * mag + 2.0 ** -11 * np.abs(want) + tiny + 2.0 ** -25
+
+
+def without_key(p, v, want, i):
+    """`want` with key i left out."""
+    total = p.sum(-1)[..., None]
+    w = p[..., i][..., None]
+    return (want * total - w * v[..., i, :]) / (total - w)
+
+
+def mark_block_edges(k, v):
+    """k, v [sequence, position, head, channel]: the first and the last position of every block of 32 get a zero key (a middling score) and
+    64 in one channel, another one from block to block, so that one of them lost or counted twice shows there."""
+    hd = v.shape[-1]
+    for i in range(k.shape[1]):
+        if i % 32 in (0, 31):
+            k[:, i] = 0
+            v[:, i, :, i // 32 % hd] = 64 if i % 64 < 32 else -64

@@ -5,17 +5,23 @@ import math
 
 import numpy as np
 import pytest
+from gpu_util import attention_bound, mark_block_edges, without_key
 
 pytestmark = pytest.mark.gpu
 
 
-def _decoder(heads, batch, max_ctx):
+def _decoder(heads, batch, max_ctx, qk_scale=None):
     from yscv_amd.decoder import Decoder
 
     nh, nkv, hd = heads
     dec = Decoder(n_layers=1, d_model=256, n_heads=nh, n_kv_heads=nkv, head_dim=hd, d_ff=256, vocab=512, group_size=32, max_batch=batch,
                   max_ctx=max_ctx, max_steps=8, rope_theta=10000.0, rms_eps=1e-5)
     dec.init_random(seed=3, nibbles=(1, 15))
+    if qk_scale:
+        rng = np.random.default_rng(5)
+        for kind, n, scale in (("q", nh * hd, qk_scale), ("k", nkv * hd, qk_scale), ("v", nkv * hd, 0.0125)):
+            nib = rng.integers(1, 16, (2, n * 128), dtype=np.uint8)
+            dec.set_linear(0, kind, nib[0] | (nib[1] << 4), np.full(n * 8, scale, np.float16), n, 256)
     dec.finalize()
     return dec
 
@@ -29,14 +35,16 @@ def _decoder(heads, batch, max_ctx):
 ], ids=["16q4kv-hd128", "32q8kv-hd128", "16q2kv-hd64", "36q2kv-hd32", "12q4kv-hd96"])
 def test_against_float64(heads, batch, max_ctx, positions):
     nh, nkv, hd = heads
-    dec = _decoder(heads, batch, max_ctx)
+    dec = _decoder(heads, batch, max_ctx, qk_scale=0.5 / 70)  # (q and the token's key of rms 1/2: no key takes all the weight)
     rng = np.random.default_rng(17)
-    k = rng.standard_normal((batch, max_ctx - 8, nkv, hd)).astype(np.float16)
+    k = (rng.standard_normal((batch, max_ctx - 8, nkv, hd)) * 0.5).astype(np.float16)
     v = rng.standard_normal((batch, max_ctx - 8, nkv, hd)).astype(np.float16)
+    mark_block_edges(k, v)
     tokens = (np.arange(batch) * 7 + 3).astype(np.int32)
     for pos in positions:
-        k[:, pos:], v[:, pos:] = np.nan, np.nan  # what lies behind the context must not be seen
-        dec.set_kv(0, k, v)
+        kp, vp = k.copy(), v.copy()
+        kp[:, pos:], vp[:, pos:] = np.nan, np.nan  # what lies behind the context must not be seen
+        dec.set_kv(0, kp, vp)
         outs = []
         for use_graph in (False, True, True):  # the slots of the merge are empty again behind every launch
             dec.reset(tokens, pos)
@@ -47,11 +55,18 @@ def test_against_float64(heads, batch, max_ctx, positions):
         kc, vc = (a.astype(np.float64).transpose(0, 2, 1, 3) for a in dec.get_kv(0, batch, 0, pos + 1))
         s = q @ kc.transpose(0, 1, 3, 2) / math.sqrt(hd)
         p = np.exp(s - s.max(-1, keepdims=True))
-        want = (p @ vc / p.sum(-1, keepdims=True)).reshape(batch, nh * hd)
-        # weights and result are rounded to fp16 (2^-11 each), v is exact; scores to 2^-22 of a few hundred
-        assert np.abs(outs[0] - want).max() <= 2.0 ** -10 * np.abs(vc).max() * 1.1, (pos, np.abs(outs[0] - want).max())
-        k = np.nan_to_num(k)
-        v = np.nan_to_num(v)
+        v4 = vc[:, :, None]
+        want = (p @ vc) / p.sum(-1)[..., None]
+        # a score: f32 sums of hd exact products, scaled; its exponential
+        score_err = hd * 2.0 ** -24 * (np.abs(q) @ np.abs(kc.transpose(0, 1, 3, 2))).max() / math.sqrt(hd) + 2.0 ** -21
+        bound = attention_bound(p, v4, want, score_err)
+        err = np.abs(outs[0].reshape(want.shape) - want)
+        assert (err <= bound).all(), (pos, float((err / bound).max()))
+        for i in range(pos):  # and a marked position lost for a kv head would show
+            if i % 32 in (0, 31):
+                ch = i // 32 % hd
+                lost = without_key(p, v4, want, i)
+                assert (np.abs(lost - want) > 2 * bound)[..., ch].all(), (pos, i)
     dec.close()
 
 

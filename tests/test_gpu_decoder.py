@@ -246,8 +246,8 @@ def test_fused_attention_equals_the_separate_rope_append(prefill, kv_dtype, head
     of it: same arithmetic, so tokens, logits, the attention output, the rotated q and the appended cache rows must be
     identical bit for bit.  The prefills put the current position at the start, the end and the middle of a
     128-position chunk and leave chunks unused.  With the int8 cache the appended row's scales span all kv heads, which
-    every workgroup that appends works out for itself.  Head shapes other than the first run the general attention
-    kernel, whose fused form patches the new row into the 16-position key block that holds it (fp16 cache only)."""
+    every workgroup that appends works out for itself.  Head shapes other than the first run decode_attention.hip (fp16 cache
+    only), which patches the new row into the 32-position block that holds it; up to 256 positions are one share there."""
     import ctypes as C
 
     from yscv_amd.capi import lib
