@@ -9,13 +9,13 @@
 //                 up with the weights of eight consecutive positions of one query head, which is
 //   O^T += V^T P^T  the B operand here; A is a slab piece of the cache as it lies (eight positions of a channel).
 // Shares of one kv head meet pairwise, two channels of a head at a time: a thread exchanges {maximum, sum of weights} with the first word of
-// a slot and, once that is there, its two sums of weighted values with the second.  Who finds the second word empty leaves; who finds it
-// full has the partner's first word, too, or finds it in the slot by now; it merges (always in the order of the positions), empties the
-// slot and goes on to the next level.  Nobody waits for another workgroup.  Two trips to memory per level (1.1 us each), the first of the
-// first level behind the merge of the waves; maximum and sum stay two f32, so that a share's weight is exact whatever the size of the
-// scores.  ({value, log of the weights' sum} in one word is one trip, a step of the 7B shape at 16 sequences 0.3 % shorter, and
-// weights that are off by |score| 2^-24.  Partials through agent-scope stores, an arrival counter and a last workgroup that reads them
-// back: three trips, 5 us.)
+// a slot and its two sums of weighted values with the second, both on their way at once.  Who finds the second word empty leaves; who
+// finds it full merges (always in the order of the positions), empties the slot and goes on to the next level.  The partner's
+// first word has been sent before its second one: it is what the exchange returned, or is about to take the place of this share's own
+// one (the sign bit of the sum tells the two apart), a wait for memory and for no other workgroup.  One trip to memory per level (1.1 us);
+// maximum and sum stay two f32, so that a share's weight is exact whatever the size of the scores.  ({value, log of the
+// weights' sum} in one word: weights that are off by |score| 2^-24.  The second word sent when the first has arrived: 0.4 us more.
+// Partials through agent-scope stores, an arrival counter and a last workgroup that reads them back: three trips, 5 us.)
 // Chunks of 128 positions and a launch that merges them (attn_chunk_kernel) -> this: 32 heads over 8 of 128, 16 sequences of 2048
 // positions 27.2 + 4.8 -> 25.3 us (5.3 TB/s; a step of 32 layers 2757 -> 2571), 8 sequences 2205 -> 2117 a step.  With fewer than 64
 // (sequence, kv head) pairs a workgroup has to take in more than it can at 50 .. 60 GB/s, or the merge gets deep: 4 sequences of 1000
@@ -39,9 +39,10 @@ constexpr uint64_t kEmpty = ~(uint64_t)0;  // a word nobody has been to (no pair
 
 typedef float float2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float2_t word_pair(uint64_t w) { return float2_t{__uint_as_float((uint32_t)w), __uint_as_float((uint32_t)(w >> 32))}; }
-__device__ __forceinline__ uint64_t swap_pair(uint64_t *slot, float x, float y) {
-  y = y == y ? y : __uint_as_float(0x7fc00000u);
-  return __hip_atomic_exchange(slot, ((uint64_t)__float_as_uint(y) << 32) | __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// mark: into the sign bit of y, which then is no negative number
+__device__ __forceinline__ uint64_t swap_pair(uint64_t *slot, float x, float y, uint32_t mark = 0) {
+  const uint32_t hi = (y == y ? __float_as_uint(y) : 0x7fc00000u) | mark << 31;
+  return __hip_atomic_exchange(slot, ((uint64_t)hi << 32) | __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 struct AttnDecodeArgs {
@@ -283,23 +284,20 @@ __global__ void __launch_bounds__(AD_THREADS, 2) attn_decode_kernel(AttnDecodeAr
     }
   };
   lds_barrier();
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): no block's load is pending, so that the compiler need not wait for the exchange with them
   uint64_t ml = kEmpty;
   if (tid < nq * HALF) {
     sums(tid / HALF);
-    if (meets) ml = swap_pair(nodes + 2 * tid + (size_t)(split >> 1) * node, m, l);  // on its way while the waves' outputs are added up
+    if (meets) ml = swap_pair(nodes + 2 * tid + (size_t)(split >> 1) * node, m, l, split & 1);  // on its way while the waves' outputs are added up
   }
   if (r < nq) {
 #pragma unroll
     for (int t = 0; t < DT; t++) *reinterpret_cast<float4_t *>(&o_s[(wave * nq + r) * OP + 16 * t + 4 * c]) = o[t];
   }
   lds_barrier();
-  for (int idx = tid; idx < nq * HALF; idx += AD_THREADS) {
+  auto meet = [&](int idx) __attribute__((always_inline)) {
     const int h = idx / HALF, d = idx % HALF * 2;
     uint64_t *level = nodes + 2 * idx;
-    if (idx != tid) {
-      sums(h);
-      if (meets) ml = swap_pair(level + (size_t)(split >> 1) * node, m, l);
-    }
     float2_t o = {0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < AD_WAVES; w++) o += *reinterpret_cast<const float2_t *>(&o_s[(w * nq + h) * OP + d]) * f[w];
@@ -310,17 +308,16 @@ __global__ void __launch_bounds__(AD_THREADS, 2) attn_decode_kernel(AttnDecodeAr
         uint64_t *slot = level + (size_t)(at >> 1) * node;
         level += (size_t)(width >> 1) * node;
         if ((at ^ 1) >= count) continue;
-        if (bit > 1) ml = swap_pair(slot, m, l);
-        asm volatile("s_waitcnt vmcnt(0)" : "+v"(ml)::"memory");  // the first word is there before the second one goes
+        if (bit > 1) ml = swap_pair(slot, m, l, at & 1);
         const uint64_t ov = swap_pair(slot + 1, o[0], o[1]);
         if (ov == kEmpty) {
           top = false;
           break;
         }
         met |= bit;
-        // (found the first slot empty and the second one full: the partner's first word has taken this one's place since)
-        if (ml == kEmpty) ml = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const float2_t om = word_pair(ov), other = word_pair(ml);
+        // the first word empty and the second one full: the partner's first word, sent before its second, takes the place of this share's
+        while (ml == kEmpty || (uint32_t)(ml >> 63) == (uint32_t)(at & 1)) ml = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const float2_t om = word_pair(ov), other = word_pair(ml & ~((uint64_t)1 << 63));
         const float mo = other[0], lo = other[1], mx = fmaxf(m, mo);
         const float own = m == mx ? 1.0f : __expf(m - mx), theirs = mo == mx ? 1.0f : __expf(mo - mx);
         const bool second = (at & 1) != 0;  // always added in the order of the positions
@@ -345,6 +342,13 @@ __global__ void __launch_bounds__(AD_THREADS, 2) attn_decode_kernel(AttnDecodeAr
       const float2_t v = l > 0.0f ? float2_t{o[0] / l, o[1] / l} : o * 0.0f;  // (a NaN stays one)
       *reinterpret_cast<half2_t *>(a.out + ((size_t)b * a.hq + head0 + h) * HD + d) = half2_t{(_Float16)v[0], (_Float16)v[1]};
     }
+  };
+  // (not as the first turn of the loop: its registers might be those of an exchange of the turn before, and it would start with a wait)
+  if (tid < nq * HALF) meet(tid);
+  for (int idx = tid + AD_THREADS; idx < nq * HALF; idx += AD_THREADS) {
+    sums(idx / HALF);
+    if (meets) ml = swap_pair(nodes + 2 * idx + (size_t)(split >> 1) * node, m, l, split & 1);
+    meet(idx);
   }
 }
 
