@@ -17,7 +17,7 @@
 // weights' sum} in one word: weights that are off by |score| 2^-24.  The second word sent when the first has arrived: 0.4 us more.
 // Partials through agent-scope stores, an arrival counter and a last workgroup that reads them back: three trips, 5 us.)
 // Chunks of 128 positions and a launch that merges them (attn_chunk_kernel) -> this: 32 heads over 8 of 128, 16 sequences of 2048
-// positions 27.2 + 4.8 -> 25.3 us (5.3 TB/s; a step of 32 layers 2757 -> 2571), 8 sequences 2205 -> 2117 a step.  With fewer than 64
+// positions 27.2 + 4.8 -> 25.6 us (5.2 TB/s; a step of 32 layers 2757 -> 2584), 8 sequences 2205 -> 2117 a step.  With fewer than 64
 // (sequence, kv head) pairs a workgroup has to take in more than it can at 50 .. 60 GB/s, or the merge gets deep: 4 sequences of 1000
 // positions 1697 -> 1739 a step, 2 of 2048 1547 -> 1602 (2 of 100: 1497 -> 1425).  16 heads over 2 of 64, where one workgroup per head
 // and sequence walked all positions: 16 sequences of 2000 positions 1573 -> 963 us a step of 24 layers, 4 of 1000 950 -> 782, 16 of 360

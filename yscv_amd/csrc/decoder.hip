@@ -710,7 +710,7 @@ static int32_t finish_setup(yscv_hip_decoder *d) {
     const Context *ctx = nullptr;
     YSCV_TRY(ensure_context(&ctx));
     // (a consuming projection adds up at most 256 partial sums per row, four rows per wave of 512 k.  Sixteen rows of up to 64 sums
-    // would fit a wave, 947 -> 858 us a step of 24 layers of d_model 1024 at batch 16; those batches have the norm in f32 with one rounding
+    // would fit a wave, 897 -> 834 us a step of 24 layers of d_model 1024 at batch 16; those batches have the norm in f32 with one rounding
     // at its end, whatever a row's growth within an update, and unnormalised fp16 rows bound it)
     bool ok = d->cfg.d_model % 256 == 0 && d->cfg.d_model <= 4096 && d->fold_norm_wanted;
     auto consumes = [&](const yscv_hip_int4_weight *w) {
