@@ -260,8 +260,6 @@ __global__ void __launch_bounds__(WG_THREADS, 1) int4_gemm_wide_kernel(WideArgs 
   };
   const std::integral_constant<int, 0> K0;
   const std::integral_constant<int, 1> K1;
-  const std::integral_constant<int, 2> K2;
-  const std::integral_constant<int, 3> K3;
   // The matrix pipe takes an MFMA every 16 cycles, two vector instructions of the SIMD fit in between and a third makes it wait
   // (measured: 7.2, 7.3, 7.5, 9.1, 11.1 ns per MFMA with 0 .. 4 of them).  So the decode is dealt out evenly: the instructions
   // whose turn it is behind MFMA `at` of a k-step, counted from MFMA FROM on.
