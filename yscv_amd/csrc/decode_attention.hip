@@ -17,7 +17,7 @@
 // weights' sum} in one word: weights that are off by |score| 2^-24.  The second word sent when the first has arrived: 0.4 us more.
 // Partials through agent-scope stores, an arrival counter and a last workgroup that reads them back: three trips, 5 us.)
 // Chunks of 128 positions and a launch that merges them (attn_chunk_kernel) -> this: 32 heads over 8 of 128, 16 sequences of 2048
-// positions 27.2 + 4.8 -> 25.6 us (5.2 TB/s; a step of 32 layers 2757 -> 2584), 8 sequences 2205 -> 2117 a step.  With fewer than 64
+// positions 27.2 + 4.8 -> 25.4 us (5.3 TB/s; a step of 32 layers 2757 -> 2571), 8 sequences 2205 -> 2117 a step.  With fewer than 64
 // (sequence, kv head) pairs a workgroup has to take in more than it can at 50 .. 60 GB/s, or the merge gets deep: 4 sequences of 1000
 // positions 1697 -> 1739 a step, 2 of 2048 1547 -> 1602 (2 of 100: 1497 -> 1425).  16 heads over 2 of 64, where one workgroup per head
 // and sequence walked all positions: 16 sequences of 2000 positions 1573 -> 963 us a step of 24 layers, 4 of 1000 950 -> 782, 16 of 360
@@ -269,6 +269,7 @@ __global__ void __launch_bounds__(AD_THREADS, 2) attn_decode_kernel(AttnDecodeAr
   const int pair = ((int)b * a.hkv + kvh) * qblocks + qb;
   uint64_t *nodes = a.meet + (size_t)pair * (size_t)a.splits * min(AD_Q, group) * HD;  // (the last block of heads may be smaller)
   const size_t node = (size_t)nq * HD;
+  const int second_word = nq * HALF;  // a node's first words, then its second ones: lanes side by side (in turn: 0.4 us a launch more)
   const bool meets = live > 1 && (split ^ 1) < live;  // at the first level (the last share of an odd number goes on by itself)
   // a thread's two channels of a head: the share's maximum and sum
   float m, l, f[AD_WAVES];
@@ -288,7 +289,7 @@ __global__ void __launch_bounds__(AD_THREADS, 2) attn_decode_kernel(AttnDecodeAr
   uint64_t ml = kEmpty;
   if (tid < nq * HALF) {
     sums(tid / HALF);
-    if (meets) ml = swap_pair(nodes + 2 * tid + (size_t)(split >> 1) * node, m, l, split & 1);  // on its way while the waves' outputs are added up
+    if (meets) ml = swap_pair(nodes + tid + (size_t)(split >> 1) * node, m, l, split & 1);  // on its way while the waves' outputs are added up
   }
   if (r < nq) {
 #pragma unroll
@@ -297,7 +298,7 @@ __global__ void __launch_bounds__(AD_THREADS, 2) attn_decode_kernel(AttnDecodeAr
   lds_barrier();
   auto meet = [&](int idx) __attribute__((always_inline)) {
     const int h = idx / HALF, d = idx % HALF * 2;
-    uint64_t *level = nodes + 2 * idx;
+    uint64_t *level = nodes + idx;
     float2_t o = {0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < AD_WAVES; w++) o += *reinterpret_cast<const float2_t *>(&o_s[(w * nq + h) * OP + d]) * f[w];
@@ -309,7 +310,7 @@ __global__ void __launch_bounds__(AD_THREADS, 2) attn_decode_kernel(AttnDecodeAr
         level += (size_t)(width >> 1) * node;
         if ((at ^ 1) >= count) continue;
         if (bit > 1) ml = swap_pair(slot, m, l, at & 1);
-        const uint64_t ov = swap_pair(slot + 1, o[0], o[1]);
+        const uint64_t ov = swap_pair(slot + second_word, o[0], o[1]);
         if (ov == kEmpty) {
           top = false;
           break;
@@ -328,12 +329,12 @@ __global__ void __launch_bounds__(AD_THREADS, 2) attn_decode_kernel(AttnDecodeAr
         m = mx;
       }
       // the slots are emptied at the end: a store in front of the next exchange would be waited for with it
-      level = nodes + 2 * idx;
+      level = nodes + idx;
       for (int at = split, width = a.splits; met != 0; at >>= 1, width >>= 1, met >>= 1) {
         uint64_t *slot = level + (size_t)(at >> 1) * node;
         if (met & 1) {
           __hip_atomic_store(slot, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(slot + 1, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(slot + second_word, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         level += (size_t)(width >> 1) * node;
       }
@@ -347,7 +348,7 @@ __global__ void __launch_bounds__(AD_THREADS, 2) attn_decode_kernel(AttnDecodeAr
   if (tid < nq * HALF) meet(tid);
   for (int idx = tid + AD_THREADS; idx < nq * HALF; idx += AD_THREADS) {
     sums(idx / HALF);
-    if (meets) ml = swap_pair(nodes + 2 * idx + (size_t)(split >> 1) * node, m, l, split & 1);
+    if (meets) ml = swap_pair(nodes + idx + (size_t)(split >> 1) * node, m, l, split & 1);
     meet(idx);
   }
 }
