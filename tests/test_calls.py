@@ -28,9 +28,9 @@ def test_calls_that_are_not_taken_go_the_general_way():
         _calls.bind(1)
 
 
-@pytest.mark.parametrize("module", ["None", "types.SimpleNamespace(torch_version=lambda: '0.0')"])
+@pytest.mark.parametrize("module", ["None", "types.SimpleNamespace(torch_version=lambda: '0.0')", "types.SimpleNamespace()"])
 def test_without_a_module_that_fits(module):
-    """Not built, or built for another torch: the package is there all the same, and every call goes the general way."""
+    """Not built, built for another torch, or an older build that does not say for which: the package is there all the same, and every call goes the general way."""
     code = f"""
 import sys, types, warnings
 warnings.simplefilter("ignore")

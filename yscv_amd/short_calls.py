@@ -20,8 +20,9 @@ def _load():
         from . import _calls
     except ImportError:  # not built, or symbols that this torch does not have
         return _None()
-    if _calls.torch_version() != torch.__version__:
-        warnings.warn(f"yscv_amd/_calls.so was built for torch {_calls.torch_version()}, not {torch.__version__}: calls go through ctypes "
+    built_for = _calls.torch_version() if hasattr(_calls, "torch_version") else "of an unknown version"  # (a build older than this file)
+    if built_for != torch.__version__:
+        warnings.warn(f"yscv_amd/_calls.so was built for torch {built_for}, not {torch.__version__}: calls go through ctypes "
                       "(make -C yscv_amd/csrc builds it anew)", RuntimeWarning)
         return _None()
     return _calls
