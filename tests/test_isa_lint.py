@@ -14,6 +14,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hi
          "-Xclang", "-packed-fp32-ops", "-S", "--cuda-device-only"]
 # the sources with asm loads or hand-counted waits, and their extra flags in the Makefile
 SOURCES = {"int4_gemm_ring.hip": [], "decode_persistent.hip": [], "i8_gemm.hip": ["-ffp-contract=off"], "int4_gemm_wide.hip": [],
+           "i8_gemm_wide.hip": ["-ffp-contract=off"],
            "int4_ksplit.hip": [], "i8_ksplit.hip": ["-ffp-contract=off"], "glue_ops.hip": [], "decode_layers.hip": [], "decode_wide.hip": []}
 # sources whose asm loads have nothing to overlap: each waits in its own statement
 WAITS_AT_ONCE = ("decode_layers.hip", "decode_wide.hip")

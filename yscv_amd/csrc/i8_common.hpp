@@ -14,14 +14,25 @@ __device__ __forceinline__ float round_half_away(float v) {
   return (d >= 0.5f) ? __fadd_rn(t, copysignf(1.0f, v)) : t;
 }
 
+// clamp(round(a * comp + y_zp), lo, hi) as an int, a NaN as 0 (clamp keeps it, `as i8` makes it 0).  Rounding is monotonic and leaves lo and hi
+// as they are, so the clamp comes first: what is rounded is then finite or a NaN, and half away from zero is trunc(v) + trunc(2 (v - trunc(v))).
+template <bool HALF_AWAY>
+__device__ __forceinline__ int requant_int(int32_t a, float comp, float y_zp, float lo, float hi) {
+  float v = __fadd_rn(__fmul_rn((float)a, comp), y_zp);  // two roundings, never an FMA
+  v = __builtin_elementwise_minimum(__builtin_elementwise_maximum(v, lo), hi);  // (these keep a NaN)
+  if constexpr (HALF_AWAY) {
+    const float t = truncf(v), d = __fsub_rn(v, t);
+    v = __fadd_rn(t, truncf(__fadd_rn(d, d)));
+  } else {
+    v = rintf(v);
+  }
+  return (int)v;
+}
+
 __device__ __forceinline__ int requant_one(int32_t acc, int32_t corr, float comp, float y_zp, int round_mode,
                                            float lo, float hi) {
-  int32_t a = (int32_t)((uint32_t)acc + (uint32_t)corr);         // wrapping_add
-  float v = __fadd_rn(__fmul_rn((float)a, comp), y_zp);          // two roundings, never an FMA
-  float r = round_mode == YSCV_HIP_ROUND_HALF_AWAY ? round_half_away(v) : rintf(v);
-  if (r != r) return 0;                                          // clamp keeps NaN, `as i8` -> 0
-  r = fminf(fmaxf(r, lo), hi);
-  return (int)r;
+  const int32_t a = (int32_t)((uint32_t)acc + (uint32_t)corr);  // wrapping_add
+  return round_mode == YSCV_HIP_ROUND_HALF_AWAY ? requant_int<true>(a, comp, y_zp, lo, hi) : requant_int<false>(a, comp, y_zp, lo, hi);
 }
 
 // requantise, then DequantizeLinear of the quantised value: (q - y_zp) * dq_scale (crates/yscv-onnx/src/runner/misc.rs:124-128)
@@ -64,9 +75,13 @@ struct I8Args {
 
 static_assert(sizeof(I8Args) + 2 * sizeof(int) <= kCheapArgs, "arguments of a launch");
 
-// Shapes whose tiles leave the ring kernel's grid short of the CUs (i8_ksplit.hip): 16-byte aligned a with an lda that is a
-// multiple of 64, m * lda below 2 GiB.
-bool i8_ksplit_takes(size_t m, size_t n, size_t ksteps, int num_cus);
+// The matrix kernels, on 16-byte aligned a with an lda that is a multiple of 64, m * lda below 2 GiB, and the us that a launch is
+// estimated to take: small tiles whose waves split K (i8_ksplit.hip; the tiles that all run at once, 1e30 where none do), and large ones
+// (i8_gemm_wide.hip; two k-steps at least).
+double i8_ksplit_us(size_t m, size_t n, size_t ksteps, size_t cus);
 int32_t launch_i8_ksplit(const I8Args &p, int num_cus, hipStream_t s);
+enum : int { IW_64x128, IW_128x256 };
+double i8_wide_us(int tile, size_t m, size_t n, size_t ksteps, bool requant, size_t cus);
+int32_t launch_i8_gemm_wide(const I8Args &p, int tile, hipStream_t s);
 
 }  // namespace yscv

@@ -1,14 +1,14 @@
 // int8 x int8 -> int32 GEMM for shapes with few tiles: y[m][n] = sum_k a[m][k] * b[k][n], zero-point correction and
 // requantising epilogue fused as in i8_gemm.hip.  Replaces int8_matmul_dispatch / int8_matmul_prepacked_dispatch
-// (crates/yscv-kernels/src/ops/int8_matmul.rs:2407-2425) where the ring kernel's 64 x 128 tiles are fewer than the CUs.
+// (crates/yscv-kernels/src/ops/int8_matmul.rs:2407-2425) where i8_gemm_wide.hip's tiles are fewer than the CUs.
 //
-// Such a call is bound by latency, not by bytes or MFMAs, and the ring kernel makes its chain long: few workgroups, each of
-// which walks the whole K stage by stage with a barrier between producers and consumers.  Here a workgroup owns a small
+// Such a call is bound by latency, not by bytes or MFMAs, and large tiles make its chain long: few workgroups, each of
+// which walks the whole K stage by stage with barriers between.  Here a workgroup owns a small
 // tile of 16 MT rows x 16 NT columns, its waves split the K of the tile, and every wave feeds itself through slots of LDS
 // of its own, filled by LDS-direct loads (A in whole 128-byte lines, B as it is packed): no barrier until the waves' tiles
 // are added (integers, so in any order) and stored as whole rows.
 // A pair is two k-steps of 64, 128 bytes of every row of the tile; a wave keeps NP pairs in flight, 96 .. 144 KB per CU.
-// us, ring kernel -> this one (m x n x k): 1 x 4096 x 4096 17.2 -> 5.7, 16 x 256 x 8192 20.5 -> 5.9, 64 x 4096 x 4096
+// us, tiles of 64 x 128 whose waves walk all of K -> this one (m x n x k): 1 x 4096 x 4096 17.2 -> 5.7, 16 x 256 x 8192 20.5 -> 5.9, 64 x 4096 x 4096
 // 18.5 -> 6.8, 128 x 4096 x 1024 9.2 -> 5.1, 197 x 768 x 3072 12.3 -> 5.1, 256 x 4096 x 4096 16.8 -> 12.3,
 // 512 x 1024 x 1024 8.5 -> 5.0, 1024 x 768 x 768 8.4 -> 6.7.  What is left is launch, first loads and the last store (3 us)
 // and, with the large tiles, the fill of a CU's LDS (64 x 64 tiles, K 4096: 512 KB per CU in 9 us).
@@ -224,15 +224,14 @@ struct IksShape {
   double fixed, per_pair;
 };
 constexpr IksShape kIksShapes[] = {{1, 1, 8, 2.7, 0.42}, {1, 2, 8, 2.85, 0.44}, {1, 4, 4, 3.1, 0.54}, {2, 1, 8, 2.85, 0.45}, {2, 2, 8, 3.1, 0.50},
-                                   {2, 4, 4, 3.8, 0.55}, {4, 2, 4, 3.7, 0.55}, {4, 4, 4, 5.3, 0.80}};
+                                   {2, 4, 4, 3.8, 0.55}, {4, 2, 4, 3.75, 0.68}, {4, 4, 4, 4.5, 1.0}};
 constexpr int kIksShapeCount = sizeof(kIksShapes) / sizeof(kIksShapes[0]);
 
-// The shape with the shortest estimate among those whose workgroups all run at once.  There every shape measured was faster
-// than the ring kernel; from two rounds over the CUs on the ring kernel's larger tiles win (512 x 4096 x 4096: 17.0 against
-// 21.8 us with 64 x 64 tiles), as they share operands among more MFMAs.
-int iks_pick(size_t m, size_t n, size_t ksteps, size_t cus) {
+// The shape with the shortest estimate among those whose workgroups all run at once, and that estimate.  (From two rounds over the
+// CUs on the large tiles win, as they share operands among more MFMAs.)
+int iks_pick(size_t m, size_t n, size_t ksteps, size_t cus, double &best_us) {
   int best = -1;
-  double best_us = 1e30;
+  best_us = 1e30;
   for (int i = 0; i < kIksShapeCount; i++) {
     const IksShape &sh = kIksShapes[i];
     const size_t tiles = ceil_div(m, (size_t)16 * sh.mt) * ceil_div(n, (size_t)16 * sh.nt);
@@ -261,11 +260,16 @@ int32_t iks_launch_shape(int shape, const I8Args &p, hipStream_t s) {
 
 }  // namespace
 
-bool i8_ksplit_takes(size_t m, size_t n, size_t ksteps, int num_cus) { return iks_pick(m, n, ksteps, num_cus > 0 ? (size_t)num_cus : 256) >= 0; }
+double i8_ksplit_us(size_t m, size_t n, size_t ksteps, size_t cus) {
+  double us;
+  (void)iks_pick(m, n, ksteps, cus, us);
+  return us;
+}
 
 int32_t launch_i8_ksplit(const I8Args &p, int num_cus, hipStream_t s) {
-  const int shape = iks_pick((size_t)p.m, (size_t)p.n, (size_t)p.ksteps, num_cus > 0 ? (size_t)num_cus : 256);
-  if (shape < 0) return set_error(YSCV_HIP_ERR_INVALID_ARG, "%d x %d has too many tiles for the K-split kernel", p.m, p.n);
+  double us;
+  int shape = iks_pick((size_t)p.m, (size_t)p.n, (size_t)p.ksteps, num_cus > 0 ? (size_t)num_cus : 256, us);
+  if (shape < 0) shape = kIksShapeCount - 1;  // (a K of 64 with more tiles than CUs)
   return iks_launch_shape(shape, p, s);
 }
 
