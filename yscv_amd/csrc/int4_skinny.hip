@@ -6,10 +6,11 @@
 // issue per byte streamed (about 80 VALU slots per KiB of weights at 8 TB/s), so everything in the
 // inner loop is there to keep that count low:
 //   * weights stream from HBM exactly once, as 1 KiB coalesced tiles (one 128-bit load per lane,
-//     layout in int4_common.hpp); a ring of P register slots keeps P-1 blocks in flight per wave.
+//     layout in int4_common.hpp); a ring of register slots keeps two to four blocks in flight per wave.
 //     Every iteration issues the same loads (requests past the last block repeat it, served by the
-//     caches), so the compiler's s_waitcnt counts are exact; the first P blocks are requested
-//     before the activations are fetched, and no load in the kernel sits behind a per-load branch
+//     caches), so the compiler's s_waitcnt counts are exact; the first blocks are requested
+//     right behind five or more activation rows and before fewer of them (loads return in order),
+//     and no load in the kernel sits behind a per-load branch
 //     (a guarded load costs one memory round trip each, under load more than a microsecond);
 //   * the activation rows sit in registers for the whole kernel, as fp16 hi (+ lo for f32 input),
 //     already in MFMA A-operand order: the inner loop reads neither LDS nor L2 for them;
@@ -119,11 +120,21 @@ __device__ __forceinline__ void zp_consts(uint32_t zp, half2_t &c1, half2_t &c2)
 // 64 bytes apart modulo the bank cycle so the sixteen lanes that carry a row read conflict-free
 constexpr int kStageRow = 512 * 2 + 64, kStageWave = 2 * 4 * kStageRow;
 constexpr int skinny_ub(int ni, int p) { return p % 4 == 0 ? 4 : (p % 2 == 0 && ni > 1 ? 2 : 1); }
+// Blocks in flight per wave, of a kernel whose loop takes P in a round.  A CU has some 70 KB of loads in flight and no more: a wave that asks
+// for further blocks stands still until the first ones are there, with nobody to work on them.  So two blocks, of eight waves 73 KB, and the
+// activations in front of them (loads return in order, to all waves of a CU): 28672 x 4096, 16 bf16 rows 19.5 -> 17.7 us, 4096 x 4096 7.4 -> 6.7,
+// 4096 x 14336 14.9 -> 13.9 (three quarters of it behind a full ring of four: first products 5.4 us into the kernel, waves four to seven 11).
+// Long streams take four: their ring is never empty, and two leave a gap between a block's products and the next request (128256 x 4096 58.1 us,
+// with two 60.6; 40000 x 2048, ten rounds, 16.8 and 17.2).
+constexpr int kDeep = 8;  // P of those: rounds of four too
+constexpr int skinny_round(int p) { return p == kDeep ? 4 : p; }
+constexpr int skinny_ring(int ni, int p, int xm, bool early) { return early && xm != 1 && ni > 1 && p == 4 ? 2 : skinny_round(p); }
 
 // XM: where the activations come from -- 0 prepared fp16 (hi [+ lo]), 1 raw f32 (split into hi + lo here), 2 raw bf16
 // FOLD: a norm is folded into this call; other calls leave that code out
-template <int SPLIT, int NI, int GM, bool SF16, bool HAS_ZP, int P, int XM, bool FOLD>
+template <int SPLIT, int NI, int GM, bool SF16, bool HAS_ZP, int FORM, int XM, bool FOLD>
 __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
+  constexpr int P = skinny_round(FORM);
   constexpr bool RAWX = XM != 0;
   static_assert(XM != 1 || SPLIT == 2, "raw f32 activations are split into hi + lo");
   static_assert(XM != 2 || SPLIT == 1, "bf16 activations fit one fp16 operand exactly");
@@ -194,21 +205,24 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
     if constexpr (HAS_ZP) zp += z_step;
   };
 
-  // ---- the first P blocks are requested before the activation set-up (EARLY, where the registers allow it: their
-  // HBM latency then overlaps the set-up) or right after it ----
+  // ---- the first blocks are requested before the activation set-up (EARLY, where the registers allow it: their
+  // HBM latency then overlaps the set-up), inside it (X_FIRST: the activations of many rows are as many bytes as a block and
+  // would wait for it) or right after it ----
   // Block `it` of this workgroup is 16-row block blockIdx.x + it * stride.  Requests past the last block are clamped
   // to it (a repeat served by the caches) so that every iteration issues the same number of loads and the
   // compiler's s_waitcnt counts stay exact.
   constexpr bool EARLY = (SPLIT == 1 || (XM == 1 && NI == 1)) && !HAS_ZP;
+  constexpr bool X_FIRST = EARLY && XM != 1 && NI > 1 && FORM != kDeep;  // the activations in front of the first blocks
+  constexpr int R = skinny_ring(NI, FORM, XM, EARLY);                     // blocks in flight
   const int iters = (a.nt - (int)blockIdx.x + stride - 1) / stride;  // >= 1, uniform in the workgroup
-  Regs ring[P];
+  Regs ring[R];
   auto fill_ring = [&]() {
-    if (wave_active) {
+    if (X_FIRST || wave_active) {  // (an idle wave's requests repeat the first slice: behind a test the compiler would wait for the ring with the activations)
 #pragma unroll
-      for (int sl = 0; sl < P; sl++) issue(ring[sl], sl < iters ? sl : iters - 1);
+      for (int sl = 0; sl < R; sl++) issue(ring[sl], sl < iters ? sl : iters - 1);
     }
   };
-  if constexpr (EARLY) fill_ring();
+  if constexpr (EARLY && !X_FIRST) fill_ring();
   // folded norm, consumer side: this wave's share of the partial sums of squares (see further down), requested
   // here so that their round trip overlaps the activations'
   // Rows wave, wave + waves, ...: the launcher checks that four per wave cover m.  Four partial sums per lane (those past the end of a row
@@ -281,11 +295,16 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
         for (int t = 0; t < TPW; t++)
 #pragma unroll
           for (int j = 0; j < 4; j++) raw[t][j] = *reinterpret_cast<const uint4_t *>(src + block_k(t, j));
+      }
+      if constexpr (X_FIRST) {
+        asm volatile("" ::: "memory");
+        fill_ring();
+      }
+      if (!whole) {
 #pragma unroll
         for (int t = 0; t < TPW; t++)
 #pragma unroll
-          for (int j = 0; j < 4; j++)
-            if (!block_in(t, j)) raw[t][j] = uint4_t{0, 0, 0, 0};
+          for (int j = 0; j < 4; j++) raw[t][j] &= block_in(t, j) ? ~0u : 0u;
       }
       uint32_t amax_bits = 0;  // |bf16| orders like its bit pattern
 #pragma unroll
@@ -438,7 +457,6 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
       }
     } else {
       const size_t row_off = (size_t)(valid ? mrow : 0) * a.ldx + c * 8;
-      const half8_t hz = {0, 0, 0, 0, 0, 0, 0, 0};
       if (whole) {
 #pragma unroll
         for (int t = 0; t < TPW; t++)
@@ -457,24 +475,26 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
             xa[t][j][0] = *reinterpret_cast<const half8_t *>(xh + off);
             if constexpr (SPLIT == 2) xa[t][j][1] = *reinterpret_cast<const half8_t *>(a.xl + off);
           }
+      }
+      if constexpr (X_FIRST) {
+        asm volatile("" ::: "memory");
+        fill_ring();
+        if (!(whole && wave_active && a.m == 4 * NI)) {  // uniform: rows or k-blocks that there are not
+#pragma unroll
+          for (int t = 0; t < TPW; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) xa[t][j][0] = __builtin_bit_cast(half8_t, __builtin_bit_cast(uint4_t, xa[t][j][0]) & (valid && block_in(t, j) ? ~0u : 0u));
+        }
+      } else {
+        const half8_t hz = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int t = 0; t < TPW; t++)
 #pragma unroll
-          for (int j = 0; j < 4; j++)
-            if (!block_in(t, j)) {
-              xa[t][j][0] = hz;
-              if constexpr (SPLIT == 2) xa[t][j][1] = hz;
-            }
-      }
-#pragma unroll
-      for (int t = 0; t < TPW; t++) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          if (!valid) xa[t][j][0] = hz;
-          if constexpr (SPLIT == 2) {
-            if (!valid) xa[t][j][1] = hz;
+          for (int j = 0; j < 4; j++) {
+            const bool in = valid && (whole || block_in(t, j));
+            xa[t][j][0] = in ? xa[t][j][0] : hz;
+            if constexpr (SPLIT == 2) xa[t][j][1] = in ? xa[t][j][1] : hz;
           }
-        }
       }
     }
   }
@@ -744,7 +764,7 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
     }
   };
 
-  // ---- main loop: slot it % P holds block it; after its dot products the slot is refilled with block it + P ----
+  // ---- main loop: slot it % R holds block it; after its dot products the slot is refilled with block it + R ----
   int nt = blockIdx.x;  // first block of the current group of UB
   int it = 0, ex = 0;
   float accs[UB][NI];
@@ -759,13 +779,13 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
     return;
   }
 
-  const int steady = (iters + P - 1) / P - 1;  // groups of P iterations that refill; the last group only drains
+  const int steady = (iters + P - 1) / P - 1;  // groups of P iterations that all refill; the last group's last R only drain
   for (int g = 0; g < steady; g++) {
 #pragma unroll
     for (int sl = 0; sl < P; sl++) {
-      dots(ring[sl], accs[sl % UB]);
-      const int left = iters - 1 - it;  // blocks after this one (>= P - sl, as one more group follows)
-      issue(ring[sl], left < P ? left : P);
+      dots(ring[sl % R], accs[sl % UB]);
+      const int left = iters - 1 - it;  // blocks after this one
+      issue(ring[sl % R], left < R ? left : R);
       if (sl % UB == UB - 1) {
         reduce_store(accs, nt, ex);
         nt += UB * stride;
@@ -778,16 +798,21 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
 #pragma unroll
   for (int sl = 0; sl < P; sl++) {
     if (it < iters) {
-      dots(ring[sl], accs[sl % UB]);
+      dots(ring[sl % R], accs[sl % UB]);
     } else {
 #pragma unroll
       for (int i = 0; i < NI; i++) accs[sl % UB][i] = 0.0f;
+    }
+    if (sl + R < P) {
+      const int left = iters - 1 - it;
+      issue(ring[sl % R], left < 0 ? 0 : (left < R ? left : R));
     }
     if (sl % UB == UB - 1) {
       if (it - (UB - 1) < iters) reduce_store(accs, nt, ex);  // the group's first block exists
       nt += UB * stride;
       ex++;
     }
+    if (sl + R < P && it + 1 < iters) advance();
     it++;
   }
 }
@@ -906,7 +931,7 @@ static unsigned skinny_groups(const SkinnyArgs &a) {
 
 template <int SPLIT, int NI, int GM, bool SF16, bool HAS_ZP, int P>
 static int32_t launch_p(const SkinnyArgs &a, const SkinnyPlan &plan, bool xraw, const SkinnyFold *fold, hipStream_t s) {
-  constexpr int UB = skinny_ub(NI, P);
+  constexpr int UB = skinny_ub(NI, skinny_round(P));
   const size_t lds = (size_t)2 * plan.waves * UB * NI * 64 * sizeof(float) + 64;  // + the sixteen row factors of a folded norm
   if constexpr (SPLIT == 2) {
     if (xraw) {
@@ -965,6 +990,9 @@ static int32_t launch_one(const SkinnyArgs &a, const SkinnyPlan &plan, bool xraw
       const int blocks_per_wg = (a.nt + plan.grid_x - 1) / plan.grid_x;
       if (blocks_per_wg == 1) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 1>(a, plan, xraw, fold, s);
       if (blocks_per_wg == 2) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 2>(a, plan, xraw, fold, s);
+      if constexpr (P == 4 && NI > 1) {
+        if (blocks_per_wg > 8) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, kDeep>(a, plan, xraw, fold, s);
+      }
     }
     return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, P>(a, plan, xraw, fold, s);
   }
