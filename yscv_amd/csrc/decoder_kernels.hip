@@ -109,27 +109,22 @@ __global__ void __launch_bounds__(256) embed_norm_kernel(const int32_t *__restri
 }
 
 // ---- RMSNorm: f32 residual -> fp16 normalised activations -----------------------------------------
+// A row of up to KEEP x 1024 values and gamma wait in registers: one memory round trip; KEEP 0: longer rows are read twice
+template <int KEEP>
 __global__ void __launch_bounds__(256) rmsnorm_kernel(const float *__restrict__ h, const float *__restrict__ gamma,
                                                       int d, float eps, _Float16 *__restrict__ out) {
   __shared__ float red[4];
   const int b = blockIdx.x;
   const float *row = h + (size_t)b * d;
-  // a row of up to 8192 values stays in registers between the two passes (one memory round trip instead of two);
-  // longer rows are read again
-  constexpr int KEEP = 8;
-  float4_t keep[KEEP];
-  const bool fits = d <= KEEP * 256 * 4;
+  constexpr int REGS = KEEP > 0 ? KEEP : 1;
+  float4_t keep[REGS], gain[REGS];
   float ss = 0.0f;
-  if (fits) {
-#pragma unroll
-    for (int u = 0; u < KEEP; u++) {
-      const int i = (u * 256 + (int)threadIdx.x) * 4;
-      keep[u] = i < d ? *reinterpret_cast<const float4_t *>(row + i) : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+  if constexpr (KEEP > 0) {
+    norm_load<KEEP>(row, gamma, d, keep, gain);
 #pragma unroll
     for (int u = 0; u < KEEP; u++) {
       const float4_t v = keep[u];
-      if ((u * 256 + (int)threadIdx.x) * 4 < d) ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+      ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
     }
   } else {
     for (int i = threadIdx.x * 4; i < d; i += 256 * 4) {
@@ -137,33 +132,26 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(const float *__restrict__ 
       ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
     }
   }
-  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+  ss = wave_sum_far_first(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
   ss = red[0] + red[1] + red[2] + red[3];
   const float inv = 1.0f / sqrtf(ss / (float)d + eps);
-  if (fits) {
-#pragma unroll
-    for (int u = 0; u < KEEP; u++) {
-      const int i = (u * 256 + (int)threadIdx.x) * 4;
-      if (i < d) {
-        const float4_t v = keep[u];
-        const float4_t g = *reinterpret_cast<const float4_t *>(gamma + i);
-        half4_t o;
-#pragma unroll
-        for (int e = 0; e < 4; e++) o[e] = (_Float16)(v[e] * inv * g[e]);
-        *reinterpret_cast<half4_t *>(out + (size_t)b * d + i) = o;
-      }
-    }
-    return;
-  }
-  for (int i = threadIdx.x * 4; i < d; i += 256 * 4) {
-    float4_t v = *reinterpret_cast<const float4_t *>(row + i);
-    float4_t g = *reinterpret_cast<const float4_t *>(gamma + i);
+  auto put = [&](int i, const float4_t &v, const float4_t &g) {
     half4_t o;
 #pragma unroll
     for (int e = 0; e < 4; e++) o[e] = (_Float16)(v[e] * inv * g[e]);
     *reinterpret_cast<half4_t *>(out + (size_t)b * d + i) = o;
+  };
+  if constexpr (KEEP > 0) {
+#pragma unroll
+    for (int u = 0; u < KEEP; u++) {
+      const int i = (u * 256 + (int)threadIdx.x) * 4;
+      if (i < d) put(i, keep[u], gain[u]);
+    }
+  } else {
+    for (int i = threadIdx.x * 4; i < d; i += 256 * 4)
+      put(i, *reinterpret_cast<const float4_t *>(row + i), *reinterpret_cast<const float4_t *>(gamma + i));
   }
 }
 
@@ -1307,7 +1295,11 @@ int32_t launch_embed_norm(const int32_t *tokens, const _Float16 *table, int batc
 
 int32_t launch_rmsnorm(const float *h, const float *gamma, int batch, int d, float eps, _Float16 *out,
                        hipStream_t s) {
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3(batch), dim3(256), 0, s, h, gamma, d, eps, out);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(batch), dim3(256), 0, s, h, gamma, d, eps, out); };
+  if (d <= 1024) go(rmsnorm_kernel<1>);
+  else if (d <= 4096) go(rmsnorm_kernel<4>);
+  else if (d <= 8192) go(rmsnorm_kernel<8>);
+  else go(rmsnorm_kernel<0>);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }

@@ -1035,24 +1035,21 @@ int32_t gqa_flat_launch(FlatArgs p, int B, int num_cus, hipStream_t s) {
 }
 
 // ---- RMSNorm over the last axis, f32 in and out ---------------------------------------------------------------
+// Latency- and HBM-bound: the row (KEEP x 1024 values, sixteen bytes per lane and load) and gamma behind it are asked for at once and wait
+// in registers, so that one memory round trip is all there is between launch and stores (each load of the row was waited for inside its
+// test, and gamma behind the sum).  us: 512 x 8192 6.3 -> 5.7, 4096 x 1024 6.3 -> 5.1, 2048 x 4096 10.7 -> 10.3, 512 x 4096 with the
+// attention behind it 19.5 -> 19.1.  KEEP 0: longer, odd or unaligned rows, read twice.
+template <int KEEP>
 __global__ void __launch_bounds__(256) rms_norm_f32_kernel(const float *__restrict__ x, const float *__restrict__ gamma, int d,
                                                            float eps, float *__restrict__ y) {
   __shared__ float red[4];
   const float *row = x + (size_t)blockIdx.x * d;
   float *out = y + (size_t)blockIdx.x * d;
-  // HBM-bound: the row stays in registers between its two uses (up to KEEP x 1024 values, sixteen bytes per lane and
-  // load); longer, odd or unaligned rows are read twice
-  constexpr int KEEP = 8;
-  const bool vec = (d & 3) == 0 && d <= KEEP * 1024 &&
-                   ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(gamma)) & 15) == 0;
-  float4_t v[KEEP];
+  constexpr int REGS = KEEP > 0 ? KEEP : 1;
+  float4_t v[REGS], g[REGS];
   float ss = 0.0f;
-  if (vec) {
-#pragma unroll
-    for (int j = 0; j < KEEP; j++) {
-      const int i = (j * 256 + (int)threadIdx.x) * 4;
-      v[j] = i < d ? *reinterpret_cast<const float4_t *>(row + i) : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+  if constexpr (KEEP > 0) {
+    norm_load<KEEP>(row, gamma, d, v, g);
 #pragma unroll
     for (int j = 0; j < KEEP; j++) ss += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
   } else {
@@ -1064,11 +1061,11 @@ __global__ void __launch_bounds__(256) rms_norm_f32_kernel(const float *__restri
   ss = red[0] + red[1] + red[2] + red[3];
   // rms = sqrt(sum / n + eps); inv_rms = 1 / rms; y = x * inv_rms * gamma (ops/norm.rs:1507-1516, in that order)
   const float inv_rms = 1.0f / sqrtf(ss / (float)d + eps);
-  if (vec) {
+  if constexpr (KEEP > 0) {
 #pragma unroll
     for (int j = 0; j < KEEP; j++) {
       const int i = (j * 256 + (int)threadIdx.x) * 4;
-      if (i < d) *reinterpret_cast<float4_t *>(out + i) = v[j] * inv_rms * *reinterpret_cast<const float4_t *>(gamma + i);
+      if (i < d) *reinterpret_cast<float4_t *>(out + i) = v[j] * inv_rms * g[j];
     }
   } else {
     for (int i = threadIdx.x; i < d; i += 256) out[i] = row[i] * inv_rms * gamma[i];
@@ -1218,9 +1215,15 @@ int32_t yscv_hip_rms_norm_dev(const float *x, const float *gamma, size_t rows, s
   YSCV_REQUIRE(std::isfinite(eps) && eps > 0.0f, "rms_norm: epsilon must be finite and > 0");
   YSCV_REQUIRE(d > 0 && d < ((size_t)1 << 31) && rows < ((size_t)1 << 31), "rms_norm: bad shape %zu x %zu", rows, d);
   const size_t step = (size_t)1 << 23;  // a grid holds less than 2^32 threads
+  const bool vec = d % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(gamma)) & 15) == 0;
   for (size_t r0 = 0; r0 < rows; r0 += step) {
-    hipLaunchKernelGGL(rms_norm_f32_kernel, dim3((unsigned)std::min(step, rows - r0)), dim3(256), 0, as_stream(stream), x + r0 * d, gamma,
-                       (int)d, eps, y + r0 * d);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(step, rows - r0)), dim3(256), 0, as_stream(stream), x + r0 * d, gamma, (int)d, eps, y + r0 * d);
+    };
+    if (!vec || d > 8192) go(rms_norm_f32_kernel<0>);
+    else if (d <= 1024) go(rms_norm_f32_kernel<1>);
+    else if (d <= 4096) go(rms_norm_f32_kernel<4>);
+    else go(rms_norm_f32_kernel<8>);
     YSCV_HIP_TRY(hipGetLastError());
   }
   return YSCV_HIP_OK;

@@ -255,6 +255,18 @@ __device__ __forceinline__ float row_max16(float v) {
   return v;
 }
 __device__ __forceinline__ float wave_sum(float v) { return sum_xor16_xor32(row_sum16(v)); }
+// the same in the order of a loop of __shfl_xor over 32, 16, .. 1 (lanes that already agree turn a rotation into that exchange)
+__device__ __forceinline__ float wave_sum_far_first(float v) {
+  float x, y;
+  xor32_pair(v, x, y);
+  v = x + y;
+  xor16_pair(v, x, y);
+  v = x + y;
+  v += dpp_move<DPP_ROR8>(v);
+  v += dpp_move<DPP_ROR4>(v);
+  v += dpp_move<DPP_XOR2>(v);
+  return v + dpp_move<DPP_XOR1>(v);
+}
 __device__ __forceinline__ float max_xor16_xor32(float v) {  // max(v, v[lane ^ 16]), then the same over lane ^ 32
   float x, y;
   xor16_pair(v, x, y);
@@ -263,6 +275,22 @@ __device__ __forceinline__ float max_xor16_xor32(float v) {  // max(v, v[lane ^ 
   return fmaxf(x, y);
 }
 __device__ __forceinline__ float wave_max(float v) { return max_xor16_xor32(row_max16(v)); }
+
+// A row of up to KEEP x 1024 values (d % 4 == 0) and its norm's gamma into the registers of 256 threads, v zero past the end.  The row comes
+// first: loads return in order, and the sum of squares needs nothing else.  Requests past the end repeat the last four values: behind a
+// test each load would be waited for inside it, one memory round trip after the other.
+template <int KEEP>
+__device__ __forceinline__ void norm_load(const float *__restrict__ row, const float *__restrict__ gamma, int d, float4_t (&v)[KEEP], float4_t (&g)[KEEP]) {
+  const int i = (int)threadIdx.x * 4;
+#pragma unroll
+  for (int j = 0; j < KEEP; j++) v[j] = *reinterpret_cast<const float4_t *>(row + min(i + j * 1024, d - 4));
+#pragma unroll
+  for (int j = 0; j < KEEP; j++) g[j] = *reinterpret_cast<const float4_t *>(gamma + min(i + j * 1024, d - 4));
+#pragma unroll
+  for (int j = 0; j < KEEP; j++) {
+    if (i + j * 1024 >= d) v[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+}
 
 // The power of two at or below 1 / (4 rms), rms = 1 / inv_rms, kept within 2^-40 .. 2^40 (NormFold, kernels.hpp)
 __device__ __forceinline__ float norm_fold_prescale(float inv_rms) {
