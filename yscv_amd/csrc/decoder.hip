@@ -1590,14 +1590,16 @@ static int32_t prefill_chunk(yscv_hip_decoder *d, const int32_t *tokens_dev, int
     return at;
   };
   const size_t at_h = place(R * D * 4), at_xn = place(R * D * 2), at_qkv = place(R * qkv_n * 2), at_ao = place(R * hq * 2),
-               at_act = place(R * ff * 2), at_tk = place(t_bytes), at_tv = place(t_bytes), at_ws = place(ws_bytes);
+               at_act = place(R * ff * 2), at_tk = place(t_bytes), at_tv = place(t_bytes),
+               at_angles = place(i8 ? 0 : prefill_angles_bytes(R, c.head_dim)), at_ws = place(ws_bytes);
   YSCV_TRY(keep_prefill_buffer(d, need));
   char *base = static_cast<char *>(d->pf_buf);
   float *h = reinterpret_cast<float *>(base + at_h);
   _Float16 *xn = reinterpret_cast<_Float16 *>(base + at_xn), *qkv = reinterpret_cast<_Float16 *>(base + at_qkv),
            *ao = reinterpret_cast<_Float16 *>(base + at_ao), *act = reinterpret_cast<_Float16 *>(base + at_act),
            *tk = reinterpret_cast<_Float16 *>(base + at_tk), *tv = reinterpret_cast<_Float16 *>(base + at_tv);
-  void *pws = base + at_ws;
+  void *pws = base + at_ws, *angles = base + at_angles;
+  if (!i8) YSCV_TRY(launch_prefill_angles(rows, start_pos, c.head_dim, c.rope_theta, angles, s));
   YSCV_TRY(launch_embed(tokens_dev, d->emb, rows, (int)D, c.vocab, h, s));
   for (auto &L : d->layers) {
     YSCV_TRY(launch_rmsnorm(h, L.attn_norm, rows, (int)D, c.rms_eps, xn, s));
@@ -1610,8 +1612,7 @@ static int32_t prefill_chunk(yscv_hip_decoder *d, const int32_t *tokens_dev, int
       YSCV_TRY(launch_gqa_cache(qkv, tk, tv, rows, start_pos, c.n_heads,
                                 c.n_kv_heads, c.head_dim, t_ctx, ao, s));
     } else {
-      YSCV_TRY(launch_prefill_rope_append(qkv, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim, c.rope_theta,
-                                          c.max_ctx, L.kc, L.vc, s));
+      YSCV_TRY(launch_prefill_rope_append(qkv, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim, angles, c.max_ctx, L.kc, L.vc, s));
       YSCV_TRY(launch_gqa_cache(qkv, L.kc, L.vc, rows, start_pos, c.n_heads, c.n_kv_heads, c.head_dim,
                                 c.max_ctx, ao, s));
     }

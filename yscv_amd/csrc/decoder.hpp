@@ -84,7 +84,10 @@ int32_t launch_kv_random_fill(_Float16 *buf, size_t n, uint64_t seed, hipStream_
 // of query heads per kv head): `rows` consecutive positions start_pos .. of batch row 0, causal, q rotated, the rows in the cache.
 int32_t launch_gqa_cache(const _Float16 *qkv, const _Float16 *kc, const _Float16 *vc, int rows, int start_pos, int hq, int hkv, int hd,
                          int max_ctx, _Float16 *out, hipStream_t s);
-int32_t launch_prefill_rope_append(_Float16 *qkv, int rows, int start_pos, int hq, int hkv, int hd, float theta, int max_ctx,
+// {cos, sin} of every pair at positions start_pos .. start_pos + rows - 1, for the launches of all layers of a pass
+size_t prefill_angles_bytes(size_t rows, int hd);
+int32_t launch_prefill_angles(int rows, int start_pos, int hd, float theta, void *angles, hipStream_t s);
+int32_t launch_prefill_rope_append(_Float16 *qkv, int rows, int start_pos, int hq, int hkv, int hd, const void *angles, int max_ctx,
                                    _Float16 *kc, _Float16 *vc, hipStream_t s);
 int32_t launch_bias_add_f16(_Float16 *x, const _Float16 *bias, size_t rows, size_t n, hipStream_t s);
 

@@ -33,6 +33,7 @@
 #include "int4_common.hpp"
 #include "decoder.hpp"
 #include "kernels.hpp"
+#include "rope.hpp"
 
 namespace yscv {
 
@@ -1090,64 +1091,90 @@ __global__ void __launch_bounds__(64) rope_f32_kernel(float *__restrict__ x, int
 
 
 // ---- small kernels of the prompt pass (rows = consecutive positions of one sequence) ------------------------------
+// {cos, sin} of every pair at the positions of a prompt pass, row p of the table for position p0 + p: once for all layers and heads
+__global__ void __launch_bounds__(256) prefill_angles_kernel(int p0, int positions, int hd, float theta, float2 *__restrict__ angles) {
+  const int idx = (int)(blockIdx.x * 256 + threadIdx.x), half_d = hd / 2;
+  if (idx >= positions * half_d) return;
+  const SinCos a = rope_sincos(theta, idx % half_d, hd, p0 + idx / half_d);
+  angles[idx] = float2{a.cs, a.sn};
+}
+
 // RoPE on the q and k heads of every row (row i sits at position start_pos + i), k and v appended to batch row 0 of
-// the cache: the arithmetic of the decode step's rope + append, one launch for all rows.  A workgroup takes the (up
-// to eight) rows whose positions share one 8-position slab of the V layout: the angle of a pair is worked out once per
-// position for all heads, and the values of a channel at the slab's positions leave as one 16-byte store where the
-// whole slab is new.
+// the cache: the arithmetic of the decode step's rope + append, one launch for all rows.  Workgroups take the (up
+// to eight) rows whose positions share one 8-position slab of the V layout; the values of a channel at the slab's positions leave as one
+// 16-byte store where the whole slab is new.  Memory-bound: a thread has eight pairs of one position, whose angles it keeps, in up to
+// ROPE_HEADS heads, and asks for all of that and its first channel of v at once: one memory round trip.  With the angles worked out here,
+// once per layer and workgroup, and an item at a time behind them it was 6 .. 8 in turn.  us a launch, 40 heads of 128: 2048 rows 12.2 -> 9.8
+(5.1 TB/s), 1500 10.6 -> 7.8, 700 7.0 -> 5.9; 18 heads of 64: 43 rows 4.3 -> 3.1, from 500 rows on no change; the angles take 3.3 a pass.
+constexpr int ROPE_HEADS = 3;
 __global__ void __launch_bounds__(256) prefill_rope_append_kernel(_Float16 *__restrict__ qkv, int rows, int start_pos, int hq, int hkv,
-                                                                  int hd, float theta, int max_ctx, _Float16 *__restrict__ kc,
+                                                                  int hd, const float2 *__restrict__ angles, int max_ctx, _Float16 *__restrict__ kc,
                                                                   _Float16 *__restrict__ vc, int parts) {
-  const int tid = threadIdx.x;
   const int slab = start_pos / 8 + (int)blockIdx.x;
   const int p_lo = max(start_pos, slab * 8), p_hi = min(start_pos + rows, slab * 8 + 8);  // positions [p_lo, p_hi)
   const size_t row_elems = (size_t)(hq + 2 * hkv) * hd;
-  const int half_d = hd / 2;
-  // the angle of pair i at each of the slab's positions, once for all heads
-  __shared__ float cs_s[8][64], sn_s[8][64];
-  const int n_pos = p_hi - p_lo;
-  for (int idx = tid; idx < n_pos * half_d; idx += 256) {
-    const int e = idx / half_d, i = idx % half_d;
-    const float inv_freq = 1.0f / powf(theta, (float)(2 * i) / (float)hd);
-    sincosf(inv_freq * (float)(p_lo + e), &sn_s[e][i], &cs_s[e][i]);
-  }
-  __syncthreads();
-  const int slots = hq + hkv, vecs = half_d / 8;  // eight pairs per item: 16-byte loads and stores
-#pragma unroll 2
-  // blockIdx.y takes every parts-th item of the slab (short prompts have few slabs and would leave the CUs idle)
-  for (int item = tid + 256 * (int)blockIdx.y; item < n_pos * slots * vecs; item += 256 * parts) {
-    const int i0 = (item % vecs) * 8, slot = (item / vecs) % slots, e = item / (vecs * slots);
-    const int pos = p_lo + e;
-    _Float16 *src = qkv + (size_t)(pos - start_pos) * row_elems + (size_t)slot * hd;
-    const half8_t x0 = *reinterpret_cast<const half8_t *>(src + i0), x1 = *reinterpret_cast<const half8_t *>(src + i0 + half_d);
-    half8_t y0, y1;
+  const int half_d = hd / 2, slots = hq + hkv, vecs = half_d / 8, channels = hkv * hd;
+  const int first = (int)threadIdx.x + 256 * (int)blockIdx.y, step = 256 * parts;
+  // Thread `first` of the slab's step: the (first % width)-th eight pairs of a head, positions last, in heads head0, head0 + stride, ..
+  // Requests past the ends repeat a neighbour's and are not stored.
+  const int width = 8 * vecs, stride = step / width, head0 = first / width, pair8 = first % width;
+  const int pos = slab * 8 + pair8 / vecs, i0 = pair8 % vecs * 8, row = min(max(pos, p_lo), p_hi - 1) - start_pos;
+  _Float16 *at = qkv + (size_t)row * row_elems + i0;
+  half8_t x0[ROPE_HEADS], x1[ROPE_HEADS];
+  float4_t ang[4];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const float cs = cs_s[e][i0 + j], sn = sn_s[e][i0 + j];
-      const float a = (float)x0[j], b = (float)x1[j];
-      float f0 = fmaf(a, cs, -(b * sn)), f1 = fmaf(a, sn, b * cs);
-      asm volatile("" : "+v"(f0), "+v"(f1));  // the f32 value exists before it is narrowed (no mixed-precision fma)
-      y0[j] = (_Float16)f0;
-      y1[j] = (_Float16)f1;
-    }
-    _Float16 *dst = slot < hq ? src : kc + ((size_t)(slot - hq) * max_ctx + pos) * hd;
-    *reinterpret_cast<half8_t *>(dst + i0) = y0;
-    *reinterpret_cast<half8_t *>(dst + i0 + half_d) = y1;
+  for (int u = 0; u < ROPE_HEADS; u++) {
+    const _Float16 *src = at + min(head0 + u * stride, slots - 1) * hd;
+    x0[u] = *reinterpret_cast<const half8_t *>(src);
+    x1[u] = *reinterpret_cast<const half8_t *>(src + half_d);
   }
-  // v: channel ch of kv head kvh at the slab's positions
-  const _Float16 *vsrc = qkv + (size_t)(hq + hkv) * hd;
-  const bool whole = p_hi - p_lo == 8;
-  for (int idx = tid + 256 * (int)blockIdx.y; idx < hkv * hd; idx += 256 * parts) {
+  const float4_t *arow = reinterpret_cast<const float4_t *>(angles + (size_t)row * half_d + i0);
+#pragma unroll
+  for (int j = 0; j < 4; j++) ang[j] = arow[j];
+  // v: channel ch of kv head kvh at the slab's positions; those that are not of this call repeat a neighbour and are not stored
+  half8_t v;
+  auto load_v = [&](int idx) {
+    const _Float16 *src = qkv + (size_t)slots * hd + min(idx, channels - 1);
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = src[(size_t)(min(max(slab * 8 + e, p_lo), p_hi - 1) - start_pos) * row_elems];
+  };
+  auto put_v = [&](int idx) {
+    if (idx >= channels) return;
     const int kvh = idx / hd, ch = idx % hd;
     _Float16 *dst = vc + (((size_t)kvh * (max_ctx / 8) + slab) * hd + ch) * 8;
-    if (whole) {
-      half8_t v;
-#pragma unroll
-      for (int e = 0; e < 8; e++) v[e] = vsrc[(size_t)(p_lo - start_pos + e) * row_elems + idx];
+    if (p_hi - p_lo == 8) {
       *reinterpret_cast<half8_t *>(dst) = v;
     } else {
-      for (int pos = p_lo; pos < p_hi; pos++) dst[pos & 7] = vsrc[(size_t)(pos - start_pos) * row_elems + idx];
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+        if (slab * 8 + e >= p_lo && slab * 8 + e < p_hi) dst[e] = v[e];
     }
+  };
+  load_v(first);
+  if (head0 < stride && pos >= p_lo && pos < p_hi) {  // (threads behind the last whole width have no head)
+#pragma unroll
+    for (int u = 0; u < ROPE_HEADS; u++) {
+      const int slot = head0 + u * stride;
+      if (slot >= slots) break;
+      half8_t y0, y1;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const float cs = ang[j / 2][j % 2 * 2], sn = ang[j / 2][j % 2 * 2 + 1];
+        const float a = (float)x0[u][j], b = (float)x1[u][j];
+        float f0 = fmaf(a, cs, -(b * sn)), f1 = fmaf(a, sn, b * cs);
+        asm volatile("" : "+v"(f0), "+v"(f1));  // the f32 value exists before it is narrowed (no mixed-precision fma)
+        y0[j] = (_Float16)f0;
+        y1[j] = (_Float16)f1;
+      }
+      _Float16 *dst = slot < hq ? at + slot * hd : kc + ((size_t)(slot - hq) * max_ctx + pos) * hd + i0;
+      *reinterpret_cast<half8_t *>(dst) = y0;
+      *reinterpret_cast<half8_t *>(dst + half_d) = y1;
+    }
+  }
+  put_v(first);
+  for (int idx = first + step; idx < channels; idx += step) {
+    load_v(idx);
+    put_v(idx);
   }
 }
 
@@ -1163,14 +1190,23 @@ unsigned flat_grid(size_t n) {
 
 }  // namespace
 
-int32_t launch_prefill_rope_append(_Float16 *qkv, int rows, int start_pos, int hq, int hkv, int hd, float theta, int max_ctx,
+size_t prefill_angles_bytes(size_t rows, int hd) { return rows * (hd / 2) * sizeof(float2); }
+int32_t launch_prefill_angles(int rows, int start_pos, int hd, float theta, void *angles, hipStream_t s) {
+  const size_t total = (size_t)rows * (hd / 2);
+  if (total > 0x7fffffff) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "rope: %d rows of head width %d", rows, hd);
+  hipLaunchKernelGGL(prefill_angles_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, start_pos, rows, hd, theta, static_cast<float2 *>(angles));
+  YSCV_HIP_TRY(hipGetLastError());
+  return YSCV_HIP_OK;
+}
+int32_t launch_prefill_rope_append(_Float16 *qkv, int rows, int start_pos, int hq, int hkv, int hd, const void *angles, int max_ctx,
                                    _Float16 *kc, _Float16 *vc, hipStream_t s) {
   if (hd > 128 || hd % 16 != 0) return set_error(YSCV_HIP_ERR_UNSUPPORTED, "rope + append: head width %d", hd);
-  const int slabs = (start_pos + rows - 1) / 8 - start_pos / 8 + 1;
-  int parts = 512 / slabs;  // about two workgroups per CU
-  parts = parts < 1 ? 1 : (parts > 16 ? 16 : parts);
-  hipLaunchKernelGGL(prefill_rope_append_kernel, dim3(slabs, parts), dim3(256), 0, s, qkv, rows, start_pos, hq, hkv, hd, theta, max_ctx,
-                     kc, vc, parts);
+  const int slabs = (start_pos + rows - 1) / 8 - start_pos / 8 + 1, width = hd / 2;  // width: threads of a head
+  // Workgroups of a slab: as many as cover its heads with ROPE_HEADS each; few slabs leave CUs idle and are spread further, down to a head each
+  const int heads = hq + hkv, least = ((heads + ROPE_HEADS - 1) / ROPE_HEADS * width + 255) / 256, most = (heads * width + 255) / 256;
+  const int parts = std::max(least, std::min(most, 512 / slabs));
+  hipLaunchKernelGGL(prefill_rope_append_kernel, dim3(slabs, parts), dim3(256), 0, s, qkv, rows, start_pos, hq, hkv, hd,
+                     static_cast<const float2 *>(angles), max_ctx, kc, vc, parts);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
