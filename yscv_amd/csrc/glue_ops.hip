@@ -1104,8 +1104,9 @@ __global__ void __launch_bounds__(256) prefill_angles_kernel(int p0, int positio
 // to eight) rows whose positions share one 8-position slab of the V layout; the values of a channel at the slab's positions leave as one
 // 16-byte store where the whole slab is new.  Memory-bound: a thread has eight pairs of one position, whose angles it keeps, in up to
 // ROPE_HEADS heads, and asks for all of that and its first channel of v at once: one memory round trip.  With the angles worked out here,
-// once per layer and workgroup, and an item at a time behind them it was 6 .. 8 in turn.  us a launch, 40 heads of 128: 2048 rows 12.2 -> 9.8
-(5.1 TB/s), 1500 10.6 -> 7.8, 700 7.0 -> 5.9; 18 heads of 64: 43 rows 4.3 -> 3.1, from 500 rows on no change; the angles take 3.3 a pass.
+// once per layer and workgroup, and an item at a time behind them it was 6 .. 8 in turn.  us a launch, 40 heads of 128: 2048 rows
+// 12.2 -> 9.8 (5.1 TB/s), 1500 10.6 -> 7.8, 700 7.0 -> 5.9; 18 heads of 64: 43 rows 4.3 -> 3.1, from 500 rows on no change; the angles
+// take 3.3 a pass.
 constexpr int ROPE_HEADS = 3;
 __global__ void __launch_bounds__(256) prefill_rope_append_kernel(_Float16 *__restrict__ qkv, int rows, int start_pos, int hq, int hkv,
                                                                   int hd, const float2 *__restrict__ angles, int max_ctx, _Float16 *__restrict__ kc,
