@@ -193,8 +193,9 @@ __global__ void __launch_bounds__(256) dql_quantize_kernel(const float *__restri
   __shared__ float smin[4], smax[4];
   float mn = 3.40282347e+38f, mx = -3.40282347e+38f;
   // The first four loads of x go out behind the partials' and arrive while those are reduced: one memory round trip instead of two, and
-  // the reduction is DPP moves.  us with the GEMM, before -> after: 128 x 1024 against 4096 columns 12.6 -> 11.1, against 1024 columns
-  // 1024 x 1024 15.5 -> 13.6, 1024 x 4096 25.0 -> 24.2, 1000 x 8192 34.8 -> 33.8
+  // the reduction is DPP moves.  us a launch: 2^20 values 5.8 -> 4.5 (the ranges in front 3.0 -> 2.8), 131072 3.4 -> 3.0 (2.6 -> 2.4); with
+  // the GEMM against 1024 columns 1024 x 1024 15.5 -> 13.6, 300 x 4096 17.1 -> 16.2, 1000 x 8192 35.1 -> 34.4; up to 131072 values the host's
+  // three launches take as long (11.5).
   constexpr bool AHEAD = VEC && !OWN;
   constexpr int BATCH = 4;
   const size_t n4 = len / 4, step = (size_t)nparts * 256, first = blockIdx.x * (size_t)256 + threadIdx.x;
