@@ -5,7 +5,7 @@ names the destination registers as read-write operands.  Between the two the com
 defined: if it moves them (a copy at a control-flow join, live-range splitting under register pressure), the copy
 runs before the data has landed, the later code reads the copy, and the result is wrong now and then, with no error.
 The check walks the assembly of every kernel in program order, keeps the destination registers of asm loads
-(`global_load*`, `ds_read*` between ASMSTART / ASMEND) until a wait counter retires them or an instruction overwrites
+(`global_load*`, `ds_read*` between ASMSTART / ASMEND; loads to LDS, `buffer_load* ... lds` too, have none but are counted) until a wait counter retires them or an instruction overwrites
 them, and reports every register move whose source is still in flight.  Program order is an approximation of
 control flow, good enough for the straight-line pipelines these kernels are.
 """
@@ -52,7 +52,7 @@ def copies_of_inflight_registers(asm_text):
                     lg = lg[len(lg) - n:] if n > 0 else []
                 continue
             if inasm:
-                if op.startswith("global_load_lds"):
+                if op.startswith("global_load_lds") or (op.startswith("buffer_load") and l.split()[-1] == "lds"):
                     vm.append((i + 1, set()))
                 elif op.startswith("global_load"):
                     vm.append((i + 1, _regs(l.split(",")[0])))
