@@ -77,7 +77,7 @@ static_assert(sizeof(I8Args) + 2 * sizeof(int) <= kCheapArgs, "arguments of a la
 
 // The matrix kernels, on 16-byte aligned a with an lda that is a multiple of 64, m * lda below 2 GiB, and the us that a launch is
 // estimated to take: small tiles whose waves split K (i8_ksplit.hip; the tiles that all run at once, 1e30 where none do), and large ones
-// (i8_gemm_wide.hip; two k-steps at least).
+// (i8_gemm_wide.hip).
 double i8_ksplit_us(size_t m, size_t n, size_t ksteps, size_t cus);
 int32_t launch_i8_ksplit(const I8Args &p, int num_cus, hipStream_t s);
 enum : int { IW_64x128, IW_128x256 };

@@ -238,9 +238,9 @@ size_t i8_gemm_pad_bytes(const yscv_hip_i8_weight *b, size_t m, const void *a, c
 
 // the matrix kernels on rows of p.lda bytes, whole 64-byte steps on 16-byte alignment
 static int32_t i8_gemm_rows(const I8Args &p, const yscv_hip_i8_weight *b, int num_cus, hipStream_t s) {
-  // the kernel with the shortest estimate; the wide tiles take pairs of k-steps and 32-bit offsets into a block of B
+  // the kernel with the shortest estimate; the wide tiles take 32-bit offsets into a block of B
   const size_t m = (size_t)p.m, ksteps = (size_t)p.ksteps, cus = num_cus > 0 ? (size_t)num_cus : 256;
-  if (ksteps >= 2 && ksteps <= (size_t)1 << 18) {
+  if (ksteps <= (size_t)1 << 18) {
     const bool requant = ((p.how & 255) == 1);
     const double small = i8_wide_us(IW_64x128, m, b->n, ksteps, requant, cus), big = i8_wide_us(IW_128x256, m, b->n, ksteps, requant, cus);
     if (std::min(small, big) < i8_ksplit_us(m, b->n, ksteps, cus)) return launch_i8_gemm_wide(p, big < small ? IW_128x256 : IW_64x128, s);

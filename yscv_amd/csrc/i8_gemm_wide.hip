@@ -29,7 +29,7 @@ namespace yscv {
 namespace {
 
 // A tile of MT x 4 NT blocks of 16.  Four waves stand side by side in columns, WK such rows of waves share the K of a stage; B of S
-// stages is in flight.
+// stages is in flight; one stage: all of K.
 // A stage is KS k-steps of 64 for each of a wave's rows.
 template <int MT, int NT, int WK, int S, int KS>
 struct IwTile {
@@ -48,7 +48,7 @@ __device__ __forceinline__ void iw_barrier() {
 template <int MT, int NT, int WK, int S, int KS>
 __global__ void __launch_bounds__(256 * WK, WK) i8_gemm_wide_kernel(I8Args p, int tiles_m, int tiles_n) {
   using T = IwTile<MT, NT, WK, S, KS>;
-  static_assert(MT % 4 == 0 && NT >= 2 && MT >= NT && S >= 2 && S <= 4, "");
+  static_assert(MT % 4 == 0 && NT >= 2 && MT >= NT && S >= 1 && S <= 4, "");
   constexpr int AL = MT / 4;  // A loads of a wave and k-step
   extern __shared__ __attribute__((aligned(1024))) uint8_t iw_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -62,7 +62,9 @@ __global__ void __launch_bounds__(256 * WK, WK) i8_gemm_wide_kernel(I8Args p, in
   const int tn = in_band / band_rows, tm = 8 * band + in_band % band_rows;
   const int m0 = tm * T::BM, nb0 = tn * 4 * NT + wn * NT, nb_last = (p.n + 15) / 16 - 1;
   const int nst = (p.ksteps + KS * WK - 1) / (KS * WK);
-  const int odd = p.ksteps & 1;
+  // (a single k-step is the first half of a pair at byte 0 whose second half is multiplied as zeros)
+  const bool one = S == 1 && p.ksteps == 1;
+  const int odd = one ? 0 : p.ksteps & 1;
   const uint32_t lds0 = (uint32_t)(size_t)iw_lds;
 
   // the per-column terms of the epilogue, requested ahead of the loop, wait in LDS behind the ring
@@ -74,14 +76,15 @@ __global__ void __launch_bounds__(256 * WK, WK) i8_gemm_wide_kernel(I8Args p, in
   // ---- loads.  A pair is two k-steps, 128 bytes of every row.  A: pieces [row tile][pair][half] of a stage, 1 KiB each; a wave fetches
   // those of AL row tiles and its own pairs.  Lane i of half h fetches 16-byte chunk (i & 7) ^ g of row 8 h + i / 8, g = 4 h + (i / 8) / 2, so
   // that the sixteen rows of a fragment read fall into sixteen different slots.  An odd count of k-steps: the last pair begins a
-  // k-step early, and its first half, which the pair in front has had, is multiplied as zeros.
+  // k-step early, and its first half, which the pair in front has had, is multiplied as zeros.  One k-step: the second half is fetched from
+  // where the first one is.
   uint32_t aoff[AL][2];
 #pragma unroll
   for (int i = 0; i < AL; i++)
 #pragma unroll
     for (int h = 0; h < 2; h++) {
       const int row8 = lane >> 3, row = min(m0 + 16 * (AL * wn + i) + 8 * h + row8, p.m - 1);
-      aoff[i][h] = (uint32_t)row * (uint32_t)p.lda + (uint32_t)(((lane & 7) ^ (4 * h + (row8 >> 1))) * 16);
+      aoff[i][h] = (uint32_t)row * (uint32_t)p.lda + (uint32_t)((((lane & 7) ^ (4 * h + (row8 >> 1))) & (one ? 3 : 7)) * 16);
     }
   uint32_t boff[NT];  // (column blocks past the end repeat the last one)
 #pragma unroll
@@ -89,7 +92,8 @@ __global__ void __launch_bounds__(256 * WK, WK) i8_gemm_wide_kernel(I8Args p, in
   int8_t *const frag0 = const_cast<int8_t *>(p.frag) + (size_t)min(nb0, nb_last) * p.ksteps * 1024;
   const uint64_t a_ptr = (uint64_t)p.a;
   constexpr int kAll = 0x7FFFFFFF, kNone = 0, kRaw = 0x00020000;  // bytes of a buffer (none: loads read nothing), its format
-  auto pair_k = [&](int q) { return min(2 * q, p.ksteps - 2); };  // first k-step of pair q
+  const int last_k = one ? 0 : p.ksteps - 2;
+  auto pair_k = [&](int q) { return min(2 * q, last_k); };  // first k-step of pair q
   // A load l of k-step ks of a stage, whose pair begins at byte k of the rows
   const int4_t a_rsrc = {(int)(uint32_t)a_ptr, (int)(uint32_t)(a_ptr >> 32), kAll, kRaw};
   const uint32_t a_lds = lds0 + (uint32_t)(KS * (AL * wn * WK + wk) * 1024);
@@ -206,7 +210,7 @@ __global__ void __launch_bounds__(256 * WK, WK) i8_gemm_wide_kernel(I8Args p, in
   auto first = [&](auto U, auto &self) __attribute__((always_inline)) -> void {
     constexpr int u = decltype(U)::value;
     if constexpr (u < S) {
-      const int records = u < nst ? kAll : kNone;
+      const int records = u < nst ? kAll : kNone, second = one ? kNone : records;
       if (u < nst) {
 #pragma unroll
         for (int ks = 0; ks < KS; ks++)
@@ -216,10 +220,10 @@ __global__ void __launch_bounds__(256 * WK, WK) i8_gemm_wide_kernel(I8Args p, in
 #pragma unroll
       for (int j = 0; j < NT; j++) {
         load_b(wave_pair(u, 0) * 1024, j, U, K0, records);
-        load_b(wave_pair(u, 0) * 1024, j, U, K1, records);
+        load_b(wave_pair(u, 0) * 1024, j, U, K1, second);
         if constexpr (KS == 4) {
           load_b(wave_pair(u, 1) * 1024, j, U, K2, records);
-          load_b(wave_pair(u, 1) * 1024, j, U, K3, records);
+          load_b(wave_pair(u, 1) * 1024, j, U, K3, second);
         }
       }
       self(std::integral_constant<int, u + 1>{}, self);
@@ -242,21 +246,34 @@ __global__ void __launch_bounds__(256 * WK, WK) i8_gemm_wide_kernel(I8Args p, in
       convert_if(a[0][1], e, mask);
     }
   }
+  // every accumulator has its own zeros in front of the first MFMA: left to the compiler, which sees no MFMA in an asm statement, it copied
+  // them from the first one's, between MFMAs that had written it
+#pragma unroll
+  for (int i = 0; i < MT; i++)
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+      if constexpr (WK == 1) asm volatile("" : "+a"(acc[i][j]));
+      else asm volatile("" : "+v"(acc[i][j]));
+    }
   asm volatile("s_nop 1");
   const std::integral_constant<int, -1> LOADS;
   const std::integral_constant<int, 2 % S> U2;
   const std::integral_constant<int, 3 % S> U3;
   const int full = p.ksteps / (KS * WK);  // stages without a k-step that there is not
   int st = 0;
-  for (; st + S <= full; st += S) {
-    stage(st, K0, LOADS);
-    stage(st + 1, K1, LOADS);
-    if constexpr (S > 2) stage(st + 2, U2, LOADS);
-    if constexpr (S > 3) stage(st + 3, U3, LOADS);
+  if constexpr (S > 1) {
+    for (; st + S <= full; st += S) {
+      stage(st, K0, LOADS);
+      stage(st + 1, K1, LOADS);
+      if constexpr (S > 2) stage(st + 2, U2, LOADS);
+      if constexpr (S > 3) stage(st + 3, U3, LOADS);
+    }
   }
   // no more than S stages are left and nothing to load (ways out of the loop's middle would have the accumulators copied in every round)
   if (st < nst) stage(st, K0, K0);
-  if (st + 1 < nst) stage(st + 1, K1, K1);
+  if constexpr (S > 1) {
+    if (st + 1 < nst) stage(st + 1, K1, K1);
+  }
   if constexpr (S > 2) {
     if (st + 2 < nst) stage(st + 2, U2, U2);
   }
@@ -375,6 +392,10 @@ double i8_wide_us(int tile, size_t m, size_t n, size_t ksteps, bool requant, siz
 }
 
 int32_t launch_i8_gemm_wide(const I8Args &p, int tile, hipStream_t s) {
+  // A K of one stage has a form of its own: the others ask for as many stages as they keep in flight, whether there are any or not, and with
+  // a K of 64 and tiles in several rounds i8_ksplit.hip gives a wave in four something to do.  us to int32, either of these before -> this: 20000 x
+  // 64 x 64 33.5 -> 5.6, 2048 x 8192 x 64 53.7 -> 19.0, 8192 x 512 x 128 8.0 -> 7.3, 512 x 4096 x 256 5.8 -> 5.3.
+  if (p.ksteps <= 4) return tile == IW_128x256 ? iw_launch<8, 4, 1, 1, 4>(p, s) : iw_launch<4, 2, 2, 1, 2>(p, s);
   return tile == IW_128x256 ? iw_launch<8, 4, 1, 2, 4>(p, s) : iw_launch<4, 2, 2, 3, 2>(p, s);
 }
 

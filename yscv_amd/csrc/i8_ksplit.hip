@@ -269,7 +269,7 @@ double i8_ksplit_us(size_t m, size_t n, size_t ksteps, size_t cus) {
 int32_t launch_i8_ksplit(const I8Args &p, int num_cus, hipStream_t s) {
   double us;
   int shape = iks_pick((size_t)p.m, (size_t)p.n, (size_t)p.ksteps, num_cus > 0 ? (size_t)num_cus : 256, us);
-  if (shape < 0) shape = kIksShapeCount - 1;  // (a K of 64 with more tiles than CUs)
+  if (shape < 0) shape = kIksShapeCount - 1;  // (a K above 2^24 with more tiles than CUs)
   return iks_launch_shape(shape, p, s);
 }
 
