@@ -1,4 +1,4 @@
-// Shared by the int8 GEMM kernels (i8_gemm.hip, i8_ksplit.hip): arguments and the per-element epilogue arithmetic.
+// Shared by the int8 GEMM kernels (i8_gemm.hip, i8_ksplit.hip, i8_gemm_wide.hip): arguments and the per-element epilogue arithmetic.
 #pragma once
 
 #include "int4_common.hpp"
@@ -14,6 +14,14 @@ __device__ __forceinline__ float round_half_away(float v) {
   return (d >= 0.5f) ? __fadd_rn(t, copysignf(1.0f, v)) : t;
 }
 
+// Towards zero, a NaN as 0 (`as i8`).  The instruction does that; of a cast it is undefined, and where the compiler knows of the NaN it
+// drops the result and what is done with it.  (A select in front of the cast costs two instructions a value.)
+__device__ __forceinline__ int nan_to_zero_int(float v) {
+  int r;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+
 // clamp(round(a * comp + y_zp), lo, hi) as an int, a NaN as 0 (clamp keeps it, `as i8` makes it 0).  Rounding is monotonic and leaves lo and hi
 // as they are, so the clamp comes first: what is rounded is then finite or a NaN, and half away from zero is trunc(v) + trunc(2 (v - trunc(v))).
 template <bool HALF_AWAY>
@@ -26,7 +34,7 @@ __device__ __forceinline__ int requant_int(int32_t a, float comp, float y_zp, fl
   } else {
     v = rintf(v);
   }
-  return (int)v;
+  return nan_to_zero_int(v);
 }
 
 __device__ __forceinline__ int requant_one(int32_t acc, int32_t corr, float comp, float y_zp, int round_mode,
