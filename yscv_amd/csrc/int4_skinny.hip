@@ -284,6 +284,12 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
       // values below 2^-29 of the slice maximum are lost); the power of two is undone on the wave's partial sums.
       const uint16_t *src = xb + (size_t)(valid ? mrow : 0) * a.ldx + c * 8;
       uint4_t raw[TPW][4];
+      auto zero_behind_k = [&]() {
+#pragma unroll
+        for (int t = 0; t < TPW; t++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) raw[t][j] &= block_in(t, j) ? ~0u : 0u;
+      };
       if (whole) {
         src += (size_t)t0 * 128;
 #pragma unroll
@@ -295,16 +301,12 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
         for (int t = 0; t < TPW; t++)
 #pragma unroll
           for (int j = 0; j < 4; j++) raw[t][j] = *reinterpret_cast<const uint4_t *>(src + block_k(t, j));
+        if constexpr (!X_FIRST) zero_behind_k();
       }
       if constexpr (X_FIRST) {
         asm volatile("" ::: "memory");
         fill_ring();
-      }
-      if (!whole) {
-#pragma unroll
-        for (int t = 0; t < TPW; t++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) raw[t][j] &= block_in(t, j) ? ~0u : 0u;
+        if (!whole) zero_behind_k();
       }
       uint32_t amax_bits = 0;  // |bf16| orders like its bit pattern
 #pragma unroll
@@ -457,6 +459,7 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
       }
     } else {
       const size_t row_off = (size_t)(valid ? mrow : 0) * a.ldx + c * 8;
+      const half8_t hz = {0, 0, 0, 0, 0, 0, 0, 0};
       if (whole) {
 #pragma unroll
         for (int t = 0; t < TPW; t++)
@@ -475,6 +478,18 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
             xa[t][j][0] = *reinterpret_cast<const half8_t *>(xh + off);
             if constexpr (SPLIT == 2) xa[t][j][1] = *reinterpret_cast<const half8_t *>(a.xl + off);
           }
+        // (here, and not behind both branches: two branches with nothing but loads are merged into one whose sixteen or 32 addresses are
+        // worked out ahead of the first load; 10 x 698 x 2304 in f32, the kernel: 8.6 us, 7.4 so)
+        if constexpr (!X_FIRST) {
+#pragma unroll
+          for (int t = 0; t < TPW; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+              if (!block_in(t, j)) {
+                xa[t][j][0] = hz;
+                if constexpr (SPLIT == 2) xa[t][j][1] = hz;
+              }
+        }
       }
       if constexpr (X_FIRST) {
         asm volatile("" ::: "memory");
@@ -486,15 +501,14 @@ __device__ __forceinline__ void skinny_body(SkinnyArgs a, const SkinnyFold &f) {
             for (int j = 0; j < 4; j++) xa[t][j][0] = __builtin_bit_cast(half8_t, __builtin_bit_cast(uint4_t, xa[t][j][0]) & (valid && block_in(t, j) ? ~0u : 0u));
         }
       } else {
-        const half8_t hz = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int t = 0; t < TPW; t++)
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const bool in = valid && (whole || block_in(t, j));
-            xa[t][j][0] = in ? xa[t][j][0] : hz;
-            if constexpr (SPLIT == 2) xa[t][j][1] = in ? xa[t][j][1] : hz;
-          }
+          for (int j = 0; j < 4; j++)
+            if (!valid) {
+              xa[t][j][0] = hz;
+              if constexpr (SPLIT == 2) xa[t][j][1] = hz;
+            }
       }
     }
   }
