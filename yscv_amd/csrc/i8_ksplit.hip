@@ -46,9 +46,13 @@ __global__ void __launch_bounds__(64 * WAVES) i8_ksplit_kernel(I8Args p, int til
   extern __shared__ __attribute__((aligned(1024))) uint8_t iks_ring[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, c = lane >> 4;
-  // the row tiles of one column block run on one XCD (workgroup ids that are equal modulo 8), so its B reaches one L2
-  const int tn = (int)(blockIdx.x & 7) + 8 * ((int)(blockIdx.x >> 3) / tiles_m), tm = (int)(blockIdx.x >> 3) % tiles_m;
-  if (tn >= tiles_n) return;
+  // Tiles are numbered column block by column block, and an XCD (workgroup ids equal modulo 8) takes an eighth of them in a row: the row
+  // tiles of a column block share its B in one L2, or two, and no XCD has more than its share, so that as many tiles as CUs do run at once.
+  // (Whole column blocks to each XCD left five of the eight idle for three column blocks: 1912 x 160 x 1664 10.1 us, 5.6
+  // so, 3419 x 16 x 7616 40.4 and 6.2; with 2916 x 16 .. 600 x 8192 and K 64 .. 8192 of all kinds 13 % less on average.)
+  const int tiles = tiles_m * tiles_n, share = (tiles + 7) >> 3, t = (int)(blockIdx.x & 7) * share + (int)(blockIdx.x >> 3);
+  if (t >= tiles) return;
+  const int tn = t / tiles_m, tm = t - tn * tiles_m;
   const int m0 = tm * 16 * MT, nb0 = tn * NT, nb_total = (p.n + 15) / 16;
   const int pairs = (p.ksteps + 1) >> 1;
   const int q_lo = pairs * wave / WAVES, q_hi = pairs * (wave + 1) / WAVES;
@@ -212,7 +216,7 @@ int32_t iks_launch(const I8Args &p, hipStream_t s) {
   std::call_once(once, [&] { attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS); });
   if (attr_err != hipSuccess) return set_error(YSCV_HIP_ERR_DEVICE, "cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(attr_err));
   const int tiles_m = (p.m + 16 * MT - 1) / (16 * MT), tiles_n = (p.n + 16 * NT - 1) / (16 * NT);
-  hipLaunchKernelGGL(kern, dim3((unsigned)((tiles_n + 7) / 8 * 8) * (unsigned)tiles_m), dim3(64 * WAVES), LDS, s, p, tiles_m, tiles_n);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((tiles_m * tiles_n + 7) / 8 * 8)), dim3(64 * WAVES), LDS, s, p, tiles_m, tiles_n);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
