@@ -89,7 +89,7 @@ static_assert(sizeof(I8Args) + 2 * sizeof(int) <= kCheapArgs, "arguments of a la
 double i8_ksplit_us(size_t m, size_t n, size_t ksteps, size_t cus);
 int32_t launch_i8_ksplit(const I8Args &p, int num_cus, hipStream_t s);
 enum : int { IW_64x128, IW_128x256 };
-double i8_wide_us(int tile, size_t m, size_t n, size_t ksteps, bool requant, size_t cus);
+double i8_wide_us(int tile, size_t m, size_t n, size_t ksteps, int mode, size_t cus);
 int32_t launch_i8_gemm_wide(const I8Args &p, int tile, hipStream_t s);
 
 }  // namespace yscv

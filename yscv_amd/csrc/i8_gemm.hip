@@ -241,8 +241,7 @@ static int32_t i8_gemm_rows(const I8Args &p, const yscv_hip_i8_weight *b, int nu
   // the kernel with the shortest estimate; the wide tiles take 32-bit offsets into a block of B
   const size_t m = (size_t)p.m, ksteps = (size_t)p.ksteps, cus = num_cus > 0 ? (size_t)num_cus : 256;
   if (ksteps <= (size_t)1 << 18) {
-    const bool requant = ((p.how & 255) == 1);
-    const double small = i8_wide_us(IW_64x128, m, b->n, ksteps, requant, cus), big = i8_wide_us(IW_128x256, m, b->n, ksteps, requant, cus);
+    const double small = i8_wide_us(IW_64x128, m, b->n, ksteps, p.mode(), cus), big = i8_wide_us(IW_128x256, m, b->n, ksteps, p.mode(), cus);
     if (std::min(small, big) < i8_ksplit_us(m, b->n, ksteps, cus)) return launch_i8_gemm_wide(p, big < small ? IW_128x256 : IW_64x128, s);
   }
   return launch_i8_ksplit(p, num_cus, s);

@@ -382,10 +382,13 @@ int32_t iw_launch(const I8Args &p, hipStream_t s) {
 // us of a launch: whole rounds over the CUs, and a last one that fills a part of them; 64 x 128 tiles run two to a CU, which their rounds
 // count as one after the other.  Fitted to 200 shapes of the same ranges as i8_ksplit.hip's (with those: the choice is 1.1 % slower than
 // the fastest of all on average, 8.5 % faster than before there were these tiles).
-double i8_wide_us(int tile, size_t m, size_t n, size_t ksteps, bool requant, size_t cus) {
+double i8_wide_us(int tile, size_t m, size_t n, size_t ksteps, int mode, size_t cus) {
   const bool big = tile == IW_128x256;
-  const double k = (double)ksteps, bytes = big && requant ? 2.5 : 0.0;  // (a thread of the big tile requantises 128 values)
-  const double full = big ? 1.0 + 0.43 * k + bytes : 0.6 + 0.155 * k, fast = big ? 0.30 * k + bytes : 0.145 * k;
+  // A thread of the big tile requantises 128 values with nothing else to do: bytes (mode 1), dequantised (2) and f32 carriers (4), whose rounding
+  // is the longer one.  us, big and small tiles: 4009 x 2880 x 512 dequantised 37.9 and 28.1, as carriers 40.6 and 28.5, 3994 x 3968 x 1344
+  // 56.8 and 52.5, 59.3 and 52.4, 3058 x 5248 x 3648 88.8 and 101, 91.7 and 99.8.
+  const double k = (double)ksteps, requant = !big ? 0.0 : mode == 1 ? 2.5 : mode == 2 ? 4.8 : mode == 4 ? 6.2 : 0.0;
+  const double full = big ? 1.0 + 0.43 * k + requant : 0.6 + 0.155 * k, fast = big ? 0.30 * k + requant : 0.145 * k;
   const size_t tiles = ceil_div(m, (size_t)(big ? 128 : 64)) * ceil_div(n, (size_t)(big ? 256 : 128)), rest = tiles % cus;
   const double part = full * (double)rest / (double)cus;
   return (big ? 6.0 : 4.0) + (double)(tiles / cus) * full + (rest == 0 ? 0.0 : (part > fast ? part : fast));
