@@ -1005,7 +1005,10 @@ static int32_t launch_one(const SkinnyArgs &a, const SkinnyPlan &plan, bool xraw
       if (blocks_per_wg == 1) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 1>(a, plan, xraw, fold, s);
       if (blocks_per_wg == 2) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, 2>(a, plan, xraw, fold, s);
       if constexpr (P == 4 && NI > 1) {
-        if (blocks_per_wg > 8) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, kDeep>(a, plan, xraw, fold, s);
+        // (a fifth block is a last round of its own, in which two in flight leave one wait after the other and end with requests for
+        // nothing: nine to sixteen rows of K 3072 13.8 us, with four 13.0, K 6144 16.6 and 15.7, K 8704 16.4 and 15.6; five to eight
+        // rows the other way, 13.8 and 14.4)
+        if (blocks_per_wg > 8 || (NI == 4 && blocks_per_wg == 5)) return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, kDeep>(a, plan, xraw, fold, s);
       }
     }
     return launch_p<SPLIT, NI, GM, SF16, HAS_ZP, P>(a, plan, xraw, fold, s);
