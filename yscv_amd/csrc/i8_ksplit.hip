@@ -39,6 +39,9 @@ constexpr int iks_lds(int mt, int nt, int waves, int np) {
   return slots > red ? slots : red;
 }
 
+// every XCD has a CU for each row tile of its column blocks (32 CUs)
+__host__ __device__ __forceinline__ bool iks_whole_columns(int tiles_m, int tiles_n) { return ((tiles_n + 7) >> 3) * tiles_m <= 32; }
+
 template <int MT, int NT, int WAVES, int NP>
 __global__ void __launch_bounds__(64 * WAVES) i8_ksplit_kernel(I8Args p, int tiles_m, int tiles_n) {
   constexpr int PAIR = (MT + NT) * 2048, LOADS = 2 * (MT + NT);  // LDS bytes and load instructions of one pair
@@ -46,13 +49,21 @@ __global__ void __launch_bounds__(64 * WAVES) i8_ksplit_kernel(I8Args p, int til
   extern __shared__ __attribute__((aligned(1024))) uint8_t iks_ring[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, c = lane >> 4;
-  // Tiles are numbered column block by column block, and an XCD (workgroup ids equal modulo 8) takes an eighth of them in a row: the row
-  // tiles of a column block share its B in one L2, or two, and no XCD has more than its share, so that as many tiles as CUs do run at once.
-  // (Whole column blocks to each XCD left five of the eight idle for three column blocks: 1912 x 160 x 1664 10.1 us, 5.6
-  // so, 3419 x 16 x 7616 40.4 and 6.2; with 2916 x 16 .. 600 x 8192 and K 64 .. 8192 of all kinds 13 % less on average.)
-  const int tiles = tiles_m * tiles_n, share = (tiles + 7) >> 3, t = (int)(blockIdx.x & 7) * share + (int)(blockIdx.x >> 3);
-  if (t >= tiles) return;
-  const int tn = t / tiles_m, tm = t - tn * tiles_m;
+  // The row tiles of one column block run on one XCD (workgroup ids equal modulo 8), so its B reaches one L2, where a workgroup to each of its CUs
+  // has room for them.  Where not (few column blocks, or a count just above a multiple of eight), tiles are numbered column block by column
+  // block and an XCD takes an eighth of them in a row: no XCD has more than its share, and as many tiles as CUs do run at once.
+  // us, whole column blocks and even shares: 22 x 64 x 64 2.6 and 3.0, 129 x 16 x 64 2.4 and 3.0 (an XCD that has nothing to do costs nothing),
+  // 40 x 48 x 4096 4.0 and 4.4; 1912 x 160 x 1664 10.1 and 5.6, 3419 x 16 x 7616 40.4 and 6.2.
+  int tn, tm;
+  if (iks_whole_columns(tiles_m, tiles_n)) {
+    const int at = (int)(blockIdx.x >> 3) / tiles_m;
+    tn = (int)(blockIdx.x & 7) + 8 * at, tm = (int)(blockIdx.x >> 3) - at * tiles_m;
+    if (tn >= tiles_n) return;
+  } else {
+    const int tiles = tiles_m * tiles_n, t = (int)(blockIdx.x & 7) * ((tiles + 7) >> 3) + (int)(blockIdx.x >> 3);
+    if (t >= tiles) return;
+    tn = t / tiles_m, tm = t - tn * tiles_m;
+  }
   const int m0 = tm * 16 * MT, nb0 = tn * NT, nb_total = (p.n + 15) / 16;
   const int pairs = (p.ksteps + 1) >> 1;
   const int q_lo = pairs * wave / WAVES, q_hi = pairs * (wave + 1) / WAVES;
@@ -216,7 +227,8 @@ int32_t iks_launch(const I8Args &p, hipStream_t s) {
   std::call_once(once, [&] { attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS); });
   if (attr_err != hipSuccess) return set_error(YSCV_HIP_ERR_DEVICE, "cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(attr_err));
   const int tiles_m = (p.m + 16 * MT - 1) / (16 * MT), tiles_n = (p.n + 16 * NT - 1) / (16 * NT);
-  hipLaunchKernelGGL(kern, dim3((unsigned)((tiles_m * tiles_n + 7) / 8 * 8)), dim3(64 * WAVES), LDS, s, p, tiles_m, tiles_n);
+  const int each = iks_whole_columns(tiles_m, tiles_n) ? (tiles_n + 7) / 8 * tiles_m : (tiles_m * tiles_n + 7) / 8;  // workgroups of an XCD
+  hipLaunchKernelGGL(kern, dim3(8 * (unsigned)each), dim3(64 * WAVES), LDS, s, p, tiles_m, tiles_n);
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }
