@@ -389,9 +389,12 @@ double i8_wide_us(int tile, size_t m, size_t n, size_t ksteps, int mode, size_t 
   // 56.8 and 52.5, 59.3 and 52.4, 3058 x 5248 x 3648 88.8 and 101, 91.7 and 99.8.
   const double k = (double)ksteps, requant = !big ? 0.0 : mode == 1 ? 2.5 : mode == 2 ? 4.8 : mode == 4 ? 6.2 : 0.0;
   const double full = big ? 1.0 + 0.43 * k + requant : 0.6 + 0.155 * k, fast = big ? 0.30 * k + requant : 0.145 * k;
+  // The small tile's last requantisation, and a single k-step, for which the line is too low.  With a K of 64 and 128 either is what decides against
+  // i8_ksplit.hip: 509 x 880 x 64 to bytes 5.0 us and 4.2, as carriers 5.8 and 5.0, sums 4.4 and 4.1, 332 x 1200 x 128 to bytes 4.9 and 4.3.
+  const double ends = big ? 6.0 : 4.1 + (mode == 1 || mode == 2 || mode == 4 ? 0.3 : 0.0) + (ksteps == 1 ? 0.2 : 0.0);
   const size_t tiles = ceil_div(m, (size_t)(big ? 128 : 64)) * ceil_div(n, (size_t)(big ? 256 : 128)), rest = tiles % cus;
   const double part = full * (double)rest / (double)cus;
-  return (big ? 6.0 : 4.0) + (double)(tiles / cus) * full + (rest == 0 ? 0.0 : (part > fast ? part : fast));
+  return ends + (double)(tiles / cus) * full + (rest == 0 ? 0.0 : (part > fast ? part : fast));
 }
 
 int32_t launch_i8_gemm_wide(const I8Args &p, int tile, hipStream_t s) {
