@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(256) embed_norm_kernel(const int32_t *__restri
 
 // ---- RMSNorm: f32 residual -> fp16 normalised activations -----------------------------------------
 // A row of up to KEEP x 1024 values and gamma wait in registers: one memory round trip; KEEP 0: longer rows are read twice
-template <int KEEP>
+template <int KEEP, bool GAIN>
 __global__ void __launch_bounds__(256) rmsnorm_kernel(const float *__restrict__ h, const float *__restrict__ gamma,
                                                       int d, float eps, _Float16 *__restrict__ out) {
   __shared__ float red[4];
@@ -120,7 +120,7 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(const float *__restrict__ 
   float4_t keep[REGS], gain[REGS];
   float ss = 0.0f;
   if constexpr (KEEP > 0) {
-    norm_load<KEEP>(row, gamma, d, keep, gain);
+    norm_load<KEEP, GAIN>(row, gamma, d, keep, gain);
 #pragma unroll
     for (int u = 0; u < KEEP; u++) {
       const float4_t v = keep[u];
@@ -147,7 +147,7 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(const float *__restrict__ 
 #pragma unroll
     for (int u = 0; u < KEEP; u++) {
       const int i = (u * 256 + (int)threadIdx.x) * 4;
-      if (i < d) put(i, keep[u], gain[u]);
+      if (i < d) put(i, keep[u], GAIN ? gain[u] : *reinterpret_cast<const float4_t *>(gamma + i));
     }
   } else {
     for (int i = threadIdx.x * 4; i < d; i += 256 * 4)
@@ -1295,11 +1295,11 @@ int32_t launch_embed_norm(const int32_t *tokens, const _Float16 *table, int batc
 
 int32_t launch_rmsnorm(const float *h, const float *gamma, int batch, int d, float eps, _Float16 *out,
                        hipStream_t s) {
-  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(batch), dim3(256), 0, s, h, gamma, d, eps, out); };
-  if (d <= 1024) go(rmsnorm_kernel<1>);
-  else if (d <= 4096) go(rmsnorm_kernel<4>);
-  else if (d <= 8192) go(rmsnorm_kernel<8>);
-  else go(rmsnorm_kernel<0>);
+  const Context *ctx = nullptr;
+  YSCV_TRY(ensure_context(&ctx));
+  norm_keep((size_t)d, (size_t)batch, (size_t)ctx->num_cus, [&](auto keep, auto gain) {
+    hipLaunchKernelGGL((rmsnorm_kernel<decltype(keep)::value, decltype(gain)::value>), dim3(batch), dim3(256), 0, s, h, gamma, d, eps, out);
+  });
   YSCV_HIP_TRY(hipGetLastError());
   return YSCV_HIP_OK;
 }

@@ -1036,11 +1036,11 @@ int32_t gqa_flat_launch(FlatArgs p, int B, int num_cus, hipStream_t s) {
 }
 
 // ---- RMSNorm over the last axis, f32 in and out ---------------------------------------------------------------
-// Latency- and HBM-bound: the row (KEEP x 1024 values, sixteen bytes per lane and load) and gamma behind it are asked for at once and wait
-// in registers, so that one memory round trip is all there is between launch and stores (each load of the row was waited for inside its
+// Latency- and HBM-bound: the row (KEEP x 1024 values, sixteen bytes per lane and load) and, with GAIN, gamma behind it are asked for at once
+// and wait in registers, so that one memory round trip is all there is between launch and stores (each load of the row was waited for inside its
 // test, and gamma behind the sum).  us: 512 x 8192 6.3 -> 5.7, 4096 x 1024 6.3 -> 5.1, 2048 x 4096 10.7 -> 10.3, 512 x 4096 with the
 // attention behind it 19.5 -> 19.1.  KEEP 0: longer, odd or unaligned rows, read twice.
-template <int KEEP>
+template <int KEEP, bool GAIN>
 __global__ void __launch_bounds__(256) rms_norm_f32_kernel(const float *__restrict__ x, const float *__restrict__ gamma, int d,
                                                            float eps, float *__restrict__ y) {
   __shared__ float red[4];
@@ -1050,7 +1050,7 @@ __global__ void __launch_bounds__(256) rms_norm_f32_kernel(const float *__restri
   float4_t v[REGS], g[REGS];
   float ss = 0.0f;
   if constexpr (KEEP > 0) {
-    norm_load<KEEP>(row, gamma, d, v, g);
+    norm_load<KEEP, GAIN>(row, gamma, d, v, g);
 #pragma unroll
     for (int j = 0; j < KEEP; j++) ss += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
   } else {
@@ -1066,7 +1066,7 @@ __global__ void __launch_bounds__(256) rms_norm_f32_kernel(const float *__restri
 #pragma unroll
     for (int j = 0; j < KEEP; j++) {
       const int i = (j * 256 + (int)threadIdx.x) * 4;
-      if (i < d) *reinterpret_cast<float4_t *>(out + i) = v[j] * inv_rms * g[j];
+      if (i < d) *reinterpret_cast<float4_t *>(out + i) = v[j] * inv_rms * (GAIN ? g[j] : *reinterpret_cast<const float4_t *>(gamma + i));
     }
   } else {
     for (int i = threadIdx.x; i < d; i += 256) out[i] = row[i] * inv_rms * gamma[i];
@@ -1247,20 +1247,20 @@ int32_t launch_gqa_cache(const _Float16 *qkv, const _Float16 *kc, const _Float16
 extern "C" {
 
 int32_t yscv_hip_rms_norm_dev(const float *x, const float *gamma, size_t rows, size_t d, float eps, float *y, void *stream) {
-  YSCV_TRY(ensure_context(nullptr));
+  const Context *ctx = nullptr;
+  YSCV_TRY(ensure_context(&ctx));
   YSCV_REQUIRE(x && gamma && y, "null argument");
   YSCV_REQUIRE(std::isfinite(eps) && eps > 0.0f, "rms_norm: epsilon must be finite and > 0");
   YSCV_REQUIRE(d > 0 && d < ((size_t)1 << 31) && rows < ((size_t)1 << 31), "rms_norm: bad shape %zu x %zu", rows, d);
   const size_t step = (size_t)1 << 23;  // a grid holds less than 2^32 threads
   const bool vec = d % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(gamma)) & 15) == 0;
   for (size_t r0 = 0; r0 < rows; r0 += step) {
-    auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(step, rows - r0)), dim3(256), 0, as_stream(stream), x + r0 * d, gamma, (int)d, eps, y + r0 * d);
+    auto go = [&](auto keep, auto gain) {
+      hipLaunchKernelGGL((rms_norm_f32_kernel<decltype(keep)::value, decltype(gain)::value>), dim3((unsigned)std::min(step, rows - r0)), dim3(256), 0,
+                         as_stream(stream), x + r0 * d, gamma, (int)d, eps, y + r0 * d);
     };
-    if (!vec || d > 8192) go(rms_norm_f32_kernel<0>);
-    else if (d <= 1024) go(rms_norm_f32_kernel<1>);
-    else if (d <= 4096) go(rms_norm_f32_kernel<4>);
-    else go(rms_norm_f32_kernel<8>);
+    if (vec) norm_keep(d, rows, (size_t)ctx->num_cus, go);
+    else go(std::integral_constant<int, 0>{}, std::false_type{});
     YSCV_HIP_TRY(hipGetLastError());
   }
   return YSCV_HIP_OK;

@@ -23,6 +23,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/yscv_hip.h"
 #include "kernels.hpp"
 
@@ -276,16 +278,37 @@ __device__ __forceinline__ float max_xor16_xor32(float v) {  // max(v, v[lane ^ 
 }
 __device__ __forceinline__ float wave_max(float v) { return max_xor16_xor32(row_max16(v)); }
 
+// f(KEEP, GAIN) for the kernels that call norm_load.  KEEP: as many loads as a row of d values has, 0 for a row that does not wait in registers
+// (requests that only repeat the row's end take their time too: 3484 x 1280 in f32 6.0 us with two loads, 7.1 with four).  GAIN: gamma is
+// asked for with the row, one memory round trip less (512 x 8192, the kernel: 6.3 us and 6.8 behind the sum).  From five loads of each on that keeps
+// the CU's memory pipeline busy and up to 86 registers, so with more than four rows to a CU gamma comes behind the sum: 2048 x 5120
+// 13.2 us with it in front and 12.8, 1200 x 7168 11.6 and 11.1, 2048 x 6144 15.1 and 14.8.
+template <int KEEP = 1, typename F>
+void norm_keep(size_t d, size_t rows, size_t cus, F f) {
+  if constexpr (KEEP > 8) {
+    f(std::integral_constant<int, 0>{}, std::false_type{});
+  } else if (d > (size_t)KEEP * 1024) {
+    norm_keep<KEEP + 1>(d, rows, cus, f);
+  } else {
+    if constexpr (KEEP > 4) {
+      if (rows > 4 * cus) return f(std::integral_constant<int, KEEP>{}, std::false_type{});
+    }
+    f(std::integral_constant<int, KEEP>{}, std::true_type{});
+  }
+}
+
 // A row of up to KEEP x 1024 values (d % 4 == 0) and its norm's gamma into the registers of 256 threads, v zero past the end.  The row comes
 // first: loads return in order, and the sum of squares needs nothing else.  Requests past the end repeat the last four values: behind a
 // test each load would be waited for inside it, one memory round trip after the other.
-template <int KEEP>
+template <int KEEP, bool GAIN>
 __device__ __forceinline__ void norm_load(const float *__restrict__ row, const float *__restrict__ gamma, int d, float4_t (&v)[KEEP], float4_t (&g)[KEEP]) {
   const int i = (int)threadIdx.x * 4;
 #pragma unroll
   for (int j = 0; j < KEEP; j++) v[j] = *reinterpret_cast<const float4_t *>(row + min(i + j * 1024, d - 4));
+  if constexpr (GAIN) {
 #pragma unroll
-  for (int j = 0; j < KEEP; j++) g[j] = *reinterpret_cast<const float4_t *>(gamma + min(i + j * 1024, d - 4));
+    for (int j = 0; j < KEEP; j++) g[j] = *reinterpret_cast<const float4_t *>(gamma + min(i + j * 1024, d - 4));
+  }
 #pragma unroll
   for (int j = 0; j < KEEP; j++) {
     if (i + j * 1024 >= d) v[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
