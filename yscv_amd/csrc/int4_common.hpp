@@ -282,7 +282,8 @@ __device__ __forceinline__ float wave_max(float v) { return max_xor16_xor32(row_
 // (requests that only repeat the row's end take their time too: 3484 x 1280 in f32 6.0 us with two loads, 7.1 with four).  GAIN: gamma is
 // asked for with the row, one memory round trip less (512 x 8192, the kernel: 6.3 us and 6.8 behind the sum).  From five loads of each on that keeps
 // the CU's memory pipeline busy and up to 86 registers, so with more than four rows to a CU gamma comes behind the sum: 2048 x 5120
-// 13.2 us with it in front and 12.8, 1200 x 7168 11.6 and 11.1, 2048 x 6144 15.1 and 14.8.
+// 13.2 us with it in front and 12.8, 1200 x 7168 11.6 and 11.1, 2048 x 6144 15.1 and 14.8.  Rows and results that the 256 MB cache in front of HBM does
+// not hold gain from every load in flight again: 8192 x 5120 56.8 us with it in front and 60.7, 8192 x 8192 91.8 and 94.8.
 template <int KEEP = 1, typename F>
 void norm_keep(size_t d, size_t rows, size_t cus, F f) {
   if constexpr (KEEP > 8) {
@@ -291,7 +292,7 @@ void norm_keep(size_t d, size_t rows, size_t cus, F f) {
     norm_keep<KEEP + 1>(d, rows, cus, f);
   } else {
     if constexpr (KEEP > 4) {
-      if (rows > 4 * cus) return f(std::integral_constant<int, KEEP>{}, std::false_type{});
+      if (rows > 4 * cus && rows * d <= ((size_t)256 << 20) / 8) return f(std::integral_constant<int, KEEP>{}, std::false_type{});
     }
     f(std::integral_constant<int, KEEP>{}, std::true_type{});
   }
