@@ -399,7 +399,7 @@ def extra_kernels(torch, stream_ptr):
                                             "operand_KB_per_CU": round((64 + 128) * k / 1024.0, 0),
                                             "operand_fill_GB/s_per_CU_whole_kernel": round((64 + 128) * k / t / 1e9, 1),
                                             "note": "compare with extra.measured_peaks.lds_direct_fill_from_L2_GB/s_per_CU: the tiling "
-                                                    "that fills 256 CUs with 512 x 4096 outputs is bound by the L2 -> LDS path"}
+                                                    "that fills 256 CUs with 512 x 4096 outputs is bound by what an L2 hands its CUs and by the ends of the kernel"}
     del pb
     # config 3: int4 prefill M2048 K4096 N14336 g128, zero points 6..10, bf16
     m, k, n, g = 2048, 4096, 14336, 128

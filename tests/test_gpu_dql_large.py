@@ -1,5 +1,5 @@
 """DynamicQuantizeLinear of several blocks: more block ranges than a workgroup has threads, one load per thread and several, values
-behind the loads that go out ahead, NaN and infinite values: scale, zero point and every value as the definition gives them in f32."""
+behind the loads that go out ahead, NaN among them: scale, zero point and every value as the definition gives them in f32."""
 import numpy as np
 import pytest
 

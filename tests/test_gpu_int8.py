@@ -83,8 +83,8 @@ def test_config2_full_size_bit_exact(oracle, K, torch_cuda):
     assert q.dtype == np.int8 and np.array_equal(q.astype(np.int32), q_exp)
 
 
-# k a multiple of 64: the LDS-ring kernel.  Row / column tails, column counts that are not multiples of 4 or 16,
-# several ring revolutions, and sizes on both sides of the 64x128 / 128x128 tile switch (256 big tiles).
+# k a multiple of 64.  Row / column tails, column counts that are not multiples of 4 or 16, k of one stage and of many, and sizes that go to
+# the kernel whose waves split K and to either of the larger tiles.
 RING_SHAPES = [(1, 64, 1), (65, 256, 129), (70, 2048, 250), (130, 1024, 260), (257, 4096, 515), (33, 192, 1030),
                (2048, 512, 2048), (2100, 320, 2050), (1999, 1088, 2500)]
 

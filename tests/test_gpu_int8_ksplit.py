@@ -11,7 +11,7 @@ SHAPES = [
     (1, 64, 16), (1, 1, 1), (1, 63, 17), (2, 65, 15), (15, 127, 33), (16, 128, 4096), (17, 129, 300), (1, 8192, 257), (16, 4160, 4097),
     (33, 192, 2050), (31, 1088, 4111), (32, 1023, 8190), (63, 4096, 4096), (65, 1000, 2000), (64, 8191, 65), (127, 320, 4095),
     (129, 1024, 4100), (197, 768, 3072), (197, 3072, 768), (256, 704, 4096), (511, 1216, 301), (1025, 768, 770), (2048, 257, 510),
-    (4097, 64, 33), (600, 321, 4099), (1500, 4097, 1900),  # the last two: the ring kernel with copied rows
+    (4097, 64, 33), (600, 321, 4099), (1500, 4097, 1900),  # the last two: larger tiles on copied rows
 ]
 
 

@@ -1,11 +1,13 @@
 """int8 GEMM in tiles of 64 x 128 and 128 x 256: whole numbers, so every value has to be the exact one.  K around the pairs of k-steps of 64,
-the stages of four of them and the two or three stages in flight; rows and columns off the tiles; all forms of the result."""
+the stages of four of them and the two or three stages in flight; rows and columns off the tiles; sums and bytes (the operators' forms of the
+result: test_gpu_int8_forms.py)."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
-# more 64 x 64 tiles than any CU count: rows x columns that take the small and (two rounds of it) the large of the two tiles
+# more 64 x 64 tiles than any CU count: rows x columns that take the small tile for few k-steps and the large one for many (sums from eight and two
+# on, bytes from 24 and more on)
 SMALL, LARGE = (1025, 4097), (2113, 8201)
 KSTEPS = [2, 3, 4, 5, 6, 7, 8, 9, 11, 12, 13, 16, 17, 24]
 

@@ -4,11 +4,11 @@
 //
 // Four waves stand side by side in columns and each takes ALL rows of the tile, so nobody but one wave needs a block of B: B goes from
 // memory to the registers of that wave (it is packed as the MFMA takes it) and only A passes through LDS.  (Waves 2 x 2 with both operands
-// in LDS, four more waves to load them: 24 KB read and 12 KB written per 64 k of a 64 x 128 tile, which is what bound that kernel, not the
-// fill of the CU: an XCD's L2 gives a CU 115 GB/s, that loop took 65.)
+// in LDS, four more waves to load them: 12 KB written to LDS and 24 KB read per 64 k of a 64 x 128 tile took 184 ns.)
 //   64 x 128:  eight waves, two rows of four that take alternate pairs of k-steps; their sums meet in LDS at the end.  One wave per SIMD
-//              is bound by the instructions it can issue (70 in a k-step, five cycles each), two fill each other's gaps.  Bound by what L2
-//              delivers (79 GB/s per CU with all of them at it).
+//              is bound by the instructions it can issue (70 in a k-step, five cycles each), two fill each other's gaps.  A k-step takes
+//              in its 12 KB in 128 ns (512 rows, N 4096, K 1024 8.3 us, 4096 14.4): 96 GB/s per CU with all of them at it, where loads
+//              to LDS alone reach 70 .. 76 (yscv_hip_measure_fill).  The other 6.2 us are launch, first operands and what the end takes.
 //   128 x 256: four waves, the accumulators in the other half of the register file.  Half the bytes per MFMA; bound by issue: a SIMD takes
 //              an instruction every four cycles and an MFMA every sixteen, two more fit behind each.  So the loop is laid out by hand as in
 //              int4_gemm_wide.hip: MFMAs are statements in their order, fragments of A are read a k-step ahead and made signed two row
